@@ -30,7 +30,8 @@ typedef enum {
 /* hb_run flags */
 #define HB_FLAG_DENSE 0x1u    /* recompute every node every iteration (the reference's
                                  schedule); default skips nodes none of whose
-                                 neighbours changed, with identical results      */
+                                 neighbours changed and nodes whose sketch cannot
+                                 change any more, with identical results         */
 #define HB_FLAG_GRAPH 0x2u    /* capture one iteration in a hipGraph and replay it   */
 #define HB_FLAG_NF    0x4u    /* record the neighbourhood function N(t) each iteration */
 #define HB_FLAG_TIMING 0x8u   /* per-iteration device timing with events (read at the

@@ -180,8 +180,12 @@ struct hb_ctx {
     DevBuf<float> est, est_tmp, lc;
     DevBuf<double> dist, inv, cent;
     DevBuf<HbBiasTable> bias;
-    DevBuf<uint32_t> bits0, bits1, sched_buf, chunk_flag;
-    DevBuf<uint32_t> active, dyn;  // push iterations: bitmap; per-bin lists + 3 counts
+    DevBuf<uint32_t> sched_buf, chunk_flag;
+    // per-node bitmaps of a run, cleared together: changed nodes (2), then active nodes of
+    // push iterations (2) and saturated nodes (2) where they are used, then the bound of
+    // all sketches (2^p)
+    DevBuf<uint32_t> bits;
+    DevBuf<uint32_t> dyn;  // push iterations: per-bin lists + 3 counts
     bool sym = false;              // staged CSR is symmetric (arc multiset fingerprints)
     DevBuf<HbIterState> st;
     DevBuf<HbIterRec> rec;
@@ -243,11 +247,9 @@ struct hb_ctx {
         inv.release();
         bias.release();
         cent.release();
-        bits0.release();
-        bits1.release();
+        bits.release();
         sched_buf.release();
         chunk_flag.release();
-        active.release();
         dyn.release();
         st.release();
         rec.release();
@@ -723,8 +725,6 @@ extern "C" int hb_run(hb_ctx *c, int p, int max_iters, uint32_t flags, hb_stats 
     HB_TRY(c->est.ensure(c->n));
     HB_TRY(c->dist.ensure(c->n));
     HB_TRY(c->inv.ensure(c->n));
-    HB_TRY(c->bits0.ensure(words));
-    HB_TRY(c->bits1.ensure(words));
     HB_TRY(c->st.ensure(1));
     // No iteration cap: a run ends by the reference's rule or at max_iters.  A graph
     // cannot change a register after its diameter, so n + 2 iterations bound a correct
@@ -735,7 +735,6 @@ extern "C" int hb_run(hb_ctx *c, int p, int max_iters, uint32_t flags, hb_stats 
     HB_TRY(c->bias.ensure(1));
     if (c->snap_k) HB_TRY(c->snaps.ensure((size_t)c->snap_k * c->n));
     const bool push_ok = c->sym && p <= 10;
-    if (push_ok) HB_TRY(c->active.ensure(2 * (size_t)words));  // two, by iteration parity
     {
         int rc = ensure_layout(c);  // normally built at staging already
         default_schedule(c, p);
@@ -750,6 +749,15 @@ extern "C" int hb_run(hb_ctx *c, int p, int max_iters, uint32_t flags, hb_stats 
     HB_TRY(hipMemcpyAsync(c->bias.ptr, hb::bias_table(p), sizeof(HbBiasTable), hipMemcpyHostToDevice,
                           c->stream));
 
+    // Saturation pays where most nodes come to hold the same sketch within a few iterations,
+    // which the chain layout's graphs do not; its kernels and the dense schedule, which
+    // recomputes every node in every iteration, go without.
+    const bool chain = c->relabelled() && c->layout_used == HB_LAYOUT_CHAIN;
+    const bool sat_ok = p <= 10 && !(flags & HB_FLAG_DENSE) && !chain;
+    // rounded up so that the bound after the bitmaps is aligned for 16-byte loads
+    const size_t bit_words = ((2 + (push_ok ? 2 : 0) + (sat_ok ? 2 : 0)) * (size_t)words + 3) & ~(size_t)3;
+    HB_TRY(c->bits.ensure(bit_words + (sat_ok ? m : 0)));
+
     HbDev &d = c->dev;
     d = HbDev{};
     d.off = c->run_off();
@@ -761,8 +769,12 @@ extern "C" int hb_run(hb_ctx *c, int p, int max_iters, uint32_t flags, hb_stats 
     d.est = c->est.ptr;
     d.dist = c->dist.ptr;
     d.inv = c->inv.ptr;
-    d.bits0 = c->bits0.ptr;
-    d.bits1 = c->bits1.ptr;
+    d.bits0 = c->bits.ptr;
+    d.bits1 = d.bits0 + words;
+    if (sat_ok) {
+        d.sat_bits = d.bits1 + words + (push_ok ? 2 * words : 0);
+        d.sat_max = c->bits.ptr + bit_words;
+    }
     d.st = c->st.ptr;
     d.rec = c->rec.ptr;
     d.lc = c->lc.ptr;
@@ -775,7 +787,7 @@ extern "C" int hb_run(hb_ctx *c, int p, int max_iters, uint32_t flags, hb_stats 
     d.mid_max = c->mid_max;
     d.wave_max = c->wave_max;
     if (push_ok) {
-        d.active = c->active.ptr;
+        d.active = d.bits1 + words;
         d.dyn_list = c->dyn.ptr + 3;
         d.dyn_count = c->dyn.ptr;
         d.dyn_base[0] = 0;
@@ -792,7 +804,7 @@ extern "C" int hb_run(hb_ctx *c, int p, int max_iters, uint32_t flags, hb_stats 
     d.five_m = 5.0f * (float)m;
     d.lc_thr = kLcThreshold[p];
     d.frontier = (flags & HB_FLAG_DENSE) ? 0 : 1;
-    d.window = c->relabelled() && c->layout_used == HB_LAYOUT_CHAIN ? 1 : 0;
+    d.window = chain ? 1 : 0;
     d.rows = d.window && (p == 5 || p == 6) ? 1 : 0;
 
     HbIterState st0{};
@@ -801,10 +813,8 @@ extern "C" int hb_run(hb_ctx *c, int p, int max_iters, uint32_t flags, hb_stats 
     st0.t = 1.0;
     st0.inv_t = 1.0;
     HB_TRY(hipMemcpyAsync(c->st.ptr, &st0, sizeof st0, hipMemcpyHostToDevice, c->stream));
-    HB_TRY(hb::launch_fill(c->bits0.ptr, words, 0u, c->stream));
-    HB_TRY(hb::launch_fill(c->bits1.ptr, words, 0u, c->stream));
     // iteration t marks the active bitmap iteration t - 1 cleared; both start clear
-    if (push_ok) HB_TRY(hb::launch_fill(c->active.ptr, 2 * (uint64_t)words, 0u, c->stream));
+    HB_TRY(hb::launch_fill(c->bits.ptr, bit_words + (sat_ok ? m : 0), 0u, c->stream));
 
     hipEvent_t e0, e1, e2;
     HB_TRY(hipEventCreate(&e0));
@@ -844,7 +854,7 @@ extern "C" int hb_run(hb_ctx *c, int p, int max_iters, uint32_t flags, hb_stats 
                 rc = fail(HB_EHIP, "hipStreamBeginCapture failed");
                 break;
             }
-            e = hb::launch_iteration(d, c->sched, nf, c->stream);
+            e = hb::launch_iteration(d, c->sched, false, nf, c->stream);
             hipError_t e2c = hipStreamEndCapture(c->stream, &graph);
             if (e != hipSuccess || e2c != hipSuccess) {
                 rc = fail(HB_EHIP, "graph capture failed: %s", hipGetErrorString(e != hipSuccess ? e : e2c));
@@ -872,8 +882,9 @@ extern "C" int hb_run(hb_ctx *c, int p, int max_iters, uint32_t flags, hb_stats 
             for (uint32_t i = 0; i < k && rc == HB_OK; ++i) {
                 hipEvent_t *ev = timing ? &tev[(size_t)i * per_it] : nullptr;
                 if (ev) (void)hipEventRecord(ev[0], c->stream);
-                e = gexec ? hipGraphLaunch(gexec, c->stream)
-                          : hb::launch_iteration(d, c->sched, nf, c->stream, ktiming ? ev + 2 : nullptr);
+                const bool first = launched + i == 0;  // not part of the captured iteration
+                e = gexec && !first ? hipGraphLaunch(gexec, c->stream)
+                                    : hb::launch_iteration(d, c->sched, first, nf, c->stream, ktiming ? ev + 2 : nullptr);
                 if (e != hipSuccess) rc = fail(HB_EHIP, "iteration launch: %s", hipGetErrorString(e));
                 if (ev) (void)hipEventRecord(ev[1], c->stream);
             }

@@ -38,6 +38,7 @@
 #include <cstring>
 #include <memory>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/sparkx_hb.h"
@@ -61,6 +62,7 @@ static constexpr int kQueues = kBatchNP * kClasses;
 
 struct HbBatchRec {  // counters of one iteration of one graph
     unsigned long long inc, chg, arcs, nodes, gathered;
+    unsigned long long sat;  // degrees of the nodes that became saturated
 };
 
 struct HbBatchGraph {
@@ -69,7 +71,7 @@ struct HbBatchGraph {
     uint32_t ring_base;   // first of the graph's kRing records
     uint32_t cap;         // iterations after which a running graph is an error (n + 2)
     uint32_t overflow;    // set when the graph reached cap without stopping
-    uint32_t pad;
+    uint32_t sym;         // v -> u for every u -> v
     float am, five_m;
     double lc_thr;
     HbIterState st;
@@ -106,6 +108,12 @@ struct HbBatchDev {
     uint32_t *chunk_flag;       // 1 if the task was recomputed this iteration
     const float *lc;            // LC tables of p = 4..8 back to back (lc_off)
     const HbBiasTable *bias;    // bias windows of p = 4..8
+    // saturation, as in HbDev (null: off): every graph's bound of all sketches, a u32 per
+    // register (k_init) and packed as registers are (k_batch_bound), kScrRow entries per
+    // graph; the saturated nodes by iteration parity
+    const uint32_t *sat_max;
+    uint8_t *bound;
+    uint32_t *sat0, *sat1;
     int frontier;
 };
 
@@ -146,7 +154,8 @@ __device__ __forceinline__ HbBatchRec *ring_rec(const HbBatchDev &b, const HbBat
 }
 
 // the iteration's view of graph g (as the single-graph kernels build it)
-__device__ __forceinline__ HbView batch_view(const HbBatchDev &b, const HbBatchGraph &g, uint32_t *s_first)
+__device__ __forceinline__ HbView batch_view(const HbBatchDev &b, const HbBatchGraph &g, uint32_t gi,
+                                             uint32_t *s_first)
 {
     const uint32_t it = g.st.iter;
     HbView v;
@@ -165,25 +174,33 @@ __device__ __forceinline__ HbView batch_view(const HbBatchDev &b, const HbBatchG
     v.inv_t = g.st.inv_t;
     v.use_frontier = b.frontier && it > 1 && !g.st.skip_scan;
     v.gather_bits = v.use_frontier ? v.bitsR : nullptr;
-    v.first = it == 1;       // p <= 8: iteration 1 hashes neighbour ids instead of gathering
     v.scr = s_first;
+    v.sym = g.sym != 0;
+    if (b.sat_max) {
+        v.satR = ((it & 1u) ? b.sat0 : b.sat1) + g.bits_base;
+        v.satW = ((it & 1u) ? b.sat1 : b.sat0) + g.bits_base;
+        v.bound = (const uint4 *)(b.bound + (uint64_t)gi * kScrRow);
+        v.sat_scan = g.st.sat_scan != 0;
+    }
     return v;
 }
 
-template <int P, int T>
+template <int P, int T, bool kFirst>
 __device__ __forceinline__ void batch_nodes(const HbView &v, const HbTables &tb, const uint32_t *list,
                                             uint32_t count, HbCounts &c)
 {
     const uint32_t lane = threadIdx.x & (HB_WAVE - 1);
-    if (v.gather_bits) {
-        for (uint32_t i = lane / T; i < count; i += HB_WAVE / T) union_node<P, T, true>(v, tb, list[i], lane % T, c);
-    } else {
-        for (uint32_t i = lane / T; i < count; i += HB_WAVE / T) union_node<P, T, false>(v, tb, list[i], lane % T, c);
-    }
+    auto run = [&](auto gather) {
+        for (uint32_t i = lane / T; i < count; i += HB_WAVE / T)
+            union_node<P, T, decltype(gather)::value>(v, tb, list[i], lane % T, c);
+    };
+    if constexpr (kFirst) run(std::integral_constant<Gather, Gather::kFirst>{});
+    else if (v.gather_bits) run(std::integral_constant<Gather, Gather::kChanged>{});
+    else run(std::integral_constant<Gather, Gather::kAll>{});
 }
 
 // one hub chunk: partial union of its neighbours into scratch (as k_chunk)
-template <int P>
+template <int P, bool kFirst>
 __device__ __forceinline__ void batch_chunk(const HbBatchDev &b, const HbView &v, uint32_t task_id,
                                             const HbBatchTask &task, HbCounts &c)
 {
@@ -193,7 +210,17 @@ __device__ __forceinline__ void batch_chunk(const HbBatchDev &b, const HbView &v
     const uint32_t *__restrict__ nbh = v.orig + task.beg;  // caller's ids, hashed in iteration 1
     const uint32_t len = task.end - task.beg;
     bool active = true;
-    if (v.use_frontier) {
+    if (!kFirst && v.satR) {
+        active = !bit_test(v.satR, task.node);
+        uint32_t scanned = 0;
+        if (active && v.sat_scan && sat_neighbour<T>(v.satR, nb, len, tl, scanned)) {
+            if (tl == 0) b.chunk_flag[task_id] = 1u;
+            if (slot == 0) *(uint4 *)(b.scratch + (uint64_t)task_id * kScrRow + cl * 16) = v.bound[cl];
+            if (tl == 0) c.arcs += scanned;
+            return;
+        }
+    }
+    if (v.use_frontier && active) {
         uint32_t any = 0;
         for (uint32_t j = tl; j < len; j += T) any |= bit_test(v.bitsR, nb[j]);
         active = hb_copy_or<T>(any) != 0;
@@ -201,11 +228,14 @@ __device__ __forceinline__ void batch_chunk(const HbBatchDev &b, const HbView &v
     if (tl == 0) b.chunk_flag[task_id] = active ? 1u : 0u;
     if (!active) return;
     uint32_t gathered = 0;
-    uint4 acc = v.use_frontier
-                    ? hb_gather_union<P, S, true>(v.in, v.first, v.scr, v.bitsR, nb, nbh, len, slot, cl,
-                                                  make_uint4(0, 0, 0, 0), gathered)
-                    : hb_gather_union<P, S, false>(v.in, v.first, v.scr, nullptr, nb, nbh, len, slot, cl,
-                                                   make_uint4(0, 0, 0, 0), gathered);
+    const uint4 none = make_uint4(0, 0, 0, 0);
+    uint4 acc;
+    if constexpr (kFirst)
+        acc = hb_gather_union<P, S, Gather::kFirst>(v.in, v.scr, nullptr, nb, nbh, len, slot, cl, none, gathered);
+    else
+        acc = v.use_frontier
+                  ? hb_gather_union<P, S, Gather::kChanged>(v.in, nullptr, v.bitsR, nb, nbh, len, slot, cl, none, gathered)
+                  : hb_gather_union<P, S, Gather::kAll>(v.in, nullptr, nullptr, nb, nbh, len, slot, cl, none, gathered);
     if (cl == 0) c.gathered += gathered;
 #pragma unroll
     for (uint32_t s = G; s < T; s <<= 1) acc = hb_bmax4(acc, hb_shfl_xor4<T>(acc, s));
@@ -233,6 +263,7 @@ __device__ __forceinline__ void wave_sum_counts(HbCounts &c)
         c.arcs += __shfl_xor(c.arcs, s);
         c.nodes += __shfl_xor(c.nodes, s);
         c.gathered += __shfl_xor(c.gathered, s);
+        c.sat += __shfl_xor(c.sat, s);
     }
 }
 
@@ -243,6 +274,7 @@ __device__ __forceinline__ void add_counts(HbBatchRec *r, const HbCounts &c)
     if (c.arcs) atomicAdd(&r->arcs, c.arcs);
     if (c.nodes) atomicAdd(&r->nodes, c.nodes);
     if (c.gathered) atomicAdd(&r->gathered, c.gathered);
+    if (c.sat) atomicAdd(&r->sat, c.sat);
 }
 
 // Global wavefront index and count of the grid (wave-uniform).
@@ -254,42 +286,42 @@ __device__ __forceinline__ uint32_t wave_count() { return gridDim.x * (kBatchBlo
 // Six wavefronts per SIMD from p = 6 up (80 VGPRs: the one-copy bins spill 2-5 where
 // seven spilled 9-19): with the precisions' chains overlapping, the p = 7 chain is the
 // longest, and the 64-graph run takes 14.1 ms against 14.6 ms at seven.
-template <int P, int T>
+template <int P, int T, bool kFirst>
 __global__ __launch_bounds__(kBatchBlock) __attribute__((amdgpu_waves_per_eu(P >= 6 ? 6 : 8))) void k_batch_nodes(
     HbBatchDev b, HbBatchList l)
 {
     const uint32_t count = b.active_count[l.queue];
     if (count == 0) return;  // the whole grid leaves: no graph of this class is running
     HB_BATCH_TABLES(P, b, tbl)
-    __shared__ uint32_t s_first[kBatchBlock * 16];
+    __shared__ uint32_t s_first[kFirst ? kBatchBlock * 16 : 1];
     const uint32_t lane = threadIdx.x & (HB_WAVE - 1);
     for (uint32_t w = wave_id(); w < count; w += wave_count()) {
         const HbBatchTile tile = wave_uniform(l.tiles[b.active[l.base + w]]);
         const HbBatchGraph g = wave_uniform(b.g[tile.graph]);
         const HbTables tb = {tbl_lc, &tbl_bias, g.am, g.five_m, g.lc_thr};
-        const HbView v = batch_view(b, g, s_first);
+        const HbView v = batch_view(b, g, tile.graph, s_first);
         HbCounts c;
-        batch_nodes<P, T>(v, tb, b.lists + tile.first, tile.count, c);
+        batch_nodes<P, T, kFirst>(v, tb, b.lists + tile.first, tile.count, c);
         wave_sum_counts(c);
         if (lane == 0) add_counts(ring_rec(b, g, g.st.iter), c);
     }
 }
 
 // Partial unions of the active hub chunks of precision P, one wavefront per chunk.
-template <int P>
+template <int P, bool kFirst>
 __global__ __launch_bounds__(kBatchBlock) __attribute__((amdgpu_waves_per_eu(P >= 7 ? 7 : 8))) void k_batch_chunk(
     HbBatchDev b, HbBatchList l)
 {
     const uint32_t count = b.active_count[l.queue];
     if (count == 0) return;
-    __shared__ uint32_t s_first[kBatchBlock * 16];
+    __shared__ uint32_t s_first[kFirst ? kBatchBlock * 16 : 1];
     const uint32_t lane = threadIdx.x & (HB_WAVE - 1);
     for (uint32_t w = wave_id(); w < count; w += wave_count()) {
         const HbBatchTile tile = wave_uniform(l.tiles[b.active[l.base + w]]);
         const HbBatchGraph g = wave_uniform(b.g[tile.graph]);
-        const HbView v = batch_view(b, g, s_first);
+        const HbView v = batch_view(b, g, tile.graph, s_first);
         HbCounts c;
-        batch_chunk<P>(b, v, tile.first, wave_uniform(b.tasks[tile.first]), c);
+        batch_chunk<P, kFirst>(b, v, tile.first, wave_uniform(b.tasks[tile.first]), c);
         wave_sum_counts(c);
         if (lane == 0) add_counts(ring_rec(b, g, g.st.iter), c);
     }
@@ -339,7 +371,7 @@ __global__ __launch_bounds__(kBatchBlock) void k_batch_merge(HbBatchDev b, HbBat
         const HbBatchGraph g = wave_uniform(b.g[hub.graph]);
         if (g.st.done) continue;
         const HbTables tb = {tbl_lc, &tbl_bias, g.am, g.five_m, g.lc_thr};
-        const HbView v = batch_view(b, g, nullptr);
+        const HbView v = batch_view(b, g, hub.graph, nullptr);
         const uint32_t u = hub.node;
         HbCounts c;
         uint32_t any = 0;
@@ -350,16 +382,21 @@ __global__ __launch_bounds__(kBatchBlock) void k_batch_merge(HbBatchDev b, HbBat
                 *(uint4 *)(v.out + ((uint64_t)u << P) + cl * 16) = *(const uint4 *)(v.in + ((uint64_t)u << P) + cl * 16);
             continue;
         }
-        const uint4 own = v.first ? hb_own_from_word(hb_insertion<P>(v.node_id[u]), cl)
-                                  : *(const uint4 *)(v.in + ((uint64_t)u << P) + cl * 16);
+        const uint4 own = *(const uint4 *)(v.in + ((uint64_t)u << P) + cl * 16);
         uint4 acc = own;
         for (uint32_t j = slot; j < hub.ntask; j += S)
             if (b.chunk_flag[hub.task0 + j])
                 acc = hb_bmax4(acc, *(const uint4 *)(b.scratch + (uint64_t)(hub.task0 + j) * kScrRow + cl * 16));
 #pragma unroll
         for (uint32_t s = G; s < T; s <<= 1) acc = hb_bmax4(acc, hb_shfl_xor4<T>(acc, s));
-        const uint32_t diffw = (acc.x != own.x) | (acc.y != own.y) | (acc.z != own.z) | (acc.w != own.w);
-        const bool changed = hb_copy_or<G>(diffw) != 0;
+        uint32_t diffw = (acc.x != own.x) | (acc.y != own.y) | (acc.z != own.z) | (acc.w != own.w);
+        const bool sat = v.satR && g.st.iter > 1;
+        if (sat) {
+            const uint4 f = v.bound[cl];
+            diffw |= ((acc.x != f.x) | (acc.y != f.y) | (acc.z != f.z) | (acc.w != f.w)) << 1;
+        }
+        diffw = hb_copy_or<G>(diffw);
+        const bool changed = (diffw & 1u) != 0;
         const float curr = hb_estimate_copy<G>(tb, acc);
         if (slot == 0) *(uint4 *)(v.out + ((uint64_t)u << P) + cl * 16) = acc;
         if (tl == 0) {
@@ -370,6 +407,7 @@ __global__ __launch_bounds__(kBatchBlock) void k_batch_merge(HbBatchDev b, HbBat
                 atomicOr(v.bitsW + (u >> 5), 1u << (u & 31u));
                 c.chg += 1;
             }
+            if (sat && !(diffw & 2u)) sat_mark(v, u, v.nbr + v.off[u], v.off[u + 1] - v.off[u], c);
             c.nodes += 1;
             add_counts(ring_rec(b, g, g.st.iter), c);
         }
@@ -377,16 +415,30 @@ __global__ __launch_bounds__(kBatchBlock) void k_batch_merge(HbBatchDev b, HbBat
 }
 
 // start of an iteration: for every running graph clear the bitmap this iteration
-// writes and its ring record
+// writes and its ring record, and carry the saturated nodes over
 __global__ __launch_bounds__(kBatchBlock) void k_batch_begin(HbBatchDev b)
 {
     for (uint32_t gi = blockIdx.x; gi < b.ngraphs; gi += gridDim.x) {
         const HbBatchGraph &g = b.g[gi];
         if (g.st.done) continue;
         uint32_t *bw = ((g.st.iter & 1u) ? b.bits1 : b.bits0) + g.bits_base;
-        for (uint32_t i = threadIdx.x; i < g.words; i += blockDim.x) bw[i] = 0u;
-        if (threadIdx.x == 0) *ring_rec(b, g, g.st.iter) = HbBatchRec{0, 0, 0, 0, 0};
+        uint32_t *sw = ((g.st.iter & 1u) ? b.sat1 : b.sat0) + g.bits_base;
+        const uint32_t *sr = ((g.st.iter & 1u) ? b.sat0 : b.sat1) + g.bits_base;
+        for (uint32_t i = threadIdx.x; i < g.words; i += blockDim.x) {
+            bw[i] = 0u;
+            if (b.sat_max) sw[i] = sr[i];
+        }
+        if (threadIdx.x == 0) *ring_rec(b, g, g.st.iter) = HbBatchRec{};
     }
+}
+
+// after the register init: every graph's bound, packed as registers are
+__global__ __launch_bounds__(64) void k_batch_bound(HbBatchDev b)
+{
+    const uint32_t gi = blockIdx.x, i = threadIdx.x;
+    if (i >= (1u << b.g[gi].p) / 4) return;
+    const uint32_t *r = b.sat_max + (uint64_t)gi * kScrRow + 4 * i;
+    ((uint32_t *)(b.bound + (uint64_t)gi * kScrRow))[i] = r[0] | (r[1] << 8) | (r[2] << 16) | (r[3] << 24);
 }
 
 // end of an iteration for every running graph (hyper_ball.rs:833-849)
@@ -412,6 +464,8 @@ __global__ void k_batch_finalize(HbBatchDev b)
     st.t = st.t + 1.0;
     st.inv_t = __ddiv_rn(1.0, st.t);
     st.skip_scan = 2 * r.chg > (unsigned long long)g.n_linked;
+    st.sat_arcs += r.sat;  // as k_finalize
+    st.sat_scan = 8 * st.sat_arcs >= (unsigned long long)g.n_linked;
 }
 
 }  // namespace hb
@@ -503,7 +557,13 @@ struct hb_batch {
     uint64_t total_nodes = 0, total_arcs = 0, total_regs = 0, total_words = 0;
     // CSRs in each graph's degree order, the caller's ids (orig per arc, perm per node)
     // and the inverse numbering (sigma: caller's node -> device node)
-    DevArr<uint32_t> off, nbr, orig, perm, sigma, bits0, bits1, lists, chunk_flag;
+    DevArr<uint32_t> off, nbr, orig, perm, sigma, lists, chunk_flag;
+    // cleared at the start of a run: changed nodes and saturated nodes (2 bitmaps of
+    // total_words each), then every graph's bound of all sketches (kScrRow u32)
+    DevArr<uint32_t> bits;
+    DevArr<uint8_t> bound;
+    size_t bits_count() const { return 4 * total_words + hg.size() * hb::kScrRow; }
+    uint32_t *sat_max(size_t gi) const { return bits.ptr + 4 * total_words + gi * hb::kScrRow; }
     DevArr<uint32_t> active, active_count;  // per class: tiles of running graphs
     DevArr<uint8_t> regs0, regs1, scratch, readback;
     DevArr<float> est, lc_all, est_tmp;
@@ -554,6 +614,7 @@ static HbDev graph_dev(hb_batch *b, int gi)
     d.bias = b->bias_all.ptr + (g.p - hb::kBatchPMin);
     d.n = g.n;
     d.n_linked = g.n_linked;
+    d.sym = (int)g.sym;
     d.p = g.p;
     d.am = g.am;
     d.five_m = g.five_m;
@@ -746,8 +807,8 @@ int hb_batch_create(hb_batch **out, int device, const hb_graph_desc *graphs, int
     HB_BTRY(b->est_tmp.alloc(nodes));
     HB_BTRY(b->dist.alloc(nodes));
     HB_BTRY(b->inv.alloc(nodes));
-    HB_BTRY(b->bits0.alloc(words));
-    HB_BTRY(b->bits1.alloc(words));
+    HB_BTRY(b->bits.alloc(b->bits_count()));
+    HB_BTRY(b->bound.alloc((size_t)count * hb::kScrRow));
     HB_BTRY(b->active_count.alloc(hb::kQueues));
     HB_BTRY(b->g.alloc(count));
     HB_BTRY(b->rec.alloc((size_t)count * hb::kRing));
@@ -795,6 +856,23 @@ int hb_batch_create(hb_batch **out, int device, const hb_graph_desc *graphs, int
         }
         std::swap(b->off.ptr, roff.ptr);
         std::swap(b->nbr.ptr, rnbr.ptr);
+    }
+    // symmetric graphs leave the nodes that reach no other sketch out of the bound
+    {
+        constexpr size_t kWork = 4 + 4 * (size_t)hb::kFingerprintBlocks;
+        DevArr<unsigned long long> work, sums;
+        HB_BTRY(work.alloc(kWork));
+        HB_BTRY(sums.alloc(4 * (size_t)count));
+        std::vector<unsigned long long> h(4 * (size_t)count);
+        for (int i = 0; i < count; ++i) {
+            const hb::HbBatchGraph &g = b->hg[i];
+            HB_BTRY(hb::arc_fingerprints(b->off.ptr + g.off_base, b->nbr.ptr + g.nbr_base, g.n, graphs[i].arcs,
+                                         work.ptr, b->stream));
+            HB_BTRY(hipMemcpyAsync(sums.ptr + 4 * i, work.ptr, 32, hipMemcpyDeviceToDevice, b->stream));
+        }
+        HB_BTRY(hipMemcpyAsync(h.data(), sums.ptr, h.size() * 8, hipMemcpyDeviceToHost, b->stream));
+        HB_BTRY(hipStreamSynchronize(b->stream));
+        for (int i = 0; i < count; ++i) b->hg[i].sym = h[4 * i] == h[4 * i + 1] && h[4 * i + 2] == h[4 * i + 3];
     }
     *out = b.release();
     hb::set_error("");
@@ -851,8 +929,12 @@ int hb_batch_run(hb_batch *b, uint32_t flags, hb_batch_stats *stats)
     d.est = b->est.ptr;
     d.dist = b->dist.ptr;
     d.inv = b->inv.ptr;
-    d.bits0 = b->bits0.ptr;
-    d.bits1 = b->bits1.ptr;
+    d.bits0 = b->bits.ptr;
+    d.bits1 = d.bits0 + b->total_words;
+    d.sat0 = d.bits1 + b->total_words;
+    d.sat1 = d.sat0 + b->total_words;
+    d.bound = b->bound.ptr;
+    d.sat_max = (flags & HB_FLAG_DENSE) ? nullptr : b->sat_max(0);
     d.g = b->g.ptr;
     d.ngraphs = (uint32_t)ng;
     d.rec = b->rec.ptr;
@@ -891,7 +973,7 @@ int hb_batch_run(hb_batch *b, uint32_t flags, hb_batch_stats *stats)
     // `running`: bit pi set while a graph of precision kBatchPMin + pi may still run.  A
     // stopped graph never runs again and its kernels would return at once, so leaving
     // out a precision whose graphs have all stopped changes nothing.
-    auto launch_iter = [&](uint32_t running) -> hipError_t {
+    auto launch_iter = [&](uint32_t running, bool first) -> hipError_t {
         hb::k_batch_begin<<<(unsigned)std::min(ng, 1024), hb::kBatchBlock, 0, b->stream>>>(d);
         hb::k_batch_compact<<<hb::kQueues, 1024, 0, b->stream>>>(d, classes);
         hipError_t e = hipEventRecord(b->fork, b->stream);
@@ -909,14 +991,15 @@ int hb_batch_run(hb_batch *b, uint32_t flags, hb_batch_stats *stats)
             load[si] += pwork[order[k]];
         }
 #define HB_BATCH_LAUNCH(q, kernel)                                                                     \
-        if (lists[q].count) kernel<<<b->grid[q], hb::kBatchBlock, 0, s>>>(d, lists[q]);
+        if (lists[q].count) (kernel)<<<b->grid[q], hb::kBatchBlock, 0, s>>>(d, lists[q]);
 #define HB_BATCH_P(P)                                                                                  \
         case P: {                                                                                      \
             constexpr int G_ = (1 << P) / 16, q0 = (P - hb::kBatchPMin) * hb::kClasses;               \
-            HB_BATCH_LAUNCH(q0, (hb::k_batch_nodes<P, G_>))                                            \
-            HB_BATCH_LAUNCH(q0 + 1, (hb::k_batch_nodes<P, (4 * G_ < 64 ? 4 * G_ : 64)>))              \
-            HB_BATCH_LAUNCH(q0 + 2, (hb::k_batch_nodes<P, 64>))                                        \
-            HB_BATCH_LAUNCH(q0 + hb::kClassChunk, hb::k_batch_chunk<P>)                                \
+            constexpr int G4_ = 4 * G_ < 64 ? 4 * G_ : 64;                                             \
+            HB_BATCH_LAUNCH(q0, (first ? hb::k_batch_nodes<P, G_, true> : hb::k_batch_nodes<P, G_, false>))       \
+            HB_BATCH_LAUNCH(q0 + 1, (first ? hb::k_batch_nodes<P, G4_, true> : hb::k_batch_nodes<P, G4_, false>)) \
+            HB_BATCH_LAUNCH(q0 + 2, (first ? hb::k_batch_nodes<P, 64, true> : hb::k_batch_nodes<P, 64, false>))   \
+            HB_BATCH_LAUNCH(q0 + hb::kClassChunk, (first ? hb::k_batch_chunk<P, true> : hb::k_batch_chunk<P, false>)) \
             if (hub_lists[P - hb::kBatchPMin].count)                                                   \
                 hb::k_batch_merge<P><<<(hub_lists[P - hb::kBatchPMin].count + 3) / 4, hb::kBatchBlock, 0, s>>>( \
                     d, hub_lists[P - hb::kBatchPMin]);                                                 \
@@ -945,19 +1028,22 @@ int hb_batch_run(hb_batch *b, uint32_t flags, hb_batch_stats *stats)
     const auto t_start = std::chrono::steady_clock::now();
     do {
         if (hipMemcpyAsync(b->g.ptr, init.data(), ng * sizeof(hb::HbBatchGraph), hipMemcpyHostToDevice, b->stream) != hipSuccess ||
-            hb::launch_fill(b->bits0.ptr, b->total_words, 0u, b->stream) != hipSuccess ||
-            hb::launch_fill(b->bits1.ptr, b->total_words, 0u, b->stream) != hipSuccess ||
+            hb::launch_fill(b->bits.ptr, b->bits_count(), 0u, b->stream) != hipSuccess ||
             hipEventRecord(e0, b->stream) != hipSuccess) {
             rc = bfail(HB_EHIP, "hb_batch_run: set-up failed");
             break;
         }
-        for (int i = 0; i < ng && rc == HB_OK; ++i)
-            if (hb::launch_init(graph_dev(b, i), b->stream) != hipSuccess) rc = bfail(HB_EHIP, "init kernel failed");
+        for (int i = 0; i < ng && rc == HB_OK; ++i) {
+            HbDev gd = graph_dev(b, i);
+            gd.sat_max = d.sat_max ? b->sat_max((size_t)i) : nullptr;
+            if (hb::launch_init(gd, b->stream) != hipSuccess) rc = bfail(HB_EHIP, "init kernel failed");
+        }
         if (rc != HB_OK) break;
+        if (d.sat_max) hb::k_batch_bound<<<ng, 64, 0, b->stream>>>(d);
         (void)hipEventRecord(e1, b->stream);
         // the replayed iteration for a set of precisions, captured on first use
-        auto exec_for = [&](uint32_t running, hipGraphExec_t *out) -> int {
-            const uint32_t key = running | (d.frontier ? 0u : 1u << 16);
+        auto exec_for = [&](uint32_t running, bool first, hipGraphExec_t *out) -> int {
+            const uint32_t key = running | (d.frontier ? 0u : 1u << 16) | (first ? 1u << 17 : 0u);
             for (const auto &x : b->execs)
                 if (x.first == key) {
                     *out = x.second;
@@ -967,7 +1053,7 @@ int hb_batch_run(hb_batch *b, uint32_t flags, hb_batch_stats *stats)
             hipGraphExec_t ge = nullptr;
             if (hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal) != hipSuccess)
                 return bfail(HB_EHIP, "hipStreamBeginCapture failed");
-            const hipError_t ec = launch_iter(running);
+            const hipError_t ec = launch_iter(running, first);
             const hipError_t ee = hipStreamEndCapture(b->stream, &graph);
             const bool ok = ec == hipSuccess && ee == hipSuccess &&
                             hipGraphInstantiate(&ge, graph, nullptr, nullptr, 0) == hipSuccess;
@@ -989,10 +1075,12 @@ int hb_batch_run(hb_batch *b, uint32_t flags, hb_batch_stats *stats)
                 rc = bfail(HB_ESTATE, "hb_batch_run: %u launches without every graph stopping", launches);
                 break;
             }
-            hipGraphExec_t gexec = nullptr;
-            if (flags & HB_FLAG_GRAPH) rc = exec_for(running_p, &gexec);
             for (uint32_t i = 0; i < k && rc == HB_OK; ++i) {
-                const hipError_t el = gexec ? hipGraphLaunch(gexec, b->stream) : launch_iter(running_p);
+                const bool first = launches + i == 0;  // every graph is in iteration 1
+                hipGraphExec_t gexec = nullptr;
+                if (flags & HB_FLAG_GRAPH) rc = exec_for(running_p, first, &gexec);
+                if (rc != HB_OK) break;
+                const hipError_t el = gexec ? hipGraphLaunch(gexec, b->stream) : launch_iter(running_p, first);
                 if (el != hipSuccess) rc = bfail(HB_EHIP, "iteration launch: %s", hipGetErrorString(el));
             }
             launches += k;

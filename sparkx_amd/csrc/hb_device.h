@@ -29,6 +29,10 @@ struct HbIterState {
     uint32_t push;       // few nodes changed last iteration (symmetric graph): build the
                          // list of nodes with a changed neighbour from the changed nodes
                          // instead of scanning every neighbour list
+    uint32_t sat_scan;   // enough nodes are saturated (HbDev::sat_max) to look for one among
+                         // the neighbours before the gather
+    uint32_t pad;
+    unsigned long long sat_arcs;  // sum of the saturated nodes' degrees
 };
 
 // kernel slots of one iteration: union bins 0..2, hub chunks, hub merge
@@ -47,6 +51,7 @@ struct HbIterRec {  // per-iteration counters, per kernel slot
     unsigned long long nodes[HB_NSLOT];  // nodes recomputed
     unsigned long long chg[HB_NSLOT];    // nodes whose registers changed
     unsigned long long gathered[HB_NSLOT];  // neighbour register blocks read (arcs counts ids scanned)
+    unsigned long long sat;              // sum of the degrees of the nodes that became saturated
     unsigned long long nf_lo, nf_hi;     // N(t) * 2^40 as a 128-bit integer
     unsigned long long push;             // 1 if iteration t listed its nodes by push
 };
@@ -78,6 +83,13 @@ struct HbDev {
     uint32_t *dyn_count;   // [3]
     uint32_t dyn_base[3];
     uint32_t small_max, mid_max, wave_max;  // degree bounds of bins 0..2 (hubs above)
+    // saturation (null: off): the register-wise maximum over the insertions of every node
+    // whose sketch can reach another's (k_init), an upper bound of every sketch.  A sketch
+    // equal to it can never change again, and a node with such a neighbour becomes equal to
+    // it too, whatever its other neighbours hold.  sat_bits: two bitmaps by iteration parity
+    // (hb_saturated), bit set: the node's sketch is the bound
+    uint32_t *sat_max;     // [2^p], one register each
+    uint32_t *sat_bits;
     int sym;               // the CSR holds v -> u for every u -> v
     uint64_t arcs;         // arcs of the staged CSR
     uint32_t n;
@@ -97,6 +109,12 @@ struct HbDev {
 __device__ __forceinline__ uint32_t *hb_active(const HbDev &d, uint32_t t)
 {
     return d.active + (size_t)(t & 1u) * ((d.n + 31u) / 32u);
+}
+
+// The nodes saturated after iteration t (k_begin of iteration t copies those of t - 1)
+__device__ __forceinline__ uint32_t *hb_saturated(const HbDev &d, uint32_t t)
+{
+    return d.sat_bits + (size_t)(t & 1u) * ((d.n + 31u) / 32u);
 }
 
 // ---------------------------------------------------------------------------

@@ -41,8 +41,9 @@ const HbBiasTable *bias_table(int p);
 
 hipError_t launch_init(const HbDev &d, hipStream_t s);
 hipError_t launch_fill(uint32_t *p, uint64_t count, uint32_t value, hipStream_t s);
+// one iteration; first: iteration 1, whose kernels hash ids (p <= 10)
 // ev (nullable): 2 * HB_NSLOT events recorded around each kernel slot that launches
-hipError_t launch_iteration(const HbDev &d, const HbSchedule &sc, bool nf, hipStream_t s,
+hipError_t launch_iteration(const HbDev &d, const HbSchedule &sc, bool first, bool nf, hipStream_t s,
                             hipEvent_t *ev = nullptr);
 hipError_t launch_estimates(const HbDev &d, const uint8_t *regs, float *out, hipStream_t s);
 // arc fingerprints into work[0..3] (work holds 4 + 4 * kFingerprintBlocks values):

@@ -8,14 +8,22 @@
 //     c_t(u) = a
 // Launch sequence per iteration, all reading the device-resident HbIterState so
 // that one captured hipGraph serves every iteration:
-//     k_begin (clear next changed-bitmap)  ->  k_union<P,T> per degree bin
+//     k_begin (clear next changed-bitmap)  ->  k_union<P,T,kFirst> per degree bin
 //     (k_union_rows<P> for the dense iterations of a chain-layout id range at p = 5, 6)
-//     ->  k_chunk<P> (hub neighbour chunks) -> k_merge<P> (hubs) -> [k_nf] -> k_finalize
+//     ->  k_chunk<P,kFirst> (hub neighbour chunks) -> k_merge<P> (hubs) -> [k_nf] -> k_finalize
 // Frontier: if no neighbour of u changed at t-1 then c_t(u) = c_{t-1}(u) (union
 // of unchanged sets), so u is skipped; when u itself changed at t-1 its row is
 // copied into the output buffer so both buffers stay complete.  Results are
 // identical to recomputing every node.
+// Saturation: no sketch exceeds the register-wise maximum B of all insertions (k_init; on
+// a symmetric graph without those that reach no other node).  A node whose sketch is B is
+// done for good, and a node with such a neighbour becomes B whatever the others hold, so
+// neither gathers anything.  Graphs of small diameter reach B within a few iterations:
+// R-MAT-24 (p = 7) iterations 4, 5 and 6 take 2.5, 1.0 and 0.4 ms instead of 7.9, 7.9 and
+// 4.5, its run 24.2 instead of 40.1 ms; R-MAT-20 (p = 8) 3.3 instead of 4.7 ms.
+#include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "hb_device.h"
 #include "hb_kernels.h"
@@ -27,10 +35,11 @@ static constexpr int kBlock = 256;
 
 
 // block-wide sums of per-lane counters, one atomic per counter per block
-__device__ __forceinline__ void block_add5(unsigned long long a, unsigned long long b, unsigned long long c,
-                                           unsigned long long e, unsigned long long f, HbIterRec *rec, int slot)
+__device__ __forceinline__ void block_add(unsigned long long a, unsigned long long b, unsigned long long c,
+                                          unsigned long long e, unsigned long long f, unsigned long long g,
+                                          HbIterRec *rec, int slot)
 {
-    __shared__ unsigned long long red[5][kBlock / HB_WAVE];
+    __shared__ unsigned long long red[6][kBlock / HB_WAVE];
 #pragma unroll
     for (int s = 1; s < HB_WAVE; s <<= 1) {
         a += __shfl_xor(a, s);
@@ -38,6 +47,7 @@ __device__ __forceinline__ void block_add5(unsigned long long a, unsigned long l
         c += __shfl_xor(c, s);
         e += __shfl_xor(e, s);
         f += __shfl_xor(f, s);
+        g += __shfl_xor(g, s);
     }
     const int w = threadIdx.x / HB_WAVE;
     if ((threadIdx.x & (HB_WAVE - 1)) == 0) {
@@ -46,22 +56,25 @@ __device__ __forceinline__ void block_add5(unsigned long long a, unsigned long l
         red[2][w] = c;
         red[3][w] = e;
         red[4][w] = f;
+        red[5][w] = g;
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-        unsigned long long s0 = 0, s1 = 0, s2 = 0, s3 = 0, s4 = 0;
+        unsigned long long s0 = 0, s1 = 0, s2 = 0, s3 = 0, s4 = 0, s5 = 0;
         for (int i = 0; i < (int)(blockDim.x / HB_WAVE); ++i) {
             s0 += red[0][i];
             s1 += red[1][i];
             s2 += red[2][i];
             s3 += red[3][i];
             s4 += red[4][i];
+            s5 += red[5][i];
         }
         if (s0) atomicAdd(&rec->inc[slot], s0);
         if (s1) atomicAdd(&rec->arcs[slot], s1);
         if (s2) atomicAdd(&rec->nodes[slot], s2);
         if (s3) atomicAdd(&rec->chg[slot], s3);
         if (s4) atomicAdd(&rec->gathered[slot], s4);
+        if (s5) atomicAdd(&rec->sat, s5);
     }
 }
 
@@ -93,10 +106,29 @@ __global__ __launch_bounds__(kBlock) void k_init(HbDev d)
     const uint64_t u = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const uint64_t first = u - lane;  // the wavefront's first node
     uint32_t word = 0;                // rank | idx << 8 | (no neighbours) << 31
+    __shared__ uint32_t s_max[M];     // the block's share of the bound of all sketches
+    if (d.sat_max) {
+        for (uint32_t i = threadIdx.x; i < M; i += kBlock) s_max[i] = 0u;
+        __syncthreads();
+    }
     if (u < d.n) {
         uint32_t idx, rank;
         hb_index_rank(d.node_id ? d.node_id[u] : (uint32_t)u, P, &idx, &rank);
-        word = rank | (idx << 8) | (d.off[u + 1] == d.off[u] ? 1u << 31 : 0u);
+        const uint32_t e0 = d.off[u], deg = d.off[u + 1] - e0;
+        word = rank | (idx << 8) | (deg == 0 ? 1u << 31 : 0u);
+        // On a symmetric graph a node without neighbours and a pair of nodes that only have
+        // each other reach no other sketch; leaving them out lets the giant component of a
+        // random graph, which seldom lacks other nodes, attain the bound.
+        if (d.sat_max) {
+            const uint32_t w = d.sym && deg == 1 ? d.nbr[e0] : 0u;
+            const bool alone = d.sym && (deg == 0 || (deg == 1 && d.off[w + 1] - d.off[w] == 1));
+            if (!alone) atomicMax(s_max + idx, rank);
+        }
+    }
+    if (d.sat_max) {  // one look per register and block; few blocks still raise one
+        __syncthreads();
+        for (uint32_t i = threadIdx.x; i < M; i += kBlock)
+            if (s_max[i] > d.sat_max[i]) atomicMax(d.sat_max + i, s_max[i]);
     }
 #pragma unroll
     for (uint32_t k = 0; k < G; ++k) {
@@ -138,8 +170,8 @@ __global__ __launch_bounds__(kBlock) void k_fill_u32(uint32_t *p, uint64_t count
 // at t-1 but has no changed neighbour (hubs: k_merge copies).
 // ---------------------------------------------------------------------------
 // Start of iteration t: clear the bitmap iteration t writes (bits[t & 1]) and, where
-// push iterations can occur, the active bitmap of iteration t + 1; clear this
-// iteration's ring record; in a push iteration also clear the per-bin list counts and
+// push iterations can occur, the active bitmap of iteration t + 1; carry the saturated
+// nodes over; clear this iteration's ring record; in a push iteration also clear the per-bin list counts and
 // mark this iteration's active bitmap.  The marking reads bits[(t - 1) & 1] and writes
 // hb_active(t), neither of which the clearing touches.
 __global__ __launch_bounds__(kBlock) void k_begin(HbDev d, uint32_t words)
@@ -156,9 +188,12 @@ __global__ __launch_bounds__(kBlock) void k_begin(HbDev d, uint32_t words)
         if (push) r->push = 1ull;
     }
     uint32_t *next_active = d.active ? hb_active(d, it + 1) : nullptr;
+    uint32_t *sat = d.sat_max ? hb_saturated(d, it) : nullptr;
+    const uint32_t *sat_prev = d.sat_max ? hb_saturated(d, it - 1) : nullptr;
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < words; i += gridDim.x * blockDim.x) {
         bw[i] = 0u;
         if (next_active) next_active[i] = 0u;
+        if (sat) sat[i] = sat_prev[i];
     }
     if (!push) return;
     uint32_t *act = hb_active(d, it);
@@ -458,8 +493,19 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(7))) voi
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     }
     const bool first_lane = lane == 0;
-    block_add5(first_lane ? n_inc : 0, first_lane ? n_arcs : 0, first_lane ? n_nodes : 0, first_lane ? n_chg : 0,
-               first_lane ? n_arcs : 0, d.rec + it % HB_REC_RING, slot_id);
+    block_add(first_lane ? n_inc : 0, first_lane ? n_arcs : 0, first_lane ? n_nodes : 0, first_lane ? n_chg : 0,
+              first_lane ? n_arcs : 0, 0, d.rec + it % HB_REC_RING, slot_id);
+}
+
+// the bound of all sketches, packed as registers are, into LDS (2^P bytes at s)
+template <int P>
+__device__ __forceinline__ void stage_bound(const HbDev &d, uint32_t *s)
+{
+    for (uint32_t i = threadIdx.x; i < (1u << P) / 4; i += kBlock) {
+        const uint4 r = *(const uint4 *)(d.sat_max + 4 * i);
+        s[i] = r.x | (r.y << 8) | (r.z << 16) | (r.w << 24);
+    }
+    __syncthreads();
 }
 
 // ---------------------------------------------------------------------------
@@ -477,13 +523,13 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(7))) voi
 // 32-bit counters, 7 still leaves the run 0.2-0.3% slower).  At p <= 6 one-copy teams run at 7 (no spill, where 8
 // spilled 7 VGPRs): ER (n = 65,536, p = 6) 44.7 -> 43.5 us per launch; the k-mer graph's
 // dense iterations run k_union_rows instead.
-template <int P, int T>
+template <int P, int T, bool kFirst>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(P >= 7 ? (T >= 32 ? 6 : 8) : (T == (1 << P) / 16 ? 7 : 8)))) void k_union(
     HbDev d, const uint32_t *__restrict__ list, uint32_t base, uint32_t count, int slot_id)
 {
     const HbIterState *st = d.st;
     if (st->done) return;
-    if constexpr (T == (1 << P) / 16 && (P == 5 || P == 6))
+    if constexpr (!kFirst && T == (1 << P) / 16 && (P == 5 || P == 6))
         if (d.rows && !list && (base & 63u) == 0 && rows_iteration(d, *st)) return;  // k_union_rows runs it
     HB_TABLES_LDS(P, d, tb)
     const uint32_t it = st->iter;
@@ -508,42 +554,53 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(P >= 7 ?
     v.use_frontier = d.frontier && it > 1 && !st->skip_scan && !st->push;
     // outside dense iterations only the neighbours that changed at t-1 are gathered
     v.gather_bits = d.frontier && it > 1 && !st->skip_scan ? v.bitsR : nullptr;
-    __shared__ __attribute__((aligned(16))) uint32_t s_first[kBlock * 16];
-    v.first = it == 1 && P <= 10;
-    v.scr = s_first;
+    // iteration 1's register arrays (16 u32 per lane), the LDS window of the chain layout's
+    // dense iterations (one uint4 per lane) or the bound of all sketches (2^P bytes)
+    constexpr uint32_t kScratch = kFirst ? kBlock * 16 : T == (1 << P) / 16 ? kBlock * 4 : (1 << P) / 4;
+    __shared__ __attribute__((aligned(16))) uint32_t s_scr[kScratch];
+    static_assert(kScratch >= (1 << P) / 4, "room for the bound");
+    v.scr = s_scr;
+    v.sym = d.sym != 0;
+    if (!kFirst && d.sat_max) {
+        stage_bound<P>(d, s_scr);
+        v.satR = hb_saturated(d, it - 1);
+        v.satW = hb_saturated(d, it);
+        v.bound = reinterpret_cast<const uint4 *>(s_scr);
+        v.sat_scan = st->sat_scan != 0;
+    }
     const uint32_t tl = threadIdx.x % T;
     const uint32_t teams_per_grid = gridDim.x * (kBlock / T);
     HbCounts c;
-    if constexpr (T == (1 << P) / 16 && P != 5 && P != 6) {
+    if constexpr (!kFirst && T == (1 << P) / 16 && P != 5 && P != 6) {
         // dense iteration over an id-range bin: each wavefront's teams hold consecutive
         // nodes, and neighbours among them come from the wavefront's LDS window (at p = 5
         // and 6 k_union_rows runs these iterations)
-        if (d.window && !list && !v.first && !v.gather_bits) {
-            uint4 *win = reinterpret_cast<uint4 *>(s_first) + (threadIdx.x / HB_WAVE) * HB_WAVE;
+        if (d.window && !list && !v.gather_bits) {
+            uint4 *win = reinterpret_cast<uint4 *>(s_scr) + (threadIdx.x / HB_WAVE) * HB_WAVE;
             const uint32_t in_wave = (threadIdx.x % HB_WAVE) / T;
             for (uint32_t team = blockIdx.x * (kBlock / T) + threadIdx.x / T; team < count; team += teams_per_grid) {
                 const uint32_t lo = base + team - in_wave;
                 union_node_window<P, T>(v, tb, base + team, tl, c, lo, min(lo + HB_WAVE / T, base + count), win);
             }
-            block_add5(c.inc, c.arcs, c.nodes, c.chg, c.gathered, d.rec + it % HB_REC_RING, slot_id);
+            block_add(c.inc, c.arcs, c.nodes, c.chg, c.gathered, c.sat, d.rec + it % HB_REC_RING, slot_id);
             return;
         }
     }
-    if (v.gather_bits) {
+    auto run = [&](auto gather) {
         for (uint32_t team = blockIdx.x * (kBlock / T) + threadIdx.x / T; team < count; team += teams_per_grid)
-            union_node<P, T, true>(v, tb, list ? list[team] : base + team, tl, c);
-    } else {
-        for (uint32_t team = blockIdx.x * (kBlock / T) + threadIdx.x / T; team < count; team += teams_per_grid)
-            union_node<P, T, false>(v, tb, list ? list[team] : base + team, tl, c);
-    }
-    block_add5(c.inc, c.arcs, c.nodes, c.chg, c.gathered, d.rec + it % HB_REC_RING, slot_id);
+            union_node<P, T, decltype(gather)::value>(v, tb, list ? list[team] : base + team, tl, c);
+    };
+    if constexpr (kFirst) run(std::integral_constant<Gather, Gather::kFirst>{});
+    else if (v.gather_bits) run(std::integral_constant<Gather, Gather::kChanged>{});
+    else run(std::integral_constant<Gather, Gather::kAll>{});
+    block_add(c.inc, c.arcs, c.nodes, c.chg, c.gathered, c.sat, d.rec + it % HB_REC_RING, slot_id);
 }
 
 // ---------------------------------------------------------------------------
 // hubs, phase 1: one wavefront per chunk of a hub's neighbour list writes the
 // chunk's partial union to scratch (not the hub's own registers)
 // ---------------------------------------------------------------------------
-template <int P>
+template <int P, bool kFirst>
 __global__ __launch_bounds__(kBlock) void k_chunk(HbDev d, const uint32_t *__restrict__ tnode,
                                                   const uint32_t *__restrict__ tbeg,
                                                   const uint32_t *__restrict__ tend, uint32_t ntasks)
@@ -557,11 +614,17 @@ __global__ __launch_bounds__(kBlock) void k_chunk(HbDev d, const uint32_t *__res
     const bool use_frontier = d.frontier && it > 1 && !st->skip_scan;
     // push iteration: a hub whose active bit is clear has no changed neighbour at all
     const bool push = st->push != 0;
-    const bool first = it == 1;
-    __shared__ uint32_t s_first[kBlock * 16];
+    __shared__ __attribute__((aligned(16))) uint32_t s_scr[kFirst ? kBlock * 16 : M / 4];  // as in k_union
     const uint32_t tl = threadIdx.x % T, cl = tl % G, slot = tl / G;
     const uint32_t waves_per_grid = gridDim.x * (kBlock / T);
     unsigned long long c_arcs = 0, c_gathered = 0;
+    const uint32_t *satR = nullptr;
+    const uint4 *bound = reinterpret_cast<const uint4 *>(s_scr);
+    if (!kFirst && d.sat_max) {
+        stage_bound<P>(d, s_scr);
+        satR = hb_saturated(d, it - 1);
+    }
+    const bool sat_scan = satR && st->sat_scan;
 
     for (uint32_t task = blockIdx.x * (kBlock / T) + threadIdx.x / T; task < ntasks;
          task += waves_per_grid) {
@@ -569,27 +632,37 @@ __global__ __launch_bounds__(kBlock) void k_chunk(HbDev d, const uint32_t *__res
         const uint32_t *__restrict__ nb = d.nbr + eb;
         const uint32_t *__restrict__ nbh = d.orig + eb;
         const uint32_t len = ee - eb;
-        bool active = !(push && !bit_test(hb_active(d, it), tnode[task]));
-        if (use_frontier && active) {
+        bool active = !(push && !bit_test(hb_active(d, it), tnode[task])) && !(satR && bit_test(satR, tnode[task]));
+        uint32_t scanned = 0;
+        const bool sat = active && sat_scan && sat_neighbour<T>(satR, nb, len, tl, scanned);
+        if (use_frontier && active && !sat) {
             uint32_t any = 0;
             for (uint32_t j = tl; j < len; j += T) any |= bit_test(bitsR, nb[j]);
             active = hb_copy_or<T>(any) != 0;
         }
         if (tl == 0) d.chunk_flag[task] = active ? 1u : 0u;
         if (!active) continue;
+        if (sat) {  // the hub becomes the bound through this chunk
+            if (slot == 0) *(uint4 *)(d.scratch + ((uint64_t)task << P) + cl * 16) = bound[cl];
+            if (tl == 0) c_arcs += scanned;
+            continue;
+        }
         uint32_t gathered = 0;  // by this lane's copy
-        uint4 acc = use_frontier
-                        ? hb_gather_union<P, S, true>(in, first, s_first, bitsR, nb, nbh, len, slot, cl,
-                                                      make_uint4(0, 0, 0, 0), gathered)
-                        : hb_gather_union<P, S, false>(in, first, s_first, nullptr, nb, nbh, len, slot, cl,
-                                                       make_uint4(0, 0, 0, 0), gathered);
+        const uint4 none = make_uint4(0, 0, 0, 0);
+        uint4 acc;
+        if constexpr (kFirst)
+            acc = hb_gather_union<P, S, Gather::kFirst>(in, s_scr, nullptr, nb, nbh, len, slot, cl, none, gathered);
+        else
+            acc = use_frontier
+                      ? hb_gather_union<P, S, Gather::kChanged>(in, nullptr, bitsR, nb, nbh, len, slot, cl, none, gathered)
+                      : hb_gather_union<P, S, Gather::kAll>(in, nullptr, nullptr, nb, nbh, len, slot, cl, none, gathered);
         if (cl == 0) c_gathered += gathered;
 #pragma unroll
         for (uint32_t s = G; s < T; s <<= 1) acc = hb_bmax4(acc, hb_shfl_xor4<T>(acc, s));
         if (slot == 0) *(uint4 *)(d.scratch + ((uint64_t)task << P) + cl * 16) = acc;
         if (tl == 0) c_arcs += len;
     }
-    block_add5(0, c_arcs, 0, 0, c_gathered, d.rec + it % HB_REC_RING, HB_SLOT_CHUNK);
+    block_add(0, c_arcs, 0, 0, c_gathered, 0, d.rec + it % HB_REC_RING, HB_SLOT_CHUNK);
 }
 
 // hubs, phase 2: one wavefront per hub merges its own registers with the
@@ -612,7 +685,11 @@ __global__ __launch_bounds__(kBlock) void k_merge(HbDev d, const uint32_t *__res
     uint32_t *bitsW = (it & 1u) ? d.bits1 : d.bits0;
     const uint32_t tl = threadIdx.x % T, cl = tl % G, slot = tl / G;
     const uint32_t waves_per_grid = gridDim.x * (kBlock / T);
-    unsigned long long c_inc = 0, c_nodes = 0, c_chg = 0;
+    unsigned long long c_inc = 0, c_nodes = 0, c_chg = 0, c_sat = 0;
+    __shared__ __attribute__((aligned(16))) uint32_t s_bound[M / 4];
+    const bool sat = d.sat_max && it > 1;
+    if (sat) stage_bound<P>(d, s_bound);
+    const uint4 *bound = reinterpret_cast<const uint4 *>(s_bound);
 
     for (uint32_t h = blockIdx.x * (kBlock / T) + threadIdx.x / T; h < nhubs; h += waves_per_grid) {
         const uint32_t u = hnode[h], t0 = htask0[h], nt = hntask[h];
@@ -632,14 +709,23 @@ __global__ __launch_bounds__(kBlock) void k_merge(HbDev d, const uint32_t *__res
                 acc = hb_bmax4(acc, *(const uint4 *)(d.scratch + ((uint64_t)(t0 + j) << P) + cl * 16));
 #pragma unroll
         for (uint32_t s = G; s < T; s <<= 1) acc = hb_bmax4(acc, hb_shfl_xor4<T>(acc, s));
-        const uint32_t diffw = (acc.x != own.x) | (acc.y != own.y) | (acc.z != own.z) | (acc.w != own.w);
-        const bool changed = hb_copy_or<G>(diffw) != 0;
+        uint32_t diffw = (acc.x != own.x) | (acc.y != own.y) | (acc.z != own.z) | (acc.w != own.w);
+        if (sat) {  // bit 1: a register is below the bound
+            const uint4 f = bound[cl];
+            diffw |= ((acc.x != f.x) | (acc.y != f.y) | (acc.z != f.z) | (acc.w != f.w)) << 1;
+        }
+        diffw = hb_copy_or<G>(diffw);
+        const bool changed = (diffw & 1u) != 0;
         const float curr = hb_estimate_copy<G>(tb, acc);
         if (slot == 0) *(uint4 *)(out + ((uint64_t)u << P) + cl * 16) = acc;
         if (tl == 0) {
             const float prev = d.est[u];
             if (accumulate(d, u, prev, curr, t, inv_t)) c_inc += 1;
             d.est[u] = curr;
+            if (sat && !(diffw & 2u)) {  // a hub has many neighbours: it is part of the bound
+                atomicOr(hb_saturated(d, it) + (u >> 5), 1u << (u & 31u));
+                c_sat += d.off[u + 1] - d.off[u];
+            }
             if (changed) {
                 atomicOr(bitsW + (u >> 5), 1u << (u & 31u));
                 c_chg += 1;
@@ -647,7 +733,7 @@ __global__ __launch_bounds__(kBlock) void k_merge(HbDev d, const uint32_t *__res
             c_nodes += 1;
         }
     }
-    block_add5(c_inc, 0, c_nodes, c_chg, 0, d.rec + it % HB_REC_RING, HB_SLOT_MERGE);
+    block_add(c_inc, 0, c_nodes, c_chg, 0, c_sat, d.rec + it % HB_REC_RING, HB_SLOT_MERGE);
 }
 
 // ---------------------------------------------------------------------------
@@ -798,7 +884,7 @@ __global__ __launch_bounds__(kBlock) void k_union_wide(HbDev d, const uint32_t *
             c_nodes += 1;
         }
     }
-    block_add5(c_inc, c_arcs, c_nodes, c_chg, c_arcs, d.rec + it % HB_REC_RING, slot_id);  // gathers every row
+    block_add(c_inc, c_arcs, c_nodes, c_chg, c_arcs, 0, d.rec + it % HB_REC_RING, slot_id);  // gathers every row
 }
 
 template <int P>
@@ -893,6 +979,11 @@ __global__ void k_finalize(HbDev d)
     // push when few nodes changed (on R-MAT-24 a push pass at 24% changed nodes whose lists
     // hold 2% of the arcs measured slower than the scan with selective gathers)
     st->push = d.sym && d.p <= 10 && d.frontier && 16 * chg <= (unsigned long long)d.n_linked;
+    // a search that finds nothing costs a node about a quarter of its gather on short lists
+    // (Erdos-Renyi, n = 65,536, degree 32: 74 against 60 us an iteration), one that finds a
+    // neighbour saves all of it: search once a node has one in eight such neighbours on average
+    st->sat_arcs += d.rec[it % HB_REC_RING].sat;
+    st->sat_scan = 8 * st->sat_arcs >= (unsigned long long)d.n_linked;
     st->t = st->t + 1.0;
     st->inv_t = __ddiv_rn(1.0, st->t);
 }
@@ -944,7 +1035,7 @@ static unsigned grid_for(uint64_t threads, unsigned cap)
     return (unsigned)(b < 1 ? 1 : (b > cap ? cap : b));
 }
 
-template <int P>
+template <int P, bool kFirst>
 static hipError_t launch_union_T(const HbDev &d, const uint32_t *list, uint32_t base, uint32_t count, int T,
                                  unsigned max_blocks, int slot, hipStream_t s)
 {
@@ -954,7 +1045,7 @@ static hipError_t launch_union_T(const HbDev &d, const uint32_t *list, uint32_t 
 #define HB_CASE(TT)                                                                        \
     case TT:                                                                               \
         if constexpr (TT >= G) {                                                           \
-            k_union<P, TT><<<grid, kBlock, 0, s>>>(d, list, base, count, slot);            \
+            k_union<P, TT, kFirst><<<grid, kBlock, 0, s>>>(d, list, base, count, slot);            \
             return hipGetLastError();                                                      \
         }                                                                                  \
         break;
@@ -1014,7 +1105,7 @@ hipError_t launch_fill(uint32_t *p, uint64_t count, uint32_t value, hipStream_t 
     return hipGetLastError();
 }
 
-hipError_t launch_iteration(const HbDev &d, const HbSchedule &sc, bool nf, hipStream_t s,
+hipError_t launch_iteration(const HbDev &d, const HbSchedule &sc, bool first, bool nf, hipStream_t s,
                             hipEvent_t *ev)
 {
     const uint32_t words = (d.n + 31) / 32;
@@ -1024,7 +1115,7 @@ hipError_t launch_iteration(const HbDev &d, const HbSchedule &sc, bool nf, hipSt
         d, words);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    if (push_possible) {  // returns at once unless this is a push iteration
+    if (push_possible && !first) {  // returns at once unless this is a push iteration
         HB_DISPATCH_P(d.p, k_push_compact<P><<<grid_for(words, 4096), kBlock, 0, s>>>(d, words));
         e = hipGetLastError();
         if (e != hipSuccess) return e;
@@ -1047,8 +1138,11 @@ hipError_t launch_iteration(const HbDev &d, const HbSchedule &sc, bool nf, hipSt
                 e = hipGetLastError();
                 if (e != hipSuccess) return e;
             }
-            HB_DISPATCH_P(d.p, e = launch_union_T<P>(d, sc.bin_list[b], sc.bin_base[b], sc.bin_count[b],
-                                                     sc.bin_team[b], sc.max_blocks, b, s));
+            if (!(first && rows_bin(d, sc, b)))
+                HB_DISPATCH_P(d.p, {
+                    auto *launch = first ? launch_union_T<P, true> : launch_union_T<P, false>;
+                    e = launch(d, sc.bin_list[b], sc.bin_base[b], sc.bin_count[b], sc.bin_team[b], sc.max_blocks, b, s);
+                });
         }
         if (ev) (void)hipEventRecord(ev[2 * b + 1], s);
         if (e != hipSuccess) return e;
@@ -1056,7 +1150,8 @@ hipError_t launch_iteration(const HbDev &d, const HbSchedule &sc, bool nf, hipSt
     if (sc.ntasks) {
         HB_DISPATCH_P(d.p, {
             if (ev) (void)hipEventRecord(ev[2 * HB_SLOT_CHUNK], s);
-            k_chunk<P><<<grid_for((uint64_t)sc.ntasks * HB_WAVE, sc.max_blocks), kBlock, 0, s>>>(
+            auto *chunk = first ? k_chunk<P, true> : k_chunk<P, false>;
+            chunk<<<grid_for((uint64_t)sc.ntasks * HB_WAVE, sc.max_blocks), kBlock, 0, s>>>(
                 d, sc.task_node, sc.task_beg, sc.task_end, sc.ntasks);
             if (ev) (void)hipEventRecord(ev[2 * HB_SLOT_CHUNK + 1], s);
             if (ev) (void)hipEventRecord(ev[2 * HB_SLOT_MERGE], s);
@@ -1085,10 +1180,14 @@ hipError_t arc_fingerprints(const uint32_t *off, const uint32_t *nbr, uint32_t n
                             unsigned long long *work, hipStream_t s)
 {
     if (n == 0) return hipSuccess;
-    k_arc_fingerprint<<<kFingerprintBlocks, kBlock, 0, s>>>(off, nbr, n, arcs, work + 4);
+    // no more blocks than there are arcs for their lanes: a small graph's search and sum
+    // take 7 us instead of 37
+    const uint64_t want = (arcs + (uint64_t)kBlock * kFpArcs - 1) / ((uint64_t)kBlock * kFpArcs);
+    const uint32_t blocks = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(want, kFingerprintBlocks));
+    k_arc_fingerprint<<<blocks, kBlock, 0, s>>>(off, nbr, n, arcs, work + 4);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    return sum_columns(work + 4, kFingerprintBlocks, 4, work, s);
+    return sum_columns(work + 4, blocks, 4, work, s);
 }
 
 // out[k] = sum over r < rows of part[r * cols + k], one block per column, a fixed

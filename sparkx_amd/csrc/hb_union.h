@@ -12,14 +12,22 @@
 
 namespace hb {
 
+// What an iteration reads of the neighbours.  Each kind is a kernel of its own: together
+// in one, they cost every one of them registers (k_union<7, 8> spills 10 VGPRs at eight
+// wavefronts per SIMD with all three, none with the first iteration's apart) and LDS.
+enum class Gather {
+    kAll,      // every neighbour's registers
+    kChanged,  // those of the neighbours in HbView::gather_bits
+    kFirst,    // iteration 1 with P <= 10: sketches hold only their own insertion, so ids are hashed
+};
+
 // one graph's state as seen by one iteration
 struct HbView {
     const uint32_t *off, *nbr;
     const uint32_t *orig;      // hashed id of each arc's head (iteration 1)
     const uint32_t *node_id;   // hashed id of each node (null: its index)
     const uint8_t *in;
-    bool first;             // iteration 1 with P <= 10: sketches hold only their own insertion
-    uint32_t *scr;          // LDS, 16 u32 per lane of the block (iteration 1 only)
+    uint32_t *scr;          // LDS, 16 u32 per lane of the block (Gather::kFirst only)
     uint8_t *out;
     float *est;
     double *dist, *inv;
@@ -28,6 +36,13 @@ struct HbView {
     uint32_t *bitsW;        // registers changed at t
     double t, inv_t;
     bool use_frontier;
+    // saturation (null: not used in this iteration): the nodes whose sketch is the upper
+    // bound of all sketches at t-1 and at t, and the bound itself (LDS, G uint4)
+    const uint32_t *satR = nullptr;
+    uint32_t *satW = nullptr;
+    const uint4 *bound = nullptr;
+    bool sat_scan = false;  // look for a saturated neighbour before the gather
+    bool sym = false;
 };
 
 // One lane's counts over its share of a launch.  32 bits suffice (a lane's sums are at
@@ -36,6 +51,7 @@ struct HbView {
 struct HbCounts {
     uint32_t inc = 0, arcs = 0, nodes = 0, chg = 0;
     uint32_t gathered = 0;  // neighbour register blocks read
+    uint32_t sat = 0;       // degrees of the nodes that became saturated
 };
 
 __device__ __forceinline__ bool bit_test(const uint32_t *bits, uint32_t v)
@@ -105,16 +121,16 @@ __device__ __forceinline__ void hb_put_max(uint4 &a, uint32_t w, uint32_t cl)
 
 // Union of the sketches of nb[slot], nb[slot + S], ... (j < len) into `start`,
 // for the 16 registers of copy lane cl (the copy is G = 2^P/16 consecutive lanes).
-// With `changed` (the nodes whose registers changed at t-1) only those neighbours are
+// kChanged: only the neighbours in `changed` (the nodes whose registers changed at t-1) are
 // gathered: an unchanged neighbour v has c_{t-1}(v) = c_{t-2}(v), which c_{t-1}(u)
 // already contains (v is u's neighbour), so leaving it out changes nothing.
-// In iteration 1 (`first`) every neighbour's sketch is still its own insertion, so
+// kFirst: in iteration 1 every neighbour's sketch is still its own insertion, so
 // instead of gathering its 2^P-byte register block the copy's lanes hash the
 // neighbour ids, one each, and raise register idx to the rank with an LDS atomic max
 // on a u32 per register (`scr`: 16 u32 per lane, the copy's registers contiguous
 // from the copy's first lane); no random global memory access at all.
-template <int P, uint32_t S, bool SEL>
-__device__ __forceinline__ uint4 hb_gather_union(const uint8_t *__restrict__ in, bool first, uint32_t *scr,
+template <int P, uint32_t S, Gather kGather>
+__device__ __forceinline__ uint4 hb_gather_union(const uint8_t *__restrict__ in, uint32_t *scr,
                                                  const uint32_t *__restrict__ changed,
                                                  const uint32_t *__restrict__ nb,
                                                  const uint32_t *__restrict__ nbh, uint32_t len, uint32_t slot,
@@ -122,7 +138,7 @@ __device__ __forceinline__ uint4 hb_gather_union(const uint8_t *__restrict__ in,
 {
     constexpr uint32_t G = (1u << P) / 16;
     uint32_t j = slot;
-    if (first) {
+    if constexpr (kGather == Gather::kFirst) {
         uint32_t *mine = scr + threadIdx.x * 16u;              // this lane's 16 registers
         uint32_t *copy = scr + (threadIdx.x - cl) * 16u;       // register idx of the copy at copy[idx]
         const uint32_t sw[4] = {start.x, start.y, start.z, start.w};
@@ -142,7 +158,7 @@ __device__ __forceinline__ uint4 hb_gather_union(const uint8_t *__restrict__ in,
         return make_uint4(r[0], r[1], r[2], r[3]);
     }
     HbAcc pa = hb_acc(start);
-    if constexpr (SEL) {
+    if constexpr (kGather == Gather::kChanged) {
         const uint4 z = make_uint4(0, 0, 0, 0);  // registers are >= 0: max with 0 is a no-op
         for (; j + 3 * S < len; j += 4 * S) {
             const uint32_t v0 = nb[j], v1 = nb[j + S], v2 = nb[j + 2 * S], v3 = nb[j + 3 * S];
@@ -185,9 +201,32 @@ __device__ __forceinline__ uint4 hb_gather_union(const uint8_t *__restrict__ in,
     return hb_acc_get(pa);
 }
 
-// SEL: gather only the neighbours in v.gather_bits (a separate instantiation, so the
-// dense path's code is unchanged by the selective one)
-template <int P, int T, bool SEL = false>
+// Whether one of the first neighbours of a list is saturated, asked by a team of T lanes
+// (all of them return it).  The degree layout lists the high-degree nodes, which saturate
+// first, at the front, so a node with a saturated neighbour nearly always shows it within
+// the first 2 T ids; missing one only costs the gather.
+template <int T>
+__device__ __forceinline__ bool sat_neighbour(const uint32_t *__restrict__ sat, const uint32_t *__restrict__ nb,
+                                              uint32_t len, uint32_t tl, uint32_t &scanned)
+{
+    for (uint32_t k = 0; k < 2 && k * T < len; ++k) {
+        const uint32_t j = k * T + tl;
+        scanned = min(len, (k + 1) * T);
+        if (hb_copy_or<T>(j < len ? (uint32_t)bit_test(sat, nb[j]) : 0u)) return true;
+    }
+    return false;
+}
+
+// Marks u saturated after this iteration: its sketch is the bound.  Two nodes that are
+// each other's only neighbour are left out of the bound (k_init), so neither is marked.
+__device__ __forceinline__ void sat_mark(const HbView &v, uint32_t u, const uint32_t *nb, uint32_t deg, HbCounts &c)
+{
+    if (v.sym && deg == 1 && v.off[nb[0] + 1] - v.off[nb[0]] == 1) return;
+    atomicOr(v.satW + (u >> 5), 1u << (u & 31u));
+    c.sat += deg;
+}
+
+template <int P, int T, Gather kGather>
 __device__ __forceinline__ void union_node(const HbView &v, const HbTables &tb, uint32_t u, uint32_t tl,
                                            HbCounts &c)
 {
@@ -198,7 +237,20 @@ __device__ __forceinline__ void union_node(const HbView &v, const HbTables &tb, 
     const uint32_t e0 = v.off[u], deg = v.off[u + 1] - e0;
     const uint32_t *__restrict__ nb = v.nbr + e0;
     const uint32_t *__restrict__ nbh = v.orig + e0;
-    if (v.use_frontier) {
+    bool sat = false;  // a neighbour is saturated, so this node becomes so
+    uint32_t scanned = deg;
+    if (kGather != Gather::kFirst && v.satR) {
+        if (bit_test(v.satR, u)) {  // nothing can change; keep both buffers complete
+            if (slot == 0 && bit_test(v.bitsR, u)) *(uint4 *)(v.out + ((uint64_t)u << P) + cl * 16) = v.bound[cl];
+            return;
+        }
+        if (v.sat_scan) {
+            uint32_t k = 0;
+            sat = sat_neighbour<T>(v.satR, nb, deg, tl, k);
+            if (sat) scanned = k;
+        }
+    }
+    if (kGather == Gather::kChanged && v.use_frontier && !sat) {
         uint32_t any = 0;
         for (uint32_t j = tl; j < deg; j += T) any |= bit_test(v.bitsR, nb[j]);
         if (hb_copy_or<T>(any) == 0) {
@@ -209,17 +261,30 @@ __device__ __forceinline__ void union_node(const HbView &v, const HbTables &tb, 
             return;
         }
     }
-    const uint4 own = v.first ? hb_own_from_word(hb_insertion<P>(v.node_id ? v.node_id[u] : u), cl)
-                              : *(const uint4 *)(v.in + ((uint64_t)u << P) + cl * 16);
-    uint32_t gathered = 0;  // by this lane's copy
-    uint4 acc = hb_gather_union<P, S, SEL>(v.in, v.first, v.scr, v.gather_bits, nb, nbh, deg, slot, cl, own,
-                                                   gathered);
-    if (cl == 0) c.gathered += gathered;
+    uint4 acc;
+    uint32_t diffw;  // bit 0: a register rose; bit 1: a register is below the bound
+    if (sat) {
+        acc = v.bound[cl];
+        diffw = 1u;  // an unmarked sketch below a saturated neighbour's rises
+    } else {
+        uint4 own;
+        if constexpr (kGather == Gather::kFirst)
+            own = hb_own_from_word(hb_insertion<P>(v.node_id ? v.node_id[u] : u), cl);
+        else
+            own = *(const uint4 *)(v.in + ((uint64_t)u << P) + cl * 16);
+        uint32_t gathered = 0;  // by this lane's copy
+        acc = hb_gather_union<P, S, kGather>(v.in, v.scr, v.gather_bits, nb, nbh, deg, slot, cl, own, gathered);
+        if (cl == 0) c.gathered += gathered;
 #pragma unroll
-    for (uint32_t s = G; s < T; s <<= 1) acc = hb_bmax4(acc, hb_shfl_xor4<T>(acc, s));
-
-    const uint32_t diffw = (acc.x != own.x) | (acc.y != own.y) | (acc.z != own.z) | (acc.w != own.w);
-    const bool changed = hb_copy_or<G>(diffw) != 0;
+        for (uint32_t s = G; s < T; s <<= 1) acc = hb_bmax4(acc, hb_shfl_xor4<T>(acc, s));
+        diffw = (acc.x != own.x) | (acc.y != own.y) | (acc.z != own.z) | (acc.w != own.w);
+        if (kGather != Gather::kFirst && v.satR) {
+            const uint4 f = v.bound[cl];
+            diffw |= ((acc.x != f.x) | (acc.y != f.y) | (acc.z != f.z) | (acc.w != f.w)) << 1;
+        }
+        diffw = hb_copy_or<G>(diffw);
+    }
+    const bool changed = (diffw & 1u) != 0;
     const float curr = hb_estimate_copy<G>(tb, acc);
     if (slot == 0) *(uint4 *)(v.out + ((uint64_t)u << P) + cl * 16) = acc;
     if (tl == 0) {
@@ -230,7 +295,8 @@ __device__ __forceinline__ void union_node(const HbView &v, const HbTables &tb, 
             atomicOr(v.bitsW + (u >> 5), 1u << (u & 31u));
             c.chg += 1;
         }
-        c.arcs += deg;
+        if (kGather != Gather::kFirst && v.satR && !(diffw & 2u)) sat_mark(v, u, nb, deg, c);
+        c.arcs += scanned;
         c.nodes += 1;
     }
 }
