@@ -315,8 +315,8 @@ int hb_walk_features(hb_ctx *ctx, int passes, float *features, double *ms);
 int hb_surrogate_walks(hb_ctx *ctx, hb_mlp *m, int passes, float *pred, float *features, double *ms);
 
 /* ---- exact BFS centralities ---------------------------------------------------
- * One breadth-first search per source over the staged graph, 64 sources per pass
- * (one bit lane each), following arcs forwards as the reference's BFSDists does
+ * One breadth-first search per source over the staged graph, thousands of sources side by
+ * side (one bit lane each), following arcs forwards as the reference's BFSDists does
  * (trails/bfs.rs:199-234), including its quirk: the source is not marked visited, so
  * it is rediscovered and counted.  Sources are [src_begin, src_end) (a sample, or
  * 0..n for every node).

@@ -138,6 +138,10 @@ struct DevBuf {
         if (n <= count && ptr) return hipSuccess;
         release();
         hipError_t e = hipMalloc(&ptr, std::max<size_t>(n, 1) * sizeof(T));
+        if (e == hipErrorOutOfMemory) {
+            hb::release_held();
+            e = hipMalloc(&ptr, std::max<size_t>(n, 1) * sizeof(T));
+        }
         if (e == hipSuccess) count = n;
         else ptr = nullptr;
         return e;

@@ -1,5 +1,6 @@
-// hb_exact.hip -- exact BFS centralities on the GPU: 64 breadth-first searches at
-// once, one bit lane per source in a u64 per node, advanced one level per launch.
+// hb_exact.hip -- exact BFS centralities on the GPU: up to 2,048 breadth-first searches at
+// once in a slice (one bit lane per source, SW u64 words per node), several slices side
+// by side, advanced one level per set of launches.
 //
 // Semantics follow the reference's BFS (src/trails/bfs.rs:199-234): the source is
 // queued with distance 0 but not marked visited, so it is rediscovered one step
@@ -9,10 +10,21 @@
 //     level d: next = nodes with an arc from a frontier node;  newly = next \ visited
 //              visited |= newly, frontier = newly, reachable += |newly|, total += d |newly|
 // which discovers exactly the nodes (and distances) of the reference's FIFO queue.
-// Arcs are followed forwards (push), so directed graphs are searched as the
-// reference searches them; on symmetric graphs a level with a large frontier pulls
-// instead (each node not yet reached ORs its neighbours' frontier words), which
-// computes the same `next` without atomics.
+//
+// Level 1 pushes the sources' own arcs (k_bfs_sources); every later level pulls: a node
+// that some live source has not reached ORs the frontier rows of the nodes with an arc to
+// it (its list on a symmetric CSR; otherwise the reversed CSR, built once per call).  No
+// atomics, and a row of 2,048 searches costs two cache lines where a single 8-byte word takes
+// one: the pull is bound by the rate of random requests, not by bytes, so the searches of a
+// slice share them.  2,048 sources of R-MAT-20 (31.4M arcs): 4.6 ms of pulls over 7 levels (64
+// sources at a time: 22 ms of pulls and 9 of per-pass bookkeeping); all 16,384 sources of a de
+// Bruijn graph (131,068 arcs): 0.8 ms for the call instead of 64.
+// What keeps a level cheap when little is left to do:
+//   - a byte per node says whether its frontier row holds any bit; rows without are neither
+//     written nor read, and an arc costs its id and that byte;
+//   - a source whose last level found nothing leaves the live mask, so that nodes it cannot
+//     reach do not look for it again;
+//   - a list is left as soon as every wanted bit has appeared.
 //
 // Per-source sums, bit-identical to the reference's:
 //   reachable : integer count (BFSDists::recheable)
@@ -20,13 +32,17 @@
 //               exact while it stays below 2^53 (16.7M nodes at distance 1000 is 2^34)
 //   inv_sum   : Σ_v 1/d(v) over v = 0..n-1 in node order, 1/d a correctly rounded
 //               f64 division and 0 for unreached nodes (exact.rs:386-396: an iterator
-//               sum over get_distances()), replayed sequentially per source from a
-//               u16 distance per (node, source) -- the order fixes the rounding.
+//               sum over get_distances()).  The order fixes the rounding; see k_bfs_harmonic
+//               for how all but a few of the adds are done in any order all the same.
 #include <hip/hip_runtime.h>
+#include <cstring>
+
+#include <rocprim/rocprim.hpp>
 
 #include <algorithm>
 #include <cstdarg>
 #include <cstdio>
+#include <mutex>
 #include <vector>
 
 #include "../../include/sparkx_hb.h"
@@ -35,255 +51,557 @@
 namespace hb {
 
 constexpr int kBfsBlock = 256;
+constexpr uint32_t kBfsChunk = 128;    // nodes per count: at most 128 fits a byte
+constexpr uint32_t kBfsHubDeg = 256;   // longer lists are cut into kBfsHubArcs-arc tasks
+constexpr uint32_t kBfsHubArcs = 1024;
+constexpr uint32_t kBfsPlanes = 4;     // bits of a kept distance
+constexpr uint32_t kBfsKeep = (1u << kBfsPlanes) - 1;  // levels whose distances can be kept
 
-__global__ __launch_bounds__(kBfsBlock) void k_bfs_init(uint64_t *frontier, uint64_t *visited, uint64_t *next,
-                                                        uint32_t n, uint32_t s0, uint32_t count)
-{
-    for (uint32_t u = blockIdx.x * blockDim.x + threadIdx.x; u < n; u += gridDim.x * blockDim.x) {
-        const uint32_t k = u - s0;  // wraps for u < s0
-        frontier[u] = (u >= s0 && k < count) ? (1ull << k) : 0ull;
-        visited[u] = 0ull;
-        next[u] = 0ull;
-    }
-}
+typedef unsigned long long u64;
+
+// One group of slices, all [slice]-major; a slice covers 64 SW consecutive sources from
+// src0 + 64 SW slice.
+struct BfsDev {
+    const uint32_t *off, *nbr;    // arcs as staged (level 1)
+    const uint32_t *ioff, *inbr;  // for each node the tails of the arcs to it
+    uint32_t n, src0, src_end;
+    uint32_t npad;                // flags per slice: n rounded up to whole chunks
+    u64 *visited;                 // [n][SW]
+    u64 *live;                    // [SW]: sources still searching
+    uint32_t *found;              // [64 SW]: nodes found in the level, zero between levels
+    u64 *reach, *total;           // [64 SW]
+    uint32_t *done, *levels;      // per slice: nothing found any more; last level that found something
+    const uint32_t *hub_node, *hub_first;  // hubs and their tasks (hub h: hub_first[h] ..)
+    const uint32_t *task_node, *task_beg, *task_end;
+    uint32_t hubs, tasks;
+    u64 *part;                    // [tasks][SW]
+    // distances kept for the harmonic sums (null: not), bit-sliced as the rows are: plane k,
+    // at k plane_stride, holds bit k of every distance; valid where visited is set
+    u64 *plane;
+    size_t plane_stride;
+};
+
+// The frontier after one level: rows [n][SW] (a row is only valid where its flag is set),
+// flags [npad], and the newly found nodes per source counted over kBfsChunk nodes at a time,
+// counts [chunks][64 SW] (valid where any is set), any [chunks].
+struct BfsLevel {
+    u64 *rows;
+    uint8_t *flag;
+    uint8_t *count;
+    uint8_t *any;
+};
+
+__device__ __forceinline__ uint32_t bfs_chunks(uint32_t n) { return (n + kBfsChunk - 1) / kBfsChunk; }
 
 template <typename T>
 __global__ __launch_bounds__(kBfsBlock) void k_bfs_zero(T *p, uint64_t count)
 {
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += (uint64_t)gridDim.x * blockDim.x)
-        p[i] = 0;
+        p[i] = T{};
 }
 
-// next[v] |= frontier[u] for every arc u -> v whose bits are not all visited at v.
-// A wavefront takes 64 consecutive nodes at a time: a frontier node of degree <= 64
-// is walked by its own lane, a larger one by the whole wavefront, so hubs do not
-// serialise on one lane; nodes of degree > hub_deg are left to k_bfs_hubs, which
-// spreads their lists over many wavefronts.
-__device__ __forceinline__ void hb_bfs_push_arc(const uint64_t *__restrict__ visited, uint64_t *next, uint32_t v,
-                                                uint64_t f)
+// live masks of the sources each slice holds; per-source sums and slice states cleared
+__global__ __launch_bounds__(kBfsBlock) void k_bfs_begin(BfsDev b, uint32_t sw)
 {
-    const uint64_t add = f & ~visited[v];
-    if (add) atomicOr((unsigned long long *)&next[v], (unsigned long long)add);
-}
-
-__global__ __launch_bounds__(kBfsBlock) void k_bfs_push(const uint32_t *__restrict__ off, const uint32_t *__restrict__ nbr,
-                                                        const uint64_t *__restrict__ frontier,
-                                                        const uint64_t *__restrict__ visited, uint64_t *next, uint32_t n,
-                                                        uint32_t hub_deg)
-{
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t waves = gridDim.x * (kBfsBlock / 64);
-    for (uint32_t base = (blockIdx.x * (kBfsBlock / 64) + threadIdx.x / 64) * 64; base < n; base += waves * 64) {
-        const uint32_t u = base + lane;  // uniform loop bound: every lane takes part in the ballot
-        uint64_t f = 0;
-        uint32_t e0 = 0, e1 = 0;
-        if (u < n) {
-            f = frontier[u];
-            if (f) {
-                e0 = off[u];
-                e1 = off[u + 1];
-            }
-        }
-        if (e1 - e0 <= 64)
-            for (uint32_t e = e0; e < e1; ++e) hb_bfs_push_arc(visited, next, nbr[e], f);
-        unsigned long long big = __ballot(e1 - e0 > 64 && e1 - e0 <= hub_deg);
-        while (big) {
-            const int i = __ffsll(big) - 1;
-            big &= big - 1;
-            const uint32_t b0 = (uint32_t)__shfl((int)e0, i), b1 = (uint32_t)__shfl((int)e1, i);
-            const uint64_t fi = (uint64_t)__shfl((long long)f, i);
-            for (uint32_t e = b0 + lane; e < b1; e += 64) hb_bfs_push_arc(visited, next, nbr[e], fi);
-        }
+    const uint32_t slice = blockIdx.x, cols = 64 * sw;
+    for (uint32_t c = threadIdx.x; c < cols; c += blockDim.x) {
+        const size_t i = (size_t)slice * cols + c;
+        b.found[i] = 0;
+        b.reach[i] = b.total[i] = 0;
+        const bool in = (uint64_t)b.src0 + (uint64_t)slice * cols + c < b.src_end;
+        const u64 m = __ballot(in);
+        if (c % 64 == 0) b.live[(size_t)slice * sw + c / 64] = m;
     }
+    if (threadIdx.x == 0) b.done[slice] = b.levels[slice] = 0;
 }
 
-// Level 1: the frontier is the pass's sources s0..s0+count-1, whose lists lie side by
-// side in nbr[off[s0], off[s0 + count]).  One thread per arc (its source found by a
-// binary search over the count + 1 offsets in LDS), so a pass of hub sources spreads
-// over the whole grid instead of one wavefront.  Nothing is visited yet at level 1.
-__global__ __launch_bounds__(kBfsBlock) void k_bfs_push_sources(const uint32_t *__restrict__ off,
-                                                                const uint32_t *__restrict__ nbr, uint64_t *next,
-                                                                uint32_t s0, uint32_t count)
+// Level 1: the frontier is the slice's sources, whose lists lie side by side.  One thread per
+// arc (its source found by a binary search over the offsets in LDS), so hub sources spread
+// over the grid.  Rows, visited and flags are zero before.
+template <int SW>
+__global__ __launch_bounds__(kBfsBlock) void k_bfs_sources(BfsDev b, BfsLevel out)
 {
-    __shared__ uint32_t so[65];
-    if (threadIdx.x <= count) so[threadIdx.x] = off[s0 + threadIdx.x];
+    __shared__ uint32_t so[64 * SW + 1];
+    const uint32_t slice = blockIdx.y, s0 = b.src0 + slice * 64 * SW;
+    const uint32_t count = min(64u * SW, b.src_end - s0);
+    for (uint32_t i = threadIdx.x; i <= count; i += blockDim.x) so[i] = b.off[s0 + i];
     __syncthreads();
-    const uint32_t e0 = so[0], e1 = so[count];
-    for (uint64_t e = (uint64_t)e0 + blockIdx.x * blockDim.x + threadIdx.x; e < e1; e += gridDim.x * blockDim.x) {
+    const uint64_t e1 = so[count];
+    u64 *rows = out.rows + (size_t)slice * b.n * SW, *vis = b.visited + (size_t)slice * b.n * SW;
+    for (uint64_t e = (uint64_t)so[0] + blockIdx.x * blockDim.x + threadIdx.x; e < e1; e += gridDim.x * blockDim.x) {
         uint32_t lo = 0, hi = count;  // so[lo] <= e < so[hi]
         while (hi - lo > 1) {
             const uint32_t mid = (lo + hi) >> 1;
             if (so[mid] <= e) lo = mid; else hi = mid;
         }
-        atomicOr((unsigned long long *)&next[nbr[e]], 1ull << lo);
+        const uint32_t v = b.nbr[e];
+        const size_t at = (size_t)v * SW + lo / 64;
+        atomicOr(rows + at, 1ull << (lo % 64));
+        atomicOr(vis + at, 1ull << (lo % 64));
+        out.flag[(size_t)slice * b.npad + v] = 1;
     }
 }
 
-// OR of frontier[nbr[e]] over e = b0 + lane, b0 + lane + 64, ... < b1 (this lane's
-// share of a list walked by a whole wavefront), four arcs' loads in flight at a time
-__device__ __forceinline__ uint64_t hb_bfs_or_range(const uint32_t *__restrict__ nbr,
-                                                    const uint64_t *__restrict__ frontier, uint32_t b0, uint32_t b1,
-                                                    uint32_t lane)
-{
-    uint64_t g = 0;
-    uint64_t e = (uint64_t)b0 + lane;
-    for (; e + 3 * 64 < b1; e += 4 * 64) {
-        const uint32_t w0 = nbr[e], w1 = nbr[e + 64], w2 = nbr[e + 128], w3 = nbr[e + 192];
-        g |= frontier[w0] | frontier[w1] | frontier[w2] | frontier[w3];
+// The lanes of a team (SW / 2, two words of a row each) within its wavefront
+template <int SW>
+struct BfsTeam {
+    static constexpr uint32_t L = SW / 2;
+    uint32_t lane, tl, base;
+    u64 mask;
+    __device__ BfsTeam()
+    {
+        lane = threadIdx.x & 63u;
+        tl = lane % L;
+        base = lane - tl;
+        mask = (L == 64 ? ~0ull : ((1ull << L) - 1)) << base;
     }
-    for (; e < b1; e += 64) g |= frontier[nbr[e]];
-    return g;
-}
+    __device__ bool any(bool p) const { return (__ballot(p) & mask) != 0; }
+    __device__ bool all(bool p) const { return (__ballot(p) & mask) == mask; }
+};
 
-// Pull form of one level, for symmetric CSRs (u -> v present iff v -> u): every node
-// that some source has not reached ORs the frontier words of its neighbours.  No
-// atomics; a node whose unreached sources all appear stops early.  Lane per node of
-// degree <= 64, whole wavefront per node of degree <= hub_deg (as in the push); the
-// larger ones are k_bfs_hubs' (their next[] word is left at the 0 that apply wrote).
-__global__ __launch_bounds__(kBfsBlock) void k_bfs_pull(const uint32_t *__restrict__ off, const uint32_t *__restrict__ nbr,
-                                                        const uint64_t *__restrict__ frontier,
-                                                        const uint64_t *__restrict__ visited, uint64_t *next, uint32_t n,
-                                                        uint64_t full, uint32_t hub_deg)
+// got |= the frontier rows of in[0 .. len), this lane's two words; leaves once the team has
+// every wanted bit.  The team reads L ids and their flags at a time and then the flagged
+// rows, four loads in flight.
+template <int SW>
+__device__ __forceinline__ void bfs_pull_range(const BfsTeam<SW> &t, const uint32_t *__restrict__ in,
+                                               uint32_t len, const uint8_t *__restrict__ flag,
+                                               const ulonglong2 *__restrict__ rows, ulonglong2 want, ulonglong2 &got)
 {
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t waves = gridDim.x * (kBfsBlock / 64);
-    for (uint32_t base = (blockIdx.x * (kBfsBlock / 64) + threadIdx.x / 64) * 64; base < n; base += waves * 64) {
-        const uint32_t v = base + lane;  // uniform loop bound: every lane takes part in the ballot
-        uint64_t want = 0;                // sources that have not reached v
-        uint32_t e0 = 0, e1 = 0;
-        if (v < n) {
-            want = full & ~visited[v];
-            if (want) {
-                e0 = off[v];
-                e1 = off[v + 1];
-            }
-        }
-        uint64_t got = 0;
-        if (e1 - e0 <= 64) {
-            // 8 arcs per step, loads issued together; the early stop is checked per step
-            constexpr uint32_t B = 8;
-            for (uint64_t e = e0; e < e1 && (got & want) != want; e += B) {
-                uint32_t w[B];
+    constexpr uint32_t L = BfsTeam<SW>::L;
+    // ids per trip: a narrow team takes several each, so that its loads overlap
+    constexpr uint32_t K = L >= 4 ? 1 : 4 / L;
+    for (uint32_t e = 0; e < len; e += L * K) {
+        uint32_t id[K];
+        bool f[K];
 #pragma unroll
-                for (uint32_t j = 0; j < B; ++j) w[j] = e + j < e1 ? nbr[e + j] : 0u;
+        for (uint32_t k = 0; k < K; ++k) id[k] = e + k * L + t.tl < len ? in[e + k * L + t.tl] : ~0u;
 #pragma unroll
-                for (uint32_t j = 0; j < B; ++j)
-                    if (e + j < e1) got |= frontier[w[j]];
-            }
-        }
-        if (v < n && e1 - e0 <= 64) next[v] = got & want;
-        unsigned long long big = __ballot(e1 - e0 > 64 && e1 - e0 <= hub_deg);
-        while (big) {
-            const int i = __ffsll(big) - 1;
-            big &= big - 1;
-            const uint32_t b0 = (uint32_t)__shfl((int)e0, i), b1 = (uint32_t)__shfl((int)e1, i);
-            const uint64_t wi = (uint64_t)__shfl((long long)want, i);
-            uint64_t g = hb_bfs_or_range(nbr, frontier, b0, b1, lane);
+        for (uint32_t k = 0; k < K; ++k) f[k] = id[k] != ~0u && flag[id[k]];
+        if constexpr (L == 1) {
 #pragma unroll
-            for (int o = 1; o < 64; o <<= 1) g |= (uint64_t)__shfl_xor((long long)g, o);
-            if ((int)lane == i) next[base + (uint32_t)i] = g & wi;
-        }
-    }
-}
-
-// The lists of nodes of degree > hub_deg, cut into chunks (hub_node[c], arcs
-// [hub_beg[c], hub_end[c])), one wavefront per chunk.  Pull: a chunk ORs its frontier
-// words and ORs the bits its hub still wants into next[hub] (zero before the level).
-// Push: a chunk of a frontier hub pushes the hub's word along its arcs.
-template <bool kPull>
-__global__ __launch_bounds__(kBfsBlock) void k_bfs_hubs(const uint32_t *__restrict__ nbr,
-                                                        const uint32_t *__restrict__ hub_node,
-                                                        const uint32_t *__restrict__ hub_beg,
-                                                        const uint32_t *__restrict__ hub_end, uint32_t chunks,
-                                                        const uint64_t *__restrict__ frontier,
-                                                        const uint64_t *__restrict__ visited, uint64_t *next,
-                                                        uint64_t full)
-{
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t waves = gridDim.x * (kBfsBlock / 64);
-    for (uint32_t c = blockIdx.x * (kBfsBlock / 64) + threadIdx.x / 64; c < chunks; c += waves) {
-        const uint32_t v = hub_node[c], b0 = hub_beg[c], b1 = hub_end[c];
-        if (kPull) {
-            const uint64_t want = full & ~visited[v];
-            if (!want) continue;
-            uint64_t g = hb_bfs_or_range(nbr, frontier, b0, b1, lane);
-#pragma unroll
-            for (int o = 1; o < 64; o <<= 1) g |= (uint64_t)__shfl_xor((long long)g, o);
-            if (lane == 0 && (g & want)) atomicOr((unsigned long long *)&next[v], (unsigned long long)(g & want));
+            for (uint32_t k = 0; k < K; ++k)
+                if (f[k]) {
+                    const ulonglong2 r = rows[id[k]];
+                    got.x |= r.x;
+                    got.y |= r.y;
+                }
         } else {
-            const uint64_t f = frontier[v];
-            if (!f) continue;
-            for (uint32_t e = b0 + lane; e < b1; e += 64) hb_bfs_push_arc(visited, next, nbr[e], f);
-        }
-    }
-}
-
-// newly = next & ~visited; visited |= newly; frontier = newly; per-source counts of
-// newly (one ballot per bit lane per wavefront) and the arcs of the new frontier's
-// nodes: the block's 65 values go to part[65 * block], summed by sum_columns; dist
-// (optional, [node][64] u16) records the level of each newly set bit
-constexpr uint32_t kBfsCols = 65;
-
-__global__ __launch_bounds__(kBfsBlock) void k_bfs_apply(const uint32_t *__restrict__ off, uint64_t *frontier,
-                                                         uint64_t *visited, uint64_t *next, uint16_t *dist, uint32_t n,
-                                                         uint32_t level, unsigned long long *part)
-{
-    __shared__ unsigned long long wc[kBfsBlock / 64][kBfsCols];
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    unsigned long long mine = 0;  // count of bit `lane` over this wavefront's nodes
-    unsigned long long farcs = 0;  // arcs of this lane's nodes that joined the frontier
-    // the loop bound is uniform across the wavefront, so every lane takes part in the ballots
-    for (uint32_t base = blockIdx.x * blockDim.x; base < n; base += gridDim.x * blockDim.x) {
-        const uint32_t v = base + threadIdx.x;
-        uint64_t newly = 0;
-        if (v < n) {
-            const uint64_t nx = next[v];
-            if (nx) {
-                const uint64_t vis = visited[v];
-                newly = nx & ~vis;
-                next[v] = 0ull;
-                if (newly) {
-                    visited[v] = vis | newly;
-                    farcs += off[v + 1] - off[v];
-                    if (dist) {  // the row's 16-byte pieces holding newly set bits, read-modify-write
-                        uint4 *row = (uint4 *)(dist + (size_t)v * 64);
 #pragma unroll
-                        for (int j = 0; j < 8; ++j) {
-                            const uint32_t bits = (uint32_t)(newly >> (8 * j)) & 0xffu;
-                            if (!bits) continue;
-                            uint4 w = row[j];
-                            uint32_t q[4] = {w.x, w.y, w.z, w.w};
+            for (uint32_t k = 0; k < K; ++k) {
+                u64 m = __ballot(f[k]) & t.mask;
+                while (m) {
+                    uint32_t v[4];
 #pragma unroll
-                            for (int h = 0; h < 8; ++h) {
-                                const uint32_t sh = 16u * (uint32_t)(h & 1);
-                                if ((bits >> h) & 1u) q[h >> 1] = (q[h >> 1] & ~(0xffffu << sh)) | (level << sh);
-                            }
-                            row[j] = make_uint4(q[0], q[1], q[2], q[3]);
-                        }
+                    for (int q = 0; q < 4; ++q) {  // past the last flagged id: the last again
+                        v[q] = (uint32_t)__shfl((int)id[k], __ffsll(m) - 1);
+                        if (m & (m - 1)) m &= m - 1;
+                        else if (q == 3) m = 0;
+                    }
+                    ulonglong2 r[4];
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) r[q] = rows[(size_t)v[q] * L + t.tl];
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        got.x |= r[q].x;
+                        got.y |= r[q].y;
                     }
                 }
             }
-            frontier[v] = newly;
         }
-        if (__ballot(newly != 0ull)) {
-            for (int k = 0; k < 64; ++k) {
-                const unsigned long long m = __ballot((newly >> k) & 1ull);
-                if ((int)lane == k) mine += (unsigned long long)__popcll(m);
-            }
-        }
-    }
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) farcs += (unsigned long long)__shfl_xor((long long)farcs, o);
-    wc[wave][lane] = mine;
-    if (lane == 0) wc[wave][64] = farcs;
-    __syncthreads();
-    if (threadIdx.x < kBfsCols) {
-        unsigned long long s = 0;
-        for (int w = 0; w < kBfsBlock / 64; ++w) s += wc[w][threadIdx.x];
-        part[kBfsCols * blockIdx.x + threadIdx.x] = s;
+        if (t.all((want.x & ~got.x) == 0 && (want.y & ~got.y) == 0)) return;
     }
 }
 
+// the planes of two words (at index `at` in ulonglong2) whose sources `got` were found in
+// `level`; `first`: none was found there before, so the planes hold nothing yet
+__device__ __forceinline__ void bfs_keep(const BfsDev &b, size_t at, bool first, ulonglong2 got, uint32_t level)
+{
+#pragma unroll
+    for (uint32_t k = 0; k < kBfsPlanes; ++k) {
+        ulonglong2 *p = (ulonglong2 *)(b.plane + k * b.plane_stride) + at;
+        const bool bit = (level >> k) & 1u;
+        if (first) {
+            *p = bit ? got : make_ulonglong2(0, 0);
+        } else if (bit) {
+            const ulonglong2 x = *p;
+            *p = make_ulonglong2(x.x | got.x, x.y | got.y);
+        }
+    }
+}
+
+// a node's newly found sources: visited, its row (both at index `at` in ulonglong2), its flag
+template <int SW>
+__device__ __forceinline__ void bfs_found(const BfsDev &b, const BfsTeam<SW> &t, size_t at, u64 *rows, uint8_t *flag,
+                                          ulonglong2 seen, ulonglong2 got, uint32_t level)
+{
+    const bool any = t.any((got.x | got.y) != 0);
+    if (any) {
+        ((ulonglong2 *)rows)[at] = got;
+        ((ulonglong2 *)b.visited)[at] = make_ulonglong2(seen.x | got.x, seen.y | got.y);
+        if (b.plane) bfs_keep(b, at, (seen.x | seen.y) == 0, got, level);
+    }
+    if (t.tl == 0) *flag = any ? 1 : 0;
+}
+
+// the planes after level 1, whose rows k_bfs_sources wrote
+template <int SW>
+__global__ __launch_bounds__(kBfsBlock) void k_bfs_keep_first(BfsDev b, BfsLevel l)
+{
+    constexpr uint32_t L = SW / 2;
+    const uint32_t slice = blockIdx.y;
+    const uint64_t threads = (uint64_t)gridDim.x * kBfsBlock, all = (uint64_t)b.n * L;
+    for (uint64_t i = (uint64_t)blockIdx.x * kBfsBlock + threadIdx.x; i < all; i += threads) {
+        if (!l.flag[(size_t)slice * b.npad + i / L]) continue;
+        const size_t at = (size_t)slice * b.n * L + i;
+        bfs_keep(b, at, true, ((const ulonglong2 *)l.rows)[at], 1);
+    }
+}
+
+// One level for the nodes with at most kBfsHubDeg tails: a team of SW / 2 lanes per node.
+template <int SW>
+__global__ __launch_bounds__(kBfsBlock) void k_bfs_pull(BfsDev b, BfsLevel prev, BfsLevel next, uint32_t level)
+{
+    constexpr uint32_t L = SW / 2;
+    const uint32_t slice = blockIdx.y;
+    if (b.done[slice]) return;
+    const BfsTeam<SW> t;
+    const size_t at = (size_t)slice * b.n, fat = (size_t)slice * b.npad;
+    const uint8_t *flag = prev.flag + fat;
+    const ulonglong2 *rows = (const ulonglong2 *)prev.rows + at * L;
+    const ulonglong2 live = ((const ulonglong2 *)b.live)[(size_t)slice * L + t.tl];
+    const uint32_t teams = gridDim.x * (kBfsBlock / L);
+    for (uint32_t v = blockIdx.x * (kBfsBlock / L) + threadIdx.x / L; v < b.n; v += teams) {
+        const uint32_t e0 = b.ioff[v], e1 = b.ioff[v + 1];
+        if (e1 - e0 > kBfsHubDeg) continue;  // k_bfs_hub_tasks and k_bfs_hubs
+        const size_t here = (at + v) * L + t.tl;
+        const ulonglong2 seen = ((const ulonglong2 *)b.visited)[here];
+        const ulonglong2 want = make_ulonglong2(live.x & ~seen.x, live.y & ~seen.y);
+        ulonglong2 got = make_ulonglong2(0, 0);
+        if (t.any((want.x | want.y) != 0)) bfs_pull_range<SW>(t, b.inbr + e0, e1 - e0, flag, rows, want, got);
+        got.x &= want.x;
+        got.y &= want.y;
+        bfs_found<SW>(b, t, here, next.rows, next.flag + fat + v, seen, got, level);
+    }
+}
+
+// The lists of hubs, cut into tasks: one wavefront per task, its teams every 64 / L-th run
+// of ids, their words ORed into the task's row of `part`.
+template <int SW>
+__global__ __launch_bounds__(kBfsBlock) void k_bfs_hub_tasks(BfsDev b, BfsLevel prev)
+{
+    constexpr uint32_t L = SW / 2, TEAMS = 64 / L;
+    const uint32_t slice = blockIdx.y;
+    if (b.done[slice]) return;
+    const BfsTeam<SW> t;
+    const size_t at = (size_t)slice * b.n, fat = (size_t)slice * b.npad;
+    const ulonglong2 live = ((const ulonglong2 *)b.live)[(size_t)slice * L + t.tl];
+    const uint32_t waves = gridDim.x * (kBfsBlock / 64), team = t.lane / L;
+    for (uint32_t k = blockIdx.x * (kBfsBlock / 64) + threadIdx.x / 64; k < b.tasks; k += waves) {
+        const ulonglong2 seen = ((const ulonglong2 *)b.visited)[(at + b.task_node[k]) * L + t.tl];
+        const ulonglong2 want = make_ulonglong2(live.x & ~seen.x, live.y & ~seen.y);
+        if (!t.any((want.x | want.y) != 0)) continue;  // k_bfs_hubs does not read its row either
+        const uint32_t e0 = b.task_beg[k], len = b.task_end[k] - e0, per = (len + TEAMS - 1) / TEAMS;
+        const uint32_t lo = min(len, team * per), hi = min(len, lo + per);
+        ulonglong2 got = make_ulonglong2(0, 0);
+        bfs_pull_range<SW>(t, b.inbr + e0 + lo, hi - lo, prev.flag + fat, (const ulonglong2 *)prev.rows + at * L, want, got);
+#pragma unroll
+        for (uint32_t s = L; s < 64; s <<= 1) {
+            got.x |= __shfl_xor(got.x, s);
+            got.y |= __shfl_xor(got.y, s);
+        }
+        if (team == 0) ((ulonglong2 *)b.part)[((size_t)slice * b.tasks + k) * L + t.tl] = got;
+    }
+}
+
+template <int SW>
+__global__ __launch_bounds__(kBfsBlock) void k_bfs_hubs(BfsDev b, BfsLevel next, uint32_t level)
+{
+    constexpr uint32_t L = SW / 2;
+    const uint32_t slice = blockIdx.y;
+    if (b.done[slice]) return;
+    const BfsTeam<SW> t;
+    const size_t at = (size_t)slice * b.n, fat = (size_t)slice * b.npad;
+    const ulonglong2 live = ((const ulonglong2 *)b.live)[(size_t)slice * L + t.tl];
+    const uint32_t teams = gridDim.x * (kBfsBlock / L);
+    for (uint32_t h = blockIdx.x * (kBfsBlock / L) + threadIdx.x / L; h < b.hubs; h += teams) {
+        const uint32_t v = b.hub_node[h];
+        const size_t here = (at + v) * L + t.tl;
+        const ulonglong2 seen = ((const ulonglong2 *)b.visited)[here];
+        const ulonglong2 want = make_ulonglong2(live.x & ~seen.x, live.y & ~seen.y);
+        ulonglong2 got = make_ulonglong2(0, 0);
+        if (t.any((want.x | want.y) != 0))
+            for (uint32_t k = b.hub_first[h]; k < b.hub_first[h + 1]; ++k) {
+                const ulonglong2 r = ((const ulonglong2 *)b.part)[((size_t)slice * b.tasks + k) * L + t.tl];
+                got.x |= r.x;
+                got.y |= r.y;
+            }
+        got.x &= want.x;
+        got.y &= want.y;
+        bfs_found<SW>(b, t, here, next.rows, next.flag + fat + v, seen, got, level);
+    }
+}
+
+// full adder over 64 columns at once
+__device__ __forceinline__ void bfs_csa(u64 &hi, u64 &lo, u64 a, u64 b2, u64 c)
+{
+    const u64 u = a ^ b2;
+    hi = (a & b2) | (u & c);
+    lo = u ^ c;
+}
+
+// The newly found nodes of every source, per chunk of kBfsChunk nodes.  A thread adds one
+// word of a chunk's rows, eight rows at a time, into bit-sliced counters (plane k holds bit
+// k of 64 counts), then transposes the planes into 64 bytes: 13 operations per 64 bits
+// added, where a ballot per column takes 256 per wavefront.
+template <int SW>
+__global__ __launch_bounds__(kBfsBlock) void k_bfs_count(BfsDev b, BfsLevel l)
+{
+    const uint32_t slice = blockIdx.y, chunks = bfs_chunks(b.n);
+    if (b.done[slice]) return;
+    const uint32_t w = threadIdx.x % SW;
+    const size_t at = (size_t)slice * b.n;
+    const uint32_t per_grid = gridDim.x * (kBfsBlock / SW);
+    for (uint32_t c = blockIdx.x * (kBfsBlock / SW) + threadIdx.x / SW; c < chunks; c += per_grid) {
+        u64 p[8] = {};
+        const uint32_t v1 = min(b.n, (c + 1) * kBfsChunk);
+        bool any = false;
+        for (uint32_t v = c * kBfsChunk; v < v1; v += 8) {
+            // eight flags of 0 or 1 as the low byte's bits, those past the last node dropped
+            const u64 f8 = *(const u64 *)(l.flag + (size_t)slice * b.npad + v) & 0x0101010101010101ull;
+            const uint32_t f = (uint32_t)((f8 * 0x0102040810204080ull) >> 56) & (0xffu >> (8 - min(8u, v1 - v)));
+            if (!f) continue;
+            any = true;
+            u64 x[8];
+#pragma unroll
+            for (uint32_t k = 0; k < 8; ++k) x[k] = (f >> k) & 1u ? l.rows[(at + v + k) * SW + w] : 0ull;
+            u64 two_a, two_b, four_a, four_b, eight;
+            bfs_csa(two_a, p[0], p[0], x[0], x[1]);
+            bfs_csa(two_b, p[0], p[0], x[2], x[3]);
+            bfs_csa(four_a, p[1], p[1], two_a, two_b);
+            bfs_csa(two_a, p[0], p[0], x[4], x[5]);
+            bfs_csa(two_b, p[0], p[0], x[6], x[7]);
+            bfs_csa(four_b, p[1], p[1], two_a, two_b);
+            bfs_csa(eight, p[2], p[2], four_a, four_b);
+#pragma unroll
+            for (int k = 3; k < 8; ++k) {
+                const u64 carry = p[k] & eight;
+                p[k] ^= eight;
+                eight = carry;
+            }
+        }
+        const size_t ci = (size_t)slice * chunks + c;
+        if (w == 0) l.any[ci] = any ? 1 : 0;
+        if (!any) continue;
+        u64 *out = (u64 *)(l.count + (ci * SW + w) * 64);
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {  // columns 8 q .. 8 q + 7: byte k of x from plane k, transposed
+            u64 x = 0;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) x |= ((p[k] >> (8 * q)) & 0xffull) << (8 * k);
+            u64 s = (x ^ (x >> 7)) & 0x00AA00AA00AA00AAull;
+            x ^= s ^ (s << 7);
+            s = (x ^ (x >> 14)) & 0x0000CCCC0000CCCCull;
+            x ^= s ^ (s << 14);
+            s = (x ^ (x >> 28)) & 0x00000000F0F0F0F0ull;
+            x ^= s ^ (s << 28);
+            out[q] = x;
+        }
+    }
+}
+
+// the chunk counts summed per source into b.found: four columns per thread, the chunks
+// split over blockIdx.x
+template <int SW>
+__global__ __launch_bounds__(kBfsBlock) void k_bfs_totals(BfsDev b, BfsLevel l, uint32_t splits)
+{
+    constexpr uint32_t QUADS = 16 * SW;  // four columns each
+    const uint32_t slice = blockIdx.y, chunks = bfs_chunks(b.n);
+    if (b.done[slice]) return;
+    for (uint32_t i = blockIdx.x * kBfsBlock + threadIdx.x; i < splits * QUADS; i += gridDim.x * kBfsBlock) {
+        const uint32_t quad = i % QUADS, part = i / QUADS;
+        uint32_t s[4] = {};
+        for (uint32_t c = part; c < chunks; c += splits) {
+            const size_t ci = (size_t)slice * chunks + c;
+            if (!l.any[ci]) continue;
+            const uint32_t x = ((const uint32_t *)l.count)[ci * QUADS + quad];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) s[k] += (x >> (8 * k)) & 0xffu;
+        }
+        uint32_t *f = b.found + ((size_t)slice * QUADS + quad) * 4;
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (s[k]) atomicAdd(f + k, s[k]);
+    }
+}
+
+// end of a level, one block per slice: the per-source sums, the sources still searching
+template <int SW>
+__global__ __launch_bounds__(1024) void k_bfs_level(BfsDev b, uint32_t level)
+{
+    const uint32_t slice = blockIdx.x;
+    if (b.done[slice]) return;
+    __shared__ uint32_t any;
+    if (threadIdx.x == 0) any = 0;
+    __syncthreads();
+    for (uint32_t c = threadIdx.x; c < 64 * SW; c += blockDim.x) {
+        const size_t i = (size_t)slice * 64 * SW + c;
+        const uint32_t f = b.found[i];
+        b.found[i] = 0;
+        b.reach[i] += f;
+        b.total[i] += (u64)level * f;
+        const u64 m = __ballot(f != 0);
+        if (c % 64 == 0) {
+            b.live[(size_t)slice * SW + c / 64] = m;
+            if (m) any = 1;
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        if (any) b.levels[slice] = level;
+        else b.done[slice] = 1;
+    }
+}
+
+// distances of the nodes found in the level, u16 [word][n][64]: a thread per 8 sources
+template <int SW>
+__global__ __launch_bounds__(kBfsBlock) void k_bfs_dist(BfsDev b, BfsLevel l, uint32_t level, uint16_t *dist)
+{
+    const uint32_t slice = blockIdx.y;
+    if (b.done[slice]) return;
+    const size_t at = (size_t)slice * b.n;
+    const uint64_t threads = (uint64_t)gridDim.x * kBfsBlock, all = (uint64_t)b.n * SW * 8;
+    for (uint64_t i = (uint64_t)blockIdx.x * kBfsBlock + threadIdx.x; i < all; i += threads) {
+        const uint32_t v = (uint32_t)(i / (SW * 8)), q = (uint32_t)(i % (SW * 8)), w = q / 8;
+        if (!l.flag[(size_t)slice * b.npad + v]) continue;
+        const uint32_t bits = (uint32_t)(l.rows[(at + v) * SW + w] >> (8 * (q % 8))) & 0xffu;
+        if (!bits) continue;
+        uint4 *row = (uint4 *)(dist + (((size_t)slice * SW + w) * b.n + v) * 64) + q % 8;
+        const uint4 x = *row;
+        uint32_t r[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+        for (int h = 0; h < 8; ++h) {
+            const uint32_t sh = 16u * (uint32_t)(h & 1);
+            if ((bits >> h) & 1u) r[h >> 1] = (r[h >> 1] & ~(0xffffu << sh)) | (level << sh);
+        }
+        *row = make_uint4(r[0], r[1], r[2], r[3]);
+    }
+}
+
+// the value of x in lane j (wave-uniform)
+__device__ __forceinline__ double bfs_lane(double x, int j)
+{
+    const u64 b = (u64)__double_as_longlong(x);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)b, j);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(b >> 32), j);
+    return __longlong_as_double((long long)(((u64)hi << 32) | lo));
+}
+
+// inv_sum[source] = Σ_{v=0..n-1} inv[d(v)] as the sequential f64 sum in node order rounds
+// it, inv[d] = 1/d, from the kept levels.  One wavefront per source.
+//
+// A chain of n dependent adds takes 28 ns each.  But while the running sum stays within one
+// binade [2^E, 2^(E+1)) its ulp is fixed, u = 2^(E-52), the sum is a multiple A u of it, and
+// adding x rounds to A + round(x / u): a whole number that does not depend on A unless x / u
+// lies halfway between two.  So a run of nodes adds Σ_d count_d round(2^.. / d) in any
+// order as long as the result stays below 2^53 and no distance in it is a halfway case.
+// The wavefront adds 64 chunks of kBfsChunk nodes at a time from the counts and their prefix
+// sums; only a chunk in which the sum leaves its binade (some log2 n of them) or that holds a
+// halfway case (the first binades) is replayed node by node.
+// R-MAT-20, 2,048 sources: 0.87 ms, against 29.7 ms as chains.
+template <int SW>
+__global__ __launch_bounds__(kBfsBlock) void k_bfs_harmonic(BfsDev b, const uint8_t *__restrict__ count,
+                                                            size_t count_stride, const uint8_t *__restrict__ any,
+                                                            size_t any_stride, const double *__restrict__ inv,
+                                                            uint32_t slices, double *__restrict__ out)
+{
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (kBfsBlock / 64) + threadIdx.x / 64);
+    const uint32_t slice = wave / (64 * SW), col = wave % (64 * SW);
+    if (slice >= slices || (uint64_t)b.src0 + wave >= b.src_end) return;
+    const uint32_t levels = b.levels[slice], chunks = bfs_chunks(b.n);
+    const size_t at = (size_t)slice * b.n, cat = (size_t)slice * chunks;
+    // lane d - 1 holds 1/d and, for the current binade, round(x / u) and whether it is a tie
+    const double x = lane < levels ? inv[lane + 1] : 0.0;
+    const u64 xb = (u64)__double_as_longlong(x);
+    const int xe = (int)(xb >> 52);  // biased exponent; 1/d is normal
+    const u64 xm = (xb & ((1ull << 52) - 1)) | (1ull << 52);
+    double acc = 0.0;
+    for (uint32_t base = 0; base < chunks; base += 64) {
+        const uint32_t c = base + lane;
+        uint32_t cnt[(kBfsKeep + 3) / 4] = {};  // this lane's chunk: nodes at distance 1 .. levels, a byte each
+#pragma unroll
+        for (uint32_t d = 0; d < kBfsKeep; ++d)
+            if (d < levels && c < chunks && any[d * any_stride + cat + c])
+                cnt[d / 4] |= (uint32_t)count[d * count_stride + (cat + c) * 64 * SW + col] << (8 * (d % 4));
+        uint32_t pos = 0;  // chunks base .. base + pos - 1 are in the sum
+        const uint32_t end = min(64u, chunks - base);
+        while (pos < end) {
+            const u64 ab = (u64)__double_as_longlong(acc);
+            const int ae = (int)(ab >> 52);
+            const u64 am = (ab & ((1ull << 52) - 1)) | (1ull << 52);
+            u64 q = 0;
+            bool tie = false;
+            if (lane < levels) {
+                const int sh = ae - xe;
+                if (acc == 0.0 || sh < 0) tie = true;  // leaves the binade at once
+                else if (sh == 0) q = xm;
+                else if (sh <= 53) {
+                    const u64 half = 1ull << (sh - 1);
+                    tie = (xm & (2 * half - 1)) == half;
+                    q = (xm + half) >> sh;
+                }
+            }
+            const u64 ties = __ballot(tie);
+            u64 s = 0;
+            bool stop = false;
+#pragma unroll
+            for (uint32_t d = 0; d < kBfsKeep; ++d)
+                if (d < levels) {
+                    const uint32_t k = (cnt[d / 4] >> (8 * (d % 4))) & 0xffu;
+                    s += k * __shfl(q, (int)d);
+                    stop = stop || (k && ((ties >> d) & 1u));
+                }
+            s = lane < pos || lane >= end ? 0ull : s < (1ull << 54) ? s : 1ull << 54;
+            u64 sum = s;  // inclusive prefix; 64 terms of at most 2^54
+#pragma unroll
+            for (uint32_t o = 1; o < 64; o <<= 1) {
+                const u64 y = __shfl_up(sum, o);
+                if (lane >= o) sum += y;
+            }
+            stop = lane >= pos && lane < end && (stop || am + sum >= (1ull << 53));
+            const u64 m = __ballot(stop);
+            const uint32_t first = m ? (uint32_t)(__ffsll(m) - 1) : end;
+            if (first > pos && acc != 0.0) {  // the sum before chunk `first`, an exact multiple of u
+                const u64 a = am + __shfl(sum, (int)first - 1);
+                acc = __longlong_as_double((long long)(((u64)ae << 52) | (a & ((1ull << 52) - 1))));
+            }
+            pos = first;
+            if (first == end) break;
+            // node by node: lane i takes nodes i and 64 + i of the chunk
+            const uint32_t v0 = (base + first) * kBfsChunk;
+#pragma unroll
+            for (uint32_t h = 0; h < kBfsChunk; h += 64) {
+                const uint32_t v = v0 + h + lane;
+                const size_t word = (at + v) * SW + col / 64;
+                uint32_t dist = 0;
+                if (v < b.n && ((b.visited[word] >> (col % 64)) & 1ull))
+#pragma unroll
+                    for (uint32_t k = 0; k < kBfsPlanes; ++k)
+                        dist |= (uint32_t)((b.plane[k * b.plane_stride + word] >> (col % 64)) & 1ull) << k;
+                const double term = __shfl(x, (int)(dist ? dist - 1 : 0));
+                u64 r = __ballot(dist != 0);
+                while (r) {
+                    acc = __dadd_rn(acc, bfs_lane(term, __ffsll(r) - 1));
+                    r &= r - 1;
+                }
+            }
+            ++pos;
+        }
+    }
+    if (lane == 0) out[wave] = acc;
+}
+
+// The harmonic sums of searches of more than kBfsKeep levels, add by add:
 // inv_sum[64 b + k] = Σ_{v=0..n-1} inv[dist_b[v][k]] as a sequential f64 sum in node
 // order, dist_b = dist + b n 64 the distances of pass b of a group; inv[0] = 0
 // (unreached), inv[d] = 1/d for d < entries.  One block per pass: the adds of a source
@@ -363,6 +681,28 @@ __global__ __launch_bounds__(kInvBlock) void k_bfs_inv_sum(const uint16_t *__res
     if (tid < counts[b]) out[64 * b + tid] = acc;
 }
 
+// the tail of every arc, a wavefront per list
+__global__ __launch_bounds__(kBfsBlock) void k_bfs_tails(const uint32_t *__restrict__ off, uint32_t n, uint32_t *tail)
+{
+    const uint32_t lane = threadIdx.x & 63u, waves = gridDim.x * (kBfsBlock / 64);
+    for (uint32_t u = blockIdx.x * (kBfsBlock / 64) + threadIdx.x / 64; u < n; u += waves) {
+        const uint32_t e1 = off[u + 1];
+        for (uint64_t e = (uint64_t)off[u] + lane; e < e1; e += 64) tail[e] = u;
+    }
+}
+
+// ioff from the ascending heads: arc e writes the offsets of the nodes after its predecessor's
+// head up to its own, the last arc those of the nodes past it too
+__global__ __launch_bounds__(kBfsBlock) void k_bfs_offsets(const uint32_t *__restrict__ head, uint64_t arcs,
+                                                           uint32_t n, uint32_t *ioff)
+{
+    for (uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; e < arcs; e += (uint64_t)gridDim.x * blockDim.x) {
+        for (uint64_t v = e ? (uint64_t)head[e - 1] + 1 : 0; v <= head[e]; ++v) ioff[v] = (uint32_t)e;
+        if (e + 1 == arcs)
+            for (uint64_t v = (uint64_t)head[e] + 1; v <= n; ++v) ioff[v] = (uint32_t)arcs;
+    }
+}
+
 }  // namespace hb
 
 namespace {
@@ -379,9 +719,11 @@ int efail(int code, const char *fmt, ...)
 
 struct Scoped {
     void *p = nullptr;
-    ~Scoped()
+    ~Scoped() { release(); }
+    void release()
     {
         if (p) (void)hipFree(p);
+        p = nullptr;
     }
 };
 }  // namespace
@@ -395,6 +737,199 @@ struct Scoped {
     } while (0)
 
 namespace hb {
+namespace {
+
+constexpr uint64_t kBfsBudget = 16ull << 30;  // device memory of one group of slices
+// What a group needs is kept between calls up to this much, one block per device: the driver
+// clears freed device memory at some 40 GB/s before it hands it out again, so a call of 12 ms
+// that takes and frees 5 GB soon waits 130 ms for it.  Given back as soon as an allocation
+// of the engine fails (release_held).  A block in use belongs to one call; a second call at the same time takes
+// memory of its own.
+constexpr uint64_t kBfsHold = 2ull << 30;
+constexpr int kBfsDevices = 16;
+
+struct BfsHeld {
+    std::mutex mu;
+    void *p[kBfsDevices] = {};
+    size_t bytes[kBfsDevices] = {};
+} g_bfs_held;
+
+struct BfsMemory {
+    void *p = nullptr;
+    size_t bytes = 0;
+    int device = -1;
+    hipStream_t stream = nullptr;
+
+    explicit BfsMemory(hipStream_t s) : stream(s) {}
+    ~BfsMemory() { release(); }
+    hipError_t take(size_t want)
+    {
+        if (device < 0) {
+            const hipError_t e = hipGetDevice(&device);
+            if (e != hipSuccess) return e;
+        }
+        if (device < kBfsDevices) {
+            std::lock_guard<std::mutex> lock(g_bfs_held.mu);
+            void *&held = g_bfs_held.p[device];
+            if (held && g_bfs_held.bytes[device] >= want) {
+                p = held;
+                bytes = g_bfs_held.bytes[device];
+                held = nullptr;
+                return hipSuccess;
+            }
+            if (held) (void)hipFree(held);  // too small: its place is for this one
+            held = nullptr;
+        }
+        const hipError_t e = hipMalloc(&p, want);
+        if (e != hipSuccess) p = nullptr;
+        else bytes = want;
+        return e;
+    }
+    void release()
+    {
+        if (!p) return;
+        (void)hipStreamSynchronize(stream);  // also where a call ends with an error
+        if (device < kBfsDevices && bytes <= kBfsHold) {
+            std::lock_guard<std::mutex> lock(g_bfs_held.mu);
+            if (!g_bfs_held.p[device]) {
+                g_bfs_held.p[device] = p;
+                g_bfs_held.bytes[device] = bytes;
+                p = nullptr;
+                return;
+            }
+        }
+        (void)hipFree(p);
+        p = nullptr;
+    }
+};
+
+// How a group of searches runs: kSums counts only; kKeep keeps distances and counts for
+// k_bfs_harmonic; kLong records u16 distances for k_bfs_inv_sum
+enum class BfsMode { kSums, kKeep, kLong };
+
+// the group's one allocation, cut up
+struct BfsPlan {
+    uint32_t sw = 0, slices = 0;
+    size_t rows_stride = 0, flag_stride = 0, count_stride = 0, any_stride = 0;  // per level
+    uint32_t counts = 0;  // count buffers; rows and flags have two, by level parity
+    size_t bytes = 0;
+    size_t o_vis = 0, o_rows = 0, o_flag = 0, o_count = 0, o_any = 0, o_part = 0, o_plane = 0, o_dist = 0, o_src = 0;
+    bool keep = false;
+};
+
+BfsPlan bfs_plan(uint32_t n, uint32_t tasks, uint32_t sw, uint32_t slices, BfsMode mode)
+{
+    BfsPlan p;
+    p.sw = sw;
+    p.slices = slices;
+    p.keep = mode == BfsMode::kKeep;
+    p.counts = p.keep ? kBfsKeep : 1;
+    const size_t chunks = (n + kBfsChunk - 1) / kBfsChunk, npad = chunks * kBfsChunk;
+    auto take = [&](size_t bytes) {
+        const size_t at = p.bytes;
+        p.bytes += (bytes + 255) & ~(size_t)255;
+        return at;
+    };
+    p.rows_stride = (size_t)slices * n * sw;
+    p.flag_stride = (size_t)slices * npad;
+    p.any_stride = (size_t)slices * chunks;
+    p.count_stride = p.any_stride * 64 * sw;
+    p.o_vis = take(p.rows_stride * 8);
+    p.o_rows = take(p.rows_stride * 8 * 2);
+    p.o_flag = take(p.flag_stride * 2);
+    p.o_plane = take(p.keep ? p.rows_stride * 8 * kBfsPlanes : 0);
+    p.o_count = take(p.count_stride * p.counts);
+    p.o_any = take(p.any_stride * p.counts);
+    p.o_part = take((size_t)slices * tasks * sw * 8);
+    p.o_dist = take(mode == BfsMode::kLong ? p.rows_stride * 128 : 0);
+    // per source: reach, total, sum, found; per word: live, source count; per slice: done, levels
+    p.o_src = take((size_t)slices * (sw * (64 * 28 + 12) + 8));
+    return p;
+}
+
+struct BfsGroup {
+    BfsDev b{};
+    BfsLevel level0{};
+    BfsPlan plan;
+    uint16_t *dist = nullptr;
+    double *sums = nullptr;
+    uint32_t *word_count = nullptr;
+
+    BfsLevel level(uint32_t l) const  // of level l >= 1
+    {
+        const uint32_t i = (l - 1) % 2, c = (l - 1) % plan.counts;
+        return {level0.rows + i * plan.rows_stride, level0.flag + i * plan.flag_stride,
+                level0.count + c * plan.count_stride, level0.any + c * plan.any_stride};
+    }
+    void place(char *base, const BfsPlan &p)
+    {
+        plan = p;
+        const size_t src = (size_t)p.slices * 64 * p.sw, words = (size_t)p.slices * p.sw;
+        b.visited = (u64 *)(base + p.o_vis);
+        level0 = {(u64 *)(base + p.o_rows), (uint8_t *)(base + p.o_flag), (uint8_t *)(base + p.o_count),
+                  (uint8_t *)(base + p.o_any)};
+        b.part = (u64 *)(base + p.o_part);
+        b.plane = p.keep ? (u64 *)(base + p.o_plane) : nullptr;
+        b.plane_stride = p.rows_stride;
+        dist = (uint16_t *)(base + p.o_dist);
+        b.reach = (u64 *)(base + p.o_src);
+        b.total = b.reach + src;
+        sums = (double *)(b.total + src);
+        b.live = (u64 *)(sums + src);
+        b.found = (uint32_t *)(b.live + words);
+        word_count = b.found + src;
+        b.done = word_count + words;
+        b.levels = b.done + p.slices;
+    }
+};
+
+unsigned bfs_grid(uint64_t threads, uint32_t slices)
+{
+    const uint64_t cap = std::max<uint64_t>(512, 16384 / slices);
+    return (unsigned)std::max<uint64_t>(1, std::min<uint64_t>((threads + kBfsBlock - 1) / kBfsBlock, cap));
+}
+
+// levels from .. to of every slice; returns at once where a slice is done
+template <int SW>
+hipError_t bfs_levels(const BfsGroup &g, uint32_t from, uint32_t to, uint64_t source_arcs, BfsMode mode, hipStream_t s)
+{
+    const BfsDev &b = g.b;
+    const uint32_t slices = g.plan.slices, chunks = (b.n + kBfsChunk - 1) / kBfsChunk;
+    const uint32_t splits = std::min(chunks, std::max(1u, 256u / slices));
+    for (uint32_t l = from; l <= to; ++l) {
+        const BfsLevel next = g.level(l);
+        if (l == 1) {
+            k_bfs_sources<SW><<<dim3(bfs_grid(source_arcs, slices), slices), kBfsBlock, 0, s>>>(b, next);
+            if (b.plane)
+                k_bfs_keep_first<SW><<<dim3(bfs_grid((uint64_t)b.n * (SW / 2), slices), slices), kBfsBlock, 0, s>>>(b, next);
+        } else {
+            const BfsLevel prev = g.level(l - 1);
+            k_bfs_pull<SW><<<dim3(bfs_grid((uint64_t)b.n * (SW / 2), slices), slices), kBfsBlock, 0, s>>>(b, prev, next, l);
+            if (b.tasks) {
+                k_bfs_hub_tasks<SW><<<dim3(bfs_grid((uint64_t)b.tasks * 64, slices), slices), kBfsBlock, 0, s>>>(b, prev);
+                k_bfs_hubs<SW><<<dim3(bfs_grid((uint64_t)b.hubs * (SW / 2), slices), slices), kBfsBlock, 0, s>>>(b, next, l);
+            }
+        }
+        k_bfs_count<SW><<<dim3(bfs_grid((uint64_t)chunks * SW, slices), slices), kBfsBlock, 0, s>>>(b, next);
+        k_bfs_totals<SW><<<dim3(bfs_grid((uint64_t)splits * 16 * SW, slices), slices), kBfsBlock, 0, s>>>(b, next, splits);
+        k_bfs_level<SW><<<slices, std::min(1024, 64 * SW), 0, s>>>(b, l);
+        // a level that found nothing has marked its slice done and records nothing
+        if (mode == BfsMode::kLong)
+            k_bfs_dist<SW><<<dim3(bfs_grid((uint64_t)b.n * SW * 8, slices), slices), kBfsBlock, 0, s>>>(b, next, l, g.dist);
+    }
+    return hipGetLastError();
+}
+
+}  // namespace
+
+void release_held()
+{
+    std::lock_guard<std::mutex> lock(g_bfs_held.mu);
+    for (void *&p : g_bfs_held.p) {
+        if (p) (void)hipFree(p);
+        p = nullptr;
+    }
+}
 
 int exact_bfs(const uint32_t *off, const uint32_t *h_off, const uint32_t *nbr, uint32_t n, bool symmetric,
               uint64_t s_begin,
@@ -403,135 +938,208 @@ int exact_bfs(const uint32_t *off, const uint32_t *h_off, const uint32_t *nbr, u
     if (s_begin > s_end || s_end > n) return efail(HB_EINVAL, "hb_exact_bfs: sources [%llu, %llu) outside [0, %u)",
                                                    (unsigned long long)s_begin, (unsigned long long)s_end, n);
     if (s_begin == s_end) return HB_OK;
-    Scoped bits, cnt, dist, inv, sums, cnts;
-    const unsigned grid = (unsigned)std::min<uint64_t>((n + kBfsBlock - 1) / kBfsBlock, 4096);
-    // passes of 64 sources; with harmonic sums, the distances of up to `group` passes are
-    // kept (u16 per node and source) so their sequential sums run side by side
-    const uint64_t passes = (s_end - s_begin + 63) / 64;
-    const uint64_t pass_bytes = (uint64_t)n * 64 * 2;
-    const uint32_t group = inv_sum ? (uint32_t)std::max<uint64_t>(
-                                         1, std::min<uint64_t>({32, passes, (16ull << 30) / pass_bytes}))
-                                   : 1;
-    HBX_TRY(hipMalloc(&bits.p, (size_t)3 * n * 8));
-    HBX_TRY(hipMalloc(&cnt.p, (size_t)kBfsCols * (1 + grid) * 8));  // totals, then kBfsCols per block
-    // hubs: nodes of degree > kHubDeg, their lists cut into chunks of kHubChunk arcs
-    // (one wavefront each).  A wavefront walks the lists of degree 65..kHubDeg of its
-    // 64 nodes one after another, so that range is kept short.
-    constexpr uint32_t kHubDeg = 128, kHubChunk = 1024;
     const uint32_t arcs = h_off[n];
-    std::vector<uint32_t> h_hub;  // node, beg, end per chunk, as three runs
-    {
-        std::vector<uint32_t> hn, hb_, he;
-        for (uint32_t v = 0; v < n; ++v)
-            if (h_off[v + 1] - h_off[v] > kHubDeg)
-                for (uint64_t b = h_off[v]; b < h_off[v + 1]; b += kHubChunk) {
-                    hn.push_back(v);
-                    hb_.push_back((uint32_t)b);
-                    he.push_back((uint32_t)std::min<uint64_t>(b + kHubChunk, h_off[v + 1]));
-                }
-        h_hub = hn;
-        h_hub.insert(h_hub.end(), hb_.begin(), hb_.end());
-        h_hub.insert(h_hub.end(), he.begin(), he.end());
+    BfsGroup g;
+    BfsDev &b = g.b;
+    b.off = off;
+    b.nbr = nbr;
+    b.n = n;
+    b.npad = (n + kBfsChunk - 1) / kBfsChunk * kBfsChunk;
+    // tails of the arcs to each node: the lists themselves, or the reversed arcs
+    Scoped rev, tmp;
+    std::vector<uint32_t> h_ioff;
+    if (symmetric || arcs == 0) {
+        b.ioff = off;
+        b.inbr = nbr;
+    } else {
+        // a stable sort by head (4M arcs: 0.3 ms; counting and placing them with atomics took 2)
+        HBX_TRY(hipMalloc(&rev.p, ((size_t)n + 1 + arcs) * 4));
+        uint32_t *ioff = (uint32_t *)rev.p, *inbr = ioff + n + 1;
+        const unsigned bits = std::max(1u, 32u - (unsigned)__builtin_clz(std::max(n - 1, 1u)));
+        size_t bytes = 0;
+        HBX_TRY(rocprim::radix_sort_pairs(nullptr, bytes, nbr, inbr, inbr, inbr, (size_t)arcs, 0, bits, s));
+        const size_t words = (bytes + 255) / 4 / 64 * 64;
+        HBX_TRY(hipMalloc(&tmp.p, (words + 2 * (size_t)arcs) * 4));
+        uint32_t *tail = (uint32_t *)tmp.p + words, *head = tail + arcs;
+        k_bfs_tails<<<(unsigned)std::min<uint64_t>(((uint64_t)n + 3) / 4, 16384), kBfsBlock, 0, s>>>(off, n, tail);
+        HBX_TRY(rocprim::radix_sort_pairs(tmp.p, bytes, nbr, head, tail, inbr, (size_t)arcs, 0, bits, s));
+        k_bfs_offsets<<<(unsigned)std::min<uint64_t>(((uint64_t)arcs + kBfsBlock - 1) / kBfsBlock, 16384), kBfsBlock, 0,
+                        s>>>(head, arcs, n, ioff);
+        HBX_TRY(hipGetLastError());
+        h_ioff.resize((size_t)n + 1);
+        HBX_TRY(hipMemcpyAsync(h_ioff.data(), ioff, ((size_t)n + 1) * 4, hipMemcpyDeviceToHost, s));
+        HBX_TRY(hipStreamSynchronize(s));
+        tmp.release();
+        b.ioff = ioff;
+        b.inbr = inbr;
     }
-    const uint32_t chunks = (uint32_t)(h_hub.size() / 3);
+    // hubs and their tasks
     Scoped hub;
-    if (chunks) {
-        HBX_TRY(hipMalloc(&hub.p, h_hub.size() * 4));
-        HBX_TRY(hipMemcpy(hub.p, h_hub.data(), h_hub.size() * 4, hipMemcpyHostToDevice));
-    }
-    const uint32_t *hub_node = (const uint32_t *)hub.p, *hub_beg = hub_node + chunks, *hub_end = hub_beg + chunks;
-    const unsigned hub_grid = (unsigned)std::min<uint64_t>((chunks + 3) / 4, 4096);
-    if (inv_sum) {
-        HBX_TRY(hipMalloc(&dist.p, (size_t)group * pass_bytes));
-        HBX_TRY(hipMalloc(&sums.p, (size_t)group * 64 * 8));
-        HBX_TRY(hipMalloc(&cnts.p, (size_t)group * 4));
-    }
-    uint64_t *fr = (uint64_t *)bits.p, *vis = fr + n, *nx = fr + 2 * (size_t)n;
-    unsigned long long *d_cnt = (unsigned long long *)cnt.p;
-    std::vector<unsigned long long> hc(kBfsCols);
-    std::vector<double> h_inv;
-    std::vector<uint32_t> h_counts(group);
-    for (uint64_t g0 = 0; g0 < passes; g0 += group) {
-        const uint32_t gn = (uint32_t)std::min<uint64_t>(group, passes - g0);
-        uint32_t levels = 0;
-        for (uint32_t j = 0; j < gn; ++j) {
-            const uint64_t s0 = s_begin + (g0 + j) * 64;
-            const uint32_t count = (uint32_t)std::min<uint64_t>(64, s_end - s0);
-            uint16_t *dj = dist.p ? (uint16_t *)dist.p + (size_t)j * n * 64 : nullptr;
-            h_counts[j] = count;
-            uint64_t r[64] = {}, t[64] = {};
-            const uint64_t full = count == 64 ? ~0ull : ((1ull << count) - 1);
-            // arcs leaving the frontier: the sources' own lists first
-            uint64_t frontier_arcs = h_off[s0 + count] - h_off[s0];
-            k_bfs_init<<<grid, kBfsBlock, 0, s>>>(fr, vis, nx, n, (uint32_t)s0, count);
-            if (dj) k_bfs_zero<uint16_t><<<4096, kBfsBlock, 0, s>>>(dj, (uint64_t)n * 64);
-            for (uint32_t level = 1;; ++level) {
-                if (dj && level > 65535u)
-                    return efail(HB_ERANGE, "hb_exact_bfs: eccentricity above 65535 (harmonic sums need u16 distances)");
-                // direction (symmetric graphs only): pull when the frontier's arcs exceed
-                // 1/8 of all arcs -- a pull scans every unreached node's list once without
-                // atomics, a push walks the frontier's lists with an atomic OR per arc
-                if (level == 1) {
-                    const unsigned sg = (unsigned)std::max<uint64_t>(
-                        1, std::min<uint64_t>((frontier_arcs + kBfsBlock - 1) / kBfsBlock, 4096));
-                    k_bfs_push_sources<<<sg, kBfsBlock, 0, s>>>(off, nbr, nx, (uint32_t)s0, count);
-                } else if (symmetric && frontier_arcs * 8 > arcs) {
-                    k_bfs_pull<<<grid, kBfsBlock, 0, s>>>(off, nbr, fr, vis, nx, n, full, kHubDeg);
-                    if (chunks)
-                        k_bfs_hubs<true><<<hub_grid, kBfsBlock, 0, s>>>(nbr, hub_node, hub_beg, hub_end, chunks, fr,
-                                                                        vis, nx, full);
-                } else {
-                    k_bfs_push<<<grid, kBfsBlock, 0, s>>>(off, nbr, fr, vis, nx, n, kHubDeg);
-                    if (chunks)
-                        k_bfs_hubs<false><<<hub_grid, kBfsBlock, 0, s>>>(nbr, hub_node, hub_beg, hub_end, chunks, fr,
-                                                                         vis, nx, full);
-                }
-                k_bfs_apply<<<grid, kBfsBlock, 0, s>>>(off, fr, vis, nx, dj, n, level, d_cnt + kBfsCols);
-                HBX_TRY(sum_columns(d_cnt + kBfsCols, grid, kBfsCols, d_cnt, s));
-                HBX_TRY(hipMemcpyAsync(hc.data(), d_cnt, kBfsCols * 8, hipMemcpyDeviceToHost, s));
-                HBX_TRY(hipStreamSynchronize(s));
-                bool any = false;
-                for (int k = 0; k < 64; ++k) any = any || hc[k] != 0;
-                frontier_arcs = hc[64];
-                if (!any) break;
-                levels = std::max(levels, level);
-                for (int k = 0; k < 64; ++k) {
-                    r[k] += hc[k];
-                    t[k] += (uint64_t)level * hc[k];
-                }
-            }
-            for (uint32_t k = 0; k < count; ++k) {
-                if (reach) reach[s0 - s_begin + k] = r[k];
-                if (total) total[s0 - s_begin + k] = t[k];
+    {
+        const uint32_t *ho = h_ioff.empty() ? h_off : h_ioff.data();
+        std::vector<uint32_t> node, first, tnode, tbeg, tend;
+        for (uint32_t v = 0; v < n; ++v) {
+            if (ho[v + 1] - ho[v] <= kBfsHubDeg) continue;
+            node.push_back(v);
+            first.push_back((uint32_t)tnode.size());
+            for (uint64_t e = ho[v]; e < ho[v + 1]; e += kBfsHubArcs) {
+                tnode.push_back(v);
+                tbeg.push_back((uint32_t)e);
+                tend.push_back((uint32_t)std::min<uint64_t>(e + kBfsHubArcs, ho[v + 1]));
             }
         }
-        if (inv_sum) {
-            // 1/d as correctly rounded host divisions, d = 1..levels; entry 0 is an unreached node
-            if (h_inv.size() < (size_t)levels + 1) {
-                const size_t from = h_inv.empty() ? 1 : h_inv.size();
-                h_inv.resize((size_t)levels + 1);
-                h_inv[0] = 0.0;
-                for (size_t d = from; d <= levels; ++d) h_inv[d] = 1.0 / (double)d;
-                if (inv.p) (void)hipFree(inv.p), inv.p = nullptr;
-                HBX_TRY(hipMalloc(&inv.p, h_inv.size() * 8));
-                HBX_TRY(hipMemcpyAsync(inv.p, h_inv.data(), h_inv.size() * 8, hipMemcpyHostToDevice, s));
+        b.hubs = (uint32_t)node.size();
+        b.tasks = (uint32_t)tnode.size();
+        first.push_back(b.tasks);
+        if (b.hubs) {
+            std::vector<uint32_t> h;
+            for (const auto *v : {&node, &first, &tnode, &tbeg, &tend}) h.insert(h.end(), v->begin(), v->end());
+            HBX_TRY(hipMalloc(&hub.p, h.size() * 4));
+            HBX_TRY(hipMemcpy(hub.p, h.data(), h.size() * 4, hipMemcpyHostToDevice));
+            b.hub_node = (const uint32_t *)hub.p;
+            b.hub_first = b.hub_node + b.hubs;
+            b.task_node = b.hub_first + b.hubs + 1;
+            b.task_beg = b.task_node + b.tasks;
+            b.task_end = b.task_beg + b.tasks;
+        }
+    }
+    BfsMode mode = inv_sum ? BfsMode::kKeep : BfsMode::kSums;
+    Scoped inv;
+    BfsMemory mem(s);
+    std::vector<double> h_inv(1, 0.0);  // 1/d as correctly rounded host divisions; entry 0: unreached
+    auto inverses = [&](uint32_t levels) -> int {
+        if (inv.p && h_inv.size() > levels) return HB_OK;
+        for (size_t d = h_inv.size(); d <= levels; ++d) h_inv.push_back(1.0 / (double)d);
+        inv.release();
+        HBX_TRY(hipMalloc(&inv.p, h_inv.size() * 8));
+        HBX_TRY(hipMemcpyAsync(inv.p, h_inv.data(), h_inv.size() * 8, hipMemcpyHostToDevice, s));
+        return HB_OK;
+    };
+    for (uint64_t s0 = s_begin; s0 < s_end;) {
+        if (!mem.p) {
+            // the widest rows and then the most slices that fit into memory that is kept, with
+            // rows of at least 64 bytes (half a cache line), else into the budget
+            const uint64_t words = (s_end - s0 + 63) / 64;
+            auto bytes = [&](uint32_t w, uint32_t k) { return (uint64_t)bfs_plan(n, b.tasks, w, k, mode).bytes; };
+            uint32_t wide = 2;
+            while (wide < 32 && wide < words) wide *= 2;
+            uint32_t sw = wide;
+            uint64_t budget = kBfsHold;
+            while (sw > 8 && bytes(sw, 1) > budget) sw /= 2;
+            if (bytes(sw, 1) > budget) {
+                sw = wide;
+                budget = kBfsBudget;
+                while (sw > 2 && bytes(sw, 1) > budget) sw /= 2;
             }
-            HBX_TRY(hipMemcpyAsync(cnts.p, h_counts.data(), (size_t)gn * 4, hipMemcpyHostToDevice, s));
-            const uint32_t entries = (uint32_t)h_inv.size();
-            if (entries <= kInvLds)
-                k_bfs_inv_sum<true><<<gn, kInvBlock, 0, s>>>((const uint16_t *)dist.p, (const double *)inv.p, entries, n,
-                                                      (const uint32_t *)cnts.p, (double *)sums.p);
-            else
-                k_bfs_inv_sum<false><<<gn, kInvBlock, 0, s>>>((const uint16_t *)dist.p, (const double *)inv.p, entries, n,
-                                                       (const uint32_t *)cnts.p, (double *)sums.p);
-            HBX_TRY(hipGetLastError());
-            std::vector<double> hs((size_t)gn * 64);
-            HBX_TRY(hipMemcpyAsync(hs.data(), sums.p, hs.size() * 8, hipMemcpyDeviceToHost, s));
+            uint32_t slices = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((words + sw - 1) / sw, budget / bytes(sw, 1)));
+            while (slices > 1 && bytes(sw, slices) > budget) --slices;
+            for (;;) {
+                const BfsPlan p = bfs_plan(n, b.tasks, sw, slices, mode);
+                const hipError_t e = mem.take(p.bytes);
+                if (e == hipSuccess) {
+                    g.place((char *)mem.p, p);
+                    break;
+                }
+                if (e != hipErrorOutOfMemory || (sw == 2 && slices == 1)) HBX_TRY(e);
+                (void)hipGetLastError();
+                if (slices > 1) slices /= 2;
+                else sw /= 2;
+            }
+        }
+        const uint32_t per_slice = 64 * g.plan.sw;
+        // the last group may need fewer slices; the buffers keep their strides
+        const uint32_t slices = (uint32_t)std::min<uint64_t>(g.plan.slices, (s_end - s0 + per_slice - 1) / per_slice);
+        BfsGroup r = g;
+        r.plan.slices = slices;
+        r.b.src0 = (uint32_t)s0;
+        r.b.src_end = (uint32_t)s_end;
+        const uint64_t group_end = std::min<uint64_t>(s_end, s0 + (uint64_t)slices * per_slice);
+        uint64_t source_arcs = 0;
+        for (uint32_t i = 0; i < slices; ++i) {
+            const uint64_t a = s0 + (uint64_t)i * per_slice, e = std::min<uint64_t>(a + per_slice, s_end);
+            source_arcs = std::max<uint64_t>(source_arcs, h_off[e] - h_off[a]);
+        }
+        const uint64_t row_words = (uint64_t)slices * n * g.plan.sw;
+        const unsigned zgrid = (unsigned)std::min<uint64_t>((row_words / 2 + kBfsBlock - 1) / kBfsBlock, 16384);
+        k_bfs_zero<uint4><<<zgrid, kBfsBlock, 0, s>>>((uint4 *)r.b.visited, row_words / 2);
+        k_bfs_zero<uint4><<<zgrid, kBfsBlock, 0, s>>>((uint4 *)r.level(1).rows, row_words / 2);
+        k_bfs_zero<uint4><<<zgrid, kBfsBlock, 0, s>>>((uint4 *)r.level(1).flag, (uint64_t)slices * r.b.npad / 16);
+        if (mode == BfsMode::kLong) k_bfs_zero<uint4><<<zgrid, kBfsBlock, 0, s>>>((uint4 *)r.dist, row_words * 8);
+        k_bfs_begin<<<slices, kBfsBlock, 0, s>>>(r.b, r.plan.sw);
+        // launches past a slice's last level return at once, so the host looks every 4, 8, ..
+        // levels only
+        std::vector<uint32_t> state(2 * (size_t)g.plan.slices);
+        uint32_t at = 0;  // levels launched
+        bool all = false;
+        while (!all) {
+            uint32_t to = at + (at < 8 ? 4 : std::min(64u, at / 2));
+            if (mode == BfsMode::kKeep) to = std::min(to, kBfsKeep);
+            if (mode == BfsMode::kLong) to = std::min(to, 65535u);
+            if (to == at) break;
+            hipError_t e = hipErrorInvalidValue;
+            switch (r.plan.sw) {
+            case 2: e = bfs_levels<2>(r, at + 1, to, source_arcs, mode, s); break;
+            case 4: e = bfs_levels<4>(r, at + 1, to, source_arcs, mode, s); break;
+            case 8: e = bfs_levels<8>(r, at + 1, to, source_arcs, mode, s); break;
+            case 16: e = bfs_levels<16>(r, at + 1, to, source_arcs, mode, s); break;
+            case 32: e = bfs_levels<32>(r, at + 1, to, source_arcs, mode, s); break;
+            }
+            HBX_TRY(e);
+            HBX_TRY(hipMemcpyAsync(state.data(), r.b.done, state.size() * 4, hipMemcpyDeviceToHost, s));
             HBX_TRY(hipStreamSynchronize(s));
-            for (uint32_t j = 0; j < gn; ++j)
-                for (uint32_t k = 0; k < h_counts[j]; ++k)
-                    inv_sum[(g0 + j) * 64 + k] = hs[(size_t)j * 64 + k];
+            at = to;
+            all = true;
+            for (uint32_t i = 0; i < slices; ++i) all = all && state[i];
         }
+        if (!all && mode == BfsMode::kKeep) {  // long searches: this group again, and the rest, by distances
+            mode = BfsMode::kLong;
+            mem.release();
+            continue;
+        }
+        if (!all)
+            return efail(HB_ERANGE, "hb_exact_bfs: eccentricity above 65535 (harmonic sums need u16 distances)");
+        const size_t sources = (size_t)(group_end - s0);
+        std::vector<u64> h_sums(2 * (size_t)g.plan.slices * per_slice);
+        if (reach || total)
+            HBX_TRY(hipMemcpyAsync(h_sums.data(), r.b.reach, h_sums.size() * 8, hipMemcpyDeviceToHost, s));
+        if (inv_sum) {
+            uint32_t levels = 0;
+            for (uint32_t i = 0; i < slices; ++i) levels = std::max(levels, state[g.plan.slices + i]);
+            if (int rc = inverses(std::max(levels, kBfsKeep))) return rc;
+            if (mode == BfsMode::kKeep) {
+                const BfsPlan &p = g.plan;
+                const unsigned grid = (unsigned)((sources + kBfsBlock / 64 - 1) / (kBfsBlock / 64));
+#define HB_BFS_HARMONIC(SW)                                                                                       \
+    case SW:                                                                                                      \
+        k_bfs_harmonic<SW><<<grid, kBfsBlock, 0, s>>>(r.b, r.level0.count, p.count_stride, r.level0.any, p.any_stride, \
+                                                      (const double *)inv.p, slices, r.sums);                      \
+        break;
+                switch (p.sw) { HB_BFS_HARMONIC(2) HB_BFS_HARMONIC(4) HB_BFS_HARMONIC(8) HB_BFS_HARMONIC(16) HB_BFS_HARMONIC(32) }
+#undef HB_BFS_HARMONIC
+            } else {
+                const uint32_t passes = (uint32_t)((sources + 63) / 64);
+                std::vector<uint32_t> counts(passes, 64u);
+                counts.back() = (uint32_t)(sources - (size_t)(passes - 1) * 64);
+                HBX_TRY(hipMemcpyAsync(r.word_count, counts.data(), passes * 4, hipMemcpyHostToDevice, s));
+                HBX_TRY(hipStreamSynchronize(s));  // `counts` is a pageable host buffer
+                const uint32_t entries = levels + 1;
+                if (entries <= kInvLds)
+                    k_bfs_inv_sum<true><<<passes, kInvBlock, 0, s>>>(r.dist, (const double *)inv.p, entries, n,
+                                                                     r.word_count, r.sums);
+                else
+                    k_bfs_inv_sum<false><<<passes, kInvBlock, 0, s>>>(r.dist, (const double *)inv.p, entries, n,
+                                                                      r.word_count, r.sums);
+            }
+            HBX_TRY(hipGetLastError());
+            HBX_TRY(hipMemcpyAsync(inv_sum + (s0 - s_begin), r.sums, sources * 8, hipMemcpyDeviceToHost, s));
+        }
+        HBX_TRY(hipStreamSynchronize(s));
+        const size_t half = (size_t)g.plan.slices * per_slice;
+        for (size_t i = 0; i < sources; ++i) {
+            if (reach) reach[s0 - s_begin + i] = h_sums[i];
+            if (total) total[s0 - s_begin + i] = h_sums[half + i];
+        }
+        s0 = group_end;
     }
     return HB_OK;
 }

@@ -121,6 +121,8 @@ hipError_t launch_surrogate_tail(struct ::hb_mlp *n, const uint32_t *off, const 
                                  uint32_t infer_nodes, bool standardized_x, float *x_dev, float *out_dev,
                                  hipStream_t s);
 int mlp_device(const struct ::hb_mlp *n);
+// frees the device memory exact_bfs keeps between calls (not what a call is using)
+void release_held();
 // exact BFS sums of sources [s_begin, s_end) over a staged CSR (hb_exact.hip), h_off
 // the host copy of its offsets; symmetric: the CSR holds v -> u for every u -> v (levels
 // may then pull)

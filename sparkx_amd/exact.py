@@ -4,7 +4,7 @@ Mirrors ExactClosenessCentrality, ExactHarmonicCentrality and ExactLinCentrality
 (src/centralities/exact.rs:10-226, :228-466, :468-644): `new(g, normalized)` runs
 at once, `centralities()` and `get_node_centrality(idx)` read the result.  The
 searches run in the HIP engine (hb_exact_bfs / hb_exact_centrality of
-libsparkx_hb.so), 64 sources per pass; `sources` (an extension) restricts the run
+libsparkx_hb.so), thousands of sources side by side; `sources` (an extension) restricts the run
 to a contiguous range of source nodes, e.g. a sample for rank correlation on
 graphs where one BFS per node is too long.  Values follow BFSDists
 (src/trails/bfs.rs:199-234) including its quirk: the source is rediscovered and
