@@ -187,7 +187,7 @@ struct hb_ctx {
     DevBuf<uint32_t> sched_buf, chunk_flag;
     // per-node bitmaps of a run, cleared together: changed nodes (2), then active nodes of
     // push iterations (2) and saturated nodes (2) where they are used, then the bound of
-    // all sketches (2^p)
+    // all sketches (2^p) and the counters of the running iteration
     DevBuf<uint32_t> bits;
     DevBuf<uint32_t> dyn;  // push iterations: per-bin lists + 3 counts
     bool sym = false;              // staged CSR is symmetric (arc multiset fingerprints)
@@ -760,7 +760,10 @@ extern "C" int hb_run(hb_ctx *c, int p, int max_iters, uint32_t flags, hb_stats 
     const bool sat_ok = p <= 10 && !(flags & HB_FLAG_DENSE) && !chain;
     // rounded up so that the bound after the bitmaps is aligned for 16-byte loads
     const size_t bit_words = ((2 + (push_ok ? 2 : 0) + (sat_ok ? 2 : 0)) * (size_t)words + 3) & ~(size_t)3;
-    HB_TRY(c->bits.ensure(bit_words + (sat_ok ? m : 0)));
+    // the bound and the iteration counters
+    const size_t count_at = (bit_words + (sat_ok ? m : 0) + 63) & ~(size_t)63;
+    const size_t all_words = count_at + 2 * HB_COUNT_COPIES * HB_COUNT_STRIDE;
+    HB_TRY(c->bits.ensure(all_words));
 
     HbDev &d = c->dev;
     d = HbDev{};
@@ -775,6 +778,7 @@ extern "C" int hb_run(hb_ctx *c, int p, int max_iters, uint32_t flags, hb_stats 
     d.inv = c->inv.ptr;
     d.bits0 = c->bits.ptr;
     d.bits1 = d.bits0 + words;
+    d.counts = (unsigned long long *)(c->bits.ptr + count_at);
     if (sat_ok) {
         d.sat_bits = d.bits1 + words + (push_ok ? 2 * words : 0);
         d.sat_max = c->bits.ptr + bit_words;
@@ -818,7 +822,7 @@ extern "C" int hb_run(hb_ctx *c, int p, int max_iters, uint32_t flags, hb_stats 
     st0.inv_t = 1.0;
     HB_TRY(hipMemcpyAsync(c->st.ptr, &st0, sizeof st0, hipMemcpyHostToDevice, c->stream));
     // iteration t marks the active bitmap iteration t - 1 cleared; both start clear
-    HB_TRY(hb::launch_fill(c->bits.ptr, bit_words + (sat_ok ? m : 0), 0u, c->stream));
+    HB_TRY(hb::launch_fill(c->bits.ptr, all_words, 0u, c->stream));
 
     hipEvent_t e0, e1, e2;
     HB_TRY(hipEventCreate(&e0));

@@ -9,6 +9,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <stddef.h>
 #include <stdint.h>
 
 #define HB_WAVE 64
@@ -56,6 +57,11 @@ struct HbIterRec {  // per-iteration counters, per kernel slot
     unsigned long long push;             // 1 if iteration t listed its nodes by push
 };
 
+static_assert(offsetof(HbIterRec, gathered) == 4 * HB_NSLOT * sizeof(unsigned long long), "five runs of slots first");
+// copies of an iteration's counters (block_add) and their distance in 8-byte words (256 B)
+#define HB_COUNT_COPIES 16
+#define HB_COUNT_STRIDE 32
+
 struct HbBiasTable;  // HLL++ bias windows of one precision (below)
 
 struct HbDev {
@@ -71,6 +77,7 @@ struct HbDev {
     uint32_t *bits0, *bits1;  // changed-node bitmaps (bit set: registers changed)
     HbIterState *st;
     HbIterRec *rec;        // ring: iteration t in rec[t % HB_REC_RING]
+    unsigned long long *counts;  // the running iteration's counters, HB_COUNT_COPIES times
     const float *lc;       // lc[z] = (float)(m ln(m/z)), z = 1..m
     const HbBiasTable *bias;  // HLL++ bias windows for this p
     float *snaps;          // estimates after iterations 1..snap_k, iteration-major
