@@ -88,8 +88,8 @@ typedef struct {
     uint64_t kernel_nodes[HB_NKERNELS];   /* nodes recomputed                         */
     uint32_t kernel_items[HB_NKERNELS];   /* nodes (bins, merge) or tasks (chunks) scheduled */
     uint32_t kernel_team[HB_NKERNELS];    /* lanes per node / task                    */
-    /* the part of kernel_arcs / kernel_nodes done in iteration 1 with p <= 10, where
-       every sketch is still a single insertion: the neighbour's (and the node's own)
+    /* the part of kernel_arcs / kernel_nodes done in iteration 1, where every sketch is
+       still a single insertion: the neighbour's (and, with p <= 10, the node's own)
        2^p-byte register block is not read, its id is hashed instead */
     uint64_t kernel_first_arcs[HB_NKERNELS];
     uint64_t kernel_first_nodes[HB_NKERNELS];

@@ -542,25 +542,30 @@ static int build_schedule(hb_ctx *c, int p)
     const std::vector<uint32_t> &h_off = c->run_hoff();
     c->n_linked = 0;
     std::vector<uint32_t> bins[3], tnode, tbeg, tend, hnode, htask0, hntask;
+    // p > 10: longer lists are cut (a wavefront reads a row of 4 KiB in about 0.7 us, so a
+    // hub of 10,000 neighbours alone would take as long as the rest of the iteration)
+    constexpr uint32_t kWideHub = 256;
+    auto split = [&](uint32_t u, uint32_t chunk) {
+        hnode.push_back(u);
+        htask0.push_back((uint32_t)tnode.size());
+        uint32_t cnt = 0;
+        for (uint64_t e = h_off[u]; e < h_off[u + 1]; e += chunk, ++cnt) {
+            tnode.push_back(u);
+            tbeg.push_back((uint32_t)e);
+            tend.push_back((uint32_t)std::min<uint64_t>(e + chunk, h_off[u + 1]));
+        }
+        hntask.push_back(cnt);
+    };
     for (uint32_t u = 0; u < n; ++u) {
         const uint32_t d = h_off[u + 1] - h_off[u];
         if (d == 0) continue;  // keeps c_0; written to both buffers at init
         ++c->n_linked;
-        if (p > 10) bins[2].push_back(u);  // one wavefront per node walks the register row
+        if (p > 10 && d <= kWideHub) bins[2].push_back(u);  // a wavefront per node
+        else if (p > 10) split(u, kWideHub);
         else if (d <= c->small_max) bins[0].push_back(u);
         else if (d <= c->mid_max) bins[1].push_back(u);
         else if (d <= c->wave_max) bins[2].push_back(u);
-        else {
-            hnode.push_back(u);
-            htask0.push_back((uint32_t)tnode.size());
-            uint32_t cnt = 0;
-            for (uint32_t e = h_off[u]; e < h_off[u + 1]; e += c->chunk, ++cnt) {
-                tnode.push_back(u);
-                tbeg.push_back(e);
-                tend.push_back(std::min(e + c->chunk, h_off[u + 1]));
-            }
-            hntask.push_back(cnt);
-        }
+        else split(u, c->chunk);
     }
     const size_t total = bins[0].size() + bins[1].size() + bins[2].size() + 3 * tnode.size() +
                          3 * hnode.size();
@@ -757,11 +762,11 @@ extern "C" int hb_run(hb_ctx *c, int p, int max_iters, uint32_t flags, hb_stats 
     // which the chain layout's graphs do not; its kernels and the dense schedule, which
     // recomputes every node in every iteration, go without.
     const bool chain = c->relabelled() && c->layout_used == HB_LAYOUT_CHAIN;
-    const bool sat_ok = p <= 10 && !(flags & HB_FLAG_DENSE) && !chain;
+    const bool sat_ok = !(flags & HB_FLAG_DENSE) && !(chain && p <= 10);
     // rounded up so that the bound after the bitmaps is aligned for 16-byte loads
     const size_t bit_words = ((2 + (push_ok ? 2 : 0) + (sat_ok ? 2 : 0)) * (size_t)words + 3) & ~(size_t)3;
-    // the bound and the iteration counters
-    const size_t count_at = (bit_words + (sat_ok ? m : 0) + 63) & ~(size_t)63;
+    // the bound, and at p > 10 its packed form; the iteration counters
+    const size_t count_at = (bit_words + (sat_ok ? m + (p > 10 ? m / 4 : 0) : 0) + 63) & ~(size_t)63;
     const size_t all_words = count_at + 2 * HB_COUNT_COPIES * HB_COUNT_STRIDE;
     HB_TRY(c->bits.ensure(all_words));
 
@@ -782,6 +787,8 @@ extern "C" int hb_run(hb_ctx *c, int p, int max_iters, uint32_t flags, hb_stats 
     if (sat_ok) {
         d.sat_bits = d.bits1 + words + (push_ok ? 2 * words : 0);
         d.sat_max = c->bits.ptr + bit_words;
+        d.sat_row = (uint8_t *)(d.sat_max + m);
+        d.sat_sym = c->sym ? 1 : 0;
     }
     d.st = c->st.ptr;
     d.rec = c->rec.ptr;
@@ -976,7 +983,7 @@ extern "C" int hb_run(hb_ctx *c, int p, int max_iters, uint32_t flags, hb_stats 
             stats->kernel_items[sl] = items[sl];
             stats->kernel_team[sl] = sl < 3 ? (uint32_t)c->sched.bin_team[sl] : 64u;
         }
-        if (p <= 10 && executed >= 1)
+        if (executed >= 1)
             for (int sl = 0; sl < HB_NSLOT; ++sl) {
                 // bins hash the ids of the neighbours and of the node itself, hub chunks
                 // those of the neighbours; the hub merge reads register blocks as always,

@@ -97,6 +97,8 @@ struct HbDev {
     // (hb_saturated), bit set: the node's sketch is the bound
     uint32_t *sat_max;     // [2^p], one register each
     uint32_t *sat_bits;
+    uint8_t *sat_row;      // p > 10: the bound packed as registers are
+    int sat_sym;           // the CSR is symmetric, whatever p
     int sym;               // the CSR holds v -> u for every u -> v
     uint64_t arcs;         // arcs of the staged CSR
     uint32_t n;

@@ -41,7 +41,7 @@ const HbBiasTable *bias_table(int p);
 
 hipError_t launch_init(const HbDev &d, hipStream_t s);
 hipError_t launch_fill(uint32_t *p, uint64_t count, uint32_t value, hipStream_t s);
-// one iteration; first: iteration 1, whose kernels hash ids (p <= 10)
+// one iteration; first: iteration 1, whose kernels hash ids
 // ev (nullable): 2 * HB_NSLOT events recorded around each kernel slot that launches
 hipError_t launch_iteration(const HbDev &d, const HbSchedule &sc, bool first, bool nf, hipStream_t s,
                             hipEvent_t *ev = nullptr);

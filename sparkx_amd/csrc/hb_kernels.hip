@@ -721,60 +721,235 @@ __global__ __launch_bounds__(kBlock) void k_merge(HbDev d, const uint32_t *__res
 }
 
 // ---------------------------------------------------------------------------
-// precisions 11..16: one wavefront per node walks the register row in 1 KiB
-// chunks (64 lanes x 16 registers); a per-wave LDS histogram of register values
-// gives zeros, the maximum and the exact integer form of sum 2^-M; a row whose
-// sum is not exact in f32 replays the sequential loop from L2.
+// precisions 11..16: one wavefront per node, 64 lanes x 16 registers to a 1 KiB chunk of
+// the row, up to four chunks at a time in registers (wider rows go in passes).  What bounds
+// it is the rows it reads, so their loads are kept in flight eight at a time; long lists are
+// cut into tasks whose partial rows the hub's wavefront then reads as if they were its
+// neighbours'; iteration 1 hashes ids as at p <= 10; outside dense iterations only changed
+// neighbours are read, and saturated nodes (HbDev::sat_max) nothing at all.
+// De Bruijn graph (n = 16,384, 131,068 arcs, p = 12): its 8 iterations take 1.07 ms, a dense one
+// 0.115 (0.67 GB of rows: 5.8 TB/s); 2.99 ms with a loop of single loads per chunk, an LDS
+// histogram for the estimate and a serial replay of the sums that are not exact.  R-MAT-15
+// (p = 13) 126 -> 3.7 ms, R-MAT-17 (p = 11) 47.9 -> 2.0 ms, where hubs were one wavefront's.
+// Three wavefronts per SIMD (up to 161 VGPRs) beat four (126 and spills: 1.24 ms).
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ void hist_add_word(uint32_t *h, uint32_t x)
+template <int P>
+struct Wide {
+    static constexpr uint32_t M = 1u << P;
+    static constexpr int CHUNKS = M / 1024, CG = CHUNKS < 4 ? CHUNKS : 4, PASSES = CHUNKS / CG;
+};
+
+// Zeros, maximum and sum of a row's registers, per lane and then over the wavefront.  s24 =
+// sum of 2^(24 - M) over the registers M <= 24: exact, and all of them unless mx > 24.
+struct WideSum {
+    uint32_t z = 0, mx = 0;
+    unsigned long long s24 = 0;
+
+    __device__ void add(uint4 a)
+    {
+        z += hb_zero_bytes(a.x) + hb_zero_bytes(a.y) + hb_zero_bytes(a.z) + hb_zero_bytes(a.w);
+        mx = max(mx, hb_max_byte(hb_bmax(hb_bmax(a.x, a.y), hb_bmax(a.z, a.w))));
+        uint32_t k = 0;  // 16 terms of at most 2^24
+        const uint32_t w[4] = {a.x, a.y, a.z, a.w};
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int b = 0; b < 4; ++b) k += (1u << 24) >> min((w[q] >> (8 * b)) & 0xffu, 31u);
+        s24 += k;
+    }
+    __device__ void reduce()
+    {
+#pragma unroll
+        for (int o = 1; o < HB_WAVE; o <<= 1) {
+            z += __shfl_xor(z, o);
+            mx = max(mx, (uint32_t)__shfl_xor(mx, o));
+            s24 += __shfl_xor(s24, o);
+        }
+    }
+};
+
+// S + the 16 registers of lane `from`, one f32 add each in register order
+__device__ __forceinline__ float wide_replay16(float S, uint4 a, int from)
 {
-    atomicAdd(h + (x & 0xffu), 1u);
-    atomicAdd(h + ((x >> 8) & 0xffu), 1u);
-    atomicAdd(h + ((x >> 16) & 0xffu), 1u);
-    atomicAdd(h + (x >> 24), 1u);
+    const uint32_t w[4] = {(uint32_t)__builtin_amdgcn_readlane((int)a.x, from),
+                           (uint32_t)__builtin_amdgcn_readlane((int)a.y, from),
+                           (uint32_t)__builtin_amdgcn_readlane((int)a.z, from),
+                           (uint32_t)__builtin_amdgcn_readlane((int)a.w, from)};
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int b = 0; b < 4; ++b) S = __fadd_rn(S, hb_pow2neg((w[q] >> (8 * b)) & 0xffu));
+    return S;
 }
 
-// estimate from a 64-bin histogram of the row (all lanes of the wave return it)
-template <int P>
-__device__ float estimate_wide(const HbDev &d, const uint32_t *h, const uint8_t *row)
+// The reference's sequential f32 sum of 2^-M over a row whose sum is not exact in f32
+// (row(c): this lane's registers of chunk c).  Let the final sum lie below 2^(E+1).  A term of
+// at least u = 2^(E-23) adds exactly to a running sum that is a multiple of u, in any order;
+// only the few smaller terms (M > 23 - E) can round, and, once one of them has left bits
+// below u in the sum, the adds that carry it into a higher binade.  So the wavefront adds
+// whole lanes (16 registers each) by prefix sums, exact in f64, up to the next lane that
+// holds such an add, and replays that lane add by add.  Rows with a register above 35, for
+// which f64 would not be exact, are replayed throughout.
+template <int CHUNKS, class Row>
+__device__ float wide_sequential_sum(uint32_t mx, Row row)
 {
-    constexpr uint32_t M = 1u << P;
     const uint32_t lane = threadIdx.x & (HB_WAVE - 1);
-    const uint32_t z = h[0];
-    if (z > 0) {
-        const float lc = d.lc[z];
+    auto lane_sum = [](uint4 a) {
+        double g = 0.0;
+        const uint32_t w[4] = {a.x, a.y, a.z, a.w};
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int b = 0; b < 4; ++b)
+                g += __longlong_as_double((long long)(1023 - ((w[q] >> (8 * b)) & 0xffu)) << 52);
+        return g;
+    };
+    float S = 0.0f;
+    if (mx > 35) {
+        for (int c = 0; c < CHUNKS; ++c) {
+            const uint4 a = row(c);
+            for (int l = 0; l < HB_WAVE; ++l) S = wide_replay16(S, a, l);
+        }
+        return S;
+    }
+    double total = 0.0;
+    for (int c = 0; c < CHUNKS; ++c) total += lane_sum(row(c));
+#pragma unroll
+    for (int o = 1; o < HB_WAVE; o <<= 1) total += __shfl_xor(total, o);
+    // no running sum exceeds the exact one by its rounding errors, 2^16 times 2^-24 of it
+    const int E = (int)((__double_as_longlong(total * 1.01) >> 52) & 0x7ff) - 1023;
+    const double per_u = __longlong_as_double((long long)(1023 - E + 23) << 52);
+    const uint32_t thr = (uint32_t)max(23 - E, 0);
+    for (int c = 0; c < CHUNKS; ++c) {
+        const uint4 a = row(c);
+        double X = lane_sum(a);
+        const bool tiny = hb_max_byte(hb_bmax(hb_bmax(a.x, a.y), hb_bmax(a.z, a.w))) > thr;
+#pragma unroll
+        for (int o = 1; o < HB_WAVE; o <<= 1) {
+            const double y = __shfl_up(X, o);
+            if ((int)lane >= o) X += y;
+        }
+        uint32_t pos = 0;
+        double before = 0.0;  // prefix sum of the lanes < pos
+        while (pos < HB_WAVE) {
+            const double s = (double)S, q = s * per_u;
+            bool stop = tiny;
+            if (q != floor(q)) {  // bits below u: the next binade rounds
+                const double next = __longlong_as_double((__double_as_longlong(s) & (0x7ffll << 52)) + (1ll << 52));
+                stop = stop || s + (X - before) >= next;
+            }
+            const unsigned long long m = __ballot(stop && lane >= pos);
+            const int first = m ? __ffsll(m) - 1 : HB_WAVE;
+            if (first > (int)pos) S = (float)(s + (__shfl(X, first - 1) - before));
+            if (first == HB_WAVE) break;
+            S = wide_replay16(S, a, first);
+            before = __shfl(X, first);
+            pos = (uint32_t)first + 1;
+        }
+    }
+    return S;
+}
+
+// estimate of a row from its (wave-reduced) sums; every lane returns it
+template <int P, class Row>
+__device__ __forceinline__ float wide_estimate(const HbDev &d, const WideSum &w, Row row)
+{
+    if (w.z > 0) {
+        const float lc = d.lc[w.z];
         if ((double)lc <= d.lc_thr) return lc;
     }
-    const uint32_t hv = h[lane];
-    uint32_t mx = hv ? lane : 0u;
-    for (int s = 1; s < HB_WAVE; s <<= 1) mx = max(mx, (uint32_t)__shfl_xor(mx, s));
-    // k = sum_v h[v] 2^(mx - v), saturated at 2^24
-    uint32_t k = 0;
-    if (hv) {
-        const uint32_t sh = mx - lane;
-        k = sh >= 24u ? (1u << 24) : min(hv << sh, 1u << 24);
-        if (sh < 24u && (hv >> (24u - sh)) != 0u) k = 1u << 24;
-    }
-    for (int s = 1; s < HB_WAVE; s <<= 1) k = min(k + (uint32_t)__shfl_xor(k, s), 1u << 24);
     float S;
-    if (k < (1u << 24)) {
-        S = ldexpf((float)k, -(int)mx);
-    } else {
-        S = 0.0f;
-        if (lane == 0) {
-            __threadfence();
-            for (uint32_t i = 0; i < M; i += 4) {
-                const uint32_t w = __hip_atomic_load((const uint32_t *)(row + i), __ATOMIC_RELAXED,
-                                                     __HIP_MEMORY_SCOPE_AGENT);
-#pragma unroll
-                for (int b = 0; b < 4; ++b) S = __fadd_rn(S, hb_pow2neg((w >> (8 * b)) & 0xffu));
-            }
-        }
-        S = __shfl(S, 0);
-    }
+    // k = sum of 2^(mx - M) as at p <= 10: below 2^24 the f32 sum is exact
+    if (w.mx <= 24 && (w.s24 >> (24 - w.mx)) < (1ull << 24))
+        S = ldexpf((float)(uint32_t)(w.s24 >> (24 - w.mx)), -(int)w.mx);
+    else
+        S = wide_sequential_sum<Wide<P>::CHUNKS>(w.mx, row);
     float est = (float)((double)d.am / (double)S);
     if (est <= d.five_m) est = (float)((double)est - hb_bias_lookup(d.bias, est));
     return est;
+}
+
+// acc[c] = max over the rows of nb[0 .. len), chunks c0 .. c0 + CG - 1.  kChanged: rows of
+// the nodes in `bits` only.
+template <int P, Gather kGather>
+__device__ __forceinline__ void wide_gather(const uint8_t *__restrict__ in, const uint32_t *__restrict__ bits,
+                                            const uint32_t *__restrict__ nb, uint32_t len, int c0, HbAcc *acc,
+                                            unsigned long long &gathered)
+{
+    constexpr int CG = Wide<P>::CG, K = CG == 2 ? 4 : 2;  // rows in flight: eight 1 KiB loads
+    const uint32_t lane = threadIdx.x & (HB_WAVE - 1);
+    const uint64_t at = (uint64_t)c0 * 1024 + lane * 16;
+    for (uint32_t j0 = 0; j0 < len; j0 += HB_WAVE) {
+        // 64 ids at a time, a lane each; the listed ones of them become wave-uniform in turn
+        const uint32_t id = j0 + lane < len ? nb[j0 + lane] : 0u;
+        bool use = j0 + lane < len;
+        if (kGather == Gather::kChanged) use = use && bit_test(bits, id);
+        unsigned long long m = __ballot(use);
+        gathered += __popcll(m);
+        while (m) {
+            uint32_t v[K];
+#pragma unroll
+            for (int k = 0; k < K; ++k) {  // past the last one: the last again
+                v[k] = (uint32_t)__builtin_amdgcn_readlane((int)id, __ffsll(m) - 1);
+                if (m & (m - 1)) m &= m - 1;
+                else if (k == K - 1) m = 0;
+            }
+            uint4 r[K][CG];
+#pragma unroll
+            for (int k = 0; k < K; ++k)
+#pragma unroll
+                for (int c = 0; c < CG; ++c) r[k][c] = *(const uint4 *)(in + ((uint64_t)v[k] << P) + at + c * 1024);
+#pragma unroll
+            for (int k = 0; k < K; ++k)
+#pragma unroll
+                for (int c = 0; c < CG; ++c) hb_acc_max(acc[c], r[k][c]);
+        }
+    }
+}
+
+// acc[c] = max over the insertions of nbh[0 .. len) (iteration 1), chunk by chunk in the
+// wavefront's 1,024 LDS words
+template <int P>
+__device__ __forceinline__ void wide_first(uint32_t *lds, const uint32_t *__restrict__ nbh, uint32_t len, int c0,
+                                           HbAcc *acc)
+{
+    const uint32_t lane = threadIdx.x & (HB_WAVE - 1);
+    uint32_t idx = ~0u, rank = 0;
+    if (len <= HB_WAVE && lane < len) hb_index_rank(nbh[lane], P, &idx, &rank);
+#pragma unroll
+    for (int c = 0; c < Wide<P>::CG; ++c) {
+        for (int k = 0; k < 16; ++k) lds[k * HB_WAVE + lane] = 0u;
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        if (len <= HB_WAVE) {
+            if (idx / 1024 == (uint32_t)(c0 + c)) atomicMax(lds + idx % 1024, rank);
+        } else {
+            for (uint32_t j = lane; j < len; j += HB_WAVE) {
+                hb_index_rank(nbh[j], P, &idx, &rank);
+                if (idx / 1024 == (uint32_t)(c0 + c)) atomicMax(lds + idx % 1024, rank);
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        uint32_t w[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const uint4 x = *(const uint4 *)(lds + lane * 16 + 4 * q);
+            w[q] = x.x | (x.y << 8) | (x.z << 16) | (x.w << 24);
+        }
+        hb_acc_max(acc[c], make_uint4(w[0], w[1], w[2], w[3]));
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+}
+
+// the bound of all sketches packed as registers are (HbDev::sat_row), after the init
+__global__ __launch_bounds__(kBlock) void k_pack_bound(HbDev d)
+{
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= (1u << d.p) / 4) return;
+    const uint4 r = *(const uint4 *)(d.sat_max + 4 * i);
+    ((uint32_t *)d.sat_row)[i] = r.x | (r.y << 8) | (r.z << 16) | (r.w << 24);
 }
 
 template <int P>
@@ -786,7 +961,8 @@ __global__ __launch_bounds__(kBlock) void k_init_wide(HbDev d)
     if (u >= d.n) return;
     uint32_t idx, rank;
     hb_index_rank(d.node_id ? d.node_id[u] : u, P, &idx, &rank);
-    const bool isolated = d.off[u + 1] == d.off[u];
+    const uint32_t e0 = d.off[u], deg = d.off[u + 1] - e0;
+    const bool isolated = deg == 0;
     for (uint32_t c = 0; c < M / 1024; ++c) {
         const uint32_t base = c * 1024 + lane * 16;
         uint32_t w[4] = {0, 0, 0, 0};
@@ -799,97 +975,234 @@ __global__ __launch_bounds__(kBlock) void k_init_wide(HbDev d)
         d.est[u] = d.lc[M - 1];  // one non-zero register: linear counting with m-1 zeros
         d.dist[u] = 0.0;
         d.inv[u] = 0.0;
+        if (d.sat_max) {  // as k_init
+            const uint32_t w = d.sat_sym && deg == 1 ? d.nbr[e0] : 0u;
+            const bool alone = d.sat_sym && (deg == 0 || (deg == 1 && d.off[w + 1] - d.off[w] == 1));
+            if (!alone && d.sat_max[idx] < rank) atomicMax(d.sat_max + idx, rank);
+        }
     }
 }
 
-template <int P>
+// kNodes: the listed nodes; kHubs: hub nodes, whose rows come from the partial rows of their
+// tasks (list: the hubs, then each one's first task, then its number of tasks)
+enum class WideKind { kNodes, kHubs };
+
+template <int P, bool kFirst, WideKind kKind>
 __global__ __launch_bounds__(kBlock) void k_union_wide(HbDev d, const uint32_t *__restrict__ list,
-                                                       uint32_t count, int slot_id)
+                                                       const uint32_t *__restrict__ htask0,
+                                                       const uint32_t *__restrict__ hntask, uint32_t count,
+                                                       int slot_id)
 {
-    constexpr uint32_t M = 1u << P;
+    using W = Wide<P>;
     const HbIterState *st = d.st;
     if (st->done) return;
-    __shared__ uint32_t hist[kBlock / HB_WAVE][64];
+    constexpr bool kHash = kFirst && kKind == WideKind::kNodes;
+    __shared__ __attribute__((aligned(16))) uint32_t s_first[kHash ? kBlock * 16 : 4];
     const uint32_t it = st->iter;
-    const double t = st->t, inv_t = st->inv_t;
-    const uint8_t *__restrict__ in = st->parity ? d.regs1 : d.regs0;
-    uint8_t *out = st->parity ? d.regs0 : d.regs1;
-    const uint32_t *__restrict__ bitsR = (it & 1u) ? d.bits0 : d.bits1;
-    uint32_t *bitsW = (it & 1u) ? d.bits1 : d.bits0;
-    const bool use_frontier = d.frontier && it > 1 && !st->skip_scan;
     const uint32_t lane = threadIdx.x & (HB_WAVE - 1), w = threadIdx.x / HB_WAVE;
-    uint32_t *h = hist[w];
-    unsigned long long c_inc = 0, c_arcs = 0, c_nodes = 0, c_chg = 0;
+    uint32_t *lds = s_first + (kHash ? w * 1024 : 0);
+    HbView v{};
+    v.off = d.off;
+    v.in = st->parity ? d.regs1 : d.regs0;
+    v.out = st->parity ? d.regs0 : d.regs1;
+    v.dist = d.dist;
+    v.inv = d.inv;
+    v.bitsR = (it & 1u) ? d.bits0 : d.bits1;
+    v.bitsW = (it & 1u) ? d.bits1 : d.bits0;
+    v.t = st->t;
+    v.inv_t = st->inv_t;
+    v.use_frontier = d.frontier && it > 1 && !st->skip_scan;
+    v.sym = d.sat_sym != 0;
+    if (d.sat_max && !kFirst) {
+        v.satR = hb_saturated(d, it - 1);
+        v.satW = hb_saturated(d, it);
+        v.sat_scan = st->sat_scan != 0;
+    }
+    HbCounts cn;
+    unsigned long long c_gathered = 0;
 
     for (uint32_t i = blockIdx.x * (kBlock / HB_WAVE) + w; i < count; i += gridDim.x * (kBlock / HB_WAVE)) {
-        const uint32_t u = list[i];
+        const uint32_t u = __builtin_amdgcn_readfirstlane(list[i]);
         const uint32_t e0 = d.off[u], deg = d.off[u + 1] - e0;
         const uint32_t *__restrict__ nb = d.nbr + e0;
-        bool active = true;
-        if (use_frontier) {
-            uint32_t any = 0;
-            for (uint32_t j = lane; j < deg; j += HB_WAVE) any |= bit_test(bitsR, nb[j]);
-            active = hb_copy_or<HB_WAVE>(any) != 0;
-        }
-        const uint8_t *own_row = in + ((uint64_t)u << P);
-        uint8_t *out_row = out + ((uint64_t)u << P);
-        if (!active) {
-            if (bit_test(bitsR, u))
-                for (uint32_t c = 0; c < M / 1024; ++c)
-                    *(uint4 *)(out_row + c * 1024 + lane * 16) = *(const uint4 *)(own_row + c * 1024 + lane * 16);
+        const uint8_t *own_row = v.in + ((uint64_t)u << P) + lane * 16;
+        uint8_t *out_row = v.out + ((uint64_t)u << P) + lane * 16;
+        const uint8_t *bound = d.sat_row + lane * 16;
+        const uint32_t t0 = kKind == WideKind::kHubs ? htask0[i] : 0u, nt = kKind == WideKind::kHubs ? hntask[i] : 0u;
+        if (v.satR && bit_test(v.satR, u)) {  // nothing can change; keep both buffers complete
+            if (bit_test(v.bitsR, u))
+                for (int c = 0; c < W::CHUNKS; ++c) *(uint4 *)(out_row + c * 1024) = *(const uint4 *)(bound + c * 1024);
             continue;
         }
-        h[lane] = 0u;
-        uint32_t diffw = 0;
-        for (uint32_t c = 0; c < M / 1024; ++c) {
-            const uint32_t off16 = c * 1024 + lane * 16;
-            const uint4 own = *(const uint4 *)(own_row + off16);
-            HbAcc pa = hb_acc(own);
-            for (uint32_t j = 0; j < deg; ++j) hb_acc_max(pa, *(const uint4 *)(in + ((uint64_t)nb[j] << P) + off16));
-            const uint4 acc = hb_acc_get(pa);
-            diffw |= (acc.x != own.x) | (acc.y != own.y) | (acc.z != own.z) | (acc.w != own.w);
-            *(uint4 *)(out_row + off16) = acc;
-            hist_add_word(h, acc.x);
-            hist_add_word(h, acc.y);
-            hist_add_word(h, acc.z);
-            hist_add_word(h, acc.w);
+        bool sat = false;
+        uint32_t scanned = deg;
+        if constexpr (kKind == WideKind::kNodes) {
+            if (v.sat_scan) {
+                uint32_t k = 0;
+                sat = sat_neighbour<HB_WAVE>(v.satR, nb, deg, lane, k);
+                if (sat) scanned = k;
+            }
         }
-        const bool changed = hb_copy_or<HB_WAVE>(diffw) != 0;
-        const float curr = estimate_wide<P>(d, h, out_row);
+        bool active = true;
+        if (kKind == WideKind::kHubs) {
+            uint32_t any = 0;
+            for (uint32_t j = lane; j < nt; j += HB_WAVE) any |= d.chunk_flag[t0 + j];
+            active = hb_copy_or<HB_WAVE>(any) != 0;
+        } else if (v.use_frontier && !sat) {
+            uint32_t any = 0;
+            for (uint32_t j = lane; j < deg; j += HB_WAVE) any |= bit_test(v.bitsR, nb[j]);
+            active = hb_copy_or<HB_WAVE>(any) != 0;
+        }
+        if (!active) {
+            if (bit_test(v.bitsR, u))
+                for (int c = 0; c < W::CHUNKS; ++c) *(uint4 *)(out_row + c * 1024) = *(const uint4 *)(own_row + c * 1024);
+            continue;
+        }
+        WideSum sum;
+        uint32_t diffw = 0;  // bit 0: a register rose; bit 1: one is below the bound
+        uint4 row[W::CG];    // the last pass's chunks: all of the row up to p = 12
+        for (int c0 = 0; c0 < W::CHUNKS; c0 += W::CG) {
+            if (sat) {
+#pragma unroll
+                for (int c = 0; c < W::CG; ++c) row[c] = *(const uint4 *)(bound + (c0 + c) * 1024);
+                diffw = 1u;
+            } else {
+                HbAcc acc[W::CG];
+                uint4 own[W::CG];
+#pragma unroll
+                for (int c = 0; c < W::CG; ++c) {
+                    own[c] = *(const uint4 *)(own_row + (c0 + c) * 1024);
+                    acc[c] = hb_acc(own[c]);
+                }
+                unsigned long long g = 0;
+                if constexpr (kKind == WideKind::kHubs) {
+                    for (uint32_t j = 0; j < nt; ++j)
+                        if (d.chunk_flag[t0 + j])
+#pragma unroll
+                            for (int c = 0; c < W::CG; ++c)
+                                hb_acc_max(acc[c], *(const uint4 *)(d.scratch + ((uint64_t)(t0 + j) << P) +
+                                                                    (c0 + c) * 1024 + lane * 16));
+                } else if constexpr (kFirst) {
+                    wide_first<P>(lds, d.orig + e0, deg, c0, acc);
+                } else if (v.use_frontier) {
+                    wide_gather<P, Gather::kChanged>(v.in, v.bitsR, nb, deg, c0, acc, g);
+                } else {
+                    wide_gather<P, Gather::kAll>(v.in, nullptr, nb, deg, c0, acc, g);
+                }
+                if (c0 == 0) c_gathered += g;
+#pragma unroll
+                for (int c = 0; c < W::CG; ++c) {
+                    row[c] = hb_acc_get(acc[c]);
+                    diffw |= (row[c].x != own[c].x) | (row[c].y != own[c].y) | (row[c].z != own[c].z) |
+                             (row[c].w != own[c].w);
+                    if (v.satR) {
+                        const uint4 f = *(const uint4 *)(bound + (c0 + c) * 1024);
+                        diffw |= ((row[c].x != f.x) | (row[c].y != f.y) | (row[c].z != f.z) | (row[c].w != f.w)) << 1;
+                    }
+                }
+            }
+#pragma unroll
+            for (int c = 0; c < W::CG; ++c) {
+                *(uint4 *)(out_row + (c0 + c) * 1024) = row[c];
+                sum.add(row[c]);
+            }
+        }
+        sum.reduce();
+        diffw = hb_copy_or<HB_WAVE>(diffw);
+        const float curr = wide_estimate<P>(d, sum, [&](int c) {
+            if constexpr (W::PASSES == 1) {
+                uint4 x = row[0];
+#pragma unroll
+                for (int k = 1; k < W::CG; ++k)
+                    if (c == k) x = row[k];
+                return x;
+            } else {
+                return *(const uint4 *)(out_row + c * 1024);  // this lane's own stores
+            }
+        });
         if (lane == 0) {
             const float prev = d.est[u];
-            if (accumulate(d, u, prev, curr, t, inv_t)) c_inc += 1;
+            if (accumulate(v, u, prev, curr)) cn.inc += 1;
             d.est[u] = curr;
-            if (changed) {
-                atomicOr(bitsW + (u >> 5), 1u << (u & 31u));
-                c_chg += 1;
+            if (diffw & 1u) {
+                atomicOr(v.bitsW + (u >> 5), 1u << (u & 31u));
+                cn.chg += 1;
             }
-            c_arcs += deg;
-            c_nodes += 1;
+            if (v.satR && !(diffw & 2u)) sat_mark(v, u, nb, deg, cn);
+            if (kKind == WideKind::kNodes) cn.arcs += scanned;
+            cn.nodes += 1;
         }
     }
-    block_add(c_inc, c_arcs, c_nodes, c_chg, c_arcs, 0, d, slot_id);  // gathers every row
+    block_add(cn.inc, cn.arcs, cn.nodes, cn.chg, lane == 0 ? c_gathered : 0, cn.sat, d, slot_id);
+}
+
+// one task of a hub's list: a wavefront per pass of its partial row
+template <int P, bool kFirst>
+__global__ __launch_bounds__(kBlock) void k_chunk_wide(HbDev d, const uint32_t *__restrict__ tnode,
+                                                       const uint32_t *__restrict__ tbeg,
+                                                       const uint32_t *__restrict__ tend, uint32_t ntasks)
+{
+    using W = Wide<P>;
+    const HbIterState *st = d.st;
+    if (st->done) return;
+    __shared__ __attribute__((aligned(16))) uint32_t s_first[kFirst ? kBlock * 16 : 4];
+    const uint32_t it = st->iter;
+    const uint32_t lane = threadIdx.x & (HB_WAVE - 1), w = threadIdx.x / HB_WAVE;
+    const uint8_t *__restrict__ in = st->parity ? d.regs1 : d.regs0;
+    const uint32_t *__restrict__ bitsR = (it & 1u) ? d.bits0 : d.bits1;
+    const bool use_frontier = d.frontier && it > 1 && !st->skip_scan;
+    const uint32_t *satR = d.sat_max && !kFirst ? hb_saturated(d, it - 1) : nullptr;
+    const bool sat_scan = satR && st->sat_scan;
+    unsigned long long c_arcs = 0, c_gathered = 0;
+    for (uint32_t i = blockIdx.x * (kBlock / HB_WAVE) + w; i < ntasks * W::PASSES; i += gridDim.x * (kBlock / HB_WAVE)) {
+        const uint32_t task = __builtin_amdgcn_readfirstlane(i / W::PASSES);
+        const int c0 = (int)(i % W::PASSES) * W::CG;
+        const uint32_t eb = tbeg[task], len = tend[task] - eb;
+        const uint32_t *__restrict__ nb = d.nbr + eb;
+        bool active = !(satR && bit_test(satR, tnode[task]));
+        uint32_t scanned = len;
+        const bool sat = active && sat_scan && sat_neighbour<HB_WAVE>(satR, nb, len, lane, scanned);
+        if (active && use_frontier && !sat) {
+            uint32_t any = 0;
+            for (uint32_t j = lane; j < len; j += HB_WAVE) any |= bit_test(bitsR, nb[j]);
+            active = hb_copy_or<HB_WAVE>(any) != 0;
+        }
+        if (lane == 0 && c0 == 0) d.chunk_flag[task] = active ? 1u : 0u;
+        if (!active) continue;
+        uint8_t *out = d.scratch + ((uint64_t)task << P) + c0 * 1024 + lane * 16;
+        if (c0 == 0) c_arcs += sat ? scanned : len;
+        if (sat) {  // the hub becomes the bound through this task
+#pragma unroll
+            for (int c = 0; c < W::CG; ++c)
+                *(uint4 *)(out + c * 1024) = *(const uint4 *)(d.sat_row + (c0 + c) * 1024 + lane * 16);
+            continue;
+        }
+        HbAcc acc[W::CG];
+#pragma unroll
+        for (int c = 0; c < W::CG; ++c) acc[c] = hb_acc(make_uint4(0, 0, 0, 0));
+        unsigned long long g = 0;
+        if constexpr (kFirst) wide_first<P>(s_first + w * 1024, d.orig + eb, len, c0, acc);
+        else if (use_frontier) wide_gather<P, Gather::kChanged>(in, bitsR, nb, len, c0, acc, g);
+        else wide_gather<P, Gather::kAll>(in, nullptr, nb, len, c0, acc, g);
+        if (c0 == 0) c_gathered += g;
+#pragma unroll
+        for (int c = 0; c < W::CG; ++c) *(uint4 *)(out + c * 1024) = hb_acc_get(acc[c]);
+    }
+    block_add(0, lane == 0 ? c_arcs : 0, 0, 0, lane == 0 ? c_gathered : 0, 0, d, HB_SLOT_CHUNK);
 }
 
 template <int P>
 __global__ __launch_bounds__(kBlock) void k_estimates_wide(HbDev d, const uint8_t *__restrict__ regs,
                                                            float *__restrict__ out)
 {
-    constexpr uint32_t M = 1u << P;
-    __shared__ uint32_t hist[kBlock / HB_WAVE][64];
     const uint32_t lane = threadIdx.x & (HB_WAVE - 1), w = threadIdx.x / HB_WAVE;
-    uint32_t *h = hist[w];
     for (uint32_t u = blockIdx.x * (kBlock / HB_WAVE) + w; u < d.n; u += gridDim.x * (kBlock / HB_WAVE)) {
-        const uint8_t *row = regs + ((uint64_t)u << P);
-        h[lane] = 0u;
-        for (uint32_t c = 0; c < M / 1024; ++c) {
-            const uint4 r = *(const uint4 *)(row + c * 1024 + lane * 16);
-            hist_add_word(h, r.x);
-            hist_add_word(h, r.y);
-            hist_add_word(h, r.z);
-            hist_add_word(h, r.w);
-        }
-        const float e = estimate_wide<P>(d, h, row);
+        const uint8_t *row = regs + ((uint64_t)u << P) + lane * 16;
+        WideSum sum;
+#pragma unroll 4
+        for (int c = 0; c < Wide<P>::CHUNKS; ++c) sum.add(*(const uint4 *)(row + c * 1024));
+        sum.reduce();
+        const float e = wide_estimate<P>(d, sum, [&](int c) { return *(const uint4 *)(row + c * 1024); });
         if (lane == 0) out[u] = e;
     }
 }
@@ -1088,6 +1401,7 @@ hipError_t launch_init(const HbDev &d, hipStream_t s)
         HB_DISPATCH_WIDE(d.p, {
             k_init_wide<P><<<(unsigned)(((uint64_t)d.n * HB_WAVE + kBlock - 1) / kBlock), kBlock, 0, s>>>(d);
         });
+        if (d.sat_max) k_pack_bound<<<((1u << d.p) / 4 + kBlock - 1) / kBlock, kBlock, 0, s>>>(d);
         return hipGetLastError();
     }
     // k_init stores the linear-counting estimate of m - 1 zeros for every node; it is what
@@ -1129,8 +1443,9 @@ hipError_t launch_iteration(const HbDev &d, const HbSchedule &sc, bool first, bo
         if (ev) (void)hipEventRecord(ev[2 * b], s);
         if (d.p > 10) {
             HB_DISPATCH_WIDE(d.p, {
-                k_union_wide<P><<<grid_for((uint64_t)sc.bin_count[b] * HB_WAVE, sc.max_blocks), kBlock, 0, s>>>(
-                    d, sc.bin_list[b], sc.bin_count[b], b);
+                auto *nodes = first ? k_union_wide<P, true, WideKind::kNodes> : k_union_wide<P, false, WideKind::kNodes>;
+                nodes<<<grid_for((uint64_t)sc.bin_count[b] * HB_WAVE, sc.max_blocks), kBlock, 0, s>>>(
+                    d, sc.bin_list[b], nullptr, nullptr, sc.bin_count[b], b);
                 e = hipGetLastError();
             });
         } else {
@@ -1151,7 +1466,22 @@ hipError_t launch_iteration(const HbDev &d, const HbSchedule &sc, bool first, bo
         if (ev) (void)hipEventRecord(ev[2 * b + 1], s);
         if (e != hipSuccess) return e;
     }
-    if (sc.ntasks) {
+    if (sc.ntasks && d.p > 10) {
+        HB_DISPATCH_WIDE(d.p, {
+            auto *chunk = first ? k_chunk_wide<P, true> : k_chunk_wide<P, false>;
+            auto *hubs = first ? k_union_wide<P, true, WideKind::kHubs> : k_union_wide<P, false, WideKind::kHubs>;
+            if (ev) (void)hipEventRecord(ev[2 * HB_SLOT_CHUNK], s);
+            chunk<<<grid_for((uint64_t)sc.ntasks * Wide<P>::PASSES * HB_WAVE, sc.max_blocks), kBlock, 0, s>>>(
+                d, sc.task_node, sc.task_beg, sc.task_end, sc.ntasks);
+            if (ev) (void)hipEventRecord(ev[2 * HB_SLOT_CHUNK + 1], s);
+            if (ev) (void)hipEventRecord(ev[2 * HB_SLOT_MERGE], s);
+            hubs<<<grid_for((uint64_t)sc.nhubs * HB_WAVE, sc.max_blocks), kBlock, 0, s>>>(
+                d, sc.hub_node, sc.hub_task0, sc.hub_ntask, sc.nhubs, HB_SLOT_MERGE);
+            if (ev) (void)hipEventRecord(ev[2 * HB_SLOT_MERGE + 1], s);
+        });
+        e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    } else if (sc.ntasks) {
         HB_DISPATCH_P(d.p, {
             if (ev) (void)hipEventRecord(ev[2 * HB_SLOT_CHUNK], s);
             auto *chunk = first ? k_chunk<P, true> : k_chunk<P, false>;

@@ -43,7 +43,7 @@ def _graph(hb, kind):  # noqa: F811
 
 
 @pytest.mark.parametrize("kind", ["pairs", "triangles", "doubled", "hubs", "directed"])
-@pytest.mark.parametrize("p", [4, 6, 7, 8, 10])
+@pytest.mark.parametrize("p", [4, 6, 7, 8, 10, 11, 13])
 def test_saturation_matches_oracle(hb, oracle, kind, p):  # noqa: F811
     g = _graph(hb, kind)
     say("saturation", kind, p, g.size(), g.width())
@@ -54,7 +54,7 @@ def test_saturation_matches_oracle(hb, oracle, kind, p):  # noqa: F811
         with hb.HyperBall(g, p, **kw) as h:
             _assert_same(h, want, oracle, p, f"{kind} p={p} {kw}")
             scanned = sum(h.stats.kernel_arcs[s] for s in range(4))
-        if kind in ("pairs", "hubs") and kw == dict(layout="degree"):
+        if p <= 10 and kind in ("pairs", "hubs") and kw == dict(layout="degree"):
             # the search ends early for most nodes of the iterations after saturation
             with hb.HyperBall(g, p, dense=True, **kw) as full:
                 assert scanned < 0.9 * sum(full.stats.kernel_arcs[s] for s in range(4))
