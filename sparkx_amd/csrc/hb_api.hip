@@ -380,56 +380,32 @@ int hb_set_layout(hb_ctx *c, int layout)
 }  // extern "C"
 
 namespace {
-// Two pinned host buffers shared by every staging call of the process (allocated on
-// first use, kept to the end: pinning host pages costs milliseconds per call);
-// g_pin_mu serialises the calls that use them.
-constexpr size_t kPinElems = size_t(8) << 20;  // u32 per buffer (32 MiB)
-std::mutex g_pin_mu;
-uint32_t *g_pin[2] = {nullptr, nullptr};
-
-// dst[i] = src[pos + i] as u32 for i < len, split over host threads; returns the
-// first arc index whose neighbour is >= n, or UINT64_MAX
-uint64_t convert_neighbours(const void *nbrs, int nbr_bytes, uint64_t pos, uint64_t len, uint64_t n,
-                            uint32_t *dst)
+// to[i - a] = neighbour i as u32 for a <= i < b; false if one of them is >= n
+bool convert_neighbours(const void *nbrs, int nbr_bytes, uint64_t a, uint64_t b, uint64_t n, uint32_t *to)
 {
-    auto run = [&](uint64_t a, uint64_t b) -> uint64_t {
-        uint64_t bad = UINT64_MAX;
-        if (nbr_bytes == 8) {
-            const uint64_t *src = (const uint64_t *)nbrs + pos;
-            for (uint64_t i = a; i < b; ++i) {
-                const uint64_t v = src[i];
-                if (v >= n && bad == UINT64_MAX) bad = pos + i;
-                dst[i] = (uint32_t)v;
-            }
-        } else {
-            const uint32_t *src = (const uint32_t *)nbrs + pos;
-            uint32_t hi = 0;
-            for (uint64_t i = a; i < b; ++i) {
-                const uint32_t v = src[i];
-                hi = std::max(hi, v);
-                dst[i] = v;
-            }
-            if (hi >= n)
-                for (uint64_t i = a; i < b; ++i)
-                    if (src[i] >= n) return pos + i;
+    uint64_t hi = 0;
+    if (nbr_bytes == 8) {
+        const uint64_t *src = (const uint64_t *)nbrs;
+        for (uint64_t i = a; i < b; ++i) {
+            hi = std::max(hi, src[i]);
+            to[i - a] = (uint32_t)src[i];
         }
-        return bad;
-    };
-    const unsigned hw = std::max(1u, std::min(8u, std::thread::hardware_concurrency()));
-    const unsigned T = len >= (1u << 20) ? hw : 1u;
-    if (T == 1) return run(0, len);
-    std::vector<uint64_t> bad(T, UINT64_MAX);
-    std::vector<std::thread> pool;
-    for (unsigned t = 0; t < T; ++t)
-        pool.emplace_back([&, t] { bad[t] = run(len * t / T, len * (t + 1) / T); });
-    for (auto &th : pool) th.join();
-    return *std::min_element(bad.begin(), bad.end());
+    } else {
+        const uint32_t *src = (const uint32_t *)nbrs;
+        uint32_t h = 0;
+        for (uint64_t i = a; i < b; ++i) {
+            h = std::max(h, src[i]);
+            to[i - a] = src[i];
+        }
+        hi = h;
+    }
+    return b == a || hi < n;
 }
 }  // namespace
 
 extern "C" {
 
-// Copies offsets/neighbours into HBM through two pinned staging buffers, converting
+// Copies offsets/neighbours into HBM through pinned memory, converting
 // to u32 and validating on the way (every neighbour id < n, offsets monotone).
 int hb_stage_csr(hb_ctx *c, const void *offsets, int off_bytes, uint64_t n, const void *nbrs,
                  int nbr_bytes, uint64_t arcs)
@@ -464,47 +440,21 @@ int hb_stage_csr(hb_ctx *c, const void *offsets, int off_bytes, uint64_t n, cons
     HB_TRY(c->nbr.ensure(arcs));
     HB_TRY(hipMemcpyAsync(c->off.ptr, h_off.data(), (n + 1) * 4, hipMemcpyHostToDevice, c->stream));
 
-    int rc = HB_OK;
     if (arcs) {
-        std::lock_guard<std::mutex> lock(g_pin_mu);
-        hipEvent_t done[2] = {nullptr, nullptr};
-        for (int b = 0; b < 2 && rc == HB_OK; ++b) {
-            if (!g_pin[b] && hipHostMalloc((void **)&g_pin[b], kPinElems * 4, hipHostMallocPortable) != hipSuccess) {
-                g_pin[b] = nullptr;
-                rc = fail(HB_ENOMEM, "hipHostMalloc of %zu bytes failed", kPinElems * 4);
-            } else if (hipEventCreateWithFlags(&done[b], hipEventDisableTiming) != hipSuccess) {
-                rc = fail(HB_EHIP, "hipEventCreate failed");
+        bool refused = false;
+        HB_TRY(hb::upload_by(
+            c->nbr.ptr, arcs, 4, c->stream,
+            [&](char *to, size_t a, size_t b) { return convert_neighbours(nbrs, nbr_bytes, a, b, n, (uint32_t *)to); },
+            &refused));
+        if (refused)  // the first of them, as a sequential check would find it
+            for (uint64_t i = 0; i < arcs; ++i) {
+                const uint64_t v = nbr_bytes == 8 ? ((const uint64_t *)nbrs)[i] : ((const uint32_t *)nbrs)[i];
+                if (v >= n)
+                    return fail(HB_EINVAL, "hb_stage_csr: neighbour %llu at arc %llu is not < n=%llu",
+                                (unsigned long long)v, (unsigned long long)i, (unsigned long long)n);
             }
-        }
-        uint64_t pos = 0;
-        int b = 0;
-        while (rc == HB_OK && pos < arcs) {
-            const uint64_t len = std::min<uint64_t>(kPinElems, arcs - pos);
-            if (hipEventSynchronize(done[b]) != hipSuccess) {  // the copy out of g_pin[b] is done
-                rc = fail(HB_EHIP, "hipEventSynchronize failed");
-                break;
-            }
-            const uint64_t bad_at = convert_neighbours(nbrs, nbr_bytes, pos, len, n, g_pin[b]);
-            if (bad_at != UINT64_MAX) {
-                const uint64_t v = nbr_bytes == 8 ? ((const uint64_t *)nbrs)[bad_at] : ((const uint32_t *)nbrs)[bad_at];
-                rc = fail(HB_EINVAL, "hb_stage_csr: neighbour %llu at arc %llu is not < n=%llu", (unsigned long long)v,
-                          (unsigned long long)bad_at, (unsigned long long)n);
-                break;
-            }
-            if (hipMemcpyAsync(c->nbr.ptr + pos, g_pin[b], len * 4, hipMemcpyHostToDevice, c->stream) != hipSuccess ||
-                hipEventRecord(done[b], c->stream) != hipSuccess) {
-                rc = fail(HB_EHIP, "staging copy failed");
-                break;
-            }
-            pos += len;
-            b ^= 1;
-        }
-        (void)hipStreamSynchronize(c->stream);  // no copy still reads the shared buffers
-        for (int i = 0; i < 2; ++i)
-            if (done[i]) (void)hipEventDestroy(done[i]);
     }
-    if (rc != HB_OK) return rc;
-    if (int rc2 = finish_stage(c, n, arcs, &h_off)) return rc2;
+    if (int rc = finish_stage(c, n, arcs, &h_off)) return rc;
     g_err.clear();
     return HB_OK;
 }
@@ -688,14 +638,12 @@ static int copy_out(hb_ctx *c, const void *src, void *dst, size_t row_bytes)
 {
     const size_t bytes = (size_t)c->n * row_bytes;
     if (!c->relabelled()) {
-        HB_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream));
-        HB_TRY(hipStreamSynchronize(c->stream));
+        HB_TRY(hb::read_back(dst, src, bytes, c->stream));
         return HB_OK;
     }
     HB_TRY(c->readback.ensure(bytes));
     HB_TRY(hb::unpermute_rows(src, c->readback.ptr, c->sigma.ptr, (uint32_t)c->n, row_bytes, c->stream));
-    HB_TRY(hipMemcpyAsync(dst, c->readback.ptr, bytes, hipMemcpyDeviceToHost, c->stream));
-    HB_TRY(hipStreamSynchronize(c->stream));
+    HB_TRY(hb::read_back(dst, c->readback.ptr, bytes, c->stream));
     return HB_OK;
 }
 
@@ -1531,7 +1479,7 @@ extern "C" int hb_stage_mtx(hb_ctx *c, const char *text, uint64_t len, hb_mtx_in
     const uint64_t body = len - h.body;
     uint8_t *dtext = nullptr;
     HB_TRY(hipMalloc(&dtext, std::max<uint64_t>(body, 1)));
-    hipError_t e = body ? hipMemcpyAsync(dtext, text + h.body, body, hipMemcpyDefault, c->stream) : hipSuccess;
+    hipError_t e = hb::upload(dtext, text + h.body, body, c->stream);
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (e == hipSuccess) e = hipEventCreate(&e0);
     if (e == hipSuccess) e = hipEventCreate(&e1);
@@ -1613,12 +1561,12 @@ extern "C" int hb_read_csr(hb_ctx *c, uint64_t *offsets, uint64_t *nbrs)
     if (!c) return fail(HB_EINVAL, "hb_read_csr: ctx is NULL");
     if (!c->off.ptr) return fail(HB_ESTATE, "hb_read_csr: no graph staged");
     if (offsets)
-        for (uint64_t i = 0; i <= c->n; ++i) offsets[i] = c->h_off[i];
+        hb::host_parallel(c->n + 1, [&](size_t a, size_t b) {
+            for (size_t i = a; i < b; ++i) offsets[i] = c->h_off[i];
+        });
     if (nbrs && c->arcs) {
         if (!set_device(c)) return fail(HB_EHIP, "hipSetDevice failed");
-        std::vector<uint32_t> tmp(c->arcs);
-        HB_TRY(hipMemcpy(tmp.data(), c->nbr.ptr, c->arcs * 4, hipMemcpyDeviceToHost));
-        for (uint64_t i = 0; i < c->arcs; ++i) nbrs[i] = tmp[i];
+        HB_TRY(hb::read_back_u64(nbrs, c->nbr.ptr, c->arcs, c->stream));
     }
     g_err.clear();
     return HB_OK;

@@ -1187,8 +1187,7 @@ static int batch_copy_out(hb_batch *b, int graph, const void *src, void *dst, si
     const size_t bytes = (size_t)g.n * row_bytes;
     if (b->readback.count < bytes) HB_BTRY(b->readback.alloc(bytes));
     HB_BTRY(hb::unpermute_rows(src, b->readback.ptr, b->sigma.ptr + g.node_base, g.n, row_bytes, b->stream));
-    HB_BTRY(hipMemcpyAsync(dst, b->readback.ptr, bytes, hipMemcpyDeviceToHost, b->stream));
-    HB_BTRY(hipStreamSynchronize(b->stream));
+    HB_BTRY(hb::read_back(dst, b->readback.ptr, bytes, b->stream));
     return HB_OK;
 }
 

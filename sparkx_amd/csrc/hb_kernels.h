@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <functional>
+
 #include "hb_device.h"
 #include "../../include/sparkx_hb.h"
 
@@ -121,6 +123,19 @@ hipError_t launch_surrogate_tail(struct ::hb_mlp *n, const uint32_t *off, const 
                                  uint32_t infer_nodes, bool standardized_x, float *x_dev, float *out_dev,
                                  hipStream_t s);
 int mlp_device(const struct ::hb_mlp *n);
+// Copies between host and device memory (hb_transfer.cpp), synchronous unless stated.
+hipError_t read_back(void *dst, const void *src, size_t bytes, hipStream_t s);
+// device u32 -> host u64
+hipError_t read_back_u64(uint64_t *dst, const uint32_t *src, size_t count, hipStream_t s);
+// not synchronous for memory that is short or known to HIP: src stays valid until s is synchronised
+hipError_t upload(void *dst, const void *src, size_t bytes, hipStream_t s);
+// dst[0 .. count) elements of `out` bytes each, written to pinned memory by get(to, first,
+// last) on several threads, each for its own range; get returns false to refuse its input
+// (*refused, dst then incomplete)
+hipError_t upload_by(void *dst, size_t count, size_t out, hipStream_t s,
+                     const std::function<bool(char *, size_t, size_t)> &get, bool *refused);
+// fn(first, last) over [0, count) on several host threads
+void host_parallel(size_t count, const std::function<void(size_t, size_t)> &fn);
 // frees the device memory exact_bfs keeps between calls (not what a call is using)
 void release_held();
 // exact BFS sums of sources [s_begin, s_end) over a staged CSR (hb_exact.hip), h_off

@@ -224,10 +224,14 @@ class HyperBall:
 
     # hyper_ball.rs:272-280
     def geodesic_distances(self) -> np.ndarray:
-        return self._accumulators()[0]
+        dist = np.empty(self.g.size(), np.float64)
+        _lib.check(self._L.hb_read_accumulators(self._ctx, _lib.ptr(dist, C.c_double), None))
+        return dist
 
     def harmonic_geodesic_distances(self) -> np.ndarray:
-        return self._accumulators()[1]
+        inv = np.empty(self.g.size(), np.float64)
+        _lib.check(self._L.hb_read_accumulators(self._ctx, None, _lib.ptr(inv, C.c_double)))
+        return inv
 
     # hyper_ball.rs:260-270: assert!(node_id < self.g.size())
     def get_geodesic_distance(self, node_id: int) -> float:
