@@ -63,7 +63,10 @@ static constexpr int kQueues = kBatchNP * kClasses;
 struct HbBatchRec {  // counters of one iteration of one graph
     unsigned long long inc, chg, arcs, nodes, gathered;
     unsigned long long sat;  // degrees of the nodes that became saturated
+    unsigned long long pad[2];
 };
+static constexpr uint32_t kCountWords = 6, kCountCopies = 16;
+static_assert(sizeof(HbBatchRec) == 64, "a copy of a graph's counters is half a cache line");
 
 struct HbBatchGraph {
     uint64_t off_base, nbr_base, reg_base, node_base, bits_base;
@@ -77,8 +80,8 @@ struct HbBatchGraph {
     HbIterState st;
 };
 
-// a tile of one precision: `team` lanes per node over lists[first ..
-// first + count) (graph-local ids), or, with team == 0, hub chunk task `first`
+// a tile of one precision: `team` lanes per node over the nodes first .. first + count - 1
+// (a degree bin is one id range), or, with team == 0, hub chunk task `first`
 struct HbBatchTile {
     uint32_t graph, first, count, team;
 };
@@ -100,9 +103,9 @@ struct HbBatchDev {
     HbBatchGraph *g;
     uint32_t ngraphs;
     HbBatchRec *rec;
+    HbBatchRec *counts;         // kCountCopies per graph, zero between iterations
     const uint32_t *active;     // per class: tiles of running graphs, at class_base[q]
     const uint32_t *active_count;  // [kQueues]
-    const uint32_t *lists;
     const HbBatchTask *tasks;
     uint8_t *scratch;           // kScrRow bytes per task
     uint32_t *chunk_flag;       // 1 if the task was recomputed this iteration
@@ -186,13 +189,12 @@ __device__ __forceinline__ HbView batch_view(const HbBatchDev &b, const HbBatchG
 }
 
 template <int P, int T, bool kFirst>
-__device__ __forceinline__ void batch_nodes(const HbView &v, const HbTables &tb, const uint32_t *list,
-                                            uint32_t count, HbCounts &c)
+__device__ __forceinline__ void batch_nodes(const HbView &v, const HbTables &tb, uint32_t first, uint32_t count,
+                                            HbCounts &c)
 {
-    const uint32_t lane = threadIdx.x & (HB_WAVE - 1);
     auto run = [&](auto gather) {
-        for (uint32_t i = lane / T; i < count; i += HB_WAVE / T)
-            union_node<P, T, decltype(gather)::value>(v, tb, list[i], lane % T, c);
+        for (uint32_t i = 0; i < count; i += HB_WAVE / T)
+            union_wave<P, T, decltype(gather)::value>(v, tb, first + i, count - i, c);
     };
     if constexpr (kFirst) run(std::integral_constant<Gather, Gather::kFirst>{});
     else if (v.gather_bits) run(std::integral_constant<Gather, Gather::kChanged>{});
@@ -254,6 +256,10 @@ __device__ __forceinline__ void batch_chunk(const HbBatchDev &b, const HbView &v
         ((uint64_t *)&name##_bias)[i_] = ((const uint64_t *)((b).bias + ((P) - kBatchPMin)))[i_]; \
     __syncthreads();
 
+// Global wavefront index and count of the grid (wave-uniform).
+__device__ __forceinline__ uint32_t wave_id() { return __builtin_amdgcn_readfirstlane(blockIdx.x * (kBatchBlock / HB_WAVE) + threadIdx.x / HB_WAVE); }
+__device__ __forceinline__ uint32_t wave_count() { return gridDim.x * (kBatchBlock / HB_WAVE); }
+
 __device__ __forceinline__ void wave_sum_counts(HbCounts &c)
 {
 #pragma unroll
@@ -267,8 +273,11 @@ __device__ __forceinline__ void wave_sum_counts(HbCounts &c)
     }
 }
 
-__device__ __forceinline__ void add_counts(HbBatchRec *r, const HbCounts &c)
+// into the copy of the graph's counters that the wavefront's number selects (k_batch_finalize
+// adds them up): thousands of tiles per graph would queue on one record
+__device__ __forceinline__ void add_counts(const HbBatchDev &b, uint32_t graph, const HbCounts &c)
 {
+    HbBatchRec *r = b.counts + (uint64_t)graph * kCountCopies + wave_id() % kCountCopies;
     if (c.inc) atomicAdd(&r->inc, c.inc);
     if (c.chg) atomicAdd(&r->chg, c.chg);
     if (c.arcs) atomicAdd(&r->arcs, c.arcs);
@@ -276,10 +285,6 @@ __device__ __forceinline__ void add_counts(HbBatchRec *r, const HbCounts &c)
     if (c.gathered) atomicAdd(&r->gathered, c.gathered);
     if (c.sat) atomicAdd(&r->sat, c.sat);
 }
-
-// Global wavefront index and count of the grid (wave-uniform).
-__device__ __forceinline__ uint32_t wave_id() { return __builtin_amdgcn_readfirstlane(blockIdx.x * (kBatchBlock / HB_WAVE) + threadIdx.x / HB_WAVE); }
-__device__ __forceinline__ uint32_t wave_count() { return gridDim.x * (kBatchBlock / HB_WAVE); }
 
 // Union over the active node tiles of one (precision P, team width T) class.  Every
 // loop has a trip count fixed by the active list and its tiles (at most 4096 nodes).
@@ -301,9 +306,9 @@ __global__ __launch_bounds__(kBatchBlock) __attribute__((amdgpu_waves_per_eu(P >
         const HbTables tb = {tbl_lc, &tbl_bias, g.am, g.five_m, g.lc_thr};
         const HbView v = batch_view(b, g, tile.graph, s_first);
         HbCounts c;
-        batch_nodes<P, T, kFirst>(v, tb, b.lists + tile.first, tile.count, c);
+        batch_nodes<P, T, kFirst>(v, tb, tile.first, tile.count, c);
         wave_sum_counts(c);
-        if (lane == 0) add_counts(ring_rec(b, g, g.st.iter), c);
+        if (lane == 0) add_counts(b, tile.graph, c);
     }
 }
 
@@ -323,7 +328,7 @@ __global__ __launch_bounds__(kBatchBlock) __attribute__((amdgpu_waves_per_eu(P >
         HbCounts c;
         batch_chunk<P, kFirst>(b, v, tile.first, wave_uniform(b.tasks[tile.first]), c);
         wave_sum_counts(c);
-        if (lane == 0) add_counts(ring_rec(b, g, g.st.iter), c);
+        if (lane == 0) add_counts(b, tile.graph, c);
     }
 }
 
@@ -404,12 +409,16 @@ __global__ __launch_bounds__(kBatchBlock) void k_batch_merge(HbBatchDev b, HbBat
             if (accumulate(v, u, prev, curr)) c.inc += 1;
             v.est[u] = curr;
             if (changed) {
-                atomicOr(v.bitsW + (u >> 5), 1u << (u & 31u));
+                bit_set(v.bitsW, u);
                 c.chg += 1;
             }
-            if (sat && !(diffw & 2u)) sat_mark(v, u, v.nbr + v.off[u], v.off[u + 1] - v.off[u], c);
+            const uint32_t e0 = v.off[u], deg = v.off[u + 1] - e0;
+            if (sat && !(diffw & 2u) && sat_allowed(v, v.nbr + e0, deg)) {
+                bit_set(v.satW, u);
+                c.sat += deg;
+            }
             c.nodes += 1;
-            add_counts(ring_rec(b, g, g.st.iter), c);
+            add_counts(b, hub.graph, c);
         }
     }
 }
@@ -441,30 +450,42 @@ __global__ __launch_bounds__(64) void k_batch_bound(HbBatchDev b)
     ((uint32_t *)(b.bound + (uint64_t)gi * kScrRow))[i] = r[0] | (r[1] << 8) | (r[2] << 16) | (r[3] << 24);
 }
 
-// end of an iteration for every running graph (hyper_ball.rs:833-849)
-__global__ void k_batch_finalize(HbBatchDev b)
+// end of an iteration, one wavefront per graph: the counter copies summed into the ring record
+// and cleared, then the stopping rule (hyper_ball.rs:833-849)
+__global__ __launch_bounds__(HB_WAVE) void k_batch_finalize(HbBatchDev b)
 {
-    const uint32_t gi = blockIdx.x * blockDim.x + threadIdx.x;
-    if (gi >= b.ngraphs) return;
+    const uint32_t gi = blockIdx.x, lane = threadIdx.x;
     HbBatchGraph &g = b.g[gi];
     HbIterState &st = g.st;
     if (st.done) return;
     const uint32_t it = st.iter;
-    const HbBatchRec &r = *ring_rec(b, g, it);
+    constexpr uint32_t kWords = sizeof(HbBatchRec) / 8, kRows = HB_WAVE / kWords;
+    unsigned long long t = 0, *words = (unsigned long long *)(b.counts + (uint64_t)gi * kCountCopies);
+#pragma unroll
+    for (uint32_t k = lane / kWords; k < kCountCopies; k += kRows) {
+        t += words[k * kWords + lane % kWords];
+        words[k * kWords + lane % kWords] = 0ull;
+    }
+#pragma unroll
+    for (uint32_t o = kWords; o < HB_WAVE; o <<= 1) t += __shfl_xor(t, o);
+    HbBatchRec &r = *ring_rec(b, g, it);
+    if (lane < kCountWords) (&r.inc)[lane] = t;
+    const unsigned long long inc = __shfl(t, 0), chg = __shfl(t, 1), sat = __shfl(t, 5);
+    if (lane != 0) return;
     const bool truncated = st.max_iters && it >= st.max_iters;
-    if (r.inc == 0 || truncated || it >= g.cap) {
+    if (inc == 0 || truncated || it >= g.cap) {
         st.done = 1;
         st.executed = it;
-        st.converged = r.inc == 0;
-        g.overflow = r.inc != 0 && !truncated;
+        st.converged = inc == 0;
+        g.overflow = inc != 0 && !truncated;
         return;
     }
     st.iter = it + 1;
     st.parity ^= 1u;
     st.t = st.t + 1.0;
     st.inv_t = __ddiv_rn(1.0, st.t);
-    st.skip_scan = 2 * r.chg > (unsigned long long)g.n_linked;
-    st.sat_arcs += r.sat;  // as k_finalize
+    st.skip_scan = 2 * chg > (unsigned long long)g.n_linked;
+    st.sat_arcs += sat;  // as k_finalize
     st.sat_scan = 8 * st.sat_arcs >= (unsigned long long)g.n_linked;
 }
 
@@ -557,12 +578,14 @@ struct hb_batch {
     uint64_t total_nodes = 0, total_arcs = 0, total_regs = 0, total_words = 0;
     // CSRs in each graph's degree order, the caller's ids (orig per arc, perm per node)
     // and the inverse numbering (sigma: caller's node -> device node)
-    DevArr<uint32_t> off, nbr, orig, perm, sigma, lists, chunk_flag;
+    DevArr<uint32_t> off, nbr, orig, perm, sigma, chunk_flag;
     // cleared at the start of a run: changed nodes and saturated nodes (2 bitmaps of
-    // total_words each), then every graph's bound of all sketches (kScrRow u32)
+    // total_words each), then every graph's bound of all sketches (kScrRow u32) and its
+    // counter copies
     DevArr<uint32_t> bits;
     DevArr<uint8_t> bound;
-    size_t bits_count() const { return 4 * total_words + hg.size() * hb::kScrRow; }
+    size_t count_at() const { return (4 * total_words + hg.size() * hb::kScrRow + 15) & ~(size_t)15; }
+    size_t bits_count() const { return count_at() + hg.size() * hb::kCountCopies * sizeof(hb::HbBatchRec) / 4; }
     uint32_t *sat_max(size_t gi) const { return bits.ptr + 4 * total_words + gi * hb::kScrRow; }
     DevArr<uint32_t> active, active_count;  // per class: tiles of running graphs
     DevArr<uint8_t> regs0, regs1, scratch, readback;
@@ -642,7 +665,6 @@ static int build_tiles(hb_batch *b)
         hb::HbBatchTile t;
         uint64_t work;
     };
-    std::vector<uint32_t> lists;
     std::vector<hb::HbBatchTask> tasks;
     std::vector<Item> items[hb::kQueues];
     std::vector<hb::HbBatchHub> hubs[hb::kBatchNP];
@@ -677,14 +699,13 @@ static int build_tiles(hb_batch *b)
             while (i < bins[k].size()) {
                 Item it{};
                 it.t.graph = (uint32_t)gi;
-                it.t.first = (uint32_t)lists.size();
+                it.t.first = bins[k][i];  // degrees descend with the id
                 it.t.team = teams[k];
                 uint64_t arcs = 0;
                 uint32_t cnt = 0;
                 // a tile holds whole waves' worth of nodes until it has tile_arcs arcs
                 while (i < bins[k].size() && (arcs < b->tile_arcs || cnt % per_wave) && cnt < 4096) {
                     const uint32_t u = bins[k][i++];
-                    lists.push_back(u);
                     arcs += off[u + 1] - off[u] + 8;
                     ++cnt;
                 }
@@ -694,7 +715,6 @@ static int build_tiles(hb_batch *b)
             }
         }
     }
-    HB_BTRY(b->lists.put(lists, b->stream));
     HB_BTRY(b->tasks.put(tasks, b->stream));
     b->ntasks = (uint32_t)tasks.size();
     HB_BTRY(b->scratch.alloc((size_t)b->ntasks * hb::kScrRow));
@@ -938,9 +958,9 @@ int hb_batch_run(hb_batch *b, uint32_t flags, hb_batch_stats *stats)
     d.g = b->g.ptr;
     d.ngraphs = (uint32_t)ng;
     d.rec = b->rec.ptr;
+    d.counts = (hb::HbBatchRec *)(b->bits.ptr + b->count_at());
     d.active = b->active.ptr;
     d.active_count = b->active_count.ptr;
-    d.lists = b->lists.ptr;
     d.tasks = b->tasks.ptr;
     d.scratch = b->scratch.ptr;
     d.chunk_flag = b->chunk_flag.ptr;
@@ -1020,7 +1040,7 @@ int hb_batch_run(hb_batch *b, uint32_t flags, hb_batch_stats *stats)
         }
 #undef HB_BATCH_P
 #undef HB_BATCH_LAUNCH
-        hb::k_batch_finalize<<<(ng + 63) / 64, 64, 0, b->stream>>>(d);
+        hb::k_batch_finalize<<<ng, HB_WAVE, 0, b->stream>>>(d);
         const hipError_t el = hipGetLastError();
         return e != hipSuccess ? e : el;
     };

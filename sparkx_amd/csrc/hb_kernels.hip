@@ -496,31 +496,28 @@ __device__ __forceinline__ void stage_bound(const HbDev &d, uint32_t *s)
 // union over the neighbours of listed nodes; a team of T lanes per node
 // (T = G: one sketch copy; T > G: S = T/G copies split the neighbours)
 // ---------------------------------------------------------------------------
-// Wavefronts per SIMD: the gathers are latency-bound, so more wavefronts in flight
-// help until the register bound makes the compiler spill.  8 (at most 64 VGPRs) took the
-// k-mer graph (p = 6, four-lane teams in the degree layout) from 59.5 to 49.5 ms per run.
-// At p >= 7 the one-copy bins run at 8 too since their per-lane counters are 32-bit
-// (HbCounts): 64 VGPRs without a spill, R-MAT-24's degree <= 256 bin 2.145 -> 2.130 ms per
-// launch against 7 (with 64-bit counters 8 spilled: 41.8 ms per run against 41.0 at 7).
-// The teams of 32 and 64 lanes spill 10-12 VGPRs at 72 (6 with the 32-bit counters); at 6
-// (80 VGPRs) they do not, and R-MAT-24's degree 257..4096 bins run 1-2% faster (with the
-// 32-bit counters, 7 still leaves the run 0.2-0.3% slower).  At p <= 6 one-copy teams run at 7 (no spill, where 8
-// spilled 7 VGPRs): ER (n = 65,536, p = 6) 44.7 -> 43.5 us per launch; the k-mer graph's
-// dense iterations run k_union_rows instead.
+// Wavefronts per SIMD: the gathers are latency-bound, so more wavefronts in flight help until
+// the register bound makes the compiler spill.  8 (at most 64 VGPRs) took the k-mer graph
+// (p = 6, four-lane teams in the degree layout) from 59.5 to 49.5 ms per run.  The one-copy
+// bins run at 7: at 8, with the saturation checks, they spill 36 VGPRs and R-MAT-24's dense
+// iterations (p = 7) take 8.13 ms against 7.97 at 7 and 8.02 at 6.  The teams of 32 and 64
+// lanes run at 6 at p >= 7 (80 VGPRs, no spill).  The k-mer graph's dense iterations run
+// k_union_rows instead.
 template <int P, int T, bool kFirst>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(P >= 7 ? (T >= 32 ? 6 : 8) : (T == (1 << P) / 16 ? 7 : 8)))) void k_union(
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(P >= 7 && T >= 32 ? 6 : T == (1 << P) / 16 ? 7 : 8))) void k_union(
     HbDev d, const uint32_t *__restrict__ list, uint32_t base, uint32_t count, int slot_id)
 {
     const HbIterState *st = d.st;
     if (st->done) return;
     if constexpr (!kFirst && T == (1 << P) / 16 && (P == 5 || P == 6))
         if (d.rows && !list && (base & 63u) == 0 && rows_iteration(d, *st)) return;  // k_union_rows runs it
-    HB_TABLES_LDS(P, d, tb)
     const uint32_t it = st->iter;
     if (st->push) {  // only the bin's nodes with a changed neighbour (k_push_compact)
         list = d.dyn_list + d.dyn_base[slot_id];
         count = d.dyn_count[slot_id];
     }
+    if (blockIdx.x * (kBlock / T) >= count) return;  // most blocks of a push iteration
+    HB_TABLES_LDS(P, d, tb)
     HbView v;
     v.off = d.off;
     v.nbr = d.nbr;
@@ -571,8 +568,19 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(P >= 7 ?
         }
     }
     auto run = [&](auto gather) {
-        for (uint32_t team = blockIdx.x * (kBlock / T) + threadIdx.x / T; team < count; team += teams_per_grid)
-            union_node<P, T, decltype(gather)::value>(v, tb, list ? list[team] : base + team, tl, c);
+        constexpr Gather kGather = decltype(gather)::value;
+        if (list) {
+            for (uint32_t team = blockIdx.x * (kBlock / T) + threadIdx.x / T; team < count; team += teams_per_grid) {
+                const uint32_t u = list[team];
+                const uint32_t r = union_node<P, T, kGather>(v, tb, u, tl, c);
+                if (tl == 0 && (r & kChangedBit)) bit_set(v.bitsW, u);
+                if (tl == 0 && (r & kSaturatedBit)) bit_set(v.satW, u);
+            }
+        } else {
+            const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / HB_WAVE);
+            for (uint32_t t0 = blockIdx.x * (kBlock / T) + wave * (HB_WAVE / T); t0 < count; t0 += teams_per_grid)
+                union_wave<P, T, kGather>(v, tb, base + t0, count - t0, c);
+        }
     };
     if constexpr (kFirst) run(std::integral_constant<Gather, Gather::kFirst>{});
     else if (v.gather_bits) run(std::integral_constant<Gather, Gather::kChanged>{});
@@ -1128,7 +1136,10 @@ __global__ __launch_bounds__(kBlock) void k_union_wide(HbDev d, const uint32_t *
                 atomicOr(v.bitsW + (u >> 5), 1u << (u & 31u));
                 cn.chg += 1;
             }
-            if (v.satR && !(diffw & 2u)) sat_mark(v, u, nb, deg, cn);
+            if (v.satR && !(diffw & 2u) && sat_allowed(v, nb, deg)) {
+                bit_set(v.satW, u);
+                cn.sat += deg;
+            }
             if (kKind == WideKind::kNodes) cn.arcs += scanned;
             cn.nodes += 1;
         }
