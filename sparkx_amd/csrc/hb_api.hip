@@ -14,10 +14,12 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <map>
 #include <memory>
 #include <mutex>
 #include <string>
 #include <thread>
+#include <utility>
 #include <vector>
 
 #include "../../include/sparkx_hb.h"
@@ -181,9 +183,8 @@ struct hb_ctx {
     int p = 0;
     bool ran = false;
     DevBuf<uint8_t> regs0, regs1, scratch;
-    DevBuf<float> est, est_tmp, lc;
+    DevBuf<float> est, est_tmp;
     DevBuf<double> dist, inv, cent;
-    DevBuf<HbBiasTable> bias;
     DevBuf<uint32_t> sched_buf, chunk_flag;
     // per-node bitmaps of a run, cleared together: changed nodes (2), then active nodes of
     // push iterations (2) and saturated nodes (2) where they are used, then the bound of
@@ -246,10 +247,8 @@ struct hb_ctx {
         scratch.release();
         est.release();
         est_tmp.release();
-        lc.release();
         dist.release();
         inv.release();
-        bias.release();
         cent.release();
         bits.release();
         sched_buf.release();
@@ -568,6 +567,85 @@ static int build_schedule(hb_ctx *c, int p)
     return HB_OK;
 }
 
+namespace {
+// The estimator's tables of one precision on one device, the same for every run: the LC table
+// (f64 then f32, as m ln(m/z)) and the bias points.  Built on first use and kept to the end of
+// the process (0.7 MB for all precisions).
+struct DeviceTables {
+    float *lc = nullptr;
+    HbBiasTable *bias = nullptr;
+};
+
+hipError_t device_tables(int device, int p, const DeviceTables **out, hipStream_t s)
+{
+    static std::mutex mu;
+    static std::map<std::pair<int, int>, DeviceTables> made;
+    std::lock_guard<std::mutex> lk(mu);
+    const auto it = made.find({device, p});
+    if (it != made.end()) {
+        *out = &it->second;
+        return hipSuccess;
+    }
+    const uint32_t m = 1u << p;
+    std::vector<float> lc(m + 1, 0.0f);
+    for (uint32_t z = 1; z <= m; ++z) lc[z] = (float)((double)m * std::log((double)m / (double)z));
+    DeviceTables t;
+    hipError_t e = hipMalloc(&t.lc, (m + 1) * sizeof(float));
+    if (e == hipSuccess) e = hipMalloc(&t.bias, sizeof(HbBiasTable));
+    if (e == hipSuccess) e = hipMemcpyAsync(t.lc, lc.data(), (m + 1) * sizeof(float), hipMemcpyHostToDevice, s);
+    if (e == hipSuccess) e = hipMemcpyAsync(t.bias, hb::bias_table(p), sizeof(HbBiasTable), hipMemcpyHostToDevice, s);
+    // in place before a kernel of any stream reads them
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    if (e != hipSuccess) {
+        if (t.lc) (void)hipFree(t.lc);
+        if (t.bias) (void)hipFree(t.bias);
+        return e;
+    }
+    *out = &made.emplace(std::make_pair(device, p), t).first->second;
+    return hipSuccess;
+}
+
+// A run's ring of records in pinned memory.  Rings come from slabs that are kept to the end
+// of the process, one ring per run under way; one that ends early waits for its launches.
+std::mutex g_ring_mu;
+std::vector<HbIterRec *> g_rings;  // free ones
+
+struct RecordSlot {
+    HbIterRec *ring = nullptr;
+    hipStream_t stream = nullptr;
+
+    hipError_t take(hipStream_t s)
+    {
+        stream = s;
+        std::lock_guard<std::mutex> lk(g_ring_mu);
+        if (g_rings.empty()) {
+            constexpr size_t kSlab = 16;
+            HbIterRec *slab = nullptr;
+            const hipError_t e =
+                hipHostMalloc((void **)&slab, kSlab * HB_REC_RING * sizeof(HbIterRec), hipHostMallocPortable);
+            if (e != hipSuccess) return e;
+            for (size_t i = 0; i < kSlab; ++i) g_rings.push_back(slab + i * HB_REC_RING);
+        }
+        ring = g_rings.back();
+        g_rings.pop_back();
+        for (int i = 0; i < HB_REC_RING; ++i) ring[i].iter = 0;
+        return hipSuccess;
+    }
+    void give()  // no launch can write it any more
+    {
+        if (!ring) return;
+        std::lock_guard<std::mutex> lk(g_ring_mu);
+        g_rings.push_back(ring);
+        ring = nullptr;
+    }
+    ~RecordSlot()
+    {
+        if (ring) (void)hipStreamSynchronize(stream);
+        give();
+    }
+};
+}  // namespace
+
 static float alpha_f32(uint32_t m)
 {
     if (m == 16) return 0.673f;
@@ -687,9 +765,11 @@ extern "C" int hb_run(hb_ctx *c, int p, int max_iters, uint32_t flags, hb_stats 
     // cannot change a register after its diameter, so n + 2 iterations bound a correct
     // run; the host loop stops there with an error rather than going on.
     const uint64_t bound = max_iters > 0 ? (uint64_t)max_iters : (uint64_t)c->n + 2;
-    HB_TRY(c->rec.ensure(HB_REC_RING));
-    HB_TRY(c->lc.ensure(m + 1));
-    HB_TRY(c->bias.ensure(1));
+    HB_TRY(c->rec.ensure(1));
+    const DeviceTables *tables = nullptr;
+    HB_TRY(device_tables(c->device, p, &tables, c->stream));
+    RecordSlot records;
+    HB_TRY(records.take(c->stream));
     if (c->snap_k) HB_TRY(c->snaps.ensure((size_t)c->snap_k * c->n));
     const bool push_ok = c->sym && p <= 10;
     {
@@ -698,13 +778,6 @@ extern "C" int hb_run(hb_ctx *c, int p, int max_iters, uint32_t flags, hb_stats 
         if (rc == HB_OK) rc = build_schedule(c, p);
         if (rc != HB_OK) return rc;
     }
-
-    // host-computed constants: LC table (f64 then f32, as m ln(m/z)), alpha m^2, bias points
-    std::vector<float> lc(m + 1, 0.0f);
-    for (uint32_t z = 1; z <= m; ++z) lc[z] = (float)((double)m * std::log((double)m / (double)z));
-    HB_TRY(hipMemcpyAsync(c->lc.ptr, lc.data(), (m + 1) * 4, hipMemcpyHostToDevice, c->stream));
-    HB_TRY(hipMemcpyAsync(c->bias.ptr, hb::bias_table(p), sizeof(HbBiasTable), hipMemcpyHostToDevice,
-                          c->stream));
 
     // Saturation pays where most nodes come to hold the same sketch within a few iterations,
     // which the chain layout's graphs do not; its kernels and the dense schedule, which
@@ -740,8 +813,9 @@ extern "C" int hb_run(hb_ctx *c, int p, int max_iters, uint32_t flags, hb_stats 
     }
     d.st = c->st.ptr;
     d.rec = c->rec.ptr;
-    d.lc = c->lc.ptr;
-    d.bias = c->bias.ptr;
+    d.host_rec = records.ring;
+    d.lc = tables->lc;
+    d.bias = tables->bias;
     d.scratch = c->scratch.ptr;
     d.chunk_flag = c->chunk_flag.ptr;
     d.sym = push_ok ? 1 : 0;
@@ -775,14 +849,16 @@ extern "C" int hb_run(hb_ctx *c, int p, int max_iters, uint32_t flags, hb_stats 
     st0.max_iters = (uint32_t)max_iters;
     st0.t = 1.0;
     st0.inv_t = 1.0;
-    HB_TRY(hipMemcpyAsync(c->st.ptr, &st0, sizeof st0, hipMemcpyHostToDevice, c->stream));
     // iteration t marks the active bitmap iteration t - 1 cleared; both start clear
-    HB_TRY(hb::launch_fill(c->bits.ptr, all_words, 0u, c->stream));
+    HB_TRY(hb::launch_start(c->st.ptr, st0, c->bits.ptr, all_words, c->stream));
 
-    hipEvent_t e0, e1, e2;
+    // ends of the batches of launches in flight; the one the run stopped in ends ms_total
+    constexpr uint32_t kInFlight = 3;
+    hipEvent_t e0, e1, eb[kInFlight + 1];
     HB_TRY(hipEventCreate(&e0));
     HB_TRY(hipEventCreate(&e1));
-    HB_TRY(hipEventCreate(&e2));
+    for (auto &ev : eb) HB_TRY(hipEventCreate(&ev));
+    hipEvent_t e2 = nullptr;
     std::vector<float> iter_ms;
     int rc = HB_OK;
     hipGraphExec_t gexec = nullptr;
@@ -793,13 +869,14 @@ extern "C" int hb_run(hb_ctx *c, int p, int max_iters, uint32_t flags, hb_stats 
     if (ktiming && (flags & HB_FLAG_GRAPH)) {
         (void)hipEventDestroy(e0);
         (void)hipEventDestroy(e1);
-        (void)hipEventDestroy(e2);
+        for (auto ev : eb) (void)hipEventDestroy(ev);
         return fail(HB_EINVAL, "hb_run: HB_FLAG_KTIMING cannot be combined with HB_FLAG_GRAPH");
     }
-    // timing: each launch of a check's batch has its own pair of events around the
-    // iteration and, with HB_FLAG_KTIMING, its own events around each kernel slot; they
-    // are read after the check, so timing adds no host round trip per iteration
-    constexpr uint32_t kMaxBatch = 8;  // launches between two checks
+    // timing: each launch of a batch has its own pair of events around the iteration and,
+    // with HB_FLAG_KTIMING, its own events around each kernel slot; they are read when the
+    // batch has ended and before the next one starts, so timing adds one host round trip per
+    // batch
+    constexpr uint32_t kMaxBatch = 8;  // launches of a batch
     const uint32_t per_it = 2 + (ktiming ? 2 * HB_NSLOT : 0);
     std::vector<hipEvent_t> tev(timing ? (size_t)kMaxBatch * per_it : 0, nullptr);
     double kms[HB_NSLOT] = {};
@@ -828,69 +905,91 @@ extern "C" int hb_run(hb_ctx *c, int p, int max_iters, uint32_t flags, hb_stats 
                 break;
             }
         }
-        // iterations: launches after convergence return at once (done flag), so a
-        // batch can run ahead of the host's check; each check drains the finished
-        // iterations' records from the device ring into c->h_rec (index t)
+        // iterations: launches after convergence return at once (done flag), so the host
+        // launches ahead of what it has seen: single iterations, two more in flight, while
+        // the run is short, then batches of 8, one more in flight (within HB_REC_RING).  It
+        // waits for the oldest batch's event and reads the records its iterations left in the
+        // ring (into c->h_rec, index t).  Nothing is launched past max_iters.
+        struct Batch {
+            uint32_t first, count;  // iterations first .. first + count - 1
+            hipEvent_t end;
+        };
+        std::vector<Batch> flying;
         uint64_t launched = 0;
-        HbIterState hs{};
-        uint32_t drained = 0;
-        HbIterRec ring[HB_REC_RING];
+        uint32_t nth = 0;
+        bool done = false;
+        HbIterRec last{};
         c->h_rec.assign(1, HbIterRec{});
-        for (;;) {
-            const uint32_t k = launched < 8 ? 2u : kMaxBatch;
-            if (launched >= bound + 16) {
-                rc = fail(HB_ESTATE, "hb_run: still changing after %llu iterations", (unsigned long long)launched);
+        while (!done) {
+            const uint32_t ahead = timing ? 0u : launched < 8 ? kInFlight - 1 : 1u;
+            uint32_t k = timing ? (launched < 8 ? 2u : kMaxBatch) : launched < 8 ? 1u : kMaxBatch;
+            if (max_iters > 0) k = (uint32_t)std::min<uint64_t>(k, (uint64_t)max_iters - launched);
+            if (k && flying.size() <= ahead) {
+                if (launched >= bound + 24) {
+                    rc = fail(HB_ESTATE, "hb_run: still changing after %llu iterations", (unsigned long long)launched);
+                    break;
+                }
+                for (uint32_t i = 0; i < k && rc == HB_OK; ++i) {
+                    hipEvent_t *ev = timing ? &tev[(size_t)i * per_it] : nullptr;
+                    if (ev) (void)hipEventRecord(ev[0], c->stream);
+                    const bool first = launched + i == 0;  // not part of the captured iteration
+                    e = gexec && !first
+                            ? hipGraphLaunch(gexec, c->stream)
+                            : hb::launch_iteration(d, c->sched, first, nf, c->stream, ktiming ? ev + 2 : nullptr);
+                    if (e != hipSuccess) rc = fail(HB_EHIP, "iteration launch: %s", hipGetErrorString(e));
+                    if (ev) (void)hipEventRecord(ev[1], c->stream);
+                }
+                if (rc != HB_OK) break;
+                flying.push_back({(uint32_t)launched + 1, k, eb[nth++ % (kInFlight + 1)]});
+                launched += k;
+                if (hipEventRecord(flying.back().end, c->stream) != hipSuccess) {
+                    rc = fail(HB_EHIP, "event record failed");
+                    break;
+                }
+                if (flying.size() <= ahead) continue;
+            }
+            if (flying.empty()) {  // max_iters launched and none of them the last: cannot be
+                rc = fail(HB_ESTATE, "hb_run: %llu iterations did not stop", (unsigned long long)launched);
                 break;
             }
-            for (uint32_t i = 0; i < k && rc == HB_OK; ++i) {
-                hipEvent_t *ev = timing ? &tev[(size_t)i * per_it] : nullptr;
-                if (ev) (void)hipEventRecord(ev[0], c->stream);
-                const bool first = launched + i == 0;  // not part of the captured iteration
-                e = gexec && !first ? hipGraphLaunch(gexec, c->stream)
-                                    : hb::launch_iteration(d, c->sched, first, nf, c->stream, ktiming ? ev + 2 : nullptr);
-                if (e != hipSuccess) rc = fail(HB_EHIP, "iteration launch: %s", hipGetErrorString(e));
-                if (ev) (void)hipEventRecord(ev[1], c->stream);
-            }
-            launched += k;
-            if (rc != HB_OK) break;
-            if (hipMemcpyAsync(&hs, c->st.ptr, sizeof hs, hipMemcpyDeviceToHost, c->stream) != hipSuccess ||
-                hipMemcpyAsync(ring, c->rec.ptr, sizeof ring, hipMemcpyDeviceToHost, c->stream) != hipSuccess ||
-                hipStreamSynchronize(c->stream) != hipSuccess) {
+            const Batch b = flying.front();
+            flying.erase(flying.begin());
+            if (hipEventSynchronize(b.end) != hipSuccess) {
                 rc = fail(HB_EHIP, "iteration failed: %s", hipGetErrorString(hipGetLastError()));
                 break;
             }
-            const uint32_t finished = hs.done ? hs.executed : hs.iter - 1;
-            for (uint32_t t = drained + 1; t <= finished; ++t) c->h_rec.push_back(ring[t % HB_REC_RING]);
-            drained = finished;
-            if (timing) {
+            for (uint32_t t = b.first; t < b.first + b.count && !done; ++t) {
+                last = records.ring[t % HB_REC_RING];
+                if (last.iter != t) {
+                    rc = fail(HB_ESTATE, "hb_run: no record of iteration %u", t);
+                    break;
+                }
+                c->h_rec.push_back(last);
+                done = last.done != 0;
+                if (!timing) continue;
                 const uint32_t counts[HB_NSLOT] = {c->sched.bin_count[0], c->sched.bin_count[1],
                                                    c->sched.bin_count[2], c->sched.ntasks, c->sched.nhubs};
-                for (uint32_t i = 0; i < k; ++i) {
-                    // launch number launched - k + i + 1 ran iteration launched - k + i + 1
-                    // unless the run had stopped before it (it then returned at once)
-                    if (hs.done && launched - k + i + 1 > hs.executed) break;
-                    const hipEvent_t *ev = &tev[(size_t)i * per_it];
-                    float ms = 0.0f;
-                    (void)hipEventElapsedTime(&ms, ev[0], ev[1]);
-                    iter_ms.push_back(ms);
-                    if (!ktiming) continue;
-                    for (int sl = 0; sl < HB_NSLOT; ++sl) {
-                        if (!counts[sl]) continue;
-                        float kms1 = 0.0f;
-                        (void)hipEventElapsedTime(&kms1, ev[2 + 2 * sl], ev[3 + 2 * sl]);
-                        kms[sl] += kms1;
-                        klaunch[sl] += 1;
-                    }
+                const hipEvent_t *ev = &tev[(size_t)(t - b.first) * per_it];
+                float ms = 0.0f;
+                (void)hipEventElapsedTime(&ms, ev[0], ev[1]);
+                iter_ms.push_back(ms);
+                for (int sl = 0; sl < HB_NSLOT && ktiming; ++sl) {
+                    if (!counts[sl]) continue;
+                    float kms1 = 0.0f;
+                    (void)hipEventElapsedTime(&kms1, ev[2 + 2 * sl], ev[3 + 2 * sl]);
+                    kms[sl] += kms1;
+                    klaunch[sl] += 1;
                 }
             }
-            if (hs.done) break;
+            if (rc != HB_OK) break;
+            e2 = b.end;
         }
         if (rc != HB_OK) break;
-        if (hipEventRecord(e2, c->stream) != hipSuccess || hipEventSynchronize(e2) != hipSuccess) {
-            rc = fail(HB_EHIP, "event sync failed");
-            break;
-        }
-        c->h_st = hs;
+        c->h_st = HbIterState{};
+        c->h_st.iter = c->h_st.executed = last.iter;
+        c->h_st.done = 1;
+        c->h_st.converged = last.converged;
+        c->h_st.parity = (last.iter - 1) & 1u;  // every iteration but the last swapped the buffers
     } while (0);
     if (gexec) (void)hipGraphExecDestroy(gexec);
     if (graph) (void)hipGraphDestroy(graph);
@@ -903,8 +1002,9 @@ extern "C" int hb_run(hb_ctx *c, int p, int max_iters, uint32_t flags, hb_stats 
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    (void)hipEventDestroy(e2);
+    for (auto ev : eb) (void)hipEventDestroy(ev);
     if (rc != HB_OK) return rc;
+    records.give();  // launches still queued return without a record
 
     const uint32_t executed = c->h_st.executed;
     // snapshot rows past the last iteration repeat its estimates (the sketches stopped changing)
@@ -1189,12 +1289,8 @@ extern "C" int hb_restore(hb_ctx *c, int p, const uint8_t *regs, const double *d
     HB_TRY(c->dist.ensure(std::max<uint32_t>(n, 1)));
     HB_TRY(c->inv.ensure(std::max<uint32_t>(n, 1)));
     HB_TRY(c->cent.ensure(std::max<uint32_t>(n, 1)));
-    HB_TRY(c->lc.ensure(m + 1));
-    HB_TRY(c->bias.ensure(1));
-    std::vector<float> lc(m + 1, 0.0f);
-    for (uint32_t z = 1; z <= m; ++z) lc[z] = (float)((double)m * std::log((double)m / (double)z));
-    HB_TRY(hipMemcpyAsync(c->lc.ptr, lc.data(), (m + 1) * 4, hipMemcpyHostToDevice, c->stream));
-    HB_TRY(hipMemcpyAsync(c->bias.ptr, hb::bias_table(p), sizeof(HbBiasTable), hipMemcpyHostToDevice, c->stream));
+    const DeviceTables *tables = nullptr;
+    HB_TRY(device_tables(c->device, p, &tables, c->stream));
     if (n) {
         if (c->relabelled()) {  // device row i = the caller's row perm[i]
             HB_TRY(hipMemcpyAsync(c->regs1.ptr, regs, rbytes, hipMemcpyHostToDevice, c->stream));
@@ -1221,8 +1317,8 @@ extern "C" int hb_restore(hb_ctx *c, int p, const uint8_t *regs, const double *d
     d.regs1 = c->regs1.ptr;
     d.dist = c->dist.ptr;
     d.inv = c->inv.ptr;
-    d.lc = c->lc.ptr;
-    d.bias = c->bias.ptr;
+    d.lc = tables->lc;
+    d.bias = tables->bias;
     d.n = n;
     d.p = (uint32_t)p;
     d.am = alpha_f32(m) * ((float)m * (float)m);

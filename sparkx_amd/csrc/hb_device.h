@@ -41,9 +41,10 @@ struct HbIterState {
 #define HB_SLOT_CHUNK 3
 #define HB_SLOT_MERGE 4
 
-// Per-iteration records live in a ring of HB_REC_RING entries (iteration t in slot
-// t % HB_REC_RING, cleared when t begins); the host drains the finished ones at every
-// check, which it makes at most 8 launches apart, so a run has no iteration cap.
+// Per-iteration records live in a ring of HB_REC_RING entries in pinned host memory, iteration
+// t in slot t % HB_REC_RING, written by its k_finalize; the host, never more than 16 launches
+// ahead, reads the finished ones as their events complete, so a run has no iteration cap and
+// no copy waits for one.
 #define HB_REC_RING 64
 
 struct HbIterRec {  // per-iteration counters, per kernel slot
@@ -55,6 +56,7 @@ struct HbIterRec {  // per-iteration counters, per kernel slot
     unsigned long long sat;              // sum of the degrees of the nodes that became saturated
     unsigned long long nf_lo, nf_hi;     // N(t) * 2^40 as a 128-bit integer
     unsigned long long push;             // 1 if iteration t listed its nodes by push
+    uint32_t iter, done, converged, pad;  // t, and whether (and how) the run stopped with it
 };
 
 static_assert(offsetof(HbIterRec, gathered) == 4 * HB_NSLOT * sizeof(unsigned long long), "five runs of slots first");
@@ -76,7 +78,8 @@ struct HbDev {
     double *dist, *inv;    // accumulators
     uint32_t *bits0, *bits1;  // changed-node bitmaps (bit set: registers changed)
     HbIterState *st;
-    HbIterRec *rec;        // ring: iteration t in rec[t % HB_REC_RING]
+    HbIterRec *rec;        // the running iteration's N(t) and push flag
+    HbIterRec *host_rec;   // the ring
     unsigned long long *counts;  // the running iteration's counters, HB_COUNT_COPIES times
     const float *lc;       // lc[z] = (float)(m ln(m/z)), z = 1..m
     const HbBiasTable *bias;  // HLL++ bias windows for this p

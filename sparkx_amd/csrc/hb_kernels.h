@@ -42,6 +42,8 @@ void set_error(const char *msg);
 const HbBiasTable *bias_table(int p);
 
 hipError_t launch_init(const HbDev &d, hipStream_t s);
+// *st = st0 and p[0 .. count) = 0
+hipError_t launch_start(HbIterState *st, const HbIterState &st0, uint32_t *p, uint64_t count, hipStream_t s);
 hipError_t launch_fill(uint32_t *p, uint64_t count, uint32_t value, hipStream_t s);
 // one iteration; first: iteration 1, whose kernels hash ids
 // ev (nullable): 2 * HB_NSLOT events recorded around each kernel slot that launches

@@ -145,6 +145,15 @@ __global__ __launch_bounds__(kBlock) void k_fill_u32(uint32_t *p, uint64_t count
         p[i] = value;
 }
 
+// start of a run: its bitmaps and counters cleared, its state as of iteration 1
+__global__ __launch_bounds__(kBlock) void k_start(HbIterState *st, HbIterState st0, uint32_t *p, uint64_t count)
+{
+    if (blockIdx.x == 0 && threadIdx.x == 0) *st = st0;
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < count;
+         i += (uint64_t)gridDim.x * blockDim.x)
+        p[i] = 0u;
+}
+
 // ---------------------------------------------------------------------------
 // push iterations (symmetric graph, few changes at t-1): u must be recomputed
 // iff one of its neighbours changed, i.e. iff u is a neighbour of a changed node.
@@ -166,10 +175,9 @@ __global__ __launch_bounds__(kBlock) void k_begin(HbDev d, uint32_t words)
     uint32_t *bw = (it & 1u) ? d.bits1 : d.bits0;
     const bool push = st->push != 0;
     if (push && blockIdx.x == 0 && threadIdx.x < 3) d.dyn_count[threadIdx.x] = 0u;
-    if (blockIdx.x == 0 && threadIdx.x == 0) {  // this iteration's ring record, cleared
-        HbIterRec *r = d.rec + it % HB_REC_RING;
-        *r = HbIterRec{};
-        if (push) r->push = 1ull;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {  // this iteration's record
+        d.rec->nf_lo = d.rec->nf_hi = 0ull;
+        d.rec->push = push ? 1ull : 0ull;
     }
     uint32_t *next_active = d.active ? hb_active(d, it + 1) : nullptr;
     uint32_t *sat = d.sat_max ? hb_saturated(d, it) : nullptr;
@@ -1249,7 +1257,7 @@ __global__ __launch_bounds__(kBlock) void k_nf(HbDev d)
         lo = nlo;
     }
     if ((threadIdx.x & (HB_WAVE - 1)) == 0) {
-        HbIterRec *r = d.rec + st->iter % HB_REC_RING;
+        HbIterRec *r = d.rec;
         const unsigned long long old = atomicAdd(&r->nf_lo, lo);
         atomicAdd(&r->nf_hi, hi + ((old + lo) < old ? 1ull : 0ull));
     }
@@ -1264,14 +1272,14 @@ __global__ __launch_bounds__(kBlock) void k_snapshot(HbDev d)
     for (uint32_t u = blockIdx.x * blockDim.x + threadIdx.x; u < d.n; u += gridDim.x * blockDim.x) dst[u] = d.est[u];
 }
 
-// end of iteration t: the counter copies summed into the ring record and cleared, the
+// end of iteration t: the counter copies summed into the host's ring record and cleared, the
 // termination rule (hyper_ball.rs:833-849) and the buffer swap; one wavefront
 __global__ __launch_bounds__(HB_WAVE) void k_finalize(HbDev d)
 {
     HbIterState *st = d.st;
     if (st->done) return;
     const uint32_t it = st->iter, lane = threadIdx.x;
-    HbIterRec &rec = d.rec[it % HB_REC_RING];
+    HbIterRec &rec = d.host_rec[it % HB_REC_RING];
     constexpr uint32_t kCounts = 5 * HB_NSLOT + 1;
     static_assert(kCounts <= HB_COUNT_STRIDE && HB_COUNT_STRIDE <= HB_WAVE / 2, "a lane per counter, two copies at a time");
     const uint32_t at = lane % HB_COUNT_STRIDE;
@@ -1295,7 +1303,14 @@ __global__ __launch_bounds__(HB_WAVE) void k_finalize(HbDev d)
     };
     const unsigned long long inc = slots(0), chg = slots(3), sat = __shfl(t, 5 * HB_NSLOT);
     if (lane != 0) return;
-    if (inc == 0 || (st->max_iters && it >= st->max_iters)) {
+    const bool stop = inc == 0 || (st->max_iters && it >= st->max_iters);
+    rec.nf_lo = d.rec->nf_lo;
+    rec.nf_hi = d.rec->nf_hi;
+    rec.push = d.rec->push;
+    rec.iter = it;
+    rec.done = stop ? 1u : 0u;
+    rec.converged = inc == 0 ? 1u : 0u;
+    if (stop) {
         st->done = 1;
         st->executed = it;
         st->converged = inc == 0;
@@ -1431,6 +1446,12 @@ hipError_t launch_fill(uint32_t *p, uint64_t count, uint32_t value, hipStream_t 
 {
     if (count == 0) return hipSuccess;
     k_fill_u32<<<grid_for(count, 4096), kBlock, 0, s>>>(p, count, value);
+    return hipGetLastError();
+}
+
+hipError_t launch_start(HbIterState *st, const HbIterState &st0, uint32_t *p, uint64_t count, hipStream_t s)
+{
+    k_start<<<grid_for(count, 4096), kBlock, 0, s>>>(st, st0, p, count);
     return hipGetLastError();
 }
 
