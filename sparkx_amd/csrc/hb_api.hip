@@ -991,7 +991,10 @@ extern "C" int hb_run(hb_ctx *c, int p, int max_iters, uint32_t flags, hb_stats 
         c->h_st.converged = last.converged;
         c->h_st.parity = (last.iter - 1) & 1u;  // every iteration but the last swapped the buffers
     } while (0);
-    if (gexec) (void)hipGraphExecDestroy(gexec);
+    if (gexec) {  // not while iterations launched past the last one are queued
+        (void)hipStreamSynchronize(c->stream);
+        (void)hipGraphExecDestroy(gexec);
+    }
     if (graph) (void)hipGraphDestroy(graph);
     for (auto &ev : tev)
         if (ev) (void)hipEventDestroy(ev);
