@@ -21,12 +21,12 @@
 // single-graph kernels run, so each graph's registers, estimates, accumulators and
 // per-iteration increase counts are its own hb_run's.
 //
-// Per-iteration counters live in a ring of kRing records per graph; the host copies
-// the new ones out at every check (at most kCheck launches apart, fewer than kRing),
-// so a run has no record cap.  A graph cannot need more than n + 1 iterations (the
-// last one changes nothing), so a graph still running after n + 2 stops the run with
-// an error rather than letting the host loop go on.  With SPARKX_HB_TRACE set in the
-// environment every check prints a progress line to stderr.
+// Per-iteration counters go to a ring of kRing records per graph in pinned host memory; the
+// host launches a few iterations ahead of the one whose records it waits for, so a run has
+// no record cap and the GPU no gap at a check.  A graph cannot need more than n + 1
+// iterations (the last one changes nothing), so a graph still running after n + 2 stops the
+// run with an error rather than letting the host loop go on.  With SPARKX_HB_TRACE set in the
+// environment every iteration prints a progress line to stderr.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -54,7 +54,6 @@ static constexpr int kBatchPMin = 4, kBatchPMax = 8, kBatchNP = kBatchPMax - kBa
 // default is 4); a fifth stream would share a queue with another chain and run after it
 static constexpr int kSide = 4;
 static constexpr uint32_t kRing = 32;    // per-graph iteration records on the device
-static constexpr uint32_t kCheck = 8;    // launches between host checks (< kRing)
 static constexpr uint32_t kScrRow = 256; // scratch bytes per hub chunk (2^p, p <= 8)
 // work classes of one precision: node bins of team width G, 4G and 64, hub chunks
 static constexpr int kClasses = 4, kClassChunk = 3;
@@ -63,7 +62,11 @@ static constexpr int kQueues = kBatchNP * kClasses;
 struct HbBatchRec {  // counters of one iteration of one graph
     unsigned long long inc, chg, arcs, nodes, gathered;
     unsigned long long sat;  // degrees of the nodes that became saturated
-    unsigned long long pad[2];
+    // of a record (not of a copy of the counters): the iteration, whether the graph stopped
+    // with it, by the rule or at its iteration limit, or should have and did not
+    uint32_t iter;
+    uint16_t done, converged;
+    unsigned long long overflow;
 };
 static constexpr uint32_t kCountWords = 6, kCountCopies = 16;
 static_assert(sizeof(HbBatchRec) == 64, "a copy of a graph's counters is half a cache line");
@@ -73,7 +76,6 @@ struct HbBatchGraph {
     uint32_t n, p, n_linked, words;
     uint32_t ring_base;   // first of the graph's kRing records
     uint32_t cap;         // iterations after which a running graph is an error (n + 2)
-    uint32_t overflow;    // set when the graph reached cap without stopping
     uint32_t sym;         // v -> u for every u -> v
     float am, five_m;
     double lc_thr;
@@ -102,7 +104,8 @@ struct HbBatchDev {
     uint32_t *bits0, *bits1;
     HbBatchGraph *g;
     uint32_t ngraphs;
-    HbBatchRec *rec;
+    HbBatchRec *rec;            // kRing per graph, in pinned host memory
+    uint32_t *stopped;          // graphs stopped so far, then what each class's list knows of it
     HbBatchRec *counts;         // kCountCopies per graph, zero between iterations
     const uint32_t *active;     // per class: tiles of running graphs, at class_base[q]
     const uint32_t *active_count;  // [kQueues]
@@ -339,6 +342,10 @@ __global__ __launch_bounds__(1024) void k_batch_compact(HbBatchDev b, HbBatchCla
     __shared__ uint32_t s_wave[1024 / HB_WAVE];
     __shared__ uint32_t s_total;
     const HbBatchList l = cl.q[blockIdx.x];
+    // the list of an earlier iteration stands until another graph stops
+    uint32_t *seen = b.stopped + 1 + blockIdx.x;
+    const uint32_t now = *b.stopped + 1;
+    if (*seen == now) return;
     uint32_t *out = (uint32_t *)b.active + l.base;
     const uint32_t lane = threadIdx.x & (HB_WAVE - 1), wv = threadIdx.x / HB_WAVE;
     if (threadIdx.x == 0) s_total = 0;
@@ -360,7 +367,10 @@ __global__ __launch_bounds__(1024) void k_batch_compact(HbBatchDev b, HbBatchCla
         }
         __syncthreads();
     }
-    if (threadIdx.x == 0) ((uint32_t *)b.active_count)[blockIdx.x] = s_total;
+    if (threadIdx.x == 0) {
+        ((uint32_t *)b.active_count)[blockIdx.x] = s_total;
+        *seen = now;
+    }
 }
 
 // hubs of precision P: one wavefront per hub merges its own registers with the
@@ -424,20 +434,19 @@ __global__ __launch_bounds__(kBatchBlock) void k_batch_merge(HbBatchDev b, HbBat
 }
 
 // start of an iteration: for every running graph clear the bitmap this iteration
-// writes and its ring record, and carry the saturated nodes over
+// writes and carry the saturated nodes over
 __global__ __launch_bounds__(kBatchBlock) void k_batch_begin(HbBatchDev b)
 {
-    for (uint32_t gi = blockIdx.x; gi < b.ngraphs; gi += gridDim.x) {
+    for (uint32_t gi = blockIdx.x; gi < b.ngraphs; gi += gridDim.x) {  // blockIdx.y: its share of the words
         const HbBatchGraph &g = b.g[gi];
         if (g.st.done) continue;
         uint32_t *bw = ((g.st.iter & 1u) ? b.bits1 : b.bits0) + g.bits_base;
         uint32_t *sw = ((g.st.iter & 1u) ? b.sat1 : b.sat0) + g.bits_base;
         const uint32_t *sr = ((g.st.iter & 1u) ? b.sat0 : b.sat1) + g.bits_base;
-        for (uint32_t i = threadIdx.x; i < g.words; i += blockDim.x) {
+        for (uint32_t i = blockIdx.y * blockDim.x + threadIdx.x; i < g.words; i += gridDim.y * blockDim.x) {
             bw[i] = 0u;
             if (b.sat_max) sw[i] = sr[i];
         }
-        if (threadIdx.x == 0) *ring_rec(b, g, g.st.iter) = HbBatchRec{};
     }
 }
 
@@ -450,8 +459,8 @@ __global__ __launch_bounds__(64) void k_batch_bound(HbBatchDev b)
     ((uint32_t *)(b.bound + (uint64_t)gi * kScrRow))[i] = r[0] | (r[1] << 8) | (r[2] << 16) | (r[3] << 24);
 }
 
-// end of an iteration, one wavefront per graph: the counter copies summed into the ring record
-// and cleared, then the stopping rule (hyper_ball.rs:833-849)
+// end of an iteration, one wavefront per graph: the counter copies summed into the host's ring
+// record and cleared, then the stopping rule (hyper_ball.rs:833-849)
 __global__ __launch_bounds__(HB_WAVE) void k_batch_finalize(HbBatchDev b)
 {
     const uint32_t gi = blockIdx.x, lane = threadIdx.x;
@@ -470,14 +479,18 @@ __global__ __launch_bounds__(HB_WAVE) void k_batch_finalize(HbBatchDev b)
     for (uint32_t o = kWords; o < HB_WAVE; o <<= 1) t += __shfl_xor(t, o);
     HbBatchRec &r = *ring_rec(b, g, it);
     if (lane < kCountWords) (&r.inc)[lane] = t;
+    static_assert(offsetof(HbBatchRec, iter) == kCountWords * 8, "counters first");
     const unsigned long long inc = __shfl(t, 0), chg = __shfl(t, 1), sat = __shfl(t, 5);
     if (lane != 0) return;
     const bool truncated = st.max_iters && it >= st.max_iters;
-    if (inc == 0 || truncated || it >= g.cap) {
+    const bool stop = inc == 0 || truncated || it >= g.cap;
+    r.iter = it;
+    r.done = stop ? 1 : 0;
+    r.converged = inc == 0 ? 1 : 0;
+    r.overflow = stop && inc != 0 && !truncated ? 1ull : 0ull;
+    if (stop) {
         st.done = 1;
-        st.executed = it;
-        st.converged = inc == 0;
-        g.overflow = inc != 0 && !truncated;
+        atomicAdd(b.stopped, 1u);
         return;
     }
     st.iter = it + 1;
@@ -569,6 +582,8 @@ struct hb_batch {
     std::vector<std::pair<uint32_t, hipGraphExec_t>> execs;
     void drop_execs()
     {
+        // not while iterations launched past the last one are queued
+        if (!execs.empty()) (void)hipStreamSynchronize(stream);
         for (const auto &x : execs) (void)hipGraphExecDestroy(x.second);
         execs.clear();
     }
@@ -585,7 +600,8 @@ struct hb_batch {
     DevArr<uint32_t> bits;
     DevArr<uint8_t> bound;
     size_t count_at() const { return (4 * total_words + hg.size() * hb::kScrRow + 15) & ~(size_t)15; }
-    size_t bits_count() const { return count_at() + hg.size() * hb::kCountCopies * sizeof(hb::HbBatchRec) / 4; }
+    size_t stopped_at() const { return count_at() + hg.size() * hb::kCountCopies * sizeof(hb::HbBatchRec) / 4; }
+    size_t bits_count() const { return stopped_at() + 1 + hb::kQueues; }
     uint32_t *sat_max(size_t gi) const { return bits.ptr + 4 * total_words + gi * hb::kScrRow; }
     DevArr<uint32_t> active, active_count;  // per class: tiles of running graphs
     DevArr<uint8_t> regs0, regs1, scratch, readback;
@@ -593,7 +609,7 @@ struct hb_batch {
     DevArr<double> dist, inv;
     DevArr<HbBiasTable> bias_all;
     DevArr<hb::HbBatchGraph> g;
-    DevArr<hb::HbBatchRec> rec;
+    hb::HbBatchRec *rec = nullptr;  // kRing per graph, pinned: written by k_batch_finalize
     DevArr<hb::HbBatchTile> tiles[hb::kQueues];  // per (precision, class)
     DevArr<hb::HbBatchHub> hubs[hb::kBatchNP];
     DevArr<hb::HbBatchTask> tasks;
@@ -616,6 +632,7 @@ struct hb_batch {
             if (side[i]) (void)hipStreamDestroy(side[i]);
         }
         if (fork) (void)hipEventDestroy(fork);
+        if (rec) (void)hipHostFree(rec);
         if (stream) (void)hipStreamDestroy(stream);
     }
 };
@@ -831,7 +848,7 @@ int hb_batch_create(hb_batch **out, int device, const hb_graph_desc *graphs, int
     HB_BTRY(b->bound.alloc((size_t)count * hb::kScrRow));
     HB_BTRY(b->active_count.alloc(hb::kQueues));
     HB_BTRY(b->g.alloc(count));
-    HB_BTRY(b->rec.alloc((size_t)count * hb::kRing));
+    HB_BTRY(hipHostMalloc((void **)&b->rec, (size_t)count * hb::kRing * sizeof(hb::HbBatchRec), hipHostMallocPortable));
     // estimator tables of p = 4..8: LC values (f64 then f32, as m ln(m/z)) and bias windows
     std::vector<float> lc(hb::kLcTotal, 0.0f);
     for (int p = hb::kBatchPMin; p <= hb::kBatchPMax; ++p) {
@@ -936,7 +953,6 @@ int hb_batch_run(hb_batch *b, uint32_t flags, hb_batch_stats *stats)
         st.max_iters = (uint32_t)b->max_iters[i];
         st.t = 1.0;
         st.inv_t = 1.0;
-        init[i].overflow = 0;
         cap_max = std::max(cap_max, st.max_iters ? std::min(st.max_iters, init[i].cap) : init[i].cap);
     }
     hb::HbBatchDev d{};
@@ -957,7 +973,8 @@ int hb_batch_run(hb_batch *b, uint32_t flags, hb_batch_stats *stats)
     d.sat_max = (flags & HB_FLAG_DENSE) ? nullptr : b->sat_max(0);
     d.g = b->g.ptr;
     d.ngraphs = (uint32_t)ng;
-    d.rec = b->rec.ptr;
+    d.rec = b->rec;
+    d.stopped = b->bits.ptr + b->stopped_at();
     d.counts = (hb::HbBatchRec *)(b->bits.ptr + b->count_at());
     d.active = b->active.ptr;
     d.active_count = b->active_count.ptr;
@@ -973,10 +990,10 @@ int hb_batch_run(hb_batch *b, uint32_t flags, hb_batch_stats *stats)
         classes.q[q] = lists[q] = {b->tiles[q].ptr, nullptr, b->ntiles[q], (uint32_t)q, b->tile_base[q]};
     for (int pi = 0; pi < hb::kBatchNP; ++pi) hub_lists[pi] = {nullptr, b->hubs[pi].ptr, b->nhubs[pi], 0, 0};
 
-    hipEvent_t e0, e1, e2;
+    hipEvent_t e0, e1, e2 = nullptr, ends[3];
     HB_BTRY(hipEventCreate(&e0));
     HB_BTRY(hipEventCreate(&e1));
-    HB_BTRY(hipEventCreate(&e2));
+    for (auto &ev : ends) HB_BTRY(hipEventCreate(&ev));
     int rc = HB_OK;
     uint32_t launches = 0;
     const bool trace = trace_on();
@@ -994,7 +1011,7 @@ int hb_batch_run(hb_batch *b, uint32_t flags, hb_batch_stats *stats)
     // stopped graph never runs again and its kernels would return at once, so leaving
     // out a precision whose graphs have all stopped changes nothing.
     auto launch_iter = [&](uint32_t running, bool first) -> hipError_t {
-        hb::k_batch_begin<<<(unsigned)std::min(ng, 1024), hb::kBatchBlock, 0, b->stream>>>(d);
+        hb::k_batch_begin<<<dim3((unsigned)std::min(ng, 1024), 8), hb::kBatchBlock, 0, b->stream>>>(d);
         hb::k_batch_compact<<<hb::kQueues, 1024, 0, b->stream>>>(d, classes);
         hipError_t e = hipEventRecord(b->fork, b->stream);
         // the running precisions' chains (the three node bins of team widths G, 4G capped at
@@ -1084,76 +1101,84 @@ int hb_batch_run(hb_batch *b, uint32_t flags, hb_batch_stats *stats)
             return HB_OK;
         };
         uint32_t running_p = (1u << hb::kBatchNP) - 1;
-        std::vector<hb::HbBatchGraph> hs(ng);
-        std::vector<hb::HbBatchRec> ring((size_t)ng * hb::kRing);
-        std::vector<uint32_t> harvested(ng, 0);  // iterations copied into history
-        for (;;) {
-            // no graph can need more than cap_max iterations; launches past that only
-            // happen if a graph failed to stop, which finalize reports as overflow
-            const uint32_t k = launches < 8 ? 2u : hb::kCheck;
-            if (launches >= cap_max + 2 * hb::kCheck) {
+        // every running graph is in iteration t at launch t: the host launches kAhead iterations
+        // beyond the one whose event it waits for, then reads that iteration's records
+        constexpr uint32_t kAhead = 2;
+        static_assert(kAhead + 1 < hb::kRing, "records in flight");
+        std::vector<uint8_t> stopped(ng, 0);
+        for (size_t i = 0; i < (size_t)ng * hb::kRing; ++i) b->rec[i].iter = 0;
+        uint32_t checked = 0;
+        int left = ng;
+        b->h_final = init;
+        while (left) {
+            // every graph stops, or finalize reports that it did not, by iteration cap_max:
+            // nothing is launched past it
+            if (checked >= cap_max) {
                 rc = bfail(HB_ESTATE, "hb_batch_run: %u launches without every graph stopping", launches);
                 break;
             }
-            for (uint32_t i = 0; i < k && rc == HB_OK; ++i) {
-                const bool first = launches + i == 0;  // every graph is in iteration 1
+            while (launches <= checked + kAhead && launches < cap_max && rc == HB_OK) {
+                const bool first = launches == 0;  // every graph is in iteration 1
                 hipGraphExec_t gexec = nullptr;
                 if (flags & HB_FLAG_GRAPH) rc = exec_for(running_p, first, &gexec);
                 if (rc != HB_OK) break;
                 const hipError_t el = gexec ? hipGraphLaunch(gexec, b->stream) : launch_iter(running_p, first);
                 if (el != hipSuccess) rc = bfail(HB_EHIP, "iteration launch: %s", hipGetErrorString(el));
+                else if (hipEventRecord(ends[launches % (kAhead + 1)], b->stream) != hipSuccess)
+                    rc = bfail(HB_EHIP, "event record failed");
+                ++launches;
             }
-            launches += k;
             if (rc != HB_OK) break;
-            if (hipMemcpyAsync(hs.data(), b->g.ptr, ng * sizeof(hb::HbBatchGraph), hipMemcpyDeviceToHost, b->stream) != hipSuccess ||
-                hipMemcpyAsync(ring.data(), b->rec.ptr, ring.size() * sizeof(hb::HbBatchRec), hipMemcpyDeviceToHost,
-                               b->stream) != hipSuccess ||
-                hipStreamSynchronize(b->stream) != hipSuccess) {
+            const uint32_t t = checked + 1;
+            e2 = ends[checked % (kAhead + 1)];
+            if (hipEventSynchronize(e2) != hipSuccess) {
                 rc = bfail(HB_EHIP, "iteration failed: %s", hipGetErrorString(hipGetLastError()));
                 break;
             }
-            bool all = true;
-            uint32_t running = 0, it_max = 0;
+            checked = t;
             running_p = 0;
             for (int i = 0; i < ng; ++i) {
-                const hb::HbBatchGraph &g = hs[i];
-                if (!g.st.done) running_p |= 1u << (g.p - hb::kBatchPMin);
-                const uint32_t complete = g.st.done ? g.st.executed : g.st.iter - 1;  // iterations finished
-                for (uint32_t t = harvested[i] + 1; t <= complete; ++t)
-                    b->history[i].push_back(ring[(size_t)i * hb::kRing + t % hb::kRing]);
-                harvested[i] = complete;
-                all = all && g.st.done;
-                running += !g.st.done;
-                it_max = std::max(it_max, complete);
+                if (stopped[i]) continue;
+                const hb::HbBatchRec r = b->rec[(size_t)i * hb::kRing + t % hb::kRing];
+                if (r.iter != t) {
+                    rc = bfail(HB_ESTATE, "hb_batch_run: no record of iteration %u of graph %d", t, i);
+                    break;
+                }
+                b->history[i].push_back(r);
+                if (!r.done) {
+                    running_p |= 1u << (b->hg[i].p - hb::kBatchPMin);
+                    continue;
+                }
+                stopped[i] = 1;
+                --left;
+                HbIterState &st = b->h_final[i].st;
+                st.done = 1;
+                st.iter = st.executed = t;
+                st.converged = r.converged;
+                st.parity = (t - 1) & 1u;  // every iteration but the last swapped the buffers
+                if (r.overflow)
+                    rc = bfail(HB_ESTATE, "hb_batch_run: graph %d still changing after %u iterations (n + 2)", i,
+                               b->hg[i].cap);
             }
             if (trace) {
-                const double s = std::chrono::duration<double>(std::chrono::steady_clock::now() - t_start).count();
-                fprintf(stderr, "[hb_batch] %.3fs launches %u: %u of %d graphs running, longest at %u iterations\n", s,
-                        launches, running, ng, it_max);
+                const double sec = std::chrono::duration<double>(std::chrono::steady_clock::now() - t_start).count();
+                fprintf(stderr, "[hb_batch] %.3fs launches %u: %d of %d graphs running, longest at %u iterations\n", sec,
+                        launches, left, ng, t);
                 fflush(stderr);
             }
-            if (all) break;
+            if (rc != HB_OK) break;
         }
-        if (rc != HB_OK) break;
-        (void)hipEventRecord(e2, b->stream);
-        (void)hipEventSynchronize(e2);
-        b->h_final = hs;
-        for (int i = 0; i < ng; ++i)
-            if (hs[i].overflow)
-                rc = bfail(HB_ESTATE, "hb_batch_run: graph %d still changing after %u iterations (n + 2)", i, hs[i].cap);
     } while (0);
     float ms_init = 0.0f, ms_loop = 0.0f;
     if (rc == HB_OK) {
         (void)hipEventElapsedTime(&ms_init, e0, e1);
         (void)hipEventElapsedTime(&ms_loop, e1, e2);
     }
+    if (rc != HB_OK) (void)hipStreamSynchronize(b->stream);
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    (void)hipEventDestroy(e2);
-    if (rc != HB_OK) {
-        (void)hipStreamSynchronize(b->stream);
-        return rc;
-    }
+    for (auto ev : ends) (void)hipEventDestroy(ev);
+    if (rc != HB_OK) return rc;
     b->ran = true;
     if (stats) {
         memset(stats, 0, sizeof *stats);
