@@ -270,10 +270,7 @@ __device__ __forceinline__ uint64_t hb_mix64(uint64_t z)
     return z ^ (z >> 31);
 }
 
-// A wavefront takes 64 consecutive nodes at a time: a node of degree <= 64 is walked
-// by its own lane, a larger one by the whole wavefront (ballot over the 64, then a
-// uniform loop), so hubs do not serialise on one lane.  Each block writes its four
-// sums to part[4 * block]; sum_columns adds the blocks in a fixed order.
+// Each block writes its four sums to part[4 * block]; sum_columns adds the blocks.
 __device__ __forceinline__ void hb_fp_add(unsigned long long *a, uint64_t u, uint64_t v)
 {
     const uint64_t hf = hb_mix64((u << 32) | v), hb = hb_mix64((v << 32) | u);
@@ -283,32 +280,77 @@ __device__ __forceinline__ void hb_fp_add(unsigned long long *a, uint64_t u, uin
     a[3] += hb * hb;
 }
 
-// every thread takes kFpArcs consecutive arcs: a binary search over the offsets finds
-// the first one's tail, then the walk advances the tail across node boundaries (empty
-// nodes between two arcs are crossed by exactly one thread), so hubs cost no more than
-// any other arcs
-constexpr uint32_t kFpArcs = 32;
+// A wavefront takes kFpArcs * 64 consecutive arcs at a time, loaded coalesced into its lanes'
+// registers.  Their tails: a 64-way search over the offsets finds the first one's, the
+// offsets that follow, read coalesced, put each node's id where its arcs start in LDS, and a
+// running maximum spreads the ids over the arcs (each lane over a run of kFpArcs, a scan over
+// the lanes joining the runs; one pad word per run keeps LDS free of bank conflicts).  Hubs
+// and runs of empty nodes cost no more than other arcs and nodes.  When each lane read and
+// walked kFpArcs = 32 arcs of its own, 128 bytes from the next lane's, 16M arcs took 583 us, 31M
+// 688, a graph of 4k nodes 24; now 77, 139 and 12 (kFpArcs of 16: 130 and 169, of 4: 77 and 130).
+constexpr uint32_t kFpArcs = 8;
 
 __global__ __launch_bounds__(kBlock) void k_arc_fingerprint(const uint32_t *off, const uint32_t *nbr, uint32_t n,
                                                             uint64_t arcs, unsigned long long *part)
 {
+    constexpr uint32_t kSpan = kFpArcs * HB_WAVE, kRun = kFpArcs + 1;
     __shared__ unsigned long long red[kBlock / HB_WAVE][4];
+    __shared__ uint32_t s_tail[kBlock / HB_WAVE][HB_WAVE * kRun];
     const uint32_t lane = threadIdx.x & (HB_WAVE - 1), wv = threadIdx.x / HB_WAVE;
+    uint32_t *tail = s_tail[wv];
     unsigned long long a[4] = {0, 0, 0, 0};
-    const uint64_t threads = (uint64_t)gridDim.x * kBlock;
-    for (uint64_t t = (uint64_t)blockIdx.x * kBlock + threadIdx.x; t * kFpArcs < arcs; t += threads) {
-        const uint64_t e_lo = t * kFpArcs, e_hi = min<uint64_t>(arcs, e_lo + kFpArcs);
-        uint32_t lo = 0, hi = n - 1;  // largest u with off[u] <= e_lo (then off[u + 1] > e_lo)
-        while (lo < hi) {
-            const uint32_t mid = lo + (hi - lo + 1) / 2;
-            if (off[mid] <= e_lo) lo = mid;
-            else hi = mid - 1;
+    const uint64_t step = (uint64_t)gridDim.x * (kBlock / HB_WAVE) * kSpan;
+    for (uint64_t base = ((uint64_t)blockIdx.x * (kBlock / HB_WAVE) + wv) * kSpan; base < arcs; base += step) {
+        const uint32_t span = (uint32_t)min<uint64_t>(kSpan, arcs - base);
+        uint32_t x[kFpArcs], run[kFpArcs];
+#pragma unroll
+        for (uint32_t k = 0; k < kFpArcs; ++k) {
+            const uint32_t i = k * HB_WAVE + lane;
+            x[k] = i < span ? nbr[base + i] : 0u;
+            tail[lane * kRun + k] = 0u;
         }
-        uint32_t u = lo;
-        for (uint64_t e = e_lo; e < e_hi; ++e) {
-            while (off[u + 1] <= e) ++u;
-            hb_fp_add(a, u, nbr[e]);
+        uint32_t lo = 0, len = n;  // the largest u with off[u] <= base is one of lo .. lo + len - 1
+        while (len > 1) {
+            const uint32_t stride = (len + HB_WAVE - 1) / HB_WAVE;
+            const uint64_t i = (uint64_t)lane * stride;
+            const unsigned long long m = __ballot(i < len && off[lo + i] <= base);
+            const uint32_t c = (uint32_t)__popcll(m) - 1u;  // off[lo] <= base
+            lo += c * stride;
+            len = min(stride, len - c * stride);
         }
+        __builtin_amdgcn_wave_barrier();  // the zeros are written
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        for (uint32_t u0 = lo + 1;; u0 += HB_WAVE) {
+            const uint32_t u = u0 + lane;
+            const uint64_t start = u < n ? off[u] : arcs;
+            const bool in = start < base + span;
+            if (in && off[u + 1] != start) {
+                const uint32_t i = (uint32_t)(start - base);
+                tail[i + i / kFpArcs] = u;
+            }
+            if (__ballot(!in)) break;
+        }
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        uint32_t top = lane == 0 ? lo : 0u;
+#pragma unroll
+        for (uint32_t k = 0; k < kFpArcs; ++k) run[k] = top = max(top, tail[lane * kRun + k]);
+        for (int o = 1; o < HB_WAVE; o <<= 1) {
+            const uint32_t below = __shfl_up(top, o);
+            if (lane >= (uint32_t)o) top = max(top, below);
+        }
+        const uint32_t before = __shfl_up(top, 1);
+#pragma unroll
+        for (uint32_t k = 0; k < kFpArcs; ++k) tail[lane * kRun + k] = lane ? max(run[k], before) : run[k];
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+        for (uint32_t k = 0; k < kFpArcs; ++k) {
+            const uint32_t i = k * HB_WAVE + lane;
+            if (i < span) hb_fp_add(a, tail[i + i / kFpArcs], x[k]);
+        }
+        __builtin_amdgcn_wave_barrier();  // every lane has read the tails
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     }
     for (int k = 0; k < 4; ++k)
         for (int o = 1; o < HB_WAVE; o <<= 1) a[k] += __shfl_xor(a[k], o);
