@@ -1251,7 +1251,12 @@ int hb_batch_read_estimates(hb_batch *b, int graph, int which, float *dst)
         return bfail(HB_EINVAL, "hb_batch_read_estimates: bad arguments");
     if (!b->ran) return bfail(HB_ESTATE, "hb_batch_read_estimates: no completed run");
     HB_BTRY(hipSetDevice(b->device));
-    HB_BTRY(hb::launch_estimates(graph_dev(b, graph), batch_regs(b, graph, which), b->est_tmp.ptr, b->stream));
+    // the run leaves the estimates of its last iteration's rows; they are the other buffer's
+    // too if that iteration changed no register
+    const uint8_t *regs = batch_regs(b, graph, which);
+    if (b->history[graph].back().chg == 0 || regs == batch_regs(b, graph, HB_REGS_LATEST))
+        return batch_copy_out(b, graph, b->est.ptr + b->hg[graph].node_base, dst, 4);
+    HB_BTRY(hb::launch_estimates(graph_dev(b, graph), regs, b->est_tmp.ptr, b->stream));
     return batch_copy_out(b, graph, b->est_tmp.ptr, dst, 4);
 }
 
