@@ -1448,9 +1448,9 @@ static int walk_surrogate(hb_ctx *c, hb_mlp *mlp, int passes, bool want_x, float
             if (ho[u + 1] - ho[u] <= hb::kWalkHub) continue;
             node.push_back(u);
             first.push_back((uint32_t)beg.size());
-            for (uint64_t b = ho[u]; b < ho[u + 1]; b += hb::kWalkHub) {
+            for (uint64_t b = ho[u]; b < ho[u + 1]; b += hb::kWalkChunk) {
                 beg.push_back((uint32_t)b);
-                end.push_back((uint32_t)std::min<uint64_t>(b + hb::kWalkHub, ho[u + 1]));
+                end.push_back((uint32_t)std::min<uint64_t>(b + hb::kWalkChunk, ho[u + 1]));
             }
         }
         first.push_back((uint32_t)beg.size());

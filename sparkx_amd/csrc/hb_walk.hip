@@ -8,11 +8,10 @@
 // wavefronts and chunks gives the same bits.
 //
 // One pass per k reads S_{k-1} at every arc's head (pass 1 the u32 degrees, half the
-// bytes of a u64 row).  Layout of a pass, as in the exact searches' pull levels: a
-// wavefront takes 64 consecutive nodes; a node of degree <= 64 is summed by its own
-// lane, one of degree <= kWalkHub by the whole wavefront, and a larger list is cut
-// into kWalkHub-arc chunks (one wavefront each) whose partial sums are combined per
-// hub in a second launch.
+// bytes of a u64 row).  Layout of a pass: a wavefront takes 64 consecutive nodes; a node of
+// degree <= 64 is summed by its own lane, one of degree <= kWalkHub by the whole wavefront,
+// and a larger list is cut into kWalkChunk-arc chunks (one wavefront each) whose partial sums
+// are combined per hub in a further launch.
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
@@ -32,51 +31,97 @@ __device__ __forceinline__ uint64_t sat_add(uint64_t a, uint64_t b)
     return r < a ? ~0ull : r;
 }
 
-// this lane's share (e = b0 + lane, b0 + lane + 64, ... < b1) of a list's sum and max
+// this lane's share (e = b0 + lane, b0 + lane + 64, ... < b1) of a list's sum and max, four
+// gathers in flight also where fewer are left: past the end the last arc is read again and
+// counts 0, which changes neither
 template <typename In>
 __device__ __forceinline__ void walk_range(const uint32_t *__restrict__ nbr, const In *__restrict__ in,
                                            uint64_t b0, uint64_t b1, uint32_t lane, uint64_t &s, uint64_t &m)
 {
-    uint64_t e = b0 + lane;
-    for (; e + 3 * 64 < b1; e += 4 * 64) {
-        const uint32_t w0 = nbr[e], w1 = nbr[e + 64], w2 = nbr[e + 128], w3 = nbr[e + 192];
-        const uint64_t x0 = in[w0], x1 = in[w1], x2 = in[w2], x3 = in[w3];
-        s = sat_add(sat_add(s, x0), sat_add(x1, sat_add(x2, x3)));
-        m = std::max(std::max(m, x0), std::max(std::max(x1, x2), x3));
-    }
-    for (; e < b1; e += 64) {
-        const uint64_t x = in[nbr[e]];
-        s = sat_add(s, x);
-        m = std::max(m, x);
+    for (uint64_t e = b0 + lane; e < b1; e += 4 * 64) {
+        uint32_t w[4];
+        uint64_t x[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) w[k] = nbr[std::min<uint64_t>(e + 64 * k, b1 - 1)];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) x[k] = in[w[k]];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if (e + 64 * k >= b1) x[k] = 0;
+            s = sat_add(s, x[k]);
+            m = std::max(m, x[k]);
+        }
     }
 }
 
+template <int kLanes = 64>
 __device__ __forceinline__ void wave_reduce(uint64_t &s, uint64_t &m)
 {
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
+    for (int o = 1; o < kLanes; o <<= 1) {
         s = sat_add(s, (uint64_t)__shfl_xor((long long)s, o));
         m = std::max(m, (uint64_t)__shfl_xor((long long)m, o));
     }
 }
 
+// arcs that a wavefront gathers at once into LDS in k_walk, and their places there: a pad word
+// per 32 keeps lists of one length (consecutive nodes in the degree layout) out of one bank
+constexpr uint32_t kWalkTile = 512;
+__device__ __forceinline__ constexpr uint32_t tile_at(uint32_t i) { return i + i / 32; }
+
 // out[u] = Σ in[v], mx[u] = max in[v] (mx nullable) over u's arcs, for every node of
-// degree <= hub_deg; the larger ones are k_walk_chunks' and k_walk_hubs'
+// degree <= hub_deg; the larger ones are k_walk_chunks' and k_walk_hubs'.
+// Bound by the rate of random gathers.  Where all 64 lists are short their arcs are
+// consecutive: ids loaded coalesced, eight gathers in flight per lane, and each lane sums its
+// list from LDS.  A lane that walks its own list instead (lists among longer ones) takes one
+// cache line of ids per lane and step, more than L1 holds for the wavefronts of a CU.
 template <typename In>
 __global__ __launch_bounds__(kBlock) void k_walk(const uint32_t *__restrict__ off, const uint32_t *__restrict__ nbr,
                                                  uint32_t n, uint32_t hub_deg, const In *__restrict__ in,
                                                  uint64_t *out, uint64_t *mx)
 {
+    __shared__ In s_tile[kBlock / 64][tile_at(kWalkTile)];
+    In *tile = s_tile[threadIdx.x / 64];
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t waves = gridDim.x * (kBlock / 64);
     for (uint32_t base = (blockIdx.x * (kBlock / 64) + threadIdx.x / 64) * 64; base < n; base += waves * 64) {
         const uint32_t v = base + lane;  // uniform loop bound: every lane takes part in the ballot
-        uint32_t e0 = 0, e1 = 0;
-        if (v < n) {
-            e0 = off[v];
-            e1 = off[v + 1];
+        const uint32_t e0 = off[std::min(v, n)], e1 = off[std::min(v + 1, n)];
+        const bool small = e1 - e0 <= 64;
+        if (__all(small)) {
+            const uint32_t lo = (uint32_t)__shfl((int)e0, 0), hi = (uint32_t)__shfl((int)e1, 63);
+            uint64_t s = 0, m = 0;
+            for (uint32_t at = 0; at < hi - lo; at += kWalkTile) {  // lo + at: the tile's first arc
+                const uint32_t span = std::min(kWalkTile, hi - lo - at);
+                const uint32_t *ids = nbr + lo + at;
+                uint32_t w[kWalkTile / 64];
+#pragma unroll
+                for (uint32_t k = 0; k < kWalkTile / 64; ++k) w[k] = ids[std::min(k * 64 + lane, span - 1)];
+                In x[kWalkTile / 64];
+#pragma unroll
+                for (uint32_t k = 0; k < kWalkTile / 64; ++k)
+                    if (k * 64 < span) x[k] = in[w[k]];
+#pragma unroll
+                for (uint32_t k = 0; k < kWalkTile / 64; ++k)
+                    if (k * 64 < span) tile[tile_at(k * 64 + lane)] = x[k];
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                const uint32_t first = std::max(e0 - lo, at) - at, last = std::min(e1 - lo, at + span);
+                for (uint32_t i = first; at + i < last; ++i) {
+                    const uint64_t y = tile[tile_at(i)];
+                    s = sat_add(s, y);
+                    m = std::max(m, y);
+                }
+                __builtin_amdgcn_wave_barrier();  // every lane has read its part of the tile
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            }
+            if (v < n) {
+                out[v] = s;
+                if (mx) mx[v] = m;
+            }
+            continue;
         }
-        if (v < n && e1 - e0 <= 64) {
+        if (v < n && small) {
             uint64_t s = 0, m = 0;
             uint32_t e = e0;
             for (; e + 4 <= e1; e += 4) {
@@ -93,7 +138,7 @@ __global__ __launch_bounds__(kBlock) void k_walk(const uint32_t *__restrict__ of
             out[v] = s;
             if (mx) mx[v] = m;
         }
-        unsigned long long big = __ballot(e1 - e0 > 64 && e1 - e0 <= hub_deg);
+        unsigned long long big = __ballot(!small && e1 - e0 <= hub_deg);
         while (big) {
             const int i = __ffsll(big) - 1;
             big &= big - 1;
@@ -129,19 +174,24 @@ __global__ __launch_bounds__(kBlock) void k_walk_chunks(const uint32_t *__restri
     }
 }
 
-// hub h owns chunks [first[h], first[h + 1]): combined into out / mx of node node[h]
+// hub h owns chunks [first[h], first[h + 1]): combined into out / mx of node node[h] by
+// kHubLanes lanes (most hubs have one chunk, the largest of a power law tens)
+constexpr uint32_t kHubLanes = 16;
 __global__ __launch_bounds__(kBlock) void k_walk_hubs(const uint32_t *__restrict__ node,
                                                       const uint32_t *__restrict__ first, uint32_t hubs,
                                                       const uint64_t *__restrict__ psum,
                                                       const uint64_t *__restrict__ pmax, uint64_t *out, uint64_t *mx)
 {
-    const uint32_t h = blockIdx.x * blockDim.x + threadIdx.x;
-    if (h >= hubs) return;
+    const uint32_t lane = threadIdx.x % kHubLanes;
+    const uint32_t h = blockIdx.x * (kBlock / kHubLanes) + threadIdx.x / kHubLanes;
+    if (h >= hubs) return;  // a team's lanes leave together
     uint64_t s = 0, m = 0;
-    for (uint32_t c = first[h]; c < first[h + 1]; ++c) {
+    for (uint32_t c = first[h] + lane; c < first[h + 1]; c += kHubLanes) {
         s = sat_add(s, psum[c]);
         m = std::max(m, pmax[c]);
     }
+    wave_reduce<kHubLanes>(s, m);
+    if (lane != 0) return;
     out[node[h]] = s;
     if (mx) mx[node[h]] = m;
 }
@@ -196,8 +246,8 @@ hipError_t walk_inputs(const uint32_t *off, const uint32_t *nbr, uint32_t n, con
     if (passes != 2 && passes != 3) return hipErrorInvalidValue;
     uint64_t *m1 = s + 3 * (uint64_t)n;
     const unsigned grid = grid_for((uint64_t)n);  // 256 nodes per block: a wavefront per 64
-    const unsigned cgrid = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>((hubs.chunks + 3) / 4, 4096));
-    const unsigned hgrid = (hubs.hubs + kBlock - 1) / kBlock;
+    const unsigned cgrid = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>((hubs.chunks + 3) / 4, 16384));
+    const unsigned hgrid = (hubs.hubs + kBlock / kHubLanes - 1) / (kBlock / kHubLanes);
     k_degrees<<<grid, kBlock, 0, st>>>(off, n, deg);
     k_walk<uint32_t><<<grid, kBlock, 0, st>>>(off, nbr, n, kWalkHub, deg, s, m1);
     if (hubs.chunks) {
