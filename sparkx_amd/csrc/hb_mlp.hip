@@ -5,8 +5,7 @@
 // instruction), products over 16 samples or the 6 (padded) inputs on
 // v_mfma_f32_16x16x16_bf16; GELU, biases, loss and the Adam update run in f32, and
 // every rounding to bf16 is the hardware's round-to-nearest-even convert.  One
-// wavefront handles a tile of 16 samples; activations move between MFMA output and
-// operand layouts through LDS.
+// wavefront handles a tile of 16 samples.
 //
 // MFMA lane layout (lane l, g = l / 16): D (M x N, both shapes): D[4 g + j][l % 16],
 // j = 0..3.  An A (M x K) register j of lane l multiplies the B (K x N) register j
@@ -37,8 +36,6 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 
 constexpr int kDIn = 6, kDH = 64;
 constexpr int oW1 = 0, oB1 = 384, oW2 = 448, oB2 = 4544, oW3 = 4608, oB3 = 4672, kNParams = 4673;
-constexpr int kBlock = 128;  // two wavefronts, one 16-sample tile each per round
-constexpr int kWaves = kBlock / 64;
 
 // round to nearest even (v_cvt_pk_bf16_f32); inputs are finite
 __device__ __forceinline__ uint16_t f2bf(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
@@ -49,7 +46,7 @@ __device__ __forceinline__ float bfr(float f) { return (float)(__bf16)f; }
 // t = 1 / (1 + p z), for z >= 0, odd in z.  About half the instructions of erff; the
 // activations it feeds are rounded to bf16 (8 bits) right after.  Training and inference
 // both use it, so the network is evaluated with the function it was trained with.
-__device__ __forceinline__ float erf_as(float x)
+__device__ __forceinline__ float erf_as(float x, float &e)
 {
     const float z = fabsf(x);
     const float t = __builtin_amdgcn_rcpf(fmaf(0.3275911f, z, 1.0f));
@@ -57,88 +54,26 @@ __device__ __forceinline__ float erf_as(float x)
     q = fmaf(t, q, 1.421413741f);
     q = fmaf(t, q, -0.284496736f);
     q = fmaf(t, q, 0.254829592f);
-    const float e = __builtin_amdgcn_exp2f(-(z * z) * 1.44269504088896341f);  // exp(-z^2)
+    e = __builtin_amdgcn_exp2f(-(z * z) * 1.44269504088896341f);  // exp(-z^2)
     return copysignf(fmaf(-(t * q), e, 1.0f), x);
 }
-__device__ __forceinline__ float gelu(float x) { return 0.5f * x * (1.0f + erf_as(x * 0.70710678118654752f)); }
-__device__ __forceinline__ float gelu_grad(float x)
+__device__ __forceinline__ float gelu(float x)
 {
-    const float cdf = 0.5f * (1.0f + erf_as(x * 0.70710678118654752f));
-    return cdf + x * (__builtin_amdgcn_exp2f(-0.5f * x * x * 1.44269504088896341f) * 0.39894228040143268f);
+    float e;
+    return 0.5f * x * (1.0f + erf_as(x * 0.70710678118654752f, e));
+}
+// gelu(x) and its derivative cdf(x) + x pdf(x); pdf(x) = exp(-x^2 / 2) / sqrt(2 pi) shares erf's
+// exponential
+__device__ __forceinline__ float gelu_grad(float x, float &grad)
+{
+    float e;
+    const float cdf2 = 1.0f + erf_as(x * 0.70710678118654752f, e);
+    grad = 0.5f * cdf2 + x * (e * 0.39894228040143268f);
+    return 0.5f * x * cdf2;
 }
 
 __device__ __forceinline__ v4f mfma(v4s a, v4s b, v4f c) { return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0); }
 __device__ __forceinline__ v4f mfma32(v8bf a, v8bf b, v4f c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
-
-struct Shared {
-    uint16_t w1[16][kDH];  // bf16, input rows 6..15 zero
-    uint16_t w2[kDH][kDH];
-    float w3[kDH];         // bf16-rounded
-    float b1[kDH], b2[kDH], b3;
-    float mean[kDIn], sd[kDIn];
-};
-
-struct Wave {
-    float xs[16][16];      // bf16(normalised input), padded
-    float h1[16][kDH];     // bf16(gelu(z1))
-    float g1[16][kDH];     // gelu'(z1)
-    float h2[16][kDH];     // bf16(gelu(z2))
-    float g2[16][kDH];     // gelu'(z2), then dz1
-    float d[16][kDH];      // dz2
-    float y[16], t[16], dy[16];
-};
-
-// operand gathers (see the layout above)
-__device__ __forceinline__ v4s opA(const float *a, int ld, int kc, int l)
-{
-    const float *p = a + (l & 15) * ld + kc + 4 * (l >> 4);
-    v4s r;
-    r[0] = (short)f2bf(p[0]);
-    r[1] = (short)f2bf(p[1]);
-    r[2] = (short)f2bf(p[2]);
-    r[3] = (short)f2bf(p[3]);
-    return r;
-}
-__device__ __forceinline__ v4s opAT(const float *src, int ld, int mc, int l)  // A[m][k] = src[k][m]
-{
-    v4s r;
-    for (int j = 0; j < 4; ++j) r[j] = (short)f2bf(src[(4 * (l >> 4) + j) * ld + mc + (l & 15)]);
-    return r;
-}
-__device__ __forceinline__ v4s opBw(const uint16_t *w, int ld, int kc, int nc, int l)  // B = W
-{
-    v4s r;
-    for (int j = 0; j < 4; ++j) r[j] = (short)w[(kc + 4 * (l >> 4) + j) * ld + nc + (l & 15)];
-    return r;
-}
-__device__ __forceinline__ v4s opBf(const float *src, int ld, int nc, int l)  // B[k][n] = src[k][n]
-{
-    v4s r;
-    for (int j = 0; j < 4; ++j) r[j] = (short)f2bf(src[(4 * (l >> 4) + j) * ld + nc + (l & 15)]);
-    return r;
-}
-
-// K = 32 gathers (k = kc + 8 g + j)
-__device__ __forceinline__ v8bf opA8(const float *a, int ld, int kc, int l)
-{
-    const float *p = a + (l & 15) * ld + kc + 8 * (l >> 4);
-    v8bf r;
-    for (int j = 0; j < 8; ++j) r[j] = (__bf16)p[j];
-    return r;
-}
-__device__ __forceinline__ v8bf opBw8(const uint16_t *w, int ld, int kc, int nc, int l)  // B = W
-{
-    v8bf r;
-    for (int j = 0; j < 8; ++j) r[j] = __builtin_bit_cast(__bf16, w[(kc + 8 * (l >> 4) + j) * ld + nc + (l & 15)]);
-    return r;
-}
-__device__ __forceinline__ v8bf opBwT8(const uint16_t *w, int ld, int kc, int nc, int l)  // B = W^T
-{
-    const uint16_t *p = w + (nc + (l & 15)) * ld + kc + 8 * (l >> 4);
-    v8bf r;
-    for (int j = 0; j < 8; ++j) r[j] = __builtin_bit_cast(__bf16, p[j]);
-    return r;
-}
 
 struct Dev {
     const float *params;  // f32 master copy
@@ -152,78 +87,6 @@ struct Dev {
     float *loss;          // sum of squared errors (training)
     float *out;           // predictions (inference)
 };
-
-__device__ void load_shared(Shared &sh, const Dev &d)
-{
-    for (int i = threadIdx.x; i < 16 * kDH; i += blockDim.x) {
-        const int r = i / kDH, c = i % kDH;
-        sh.w1[r][c] = r < kDIn ? f2bf(d.params[oW1 + r * kDH + c]) : (uint16_t)0;
-    }
-    for (int i = threadIdx.x; i < kDH * kDH; i += blockDim.x) sh.w2[i / kDH][i % kDH] = f2bf(d.params[oW2 + i]);
-    for (int i = threadIdx.x; i < kDH; i += blockDim.x) {
-        sh.w3[i] = bfr(d.params[oW3 + i]);
-        sh.b1[i] = d.params[oB1 + i];
-        sh.b2[i] = d.params[oB2 + i];
-    }
-    if (threadIdx.x < kDIn) {
-        sh.mean[threadIdx.x] = d.norm[threadIdx.x];
-        sh.sd[threadIdx.x] = d.norm[kDIn + threadIdx.x];
-    }
-    if (threadIdx.x == 0) sh.b3 = d.params[oB3];
-}
-
-// forward pass of one tile; rows >= valid are zero inputs
-__device__ void forward_tile(const Shared &sh, Wave &w, const Dev &d, uint64_t base, int valid, int l, bool training)
-{
-    for (int i = l; i < 16 * 16; i += 64) {
-        const int s = i / 16, k = i % 16;
-        float v = 0.0f;
-        if (s < valid && k < kDIn) {
-            const uint64_t row = d.idx ? d.idx[base + s] : base + s;
-            v = bfr(__fdiv_rn(__fsub_rn(d.x[row * kDIn + k], sh.mean[k]), sh.sd[k]));
-        }
-        w.xs[s][k] = v;
-    }
-    if (l < 16) {
-        float tv = 0.0f;
-        if (training && l < valid) tv = d.y[d.idx ? d.idx[base + l] : base + l];
-        w.t[l] = tv;
-    }
-    __syncthreads();
-    for (int nb = 0; nb < 4; ++nb) {
-        v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
-        acc = mfma(opA(&w.xs[0][0], 16, 0, l), opBw(&sh.w1[0][0], kDH, 0, 16 * nb, l), acc);
-        for (int j = 0; j < 4; ++j) {
-            const int s = 4 * (l >> 4) + j, n = 16 * nb + (l & 15);
-            const float z = acc[j] + sh.b1[n];
-            w.h1[s][n] = bfr(gelu(z));
-            w.g1[s][n] = gelu_grad(z);
-        }
-    }
-    __syncthreads();
-    for (int nb = 0; nb < 4; ++nb) {
-        v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
-        for (int kc = 0; kc < kDH; kc += 32)
-            acc = mfma32(opA8(&w.h1[0][0], kDH, kc, l), opBw8(&sh.w2[0][0], kDH, kc, 16 * nb, l), acc);
-        for (int j = 0; j < 4; ++j) {
-            const int s = 4 * (l >> 4) + j, n = 16 * nb + (l & 15);
-            const float z = acc[j] + sh.b2[n];
-            w.h2[s][n] = bfr(gelu(z));
-            w.g2[s][n] = gelu_grad(z);
-        }
-    }
-    __syncthreads();
-    // layer 3: lane (s, q) sums 16 features, quarters combined with xor shuffles
-    {
-        const int s = l & 15, q = l >> 4;
-        float part = 0.0f;
-        for (int k = 16 * q; k < 16 * q + 16; ++k) part += w.h2[s][k] * sh.w3[k];
-        part += __shfl_xor(part, 16);
-        part += __shfl_xor(part, 32);
-        if (q == 0) w.y[s] = part + sh.b3;
-    }
-    __syncthreads();
-}
 
 // Inference only, activations kept in registers.  Both layers are computed
 // transposed, z^T = W^T x^T, so the outputs of the layer-1 MFMAs (D[n][s]: lane l
@@ -298,83 +161,225 @@ __global__ __launch_bounds__(kInferBlock) void k_infer(Dev d)
     }
 }
 
-__global__ __launch_bounds__(kBlock) void k_train(Dev d)
+// Forward and backward of 16-sample tiles, one wavefront each, the gradients summed in
+// registers over the wavefront's tiles, then over the block in LDS, then one f32 atomic per
+// parameter and block.
+// A tile's activations have samples as rows and units as columns: lane l (g = l / 16,
+// sl = l % 16) of an MFMA result holds units 16 nb + sl of samples 4 g + j.  Those registers
+// are, without a move, the A operand (transposed: K = samples) and the B operand of the
+// weight gradients h1^T dz2 and x^T dz1, and GELU, its derivative, biases, the output layer
+// and their gradients work on them in place.  Only the A operands of h1 W2 and of dz2 W2^T
+// change layout, through LDS: a lane writes its units nb = 0..3 of a sample as 8 bytes, so
+// unit 16 nb + sl stands at place 4 sl + nb, and the K order of those two products is the order
+// of the places (w2 and w2t are stored in it, one 16-byte read per lane and operand).
+// Bound by the GELUs (128 per sample, value and derivative) at two wavefronts per SIMD (the 80
+// registers of gradient sums).  When every activation went through f32 arrays in LDS, a block
+// of two wavefronts held 54 KB and a SIMD one wavefront: 1M samples took 0.685 ms, now 0.242.
+constexpr int kTrainBlock = 256, kTrainWaves = kTrainBlock / 64;
+constexpr int kActRow = 72;  // bf16 per row of the tile in LDS: 64 and a pad of 16 bytes
+
+struct TrainLds {
+    alignas(16) uint16_t w2[2][4][64][8];   // B operands of h1 W2: K chunk, unit tile, lane
+    alignas(16) uint16_t w2t[2][4][64][8];  // of dz2 W2^T
+    alignas(16) uint16_t act[kTrainWaves][16][kActRow];
+    alignas(16) uint16_t xt[kTrainWaves][8][16];  // inputs (6, padded) x samples
+    float grad[kNParams];
+};
+
+__device__ __forceinline__ void lds_order()  // between a wavefront's LDS writes and reads
 {
-    __shared__ Shared sh;
-    __shared__ Wave wv[kWaves];
-    load_shared(sh, d);
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+
+__global__ __launch_bounds__(kTrainBlock, 2) void k_train(Dev d)
+{
+    __shared__ TrainLds sh;
+    const int l = threadIdx.x & 63, wi = threadIdx.x / 64, g = l >> 4, sl = l & 15;
+    for (int i = threadIdx.x; i < kDH * kDH; i += kTrainBlock) {
+        const uint16_t w = f2bf(d.params[oW2 + i]);
+        const int r = i / kDH, c = i % kDH;
+        const int qr = 4 * (r % 16) + r / 16, qc = 4 * (c % 16) + c / 16;  // places of units r and c
+        sh.w2[qr / 32][c / 16][(qr % 32) / 8 * 16 + c % 16][qr % 8] = w;
+        sh.w2t[qc / 32][r / 16][(qc % 32) / 8 * 16 + r % 16][qc % 8] = w;
+    }
+    for (int i = threadIdx.x; i < kNParams; i += kTrainBlock) sh.grad[i] = 0.0f;
+    v4s w1[4];
+    float b1[4], b2[4], w3[4], mean[4], sd[4];
+    for (int nb = 0; nb < 4; ++nb) {
+        const int n = 16 * nb + sl;
+        b1[nb] = d.params[oB1 + n];
+        b2[nb] = d.params[oB2 + n];
+        w3[nb] = bfr(d.params[oW3 + n]);
+        for (int j = 0; j < 4; ++j) {
+            const int k = 4 * g + j;
+            w1[nb][j] = (short)(k < kDIn ? f2bf(d.params[oW1 + k * kDH + n]) : 0);
+        }
+    }
+    for (int j = 0; j < 4; ++j) {
+        const int k = 4 * g + j;
+        mean[j] = k < kDIn ? d.norm[k] : 0.0f;
+        sd[j] = k < kDIn ? d.norm[kDIn + k] : 1.0f;
+    }
+    const float b3 = d.params[oB3];
     __syncthreads();
-    const int l = threadIdx.x & 63, wi = threadIdx.x / 64;
-    Wave &w = wv[wi];
+
     v4f gw2[4][4], gw1[4];
+    float gb1[4] = {}, gb2[4] = {}, gw3[4] = {}, gb3 = 0.0f, sse = 0.0f;
     for (int a = 0; a < 4; ++a) {
         gw1[a] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
         for (int b = 0; b < 4; ++b) gw2[a][b] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
     }
-    float gb1 = 0.0f, gb2 = 0.0f, gw3 = 0.0f, gb3 = 0.0f, sse = 0.0f;
-    const uint64_t tiles = (d.count + 15) / 16;
-    const uint64_t rounds = (tiles + (uint64_t)gridDim.x * kWaves - 1) / ((uint64_t)gridDim.x * kWaves);
-    for (uint64_t r = 0; r < rounds; ++r) {
-        const uint64_t tile = (r * gridDim.x + blockIdx.x) * kWaves + wi;
+    const uint64_t tiles = (d.count + 15) / 16, stride = (uint64_t)gridDim.x * kTrainWaves;
+    const uint64_t end = d.first + d.count;
+    // inputs 4 g + j of sample sl, targets of samples 4 g + j; those past the end are the last
+    // sample's and count nothing
+    auto load = [&](uint64_t tile, float *x, float *t) {
         const uint64_t base = d.first + tile * 16;
-        const int valid = tile < tiles ? (int)min<uint64_t>(16, d.first + d.count - base) : 0;
-        forward_tile(sh, w, d, base, valid, l, true);
-        if (l < 16) {
-            const float e = l < valid ? w.y[l] - w.t[l] : 0.0f;
-            w.dy[l] = 2.0f * e * d.inv_b;
-            sse += e * e;
-        }
-        __syncthreads();
-        // layer 3 gradients; dz2 = dy w3 gelu'(z2)
-        for (int s = 0; s < 16; ++s) gw3 += w.dy[s] * w.h2[s][l];
-        if (l == 0)
-            for (int s = 0; s < 16; ++s) gb3 += w.dy[s];
-        for (int s = 0; s < 16; ++s) {
-            const float dz = w.dy[s] * sh.w3[l] * w.g2[s][l];
-            w.d[s][l] = dz;
-            gb2 += dz;
-        }
-        __syncthreads();
-        // gW2 += a1^T bf16(dz2); dh1 = bf16(dz2) W2^T; dz1 = dh1 gelu'(z1) -> g2
-        for (int mb = 0; mb < 4; ++mb) {
-            const v4s a = opAT(&w.h1[0][0], kDH, 16 * mb, l);
-            for (int nb = 0; nb < 4; ++nb) gw2[mb][nb] = mfma(a, opBf(&w.d[0][0], kDH, 16 * nb, l), gw2[mb][nb]);
-        }
-        for (int nb = 0; nb < 4; ++nb) {
-            v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
-            for (int kc = 0; kc < kDH; kc += 32)
-                acc = mfma32(opA8(&w.d[0][0], kDH, kc, l), opBwT8(&sh.w2[0][0], kDH, kc, 16 * nb, l), acc);
-            for (int j = 0; j < 4; ++j) {
-                const int s = 4 * (l >> 4) + j, n = 16 * nb + (l & 15);
-                w.g2[s][n] = acc[j] * w.g1[s][n];
-            }
-        }
-        __syncthreads();
-        for (int s = 0; s < 16; ++s) gb1 += w.g2[s][l];
-        for (int nb = 0; nb < 4; ++nb) gw1[nb] = mfma(opAT(&w.xs[0][0], 16, 0, l), opBf(&w.g2[0][0], kDH, 16 * nb, l), gw1[nb]);
-        __syncthreads();
-    }
-    // flush this wavefront's partial gradients
-    for (int mb = 0; mb < 4; ++mb)
-        for (int nb = 0; nb < 4; ++nb)
-            for (int j = 0; j < 4; ++j) {
-                const int row = 16 * mb + 4 * (l >> 4) + j, col = 16 * nb + (l & 15);
-                atomicAdd(d.grad + oW2 + row * kDH + col, gw2[mb][nb][j]);
-            }
-    for (int nb = 0; nb < 4; ++nb)
+        const uint64_t at = min(base + sl, end - 1);
+        const uint64_t row = d.idx ? d.idx[at] : at;
+#pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const int row = 4 * (l >> 4) + j, col = 16 * nb + (l & 15);
-            if (row < kDIn) atomicAdd(d.grad + oW1 + row * kDH + col, gw1[nb][j]);
+            x[j] = d.x[row * kDIn + min(4 * g + j, kDIn - 1)];
+            const uint64_t s = min(base + 4 * g + j, end - 1);
+            t[j] = d.y[d.idx ? d.idx[s] : s];
         }
-    atomicAdd(d.grad + oB1 + l, gb1);
-    atomicAdd(d.grad + oB2 + l, gb2);
-    atomicAdd(d.grad + oW3 + l, gw3);
-    if (l == 0) atomicAdd(d.grad + oB3, gb3);
-    for (int s = 1; s < 64; s <<= 1) sse += __shfl_xor(sse, s);
-    if (l == 0) atomicAdd(d.loss, sse);
+    };
+    uint64_t tile = (uint64_t)blockIdx.x * kTrainWaves + wi;
+    float xn[4], tn[4];
+    load(tile, xn, tn);
+    for (; tile < tiles; tile += stride) {
+        const uint64_t base = d.first + tile * 16;
+        int lw = l;  // opaque, so that the weights' reads stay in the loop: 64 registers less
+        asm volatile("" : "+v"(lw));
+        v4s xa;
+        float t[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const float v = __fdiv_rn(__fsub_rn(xn[j], mean[j]), sd[j]);
+            xa[j] = (short)(4 * g + j < kDIn && base + sl < end ? f2bf(v) : 0);
+            t[j] = tn[j];
+        }
+        load(tile + stride, xn, tn);  // in flight during this tile
+        if (g < 2)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) sh.xt[wi][4 * g + j][sl] = (uint16_t)xa[j];
+        v4s h1[4];
+        float g1[4][4];
+#pragma unroll
+        for (int nb = 0; nb < 4; ++nb) {
+            const v4f z = mfma(xa, w1[nb], v4f{0.0f, 0.0f, 0.0f, 0.0f});
+#pragma unroll
+            for (int j = 0; j < 4; ++j) h1[nb][j] = (short)f2bf(gelu_grad(z[j] + b1[nb], g1[nb][j]));
+            // finished here, not where they are used: else the compiler keeps what they are
+            // computed from instead and spills 59 registers
+#pragma unroll
+            for (int j = 0; j < 4; ++j) asm volatile("" : "+v"(g1[nb][j]));
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        auto put = [&](const v4s *v) {  // rows of samples 4 g + j, places 4 sl .. 4 sl + 3
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                *(v4s *)&sh.act[wi][4 * g + j][4 * sl] = v4s{v[0][j], v[1][j], v[2][j], v[3][j]};
+            lds_order();
+        };
+        auto get = [&](int c) { return *(const v8bf *)&sh.act[wi][sl][32 * c + 8 * g]; };
+        put(h1);
+        v4s h2[4];
+        float g2[4][4], y[4] = {};
+        {
+            const v8bf a0 = get(0), a1 = get(1);
+            lds_order();
+#pragma unroll
+            for (int nb = 0; nb < 4; ++nb) {
+                v4f z = {0.0f, 0.0f, 0.0f, 0.0f};
+                z = mfma32(a0, *(const v8bf *)sh.w2[0][nb][lw], z);
+                z = mfma32(a1, *(const v8bf *)sh.w2[1][nb][lw], z);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const float h = bfr(gelu_grad(z[j] + b2[nb], g2[nb][j]));
+                    h2[nb][j] = (short)f2bf(h);
+                    y[j] += h * w3[nb];
+                }
+#pragma unroll
+                for (int j = 0; j < 4; ++j) asm volatile("" : "+v"(g2[nb][j]));
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        float dy[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            for (int o = 1; o < 16; o <<= 1) y[j] += __shfl_xor(y[j], o);
+            const float e = base + 4 * g + j < end ? y[j] + b3 - t[j] : 0.0f;
+            dy[j] = 2.0f * e * d.inv_b;
+            sse += e * e;
+            gb3 += dy[j];
+        }
+        v4s dz2[4];
+#pragma unroll
+        for (int nb = 0; nb < 4; ++nb)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                gw3[nb] += dy[j] * __uint_as_float((uint32_t)(uint16_t)h2[nb][j] << 16);
+                const float dz = dy[j] * w3[nb] * g2[nb][j];
+                gb2[nb] += dz;
+                dz2[nb][j] = (short)f2bf(dz);
+            }
+        put(dz2);
+#pragma unroll
+        for (int mb = 0; mb < 4; ++mb)
+#pragma unroll
+            for (int nb = 0; nb < 4; ++nb) gw2[mb][nb] = mfma(h1[mb], dz2[nb], gw2[mb][nb]);
+        const v8bf a0 = get(0), a1 = get(1);
+        const v4s xt = sl < 8 ? *(const v4s *)&sh.xt[wi][sl][4 * g] : v4s{0, 0, 0, 0};
+        lds_order();  // before the next tile's writes
+#pragma unroll
+        for (int nb = 0; nb < 4; ++nb) {
+            v4f a = {0.0f, 0.0f, 0.0f, 0.0f};
+            a = mfma32(a0, *(const v8bf *)sh.w2t[0][nb][lw], a);
+            a = mfma32(a1, *(const v8bf *)sh.w2t[1][nb][lw], a);
+            v4s dz1;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const float dz = a[j] * g1[nb][j];
+                gb1[nb] += dz;
+                dz1[j] = (short)f2bf(dz);
+            }
+            gw1[nb] = mfma(xt, dz1, gw1[nb]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    // the block's sums, then the grid's
+#pragma unroll
+    for (int mb = 0; mb < 4; ++mb)
+#pragma unroll
+        for (int nb = 0; nb < 4; ++nb)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                atomicAdd(&sh.grad[oW2 + (16 * mb + 4 * g + j) * kDH + 16 * nb + sl], gw2[mb][nb][j]);
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb) {
+        const int n = 16 * nb + sl;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (4 * g + j < kDIn) atomicAdd(&sh.grad[oW1 + (4 * g + j) * kDH + n], gw1[nb][j]);
+        atomicAdd(&sh.grad[oB1 + n], gb1[nb]);
+        atomicAdd(&sh.grad[oB2 + n], gb2[nb]);
+        atomicAdd(&sh.grad[oW3 + n], gw3[nb]);
+    }
+    // the lanes of a group hold the same samples
+    for (int o = 16; o < 64; o <<= 1) {
+        gb3 += __shfl_xor(gb3, o);
+        sse += __shfl_xor(sse, o);
+    }
+    if (l == 0) {
+        atomicAdd(&sh.grad[oB3], gb3);
+        atomicAdd(d.loss, sse);
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < kNParams; i += kTrainBlock) atomicAdd(d.grad + i, sh.grad[i]);
 }
 
-// Adam (Kingma & Ba 2015) on the f32 master parameters
 __global__ void k_adam(float *w, float *m, float *v, const float *g, int n, float lr, float b1, float b2,
                        float eps, float bc1, float bc2)
 {
@@ -535,7 +540,7 @@ static unsigned infer_grid(uint64_t count)
 
 static unsigned mlp_grid(uint64_t count, unsigned cap)
 {
-    const uint64_t tiles = (count + 15) / 16, blocks = (tiles + hb::mlp::kWaves - 1) / hb::mlp::kWaves;
+    const uint64_t tiles = (count + 15) / 16, blocks = (tiles + hb::mlp::kTrainWaves - 1) / hb::mlp::kTrainWaves;
     return (unsigned)std::max<uint64_t>(1, std::min<uint64_t>(blocks, cap));
 }
 
@@ -615,7 +620,7 @@ int hb_mlp_gradient(hb_mlp *n, const float *x, const float *y, uint64_t count, f
     HB_MTRY(hipMemsetAsync(n->g, 0, hb::mlp::kNParams * 4, n->stream));
     HB_MTRY(hipMemsetAsync(n->loss, 0, 4, n->stream));
     hb::mlp::Dev d{n->w, n->norm, n->x, n->y, nullptr, 0, count, (float)(1.0 / (double)count), n->g, n->loss, nullptr};
-    hb::mlp::k_train<<<mlp_grid(count, 1024), hb::mlp::kBlock, 0, n->stream>>>(d);
+    hb::mlp::k_train<<<mlp_grid(count, 512), hb::mlp::kTrainBlock, 0, n->stream>>>(d);
     HB_MTRY(hipGetLastError());
     float sse = 0.0f;
     HB_MTRY(hipMemcpyAsync(grad, n->g, hb::mlp::kNParams * 4, hipMemcpyDeviceToHost, n->stream));
@@ -663,7 +668,7 @@ int hb_mlp_train(hb_mlp *n, const float *x, const float *y, uint64_t count, int 
             const uint64_t cnt = std::min<uint64_t>(batch, count - first);
             hb::mlp::k_zero<<<(hb::mlp::kNParams + 255) / 256, 256, 0, n->stream>>>(n->g, hb::mlp::kNParams);
             hb::mlp::Dev d{n->w, n->norm, n->x, n->y, n->idx, first, cnt, (float)(1.0 / (double)cnt), n->g, n->loss, nullptr};
-            hb::mlp::k_train<<<mlp_grid(cnt, 1024), hb::mlp::kBlock, 0, n->stream>>>(d);
+            hb::mlp::k_train<<<mlp_grid(cnt, 512), hb::mlp::kTrainBlock, 0, n->stream>>>(d);
             ++n->step;
             const float bc1 = (float)(1.0 - std::pow(0.9, (double)n->step));
             const float bc2 = (float)(1.0 - std::pow(0.999, (double)n->step));
