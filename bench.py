@@ -84,7 +84,8 @@ def algorithmic_bytes(slot, arcs, nodes, items, p, gathered, first_nodes=0):
 
 
 def kernel_name(slot, p, team, layout):
-    """The kernel that does a slot's work in the dense iterations.  In the chain layout at
+    """The kernel that does a slot's work in the dense iterations (k_union has a second
+    instantiation, in the same slot, for the first one).  In the chain layout at
     p = 5 and 6 the single bin of one-copy teams (an id range from node 0) is run by
     k_union_rows after the first iteration, which k_union still runs."""
     if slot == 0 and layout == "chain" and p in (5, 6) and team == (1 << p) // 16:

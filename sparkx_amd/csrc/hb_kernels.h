@@ -104,7 +104,8 @@ hipError_t coo_to_csr(const uint32_t *src, const uint32_t *dst, uint64_t m, uint
 // chunks [first[h], first[h + 1]) (device arrays).  A wavefront of k_walk takes the lists of
 // 64 nodes one after the other, so lists near the line set its time: R-MAT-22 in the degree
 // layout took 2.7 ms for two passes when lists of up to 4,096 arcs stayed there, 1.9 at 1,024,
-// 1.6 at 512, 1.5 at 256 (chunks of 512, 1,024 or 2,048 arcs: within 0.02 ms).
+// 1.6 at 512, 1.5 at 256 (chunks of 512, 1,024 or 2,048 arcs: within 0.02 ms).  R-MAT-24 has
+// work enough to hide them: 6.5 ms with lists up to 4,096 and at 256.
 constexpr uint32_t kWalkHub = 256, kWalkChunk = 2048;
 struct WalkHubs {
     const uint32_t *beg = nullptr, *end = nullptr, *node = nullptr, *first = nullptr;
