@@ -14,7 +14,7 @@ CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libsparkx_hb.so")
 
 SOURCES = ["hb_kernels.hip", "hb_api.hip", "hb_batch.hip", "hb_mlp.hip", "hb_exact.hip", "hb_eval.hip", "hb_layout.hip", "hb_ingest.hip", "hb_walk.hip", "hb_transfer.cpp", "hb_graphgen.cpp"]
-HEADERS = ["hb_device.h", "hb_kernels.h", "hb_union.h", "hll_bias_table.inc"]
+HEADERS = ["hb_device.h", "hb_kernels.h", "hb_schedule.h", "hb_union.h", "hll_bias_table.inc"]
 ABI_HEADERS = ["sparkx_hb.h", "sparkx_hb_graphgen.h"]  # under include/ at the repo root
 
 # -ffp-contract=off: the f64 accumulators and f32 estimates must not fuse a*b+c

@@ -25,6 +25,7 @@
 #include "../../include/sparkx_hb.h"
 #include "hb_device.h"
 #include "hb_kernels.h"
+#include "hb_schedule.h"
 
 #define HB_BIAS_TABLE_QUAL static const
 #include "hll_bias_table.inc"
@@ -269,6 +270,21 @@ struct hb_ctx {
 
 static bool set_device(hb_ctx *c) { return hipSetDevice(c->device) == hipSuccess; }
 
+// A buffer of the context.  Short of memory, the partial rows of the hubs' tasks are given up
+// first: only a run needs them, and it can do with fewer (build_schedule).
+template <class T>
+static hipError_t ensure(hb_ctx *c, DevBuf<T> &b, size_t n)
+{
+    hipError_t e = b.ensure(n);
+    if (e == hipErrorOutOfMemory && c->scratch.ptr) {
+        (void)hipGetLastError();
+        c->scratch.release();
+        c->sched_p = 0;
+        e = b.ensure(n);
+    }
+    return e;
+}
+
 static int ensure_layout(hb_ctx *c);
 
 // The CSR is in c->off / c->nbr: keeps a host copy of the offsets (h_off, or read
@@ -489,12 +505,9 @@ static int build_schedule(hb_ctx *c, int p)
     const uint32_t G = std::min(64u, (1u << p) / 16u);
     const uint32_t n = (uint32_t)c->n;
     const std::vector<uint32_t> &h_off = c->run_hoff();
-    c->n_linked = 0;
+    c->sched_p = 0;  // until the new one is in place
     std::vector<uint32_t> bins[3], tnode, tbeg, tend, hnode, htask0, hntask;
-    // p > 10: longer lists are cut (a wavefront reads a row of 4 KiB in about 0.7 us, so a
-    // hub of 10,000 neighbours alone would take as long as the rest of the iteration)
-    constexpr uint32_t kWideHub = 256;
-    auto split = [&](uint32_t u, uint32_t chunk) {
+    auto split = [&](uint32_t u, uint64_t chunk) {
         hnode.push_back(u);
         htask0.push_back((uint32_t)tnode.size());
         uint32_t cnt = 0;
@@ -505,20 +518,30 @@ static int build_schedule(hb_ctx *c, int p)
         }
         hntask.push_back(cnt);
     };
-    for (uint32_t u = 0; u < n; ++u) {
-        const uint32_t d = h_off[u + 1] - h_off[u];
-        if (d == 0) continue;  // keeps c_0; written to both buffers at init
-        ++c->n_linked;
-        if (p > 10 && d <= kWideHub) bins[2].push_back(u);  // a wavefront per node
-        else if (p > 10) split(u, kWideHub);
-        else if (d <= c->small_max) bins[0].push_back(u);
-        else if (d <= c->mid_max) bins[1].push_back(u);
-        else if (d <= c->wave_max) bins[2].push_back(u);
-        else split(u, c->chunk);
+    size_t total = 0;
+    for (uint64_t wide_len = p > 10 ? hb::wide_task_len(h_off.data(), n, p) : 0;; wide_len *= 2) {
+        for (auto *v : {&bins[0], &bins[1], &bins[2], &tnode, &tbeg, &tend, &hnode, &htask0, &hntask}) v->clear();
+        c->n_linked = 0;
+        for (uint32_t u = 0; u < n; ++u) {
+            const uint32_t d = h_off[u + 1] - h_off[u];
+            if (d == 0) continue;  // keeps c_0; written to both buffers at init
+            ++c->n_linked;
+            if (p > 10 && d <= wide_len) bins[2].push_back(u);  // a wavefront per node
+            else if (p > 10) split(u, wide_len);
+            else if (d <= c->small_max) bins[0].push_back(u);
+            else if (d <= c->mid_max) bins[1].push_back(u);
+            else if (d <= c->wave_max) bins[2].push_back(u);
+            else split(u, c->chunk);
+        }
+        total = bins[0].size() + bins[1].size() + bins[2].size() + 3 * tnode.size() + 3 * hnode.size();
+        HB_TRY(c->sched_buf.ensure(total));
+        HB_TRY(c->chunk_flag.ensure(tnode.size()));
+        const hipError_t e = c->scratch.ensure(tnode.size() << p);
+        if (e == hipSuccess) break;
+        // p > 10: a run needs no tasks; where their partial rows do not fit, fewer lists are cut
+        if (e != hipErrorOutOfMemory || p <= 10 || tnode.empty()) HB_TRY(e);
+        (void)hipGetLastError();
     }
-    const size_t total = bins[0].size() + bins[1].size() + bins[2].size() + 3 * tnode.size() +
-                         3 * hnode.size();
-    HB_TRY(c->sched_buf.ensure(total));
     std::vector<uint32_t> host;
     host.reserve(total);
     hb::HbSchedule s;
@@ -557,8 +580,6 @@ static int build_schedule(hb_ctx *c, int p)
     if (!host.empty())
         HB_TRY(hipMemcpyAsync(c->sched_buf.ptr, host.data(), host.size() * 4, hipMemcpyHostToDevice,
                               c->stream));
-    HB_TRY(c->scratch.ensure((size_t)s.ntasks << p));
-    HB_TRY(c->chunk_flag.ensure(s.ntasks));
     if (c->sym && p <= 10) HB_TRY(c->dyn.ensure((size_t)s.bin_count[0] + s.bin_count[1] + s.bin_count[2] + 3));
     HB_TRY(hipStreamSynchronize(c->stream));
     c->sched = s;
@@ -673,11 +694,11 @@ static int ensure_layout(hb_ctx *c)
     if (c->layout == HB_LAYOUT_INPUT || c->laid_out || c->n == 0) return HB_OK;
     const int kind = resolve_layout(c);
     const uint32_t n = (uint32_t)c->n, arcs = (uint32_t)c->arcs;
-    HB_TRY(c->perm.ensure(n));
-    HB_TRY(c->sigma.ensure(n));
-    HB_TRY(c->roff.ensure((size_t)n + 1));
-    HB_TRY(c->rnbr.ensure(arcs));
-    HB_TRY(c->rorig.ensure(arcs));
+    HB_TRY(ensure(c, c->perm, n));
+    HB_TRY(ensure(c, c->sigma, n));
+    HB_TRY(ensure(c, c->roff, (size_t)n + 1));
+    HB_TRY(ensure(c, c->rnbr, arcs));
+    HB_TRY(ensure(c, c->rorig, arcs));
     hipEvent_t e0, e1;
     HB_TRY(hipEventCreate(&e0));
     HB_TRY(hipEventCreate(&e1));
@@ -719,7 +740,7 @@ static int copy_out(hb_ctx *c, const void *src, void *dst, size_t row_bytes)
         HB_TRY(hb::read_back(dst, src, bytes, c->stream));
         return HB_OK;
     }
-    HB_TRY(c->readback.ensure(bytes));
+    HB_TRY(ensure(c, c->readback, bytes));
     HB_TRY(hb::unpermute_rows(src, c->readback.ptr, c->sigma.ptr, (uint32_t)c->n, row_bytes, c->stream));
     HB_TRY(hb::read_back(dst, c->readback.ptr, bytes, c->stream));
     return HB_OK;
@@ -755,29 +776,24 @@ extern "C" int hb_run(hb_ctx *c, int p, int max_iters, uint32_t flags, hb_stats 
         return HB_OK;
     }
 
-    HB_TRY(c->regs0.ensure((size_t)c->n << p));
-    HB_TRY(c->regs1.ensure((size_t)c->n << p));
-    HB_TRY(c->est.ensure(c->n));
-    HB_TRY(c->dist.ensure(c->n));
-    HB_TRY(c->inv.ensure(c->n));
-    HB_TRY(c->st.ensure(1));
+    HB_TRY(ensure(c, c->regs0, (size_t)c->n << p));
+    HB_TRY(ensure(c, c->regs1, (size_t)c->n << p));
+    HB_TRY(ensure(c, c->est, c->n));
+    HB_TRY(ensure(c, c->dist, c->n));
+    HB_TRY(ensure(c, c->inv, c->n));
+    HB_TRY(ensure(c, c->st, 1));
     // No iteration cap: a run ends by the reference's rule or at max_iters.  A graph
     // cannot change a register after its diameter, so n + 2 iterations bound a correct
     // run; the host loop stops there with an error rather than going on.
     const uint64_t bound = max_iters > 0 ? (uint64_t)max_iters : (uint64_t)c->n + 2;
-    HB_TRY(c->rec.ensure(1));
+    HB_TRY(ensure(c, c->rec, 1));
     const DeviceTables *tables = nullptr;
     HB_TRY(device_tables(c->device, p, &tables, c->stream));
     RecordSlot records;
     HB_TRY(records.take(c->stream));
-    if (c->snap_k) HB_TRY(c->snaps.ensure((size_t)c->snap_k * c->n));
+    if (c->snap_k) HB_TRY(ensure(c, c->snaps, (size_t)c->snap_k * c->n));
     const bool push_ok = c->sym && p <= 10;
-    {
-        int rc = ensure_layout(c);  // normally built at staging already
-        default_schedule(c, p);
-        if (rc == HB_OK) rc = build_schedule(c, p);
-        if (rc != HB_OK) return rc;
-    }
+    if (const int rc = ensure_layout(c)) return rc;  // normally built at staging already
 
     // Saturation pays where most nodes come to hold the same sketch within a few iterations,
     // which the chain layout's graphs do not; its kernels and the dense schedule, which
@@ -789,7 +805,10 @@ extern "C" int hb_run(hb_ctx *c, int p, int max_iters, uint32_t flags, hb_stats 
     // the bound, and at p > 10 its packed form; the iteration counters
     const size_t count_at = (bit_words + (sat_ok ? m + (p > 10 ? m / 4 : 0) : 0) + 63) & ~(size_t)63;
     const size_t all_words = count_at + 2 * HB_COUNT_COPIES * HB_COUNT_STRIDE;
-    HB_TRY(c->bits.ensure(all_words));
+    HB_TRY(ensure(c, c->bits, all_words));
+    // last: how much it allocates depends on what is left
+    default_schedule(c, p);
+    if (const int rc = build_schedule(c, p)) return rc;
 
     HbDev &d = c->dev;
     d = HbDev{};
@@ -1098,7 +1117,7 @@ static int estimates_of(hb_ctx *c, int which, const float **est)
             return HB_OK;
         }
     }
-    HB_TRY(c->est_tmp.ensure(c->n));
+    HB_TRY(ensure(c, c->est_tmp, c->n));
     HB_TRY(hb::launch_estimates(c->dev, regs, c->est_tmp.ptr, c->stream));
     *est = c->est_tmp.ptr;
     return HB_OK;
@@ -1153,7 +1172,7 @@ extern "C" int hb_centrality(hb_ctx *c, int kind, int normalize, double *dst)
     if (!c->ran) return fail(HB_ESTATE, "hb_centrality: no completed run");
     if (c->n == 0) return HB_OK;
     if (!set_device(c)) return fail(HB_EHIP, "hipSetDevice failed");
-    HB_TRY(c->cent.ensure(c->n));
+    HB_TRY(ensure(c, c->cent, c->n));
     // the epilogues take the estimates of the reference's counters buffer (hyper_ball.rs:452,506,544)
     const float *est = nullptr;
     if (int rc = estimates_of(c, HB_REGS_REFERENCE, &est)) return rc;
@@ -1309,11 +1328,11 @@ extern "C" int hb_restore(hb_ctx *c, int p, const uint8_t *regs, const double *d
     const uint32_t n = (uint32_t)c->n, m = 1u << p;
     if (int rc = ensure_layout(c)) return rc;
     const size_t rbytes = (size_t)n << p;
-    HB_TRY(c->regs0.ensure(std::max<size_t>(rbytes, 1)));
-    HB_TRY(c->regs1.ensure(std::max<size_t>(rbytes, 1)));
-    HB_TRY(c->dist.ensure(std::max<uint32_t>(n, 1)));
-    HB_TRY(c->inv.ensure(std::max<uint32_t>(n, 1)));
-    HB_TRY(c->cent.ensure(std::max<uint32_t>(n, 1)));
+    HB_TRY(ensure(c, c->regs0, std::max<size_t>(rbytes, 1)));
+    HB_TRY(ensure(c, c->regs1, std::max<size_t>(rbytes, 1)));
+    HB_TRY(ensure(c, c->dist, std::max<uint32_t>(n, 1)));
+    HB_TRY(ensure(c, c->inv, std::max<uint32_t>(n, 1)));
+    HB_TRY(ensure(c, c->cent, std::max<uint32_t>(n, 1)));
     const DeviceTables *tables = nullptr;
     HB_TRY(device_tables(c->device, p, &tables, c->stream));
     if (n) {
@@ -1411,8 +1430,8 @@ extern "C" int hb_surrogate(hb_ctx *c, hb_mlp *mlp, int p_feat, float *pred, flo
     if (rc != HB_OK) return rc;
     // device time: register init + the 4 iterations (hb_run's events, host set-up excluded)
     // + features and inference
-    HB_TRY(c->feat.ensure(c->n * 6));
-    HB_TRY(c->pred.ensure(c->n));
+    HB_TRY(ensure(c, c->feat, c->n * 6));
+    HB_TRY(ensure(c, c->pred, c->n));
     hipEvent_t e0, e1;
     HB_TRY(hipEventCreate(&e0));
     HB_TRY(hipEventCreate(&e1));
@@ -1460,7 +1479,7 @@ static int walk_surrogate(hb_ctx *c, hb_mlp *mlp, int passes, bool want_x, float
         table.insert(table.end(), end.begin(), end.end());
         table.insert(table.end(), node.begin(), node.end());
         table.insert(table.end(), first.begin(), first.end());
-        HB_TRY(c->walk_hub.ensure(table.size() + n));
+        HB_TRY(ensure(c, c->walk_hub, table.size() + n));
         HB_TRY(hipMemcpyAsync(c->walk_hub.ptr, table.data(), table.size() * 4, hipMemcpyHostToDevice, c->stream));
         HB_TRY(hipStreamSynchronize(c->stream));  // `table` is a pageable host buffer
         c->walk_chunks = (uint32_t)beg.size();
@@ -1474,9 +1493,9 @@ static int walk_surrogate(hb_ctx *c, hb_mlp *mlp, int passes, bool want_x, float
     hubs.node = hubs.end + hubs.chunks;
     hubs.first = hubs.node + hubs.hubs;
     uint32_t *deg = c->walk_hub.ptr + 2 * (size_t)hubs.chunks + 2 * (size_t)hubs.hubs + 1;
-    HB_TRY(c->walk.ensure(4 * (size_t)n + 2 * (size_t)hubs.chunks));
-    HB_TRY(c->feat.ensure((size_t)n * 6));
-    if (mlp) HB_TRY(c->pred.ensure(n));
+    HB_TRY(ensure(c, c->walk, 4 * (size_t)n + 2 * (size_t)hubs.chunks));
+    HB_TRY(ensure(c, c->feat, (size_t)n * 6));
+    if (mlp) HB_TRY(ensure(c, c->pred, n));
     hipEvent_t e0, e1;
     HB_TRY(hipEventCreate(&e0));
     HB_TRY(hipEventCreate(&e1));
