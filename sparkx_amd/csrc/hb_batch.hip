@@ -497,8 +497,8 @@ __global__ __launch_bounds__(HB_WAVE) void k_batch_finalize(HbBatchDev b)
     st.parity ^= 1u;
     st.t = st.t + 1.0;
     st.inv_t = __ddiv_rn(1.0, st.t);
-    st.skip_scan = 2 * chg > (unsigned long long)g.n_linked;
-    st.sat_arcs += sat;  // as k_finalize
+    st.skip_scan = (it == 1 && b.sat_max) || 2 * chg > (unsigned long long)g.n_linked;  // as k_finalize
+    st.sat_arcs += sat;
     st.sat_scan = 8 * st.sat_arcs >= (unsigned long long)g.n_linked;
 }
 

@@ -1362,10 +1362,14 @@ __global__ __launch_bounds__(HB_WAVE) void k_finalize(HbDev d)
     }
     st->iter = it + 1;
     st->parity ^= 1u;
-    st->skip_scan = 2 * chg > (unsigned long long)d.n_linked;
+    // Iteration 1 marks no node saturated.  Iteration 2 recomputes every node, so that from then
+    // on a node whose sketch is the bound is marked, and one that a saturated neighbour raises
+    // has changed.  (Almost every node changes in iteration 1 anyway.)
+    const bool mark = it == 1 && d.sat_max;
+    st->skip_scan = mark || 2 * chg > (unsigned long long)d.n_linked;
     // push when few nodes changed (on R-MAT-24 a push pass at 24% changed nodes whose lists
     // hold 2% of the arcs measured slower than the scan with selective gathers)
-    st->push = d.sym && d.p <= 10 && d.frontier && 16 * chg <= (unsigned long long)d.n_linked;
+    st->push = !mark && d.sym && d.p <= 10 && d.frontier && 16 * chg <= (unsigned long long)d.n_linked;
     // a search that finds nothing costs a node about a quarter of its gather on short lists
     // (Erdos-Renyi, n = 65,536, degree 32: 74 against 60 us an iteration), one that finds a
     // neighbour saves all of it: search once a node has one in eight such neighbours on average

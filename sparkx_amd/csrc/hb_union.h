@@ -315,7 +315,7 @@ __device__ __forceinline__ uint32_t union_node(const HbView &v, const HbTables &
     uint32_t diffw;  // bit 0: a register rose; bit 1: a register is below the bound
     if (sat) {
         acc = v.bound[cl];
-        diffw = 1u;  // an unmarked sketch below a saturated neighbour's rises
+        diffw = 1u;  // this one is not marked, so it is below the bound and rises
     } else {
         uint4 own;
         if constexpr (kGather == Gather::kFirst)
