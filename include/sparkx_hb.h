@@ -127,6 +127,12 @@ const char *hb_last_error(void);
  * binary comes from. */
 const char *hb_build_digest(void);
 
+/* Frees the device memory the library keeps between calls: after hb_exact_bfs and
+ * hb_exact_centrality one block of at most 2 GiB per device, for the next such call.  The
+ * library gives it back by itself when an allocation of its own fails; this is for other
+ * users of the device.  No counterpart in the reference. */
+void hb_release_memory(void);
+
 /* Stages a CSR graph into HBM once, through pinned host buffers.  offsets has n+1
  * entries and nbrs has arcs entries, each 8- or 4-byte unsigned (the reference's
  * mmap'd index and edge files are 8-byte).  Neighbour ids must be < n and offsets

@@ -6,4 +6,4 @@ from .graph import Graph  # noqa: F401
 from .hyper_ball import (HyperBall, HyperBall4, HyperBall5, HyperBall6, HyperBall7,  # noqa: F401
                          HyperBall8, HyperBall9, HyperBall10, HyperBall11, HyperBall12,
                          HyperBall13, HyperBall14, HyperBall15, HyperBall16)
-from ._lib import HyperBallError  # noqa: F401
+from ._lib import HyperBallError, release_memory  # noqa: F401

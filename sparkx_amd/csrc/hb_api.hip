@@ -140,13 +140,8 @@ struct DevBuf {
     {
         if (n <= count && ptr) return hipSuccess;
         release();
-        hipError_t e = hipMalloc(&ptr, std::max<size_t>(n, 1) * sizeof(T));
-        if (e == hipErrorOutOfMemory) {
-            hb::release_held();
-            e = hipMalloc(&ptr, std::max<size_t>(n, 1) * sizeof(T));
-        }
+        const hipError_t e = hb::device_alloc(&ptr, std::max<size_t>(n, 1) * sizeof(T));
         if (e == hipSuccess) count = n;
-        else ptr = nullptr;
         return e;
     }
     void release()
@@ -155,7 +150,7 @@ struct DevBuf {
         ptr = nullptr;
         count = 0;
     }
-    void adopt(T *p, size_t n)  // takes a hipMalloc'd buffer
+    void adopt(T *p, size_t n)  // takes a buffer of device_alloc
     {
         release();
         ptr = p;
@@ -277,7 +272,6 @@ static hipError_t ensure(hb_ctx *c, DevBuf<T> &b, size_t n)
 {
     hipError_t e = b.ensure(n);
     if (e == hipErrorOutOfMemory && c->scratch.ptr) {
-        (void)hipGetLastError();
         c->scratch.release();
         c->sched_p = 0;
         e = b.ensure(n);
@@ -296,7 +290,7 @@ static int finish_stage(hb_ctx *c, uint64_t n, uint64_t arcs, std::vector<uint32
     c->sym = true;
     if (n) {
         unsigned long long *acc = nullptr, h_acc[4] = {};
-        HB_TRY(hipMalloc(&acc, (4 + 4 * hb::kFingerprintBlocks) * sizeof(unsigned long long)));
+        HB_TRY(hb::device_alloc(&acc, (4 + 4 * hb::kFingerprintBlocks) * sizeof(unsigned long long)));
         hipError_t e = hb::arc_fingerprints(c->off.ptr, c->nbr.ptr, (uint32_t)n, arcs, acc, c->stream);
         if (e == hipSuccess) e = hipMemcpyAsync(h_acc, acc, sizeof h_acc, hipMemcpyDeviceToHost, c->stream);
         if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
@@ -324,6 +318,8 @@ const char *hb_last_error(void) { return g_err.c_str(); }
 #define HB_BUILD_DIGEST "unknown"
 #endif
 const char *hb_build_digest(void) { return HB_BUILD_DIGEST; }
+
+void hb_release_memory(void) { hb::release_held(); }
 
 int hb_create(hb_ctx **out, int device_ordinal)
 {
@@ -540,7 +536,6 @@ static int build_schedule(hb_ctx *c, int p)
         if (e == hipSuccess) break;
         // p > 10: a run needs no tasks; where their partial rows do not fit, fewer lists are cut
         if (e != hipErrorOutOfMemory || p <= 10 || tnode.empty()) HB_TRY(e);
-        (void)hipGetLastError();
     }
     std::vector<uint32_t> host;
     host.reserve(total);
@@ -611,8 +606,8 @@ hipError_t device_tables(int device, int p, const DeviceTables **out, hipStream_
     std::vector<float> lc(m + 1, 0.0f);
     for (uint32_t z = 1; z <= m; ++z) lc[z] = (float)((double)m * std::log((double)m / (double)z));
     DeviceTables t;
-    hipError_t e = hipMalloc(&t.lc, (m + 1) * sizeof(float));
-    if (e == hipSuccess) e = hipMalloc(&t.bias, sizeof(HbBiasTable));
+    hipError_t e = hb::device_alloc(&t.lc, (m + 1) * sizeof(float));
+    if (e == hipSuccess) e = hb::device_alloc(&t.bias, sizeof(HbBiasTable));
     if (e == hipSuccess) e = hipMemcpyAsync(t.lc, lc.data(), (m + 1) * sizeof(float), hipMemcpyHostToDevice, s);
     if (e == hipSuccess) e = hipMemcpyAsync(t.bias, hb::bias_table(p), sizeof(HbBiasTable), hipMemcpyHostToDevice, s);
     // in place before a kernel of any stream reads them
@@ -1618,7 +1613,7 @@ extern "C" int hb_stage_mtx(hb_ctx *c, const char *text, uint64_t len, hb_mtx_in
     c->n = c->arcs = 0;
     const uint64_t body = len - h.body;
     uint8_t *dtext = nullptr;
-    HB_TRY(hipMalloc(&dtext, std::max<uint64_t>(body, 1)));
+    HB_TRY(hb::device_alloc(&dtext, std::max<uint64_t>(body, 1)));
     hipError_t e = hb::upload(dtext, text + h.body, body, c->stream);
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (e == hipSuccess) e = hipEventCreate(&e0);
@@ -1670,8 +1665,8 @@ extern "C" int hb_stage_coo(hb_ctx *c, uint64_t n, const uint32_t *src, const ui
     c->release_layout();
     c->n = c->arcs = 0;
     uint32_t *ds = nullptr, *dd = nullptr;
-    hipError_t e = hipMalloc(&ds, std::max<uint64_t>(m, 1) * 4);
-    if (e == hipSuccess) e = hipMalloc(&dd, std::max<uint64_t>(m, 1) * 4);
+    hipError_t e = hb::device_alloc(&ds, std::max<uint64_t>(m, 1) * 4);
+    if (e == hipSuccess) e = hb::device_alloc(&dd, std::max<uint64_t>(m, 1) * 4);
     if (e == hipSuccess && m) e = hipMemcpyAsync(ds, src, m * 4, hipMemcpyDefault, c->stream);
     if (e == hipSuccess && m) e = hipMemcpyAsync(dd, dst, m * 4, hipMemcpyDefault, c->stream);
     hb::CsrBuild b{};

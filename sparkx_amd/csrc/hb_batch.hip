@@ -547,7 +547,7 @@ struct DevArr {
         if (ptr) (void)hipFree(ptr);
         ptr = nullptr;
         count = n;
-        return hipMalloc(&ptr, std::max<size_t>(n, 1) * sizeof(T));
+        return hb::device_alloc(&ptr, std::max<size_t>(n, 1) * sizeof(T));
     }
     hipError_t put(const std::vector<T> &h, hipStream_t s)
     {

@@ -180,14 +180,14 @@ struct Ranker {
 
     int init(int arrays)
     {
-        HBE_TRY(hipMalloc(&kin.p, n * 8));
-        HBE_TRY(hipMalloc(&kout.p, n * 8));
-        HBE_TRY(hipMalloc(&iin.p, n * 4));
-        HBE_TRY(hipMalloc(&nan.p, arrays * 8));
+        HBE_TRY(hb::device_alloc(&kin.p, n * 8));
+        HBE_TRY(hb::device_alloc(&kout.p, n * 8));
+        HBE_TRY(hb::device_alloc(&iin.p, n * 4));
+        HBE_TRY(hb::device_alloc(&nan.p, arrays * 8));
         HBE_TRY(hipMemsetAsync(nan.p, 0xff, arrays * 8, s));
         HBE_TRY(rocprim::radix_sort_pairs_desc(nullptr, tmp_bytes, (double *)kin.p, (double *)kout.p,
                                                (uint32_t *)iin.p, (uint32_t *)iin.p, (size_t)n, 0, 64, s));
-        HBE_TRY(hipMalloc(&tmp.p, std::max<size_t>(tmp_bytes, 1)));
+        HBE_TRY(hb::device_alloc(&tmp.p, std::max<size_t>(tmp_bytes, 1)));
         grid = (unsigned)std::min<uint64_t>((n + hb::eval::kBlock - 1) / hb::eval::kBlock, 8192);
         return HB_OK;
     }
@@ -233,9 +233,9 @@ extern "C" int hb_eval_ranks(int device, const double *v, uint64_t n, uint32_t *
     StreamGuard sg;
     HBE_TRY(hipStreamCreateWithFlags(&sg.s, hipStreamNonBlocking));
     DevMem dv, order, rk;
-    HBE_TRY(hipMalloc(&dv.p, n * 8));
-    HBE_TRY(hipMalloc(&order.p, n * 4));
-    HBE_TRY(hipMalloc(&rk.p, n * 4));
+    HBE_TRY(hb::device_alloc(&dv.p, n * 8));
+    HBE_TRY(hb::device_alloc(&order.p, n * 4));
+    HBE_TRY(hb::device_alloc(&rk.p, n * 4));
     HBE_TRY(hipMemcpyAsync(dv.p, v, n * 8, hipMemcpyDefault, sg.s));
     Ranker r{fn, n, sg.s};
     if (int rc = r.init(1)) return rc;
@@ -260,15 +260,15 @@ extern "C" int hb_eval_metrics(int device, const double *a, const double *b, uin
     HBE_TRY(hipStreamCreateWithFlags(&sg.s, hipStreamNonBlocking));
     const hipStream_t s = sg.s;
     DevMem va, vb, oa, ob, rka, rkb, flag, part, tpart;
-    HBE_TRY(hipMalloc(&va.p, n * 8));
-    HBE_TRY(hipMalloc(&vb.p, n * 8));
-    HBE_TRY(hipMalloc(&oa.p, n * 4));
-    HBE_TRY(hipMalloc(&ob.p, n * 4));
-    HBE_TRY(hipMalloc(&rka.p, n * 4));
-    HBE_TRY(hipMalloc(&rkb.p, n * 4));
-    HBE_TRY(hipMalloc(&flag.p, n));
-    HBE_TRY(hipMalloc(&part.p, kSumBlocks * sizeof(Partial)));
-    HBE_TRY(hipMalloc(&tpart.p, kSumBlocks * 8));
+    HBE_TRY(hb::device_alloc(&va.p, n * 8));
+    HBE_TRY(hb::device_alloc(&vb.p, n * 8));
+    HBE_TRY(hb::device_alloc(&oa.p, n * 4));
+    HBE_TRY(hb::device_alloc(&ob.p, n * 4));
+    HBE_TRY(hb::device_alloc(&rka.p, n * 4));
+    HBE_TRY(hb::device_alloc(&rkb.p, n * 4));
+    HBE_TRY(hb::device_alloc(&flag.p, n));
+    HBE_TRY(hb::device_alloc(&part.p, kSumBlocks * sizeof(Partial)));
+    HBE_TRY(hb::device_alloc(&tpart.p, kSumBlocks * 8));
     HBE_TRY(hipMemcpyAsync(va.p, a, n * 8, hipMemcpyDefault, s));
     HBE_TRY(hipMemcpyAsync(vb.p, b, n * 8, hipMemcpyDefault, s));
     Ranker r{fn, n, s};

@@ -742,9 +742,9 @@ namespace {
 constexpr uint64_t kBfsBudget = 16ull << 30;  // device memory of one group of slices
 // What a group needs is kept between calls up to this much, one block per device: the driver
 // clears freed device memory at some 40 GB/s before it hands it out again, so a call of 12 ms
-// that takes and frees 5 GB soon waits 130 ms for it.  Given back as soon as an allocation
-// of the engine fails (release_held).  A block in use belongs to one call; a second call at the same time takes
-// memory of its own.
+// that takes and frees 5 GB soon waits 130 ms for it.  Given back when any allocation of the
+// library fails (device_alloc) and by hb_release_memory.  A block in use belongs to one call; a
+// second call at the same time takes memory of its own.
 constexpr uint64_t kBfsHold = 2ull << 30;
 constexpr int kBfsDevices = 16;
 
@@ -780,7 +780,7 @@ struct BfsMemory {
             if (held) (void)hipFree(held);  // too small: its place is for this one
             held = nullptr;
         }
-        const hipError_t e = hipMalloc(&p, want);
+        const hipError_t e = device_alloc(&p, want);
         if (e != hipSuccess) p = nullptr;
         else bytes = want;
         return e;
@@ -931,6 +931,20 @@ void release_held()
     }
 }
 
+hipError_t device_alloc(void **p, size_t bytes)
+{
+    *p = nullptr;
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        release_held();
+        e = hipMalloc(p, bytes);
+        if (e != hipSuccess) (void)hipGetLastError();
+    }
+    if (e != hipSuccess) *p = nullptr;
+    return e;
+}
+
 int exact_bfs(const uint32_t *off, const uint32_t *h_off, const uint32_t *nbr, uint32_t n, bool symmetric,
               uint64_t s_begin,
               uint64_t s_end, uint64_t *reach, uint64_t *total, double *inv_sum, hipStream_t s)
@@ -953,13 +967,13 @@ int exact_bfs(const uint32_t *off, const uint32_t *h_off, const uint32_t *nbr, u
         b.inbr = nbr;
     } else {
         // a stable sort by head (4M arcs: 0.3 ms; counting and placing them with atomics took 2)
-        HBX_TRY(hipMalloc(&rev.p, ((size_t)n + 1 + arcs) * 4));
+        HBX_TRY(device_alloc(&rev.p, ((size_t)n + 1 + arcs) * 4));
         uint32_t *ioff = (uint32_t *)rev.p, *inbr = ioff + n + 1;
         const unsigned bits = std::max(1u, 32u - (unsigned)__builtin_clz(std::max(n - 1, 1u)));
         size_t bytes = 0;
         HBX_TRY(rocprim::radix_sort_pairs(nullptr, bytes, nbr, inbr, inbr, inbr, (size_t)arcs, 0, bits, s));
         const size_t words = (bytes + 255) / 4 / 64 * 64;
-        HBX_TRY(hipMalloc(&tmp.p, (words + 2 * (size_t)arcs) * 4));
+        HBX_TRY(device_alloc(&tmp.p, (words + 2 * (size_t)arcs) * 4));
         uint32_t *tail = (uint32_t *)tmp.p + words, *head = tail + arcs;
         k_bfs_tails<<<(unsigned)std::min<uint64_t>(((uint64_t)n + 3) / 4, 16384), kBfsBlock, 0, s>>>(off, n, tail);
         HBX_TRY(rocprim::radix_sort_pairs(tmp.p, bytes, nbr, head, tail, inbr, (size_t)arcs, 0, bits, s));
@@ -994,7 +1008,7 @@ int exact_bfs(const uint32_t *off, const uint32_t *h_off, const uint32_t *nbr, u
         if (b.hubs) {
             std::vector<uint32_t> h;
             for (const auto *v : {&node, &first, &tnode, &tbeg, &tend}) h.insert(h.end(), v->begin(), v->end());
-            HBX_TRY(hipMalloc(&hub.p, h.size() * 4));
+            HBX_TRY(device_alloc(&hub.p, h.size() * 4));
             HBX_TRY(hipMemcpy(hub.p, h.data(), h.size() * 4, hipMemcpyHostToDevice));
             b.hub_node = (const uint32_t *)hub.p;
             b.hub_first = b.hub_node + b.hubs;
@@ -1011,7 +1025,7 @@ int exact_bfs(const uint32_t *off, const uint32_t *h_off, const uint32_t *nbr, u
         if (inv.p && h_inv.size() > levels) return HB_OK;
         for (size_t d = h_inv.size(); d <= levels; ++d) h_inv.push_back(1.0 / (double)d);
         inv.release();
-        HBX_TRY(hipMalloc(&inv.p, h_inv.size() * 8));
+        HBX_TRY(device_alloc(&inv.p, h_inv.size() * 8));
         HBX_TRY(hipMemcpyAsync(inv.p, h_inv.data(), h_inv.size() * 8, hipMemcpyHostToDevice, s));
         return HB_OK;
     };
@@ -1041,7 +1055,6 @@ int exact_bfs(const uint32_t *off, const uint32_t *h_off, const uint32_t *nbr, u
                     break;
                 }
                 if (e != hipErrorOutOfMemory || (sw == 2 && slices == 1)) HBX_TRY(e);
-                (void)hipGetLastError();
                 if (slices > 1) slices /= 2;
                 else sw /= 2;
             }

@@ -224,7 +224,7 @@ struct Tmp {
     {
         if (p) (void)hipFree(p);
     }
-    hipError_t alloc(size_t bytes) { return hipMalloc(&p, std::max<size_t>(bytes, 1)); }
+    hipError_t alloc(size_t bytes) { return device_alloc(&p, std::max<size_t>(bytes, 1)); }
 };
 
 #define HBI_TRY(call)                    \
@@ -240,8 +240,8 @@ hipError_t build_csr(const uint32_t *ei, const uint32_t *ej, const uint32_t *emi
     Tmp pos, total, keys, keys2, tmp;
     if (count == 0) {  // nothing emitted: n empty lists
         out->emitted = out->arcs = 0;
-        HBI_TRY(hipMalloc(&out->off, ((size_t)n + 1) * 4));
-        HBI_TRY(hipMalloc(&out->nbr, 4));
+        HBI_TRY(device_alloc(&out->off, ((size_t)n + 1) * 4));
+        HBI_TRY(device_alloc(&out->nbr, 4));
         HBI_TRY(hipMemsetAsync(out->off, 0, ((size_t)n + 1) * 4, s));
         return hipStreamSynchronize(s);
     }
@@ -267,8 +267,8 @@ hipError_t build_csr(const uint32_t *ei, const uint32_t *ej, const uint32_t *emi
     if (m >= (1ull << 32)) return hipErrorInvalidValue;  // reported as HB_ERANGE by the caller
     if (m == 0) {
         out->arcs = 0;
-        HBI_TRY(hipMalloc(&out->off, ((size_t)n + 1) * 4));
-        HBI_TRY(hipMalloc(&out->nbr, 4));
+        HBI_TRY(device_alloc(&out->off, ((size_t)n + 1) * 4));
+        HBI_TRY(device_alloc(&out->nbr, 4));
         HBI_TRY(hipMemsetAsync(out->off, 0, ((size_t)n + 1) * 4, s));
         return hipStreamSynchronize(s);
     }
@@ -303,8 +303,8 @@ hipError_t build_csr(const uint32_t *ei, const uint32_t *ej, const uint32_t *emi
         sorted = (const unsigned long long *)keys.p;
     }
     out->arcs = m;
-    HBI_TRY(hipMalloc(&out->off, ((size_t)n + 1) * 4));
-    HBI_TRY(hipMalloc(&out->nbr, std::max<size_t>(m, 1) * 4));
+    HBI_TRY(device_alloc(&out->off, ((size_t)n + 1) * 4));
+    HBI_TRY(device_alloc(&out->nbr, std::max<size_t>(m, 1) * 4));
     if (m == 0) {
         HBI_TRY(hipMemsetAsync(out->off, 0, ((size_t)n + 1) * 4, s));
     } else {

@@ -142,8 +142,20 @@ hipError_t upload_by(void *dst, size_t count, size_t out, hipStream_t s,
                      const std::function<bool(char *, size_t, size_t)> &get, bool *refused);
 // fn(first, last) over [0, count) on several host threads
 void host_parallel(size_t count, const std::function<void(size_t, size_t)> &fn);
-// frees the device memory exact_bfs keeps between calls (not what a call is using)
+// Frees the device memory exact_bfs keeps between calls (not what a call is using).
 void release_held();
+// hipMalloc, for every device buffer of the library: short of memory it gives back what
+// exact_bfs keeps and tries again.  A failure leaves *p null and no error behind for the next
+// check of a launch to report.
+hipError_t device_alloc(void **p, size_t bytes);
+template <class T>
+hipError_t device_alloc(T **p, size_t bytes)
+{
+    void *q = nullptr;
+    const hipError_t e = device_alloc(&q, bytes);
+    *p = (T *)q;
+    return e;
+}
 // exact BFS sums of sources [s_begin, s_end) over a staged CSR (hb_exact.hip), h_off
 // the host copy of its offsets; symmetric: the CSR holds v -> u for every u -> v (levels
 // may then pull)

@@ -105,13 +105,13 @@ hipError_t finish_relabel(const uint32_t *off, const uint32_t *nbr, uint32_t n, 
     size_t scan_bytes = 0;
     HBL_TRY(rocprim::inclusive_scan(nullptr, scan_bytes, degs, roff + 1, (size_t)n, rocprim::plus<uint32_t>(), s));
     Tmp scan_tmp;
-    HBL_TRY(hipMalloc(&scan_tmp.p, std::max<size_t>(scan_bytes, 1)));
+    HBL_TRY(device_alloc(&scan_tmp.p, std::max<size_t>(scan_bytes, 1)));
     HBL_TRY(rocprim::inclusive_scan(scan_tmp.p, scan_bytes, degs, roff + 1, (size_t)n, rocprim::plus<uint32_t>(), s));
     if (arcs == 0) return hipStreamSynchronize(s);
     // lists in new node order, renumbered, then each sorted by new id (carrying the old id)
     Tmp kin, vin;
-    HBL_TRY(hipMalloc(&kin.p, (size_t)arcs * 4));
-    HBL_TRY(hipMalloc(&vin.p, (size_t)arcs * 4));
+    HBL_TRY(device_alloc(&kin.p, (size_t)arcs * 4));
+    HBL_TRY(device_alloc(&vin.p, (size_t)arcs * 4));
     k_fill_lists<<<grid_for((uint64_t)n * 64), kBlock, 0, s>>>(off, nbr, perm, sigma, roff, n, (uint32_t *)kin.p,
                                                                 (uint32_t *)vin.p);
     HBL_TRY(hipGetLastError());
@@ -120,7 +120,7 @@ hipError_t finish_relabel(const uint32_t *off, const uint32_t *nbr, uint32_t n, 
     HBL_TRY(rocprim::segmented_radix_sort_pairs(nullptr, seg_bytes, (uint32_t *)kin.p, rnbr, (uint32_t *)vin.p,
                                                 rorig, arcs, n, roff, roff + 1, 0, bits, s));
     Tmp seg_tmp;
-    HBL_TRY(hipMalloc(&seg_tmp.p, std::max<size_t>(seg_bytes, 1)));
+    HBL_TRY(device_alloc(&seg_tmp.p, std::max<size_t>(seg_bytes, 1)));
     HBL_TRY(rocprim::segmented_radix_sort_pairs(seg_tmp.p, seg_bytes, (uint32_t *)kin.p, rnbr, (uint32_t *)vin.p,
                                                 rorig, arcs, n, roff, roff + 1, 0, bits, s));
     return hipStreamSynchronize(s);  // the temporaries are freed on return
@@ -200,16 +200,16 @@ hipError_t relabel_by_degree(const uint32_t *off, const uint32_t *nbr, uint32_t 
 {
     if (n == 0) return hipMemsetAsync(roff, 0, 4, s);
     Tmp deg, ids, degs, tmp;
-    HBL_TRY(hipMalloc(&deg.p, (size_t)n * 4));
-    HBL_TRY(hipMalloc(&ids.p, (size_t)n * 4));
-    HBL_TRY(hipMalloc(&degs.p, (size_t)n * 4));
+    HBL_TRY(device_alloc(&deg.p, (size_t)n * 4));
+    HBL_TRY(device_alloc(&ids.p, (size_t)n * 4));
+    HBL_TRY(device_alloc(&degs.p, (size_t)n * 4));
     k_deg_ids<<<grid_for(n), kBlock, 0, s>>>(off, n, (uint32_t *)deg.p, (uint32_t *)ids.p);
     HBL_TRY(hipGetLastError());
     // stable: equal degrees keep ascending ids
     size_t bytes = 0;
     HBL_TRY(rocprim::radix_sort_pairs_desc(nullptr, bytes, (uint32_t *)deg.p, (uint32_t *)degs.p,
                                            (uint32_t *)ids.p, perm, n, 0, 32, s));
-    HBL_TRY(hipMalloc(&tmp.p, std::max<size_t>(bytes, 1)));
+    HBL_TRY(device_alloc(&tmp.p, std::max<size_t>(bytes, 1)));
     HBL_TRY(rocprim::radix_sort_pairs_desc(tmp.p, bytes, (uint32_t *)deg.p, (uint32_t *)degs.p, (uint32_t *)ids.p,
                                            perm, n, 0, 32, s));
     return finish_relabel(off, nbr, n, arcs, perm, (const uint32_t *)degs.p, sigma, roff, rnbr, rorig, s);
@@ -222,12 +222,12 @@ hipError_t relabel_by_chain(const uint32_t *off, const uint32_t *nbr, uint32_t n
     *levels = 0;
     if (n == 0) return hipMemsetAsync(roff, 0, 4, s);
     Tmp key, keys, ids, fr0, fr1, counts, degs, tmp;
-    HBL_TRY(hipMalloc(&key.p, (size_t)n * 8));
-    HBL_TRY(hipMalloc(&keys.p, (size_t)n * 8));
-    HBL_TRY(hipMalloc(&ids.p, (size_t)n * 4));
-    HBL_TRY(hipMalloc(&fr0.p, (size_t)n * 4));
-    HBL_TRY(hipMalloc(&fr1.p, (size_t)n * 4));
-    HBL_TRY(hipMalloc(&counts.p, 8));
+    HBL_TRY(device_alloc(&key.p, (size_t)n * 8));
+    HBL_TRY(device_alloc(&keys.p, (size_t)n * 8));
+    HBL_TRY(device_alloc(&ids.p, (size_t)n * 4));
+    HBL_TRY(device_alloc(&fr0.p, (size_t)n * 4));
+    HBL_TRY(device_alloc(&fr1.p, (size_t)n * 4));
+    HBL_TRY(device_alloc(&counts.p, 8));
     uint32_t *cnt = (uint32_t *)counts.p;
     HBL_TRY(hipMemsetAsync(cnt, 0, 8, s));
     k_chain_seed<<<grid_for(n), kBlock, 0, s>>>(off, n, (unsigned long long *)key.p, (uint32_t *)fr0.p, cnt);
@@ -251,10 +251,10 @@ hipError_t relabel_by_chain(const uint32_t *off, const uint32_t *nbr, uint32_t n
     size_t bytes = 0;
     HBL_TRY(rocprim::radix_sort_pairs(nullptr, bytes, (unsigned long long *)key.p, (unsigned long long *)keys.p,
                                       (uint32_t *)ids.p, perm, n, 0, 64, s));
-    HBL_TRY(hipMalloc(&tmp.p, std::max<size_t>(bytes, 1)));
+    HBL_TRY(device_alloc(&tmp.p, std::max<size_t>(bytes, 1)));
     HBL_TRY(rocprim::radix_sort_pairs(tmp.p, bytes, (unsigned long long *)key.p, (unsigned long long *)keys.p,
                                       (uint32_t *)ids.p, perm, n, 0, 64, s));
-    HBL_TRY(hipMalloc(&degs.p, (size_t)n * 4));
+    HBL_TRY(device_alloc(&degs.p, (size_t)n * 4));
     k_perm_deg<<<grid_for(n), kBlock, 0, s>>>(off, perm, n, (uint32_t *)degs.p);
     HBL_TRY(hipGetLastError());
     return finish_relabel(off, nbr, n, arcs, perm, (const uint32_t *)degs.p, sigma, roff, rnbr, rorig, s);

@@ -523,10 +523,10 @@ struct hb_mlp {
         for (void **p : {(void **)&x, (void **)&y, (void **)&out, (void **)&idx})
             if (*p) (void)hipFree(*p), *p = nullptr;
         hipError_t e;
-        if ((e = hipMalloc(&x, n * 6 * 4)) != hipSuccess) return e;
-        if ((e = hipMalloc(&y, n * 4)) != hipSuccess) return e;
-        if ((e = hipMalloc(&out, n * 4)) != hipSuccess) return e;
-        if ((e = hipMalloc(&idx, n * 4)) != hipSuccess) return e;
+        if ((e = hb::device_alloc(&x, n * 6 * 4)) != hipSuccess) return e;
+        if ((e = hb::device_alloc(&y, n * 4)) != hipSuccess) return e;
+        if ((e = hb::device_alloc(&out, n * 4)) != hipSuccess) return e;
+        if ((e = hb::device_alloc(&idx, n * 4)) != hipSuccess) return e;
         cap = n;
         return hipSuccess;
     }
@@ -557,10 +557,10 @@ int hb_mlp_create(hb_mlp **out, int device_ordinal, uint64_t seed)
     auto n = std::make_unique<hb_mlp>();
     n->device = device_ordinal;
     HB_MTRY(hipStreamCreateWithFlags(&n->stream, hipStreamNonBlocking));
-    for (float **p : {&n->w, &n->m, &n->v, &n->g}) HB_MTRY(hipMalloc(p, hb::mlp::kNParams * 4));
-    HB_MTRY(hipMalloc(&n->norm, 12 * 4));
-    HB_MTRY(hipMalloc(&n->loss, 4));
-    HB_MTRY(hipMalloc(&n->stats, 13 * (1 + hb::mlp::kSumBlocks) * sizeof(double)));
+    for (float **p : {&n->w, &n->m, &n->v, &n->g}) HB_MTRY(hb::device_alloc(p, hb::mlp::kNParams * 4));
+    HB_MTRY(hb::device_alloc(&n->norm, 12 * 4));
+    HB_MTRY(hb::device_alloc(&n->loss, 4));
+    HB_MTRY(hb::device_alloc(&n->stats, 13 * (1 + hb::mlp::kSumBlocks) * sizeof(double)));
     // He-uniform weights for the GELU layers, zero biases; identity normalisation
     std::mt19937_64 rng(seed);
     std::vector<float> w(hb::mlp::kNParams, 0.0f);
