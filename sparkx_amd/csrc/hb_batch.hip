@@ -546,8 +546,9 @@ struct DevArr {
     {
         if (ptr) (void)hipFree(ptr);
         ptr = nullptr;
-        count = n;
-        return hb::device_alloc(&ptr, std::max<size_t>(n, 1) * sizeof(T));
+        const hipError_t e = hb::device_alloc(&ptr, std::max<size_t>(n, 1) * sizeof(T));
+        count = e == hipSuccess ? n : 0;
+        return e;
     }
     hipError_t put(const std::vector<T> &h, hipStream_t s)
     {

@@ -522,6 +522,7 @@ struct hb_mlp {
         if (n <= cap) return hipSuccess;
         for (void **p : {(void **)&x, (void **)&y, (void **)&out, (void **)&idx})
             if (*p) (void)hipFree(*p), *p = nullptr;
+        cap = 0;
         hipError_t e;
         if ((e = hb::device_alloc(&x, n * 6 * 4)) != hipSuccess) return e;
         if ((e = hb::device_alloc(&y, n * 4)) != hipSuccess) return e;
