@@ -11,7 +11,7 @@
 //              visited |= newly, frontier = newly, reachable += |newly|, total += d |newly|
 // which discovers exactly the nodes (and distances) of the reference's FIFO queue.
 //
-// Level 1 pushes the sources' own arcs (k_bfs_sources); every later level pulls: a node
+// Level 1 pushes the sources' own arcs (k_bfs_sources).  Later levels pull: a node
 // that some live source has not reached ORs the frontier rows of the nodes with an arc to
 // it (its list on a symmetric CSR; otherwise the reversed CSR, built once per call).  No
 // atomics, and a row of 2,048 searches costs two cache lines where a single 8-byte word takes
@@ -24,7 +24,11 @@
 //     written nor read, and an arc costs its id and that byte;
 //   - a source whose last level found nothing leaves the live mask, so that nodes it cannot
 //     reach do not look for it again;
-//   - a list is left as soon as every wanted bit has appeared.
+//   - a list is left as soon as every wanted bit has appeared;
+//   - with few sources (rows of two words) a level whose frontier has few arcs pushes them
+//     (k_bfs_push): a node in a component without a source wants bits for ever, and a pull scans
+//     its list in every level.  A path of 2,000 nodes beside R-MAT-18, 64 sources on the path: 45 ms,
+//     245 when every level pulled; a grid of 1,000 x 1,000, 1 source: 54 and 67 ms.
 //
 // Per-source sums, bit-identical to the reference's:
 //   reachable : integer count (BFSDists::recheable)
@@ -56,6 +60,13 @@ constexpr uint32_t kBfsHubDeg = 256;   // longer lists are cut into kBfsHubArcs-
 constexpr uint32_t kBfsHubArcs = 1024;
 constexpr uint32_t kBfsPlanes = 4;     // bits of a kept distance
 constexpr uint32_t kBfsKeep = (1u << kBfsPlanes) - 1;  // levels whose distances can be kept
+// A level of rows of two words pushes when the arcs out of its frontier are at most an eighth of
+// all arcs (a sixteenth: 64 sources of R-MAT-20 take 7% longer, paths and grids the same), on graphs
+// of at least kBfsPushArcs: below, a pull scans all arcs in about the time of the push's launch.
+// Wider rows always pull, as that one scan serves all their sources (256 sources on a path
+// beside R-MAT-18: 225 ms; 267 when passes of 64 pushed).
+constexpr uint32_t kBfsPush = 8;
+constexpr uint64_t kBfsPushArcs = 1ull << 20;
 
 typedef unsigned long long u64;
 
@@ -75,6 +86,10 @@ struct BfsDev {
     const uint32_t *task_node, *task_beg, *task_end;
     uint32_t hubs, tasks;
     u64 *part;                    // [tasks][SW]
+    // SW == 2: a level may push
+    u64 push_arcs;                // if its frontier has at most this many arcs out
+    u64 *front;                   // per slice: a bound of them, zero between levels
+    uint32_t *push;               // per slice: the next level pushes
     // distances kept for the harmonic sums (null: not), bit-sliced as the rows are: plane k,
     // at k plane_stride, holds bit k of every distance; valid where visited is set
     u64 *plane;
@@ -90,6 +105,15 @@ struct BfsLevel {
     uint8_t *count;
     uint8_t *any;
 };
+
+// The forms a level's launches hold.  kEither: both, and BfsDev::push says which one works.
+enum class BfsDir { kPull, kEither, kPush };
+
+template <int SW>
+__device__ __forceinline__ bool bfs_pushes(const BfsDev &b, uint32_t slice, BfsDir dir)
+{
+    return SW == 2 && (dir == BfsDir::kPush || (dir == BfsDir::kEither && b.push[slice]));
+}
 
 __device__ __forceinline__ uint32_t bfs_chunks(uint32_t n) { return (n + kBfsChunk - 1) / kBfsChunk; }
 
@@ -112,7 +136,10 @@ __global__ __launch_bounds__(kBfsBlock) void k_bfs_begin(BfsDev b, uint32_t sw)
         const u64 m = __ballot(in);
         if (c % 64 == 0) b.live[(size_t)slice * sw + c / 64] = m;
     }
-    if (threadIdx.x == 0) b.done[slice] = b.levels[slice] = 0;
+    if (threadIdx.x == 0) {
+        b.done[slice] = b.levels[slice] = b.push[slice] = 0;
+        b.front[slice] = 0;
+    }
 }
 
 // Level 1: the frontier is the slice's sources, whose lists lie side by side.  One thread per
@@ -257,9 +284,68 @@ __global__ __launch_bounds__(kBfsBlock) void k_bfs_keep_first(BfsDev b, BfsLevel
     }
 }
 
+// Push form of a level of rows of two words: the row of every node of the frontier, without the
+// sources that have reached the head, ORed into the head's row, whose flag is set; k_bfs_pull
+// then makes the flagged ones newly found nodes.  Rows and flags are zero before
+// (k_bfs_count).  A wavefront takes 64 nodes, the arcs of the flagged ones side by side, a lane
+// each; the lists of hubs come as tasks.
+__global__ __launch_bounds__(kBfsBlock) void k_bfs_push(BfsDev b, BfsLevel prev, BfsLevel next, BfsDir dir)
+{
+    const uint32_t slice = blockIdx.y;
+    if (b.done[slice] || !bfs_pushes<2>(b, slice, dir)) return;
+    const size_t at = (size_t)slice * b.n, fat = (size_t)slice * b.npad;
+    const uint8_t *flag = prev.flag + fat;
+    const ulonglong2 *rows = (const ulonglong2 *)prev.rows + at;
+    const uint32_t lane = threadIdx.x & 63u, waves = gridDim.x * (kBfsBlock / 64);
+    const uint32_t wave = blockIdx.x * (kBfsBlock / 64) + threadIdx.x / 64;
+    auto arc = [&](ulonglong2 r, uint32_t v) {
+        const ulonglong2 seen = ((const ulonglong2 *)b.visited)[at + v];
+        const u64 x = r.x & ~seen.x, y = r.y & ~seen.y;
+        if (x) atomicOr(next.rows + 2 * (at + v), x);
+        if (y) atomicOr(next.rows + 2 * (at + v) + 1, y);
+        if (x | y) next.flag[fat + v] = 1;
+    };
+    for (uint64_t base = (uint64_t)wave * 64; base < b.n; base += (uint64_t)waves * 64) {
+        const uint64_t u = base + lane;
+        uint32_t e0 = 0, len = 0;
+        if (u < b.n && flag[u]) {
+            e0 = b.off[u];
+            len = b.off[u + 1] - e0;
+            if (len > kBfsHubDeg) len = 0;
+        }
+        if (!__ballot(len != 0)) continue;
+        uint32_t end = len;  // of the lane's arcs among the wavefront's
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t below = __shfl_up(end, o);
+            if (lane >= (uint32_t)o) end += below;
+        }
+        const uint32_t all = __shfl(end, 63);
+        for (uint32_t i0 = 0; i0 < all; i0 += 64) {  // arc i0 + lane: of the first lane that ends past it
+            const uint32_t i = i0 + lane;
+            uint32_t j = 0;
+#pragma unroll
+            for (uint32_t step = 32; step; step >>= 1)
+                if ((uint32_t)__shfl((int)end, (int)(j + step - 1)) <= i) j += step;
+            j = min(j, 63u);
+            const uint32_t first = __shfl(e0, (int)j) - (__shfl(end, (int)j) - __shfl(len, (int)j));
+            if (i < all) arc(rows[base + j], b.nbr[(uint32_t)(first + i)]);
+        }
+    }
+    for (uint32_t k = wave; k < b.tasks; k += waves) {
+        const uint32_t u = b.task_node[k];
+        if (!flag[u]) continue;
+        const ulonglong2 r = rows[u];
+        const uint32_t e0 = b.task_beg[k], len = b.task_end[k] - e0;
+        for (uint32_t i = lane; i < len; i += 64) arc(r, b.nbr[(size_t)e0 + i]);
+    }
+}
+
 // One level for the nodes with at most kBfsHubDeg tails: a team of SW / 2 lanes per node.
+// After a push, what it left at every node.
 template <int SW>
-__global__ __launch_bounds__(kBfsBlock) void k_bfs_pull(BfsDev b, BfsLevel prev, BfsLevel next, uint32_t level)
+__global__ __launch_bounds__(kBfsBlock) void k_bfs_pull(BfsDev b, BfsLevel prev, BfsLevel next, uint32_t level,
+                                                        BfsDir dir)
 {
     constexpr uint32_t L = SW / 2;
     const uint32_t slice = blockIdx.y;
@@ -270,6 +356,14 @@ __global__ __launch_bounds__(kBfsBlock) void k_bfs_pull(BfsDev b, BfsLevel prev,
     const ulonglong2 *rows = (const ulonglong2 *)prev.rows + at * L;
     const ulonglong2 live = ((const ulonglong2 *)b.live)[(size_t)slice * L + t.tl];
     const uint32_t teams = gridDim.x * (kBfsBlock / L);
+    if constexpr (SW == 2)
+        if (bfs_pushes<SW>(b, slice, dir)) {
+            for (uint32_t v = blockIdx.x * kBfsBlock + threadIdx.x; v < b.n; v += teams)
+                if (next.flag[fat + v])
+                    bfs_found<SW>(b, t, at + v, next.rows, next.flag + fat + v, ((const ulonglong2 *)b.visited)[at + v],
+                                  ((const ulonglong2 *)next.rows)[at + v], level);
+            return;
+        }
     for (uint32_t v = blockIdx.x * (kBfsBlock / L) + threadIdx.x / L; v < b.n; v += teams) {
         const uint32_t e0 = b.ioff[v], e1 = b.ioff[v + 1];
         if (e1 - e0 > kBfsHubDeg) continue;  // k_bfs_hub_tasks and k_bfs_hubs
@@ -287,11 +381,11 @@ __global__ __launch_bounds__(kBfsBlock) void k_bfs_pull(BfsDev b, BfsLevel prev,
 // The lists of hubs, cut into tasks: one wavefront per task, its teams every 64 / L-th run
 // of ids, their words ORed into the task's row of `part`.
 template <int SW>
-__global__ __launch_bounds__(kBfsBlock) void k_bfs_hub_tasks(BfsDev b, BfsLevel prev)
+__global__ __launch_bounds__(kBfsBlock) void k_bfs_hub_tasks(BfsDev b, BfsLevel prev, BfsDir dir)
 {
     constexpr uint32_t L = SW / 2, TEAMS = 64 / L;
     const uint32_t slice = blockIdx.y;
-    if (b.done[slice]) return;
+    if (b.done[slice] || bfs_pushes<SW>(b, slice, dir)) return;
     const BfsTeam<SW> t;
     const size_t at = (size_t)slice * b.n, fat = (size_t)slice * b.npad;
     const ulonglong2 live = ((const ulonglong2 *)b.live)[(size_t)slice * L + t.tl];
@@ -314,11 +408,11 @@ __global__ __launch_bounds__(kBfsBlock) void k_bfs_hub_tasks(BfsDev b, BfsLevel 
 }
 
 template <int SW>
-__global__ __launch_bounds__(kBfsBlock) void k_bfs_hubs(BfsDev b, BfsLevel next, uint32_t level)
+__global__ __launch_bounds__(kBfsBlock) void k_bfs_hubs(BfsDev b, BfsLevel next, uint32_t level, BfsDir dir)
 {
     constexpr uint32_t L = SW / 2;
     const uint32_t slice = blockIdx.y;
-    if (b.done[slice]) return;
+    if (b.done[slice] || bfs_pushes<SW>(b, slice, dir)) return;
     const BfsTeam<SW> t;
     const size_t at = (size_t)slice * b.n, fat = (size_t)slice * b.npad;
     const ulonglong2 live = ((const ulonglong2 *)b.live)[(size_t)slice * L + t.tl];
@@ -353,23 +447,36 @@ __device__ __forceinline__ void bfs_csa(u64 &hi, u64 &lo, u64 a, u64 b2, u64 c)
 // word of a chunk's rows, eight rows at a time, into bit-sliced counters (plane k holds bit
 // k of 64 counts), then transposes the planes into 64 bytes: 13 operations per 64 bits
 // added, where a ballot per column takes 256 per wavefront.
+// Where the next level may push, the frontier before, which no kernel reads any more, is
+// cleared here, so that the level finds its rows and flags zero.
 template <int SW>
-__global__ __launch_bounds__(kBfsBlock) void k_bfs_count(BfsDev b, BfsLevel l)
+__global__ __launch_bounds__(kBfsBlock) void k_bfs_count(BfsDev b, BfsLevel l, BfsLevel prev, bool clear)
 {
     const uint32_t slice = blockIdx.y, chunks = bfs_chunks(b.n);
     if (b.done[slice]) return;
     const uint32_t w = threadIdx.x % SW;
     const size_t at = (size_t)slice * b.n;
     const uint32_t per_grid = gridDim.x * (kBfsBlock / SW);
+    if (SW == 2 && clear) {
+        ulonglong2 *pf = (ulonglong2 *)(prev.flag + (size_t)slice * b.npad);
+        for (uint32_t i = blockIdx.x * kBfsBlock + threadIdx.x; i < b.npad / 16; i += gridDim.x * kBfsBlock) {
+            const ulonglong2 f = pf[i];
+            if (!(f.x | f.y)) continue;
+            pf[i] = make_ulonglong2(0, 0);
+            for (uint32_t k = 0; k < 16; ++k)
+                if (((k < 8 ? f.x : f.y) >> (8 * (k % 8))) & 1u)
+                    ((ulonglong2 *)prev.rows)[at + 16 * (size_t)i + k] = make_ulonglong2(0, 0);
+        }
+    }
     for (uint32_t c = blockIdx.x * (kBfsBlock / SW) + threadIdx.x / SW; c < chunks; c += per_grid) {
         u64 p[8] = {};
-        const uint32_t v1 = min(b.n, (c + 1) * kBfsChunk);
+        const uint32_t v0 = c * kBfsChunk, v1 = min(b.n, v0 + kBfsChunk);
         bool any = false;
-        for (uint32_t v = c * kBfsChunk; v < v1; v += 8) {
+        auto add = [&](uint32_t v) {
             // eight flags of 0 or 1 as the low byte's bits, those past the last node dropped
             const u64 f8 = *(const u64 *)(l.flag + (size_t)slice * b.npad + v) & 0x0101010101010101ull;
             const uint32_t f = (uint32_t)((f8 * 0x0102040810204080ull) >> 56) & (0xffu >> (8 - min(8u, v1 - v)));
-            if (!f) continue;
+            if (!f) return;
             any = true;
             u64 x[8];
 #pragma unroll
@@ -388,6 +495,21 @@ __global__ __launch_bounds__(kBfsBlock) void k_bfs_count(BfsDev b, BfsLevel l)
                 p[k] ^= eight;
                 eight = carry;
             }
+        };
+        if constexpr (SW == 2) {  // few threads: one round of loads finds the eights to add
+            const ulonglong2 *q = (const ulonglong2 *)(l.flag + (size_t)slice * b.npad + v0);
+            uint32_t eights = 0;
+#pragma unroll
+            for (uint32_t i = 0; i < kBfsChunk / 16; ++i) {
+                const ulonglong2 f = q[i];
+                eights |= (f.x ? 1u << (2 * i) : 0u) | (f.y ? 2u << (2 * i) : 0u);
+            }
+            for (; eights; eights &= eights - 1) {
+                const uint32_t v = v0 + 8 * (uint32_t)(__ffs((int)eights) - 1);
+                if (v < v1) add(v);
+            }
+        } else {
+            for (uint32_t v = v0; v < v1; v += 8) add(v);
         }
         const size_t ci = (size_t)slice * chunks + c;
         if (w == 0) l.any[ci] = any ? 1 : 0;
@@ -434,7 +556,45 @@ __global__ __launch_bounds__(kBfsBlock) void k_bfs_totals(BfsDev b, BfsLevel l, 
     }
 }
 
-// end of a level, one block per slice: the per-source sums, the sources still searching
+// The same for rows of two words, whose 32 quads leave k_bfs_totals few threads (18 us a level of
+// a graph of a million nodes): eight parts of the chunks to a block, summed there before the
+// atomics.  Also the arcs out of the chunks that hold a newly found node, a bound of the next
+// frontier's.
+__global__ __launch_bounds__(kBfsBlock) void k_bfs_totals_narrow(BfsDev b, BfsLevel l)
+{
+    constexpr uint32_t QUADS = 32, PARTS = kBfsBlock / QUADS;
+    const uint32_t slice = blockIdx.y, chunks = bfs_chunks(b.n);
+    if (b.done[slice]) return;
+    __shared__ uint32_t red[PARTS][4 * QUADS];
+    __shared__ u64 red_arcs[PARTS];
+    const uint32_t quad = threadIdx.x % QUADS, part = threadIdx.x / QUADS, parts = gridDim.x * PARTS;
+    uint32_t s[4] = {};
+    u64 arcs = 0;
+    for (uint32_t c = blockIdx.x * PARTS + part; c < chunks; c += parts) {
+        const size_t ci = (size_t)slice * chunks + c;
+        if (!l.any[ci]) continue;
+        const uint32_t x = ((const uint32_t *)l.count)[ci * QUADS + quad];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) s[k] += (x >> (8 * k)) & 0xffu;
+        if (quad == 0) arcs += b.off[min(b.n, (c + 1) * kBfsChunk)] - b.off[c * kBfsChunk];
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) red[part][4 * quad + k] = s[k];
+    if (quad == 0) red_arcs[part] = arcs;
+    __syncthreads();
+    if (threadIdx.x < 4 * QUADS) {
+        uint32_t t = 0;
+        for (uint32_t p = 0; p < PARTS; ++p) t += red[p][threadIdx.x];
+        if (t) atomicAdd(b.found + (size_t)slice * 4 * QUADS + threadIdx.x, t);
+    } else if (threadIdx.x == 4 * QUADS) {
+        u64 t = 0;
+        for (uint32_t p = 0; p < PARTS; ++p) t += red_arcs[p];
+        if (t) atomicAdd(b.front + slice, t);
+    }
+}
+
+// end of a level, one block per slice: the per-source sums, the sources still searching, the
+// form of the next level
 template <int SW>
 __global__ __launch_bounds__(1024) void k_bfs_level(BfsDev b, uint32_t level)
 {
@@ -459,7 +619,30 @@ __global__ __launch_bounds__(1024) void k_bfs_level(BfsDev b, uint32_t level)
     if (threadIdx.x == 0) {
         if (any) b.levels[slice] = level;
         else b.done[slice] = 1;
+        if (SW == 2) {
+            b.push[slice] = b.front[slice] <= b.push_arcs;
+            b.front[slice] = 0;
+        }
     }
+}
+
+// level into the distances of the found sources among the 8 of piece q of node v's row
+template <int SW>
+__device__ __forceinline__ void bfs_distance(const BfsDev &b, const BfsLevel &l, uint32_t slice, size_t v, uint32_t q,
+                                             uint32_t level, uint16_t *dist)
+{
+    const uint32_t w = q / 8;
+    const uint32_t bits = (uint32_t)(l.rows[((size_t)slice * b.n + v) * SW + w] >> (8 * (q % 8))) & 0xffu;
+    if (!bits) return;
+    uint4 *row = (uint4 *)(dist + (((size_t)slice * SW + w) * b.n + v) * 64) + q % 8;
+    const uint4 x = *row;
+    uint32_t r[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+    for (int h = 0; h < 8; ++h) {
+        const uint32_t sh = 16u * (uint32_t)(h & 1);
+        if ((bits >> h) & 1u) r[h >> 1] = (r[h >> 1] & ~(0xffffu << sh)) | (level << sh);
+    }
+    *row = make_uint4(r[0], r[1], r[2], r[3]);
 }
 
 // distances of the nodes found in the level, u16 [word][n][64]: a thread per 8 sources
@@ -468,22 +651,27 @@ __global__ __launch_bounds__(kBfsBlock) void k_bfs_dist(BfsDev b, BfsLevel l, ui
 {
     const uint32_t slice = blockIdx.y;
     if (b.done[slice]) return;
-    const size_t at = (size_t)slice * b.n;
     const uint64_t threads = (uint64_t)gridDim.x * kBfsBlock, all = (uint64_t)b.n * SW * 8;
     for (uint64_t i = (uint64_t)blockIdx.x * kBfsBlock + threadIdx.x; i < all; i += threads) {
-        const uint32_t v = (uint32_t)(i / (SW * 8)), q = (uint32_t)(i % (SW * 8)), w = q / 8;
-        if (!l.flag[(size_t)slice * b.npad + v]) continue;
-        const uint32_t bits = (uint32_t)(l.rows[(at + v) * SW + w] >> (8 * (q % 8))) & 0xffu;
-        if (!bits) continue;
-        uint4 *row = (uint4 *)(dist + (((size_t)slice * SW + w) * b.n + v) * 64) + q % 8;
-        const uint4 x = *row;
-        uint32_t r[4] = {x.x, x.y, x.z, x.w};
-#pragma unroll
-        for (int h = 0; h < 8; ++h) {
-            const uint32_t sh = 16u * (uint32_t)(h & 1);
-            if ((bits >> h) & 1u) r[h >> 1] = (r[h >> 1] & ~(0xffffu << sh)) | (level << sh);
-        }
-        *row = make_uint4(r[0], r[1], r[2], r[3]);
+        const uint32_t v = (uint32_t)(i / (SW * 8));
+        if (l.flag[(size_t)slice * b.npad + v]) bfs_distance<SW>(b, l, slice, v, (uint32_t)(i % (SW * 8)), level, dist);
+    }
+}
+
+// The same for rows of two words of a large graph, few of whose nodes are found in a level: a
+// wavefront looks at 16 nodes at a time (11 us a level of a million nodes, 25 with a thread per 8
+// sources; on a few thousand nodes 7 and 2)
+__global__ __launch_bounds__(kBfsBlock) void k_bfs_dist_narrow(BfsDev b, BfsLevel l, uint32_t level, uint16_t *dist)
+{
+    constexpr uint32_t N = 16;
+    const uint32_t slice = blockIdx.y;
+    if (b.done[slice]) return;
+    const uint32_t lane = threadIdx.x & 63u, step = gridDim.x * (kBfsBlock / 64) * N;
+    for (uint64_t v0 = (blockIdx.x * (kBfsBlock / 64) + threadIdx.x / 64) * N; v0 < b.n; v0 += step) {
+        const u64 found = __ballot(lane < N && v0 + lane < b.n && l.flag[(size_t)slice * b.npad + v0 + lane]);
+        if (!found) continue;
+        for (uint32_t i = lane; i < N * 16; i += 64)
+            if ((found >> (i / 16)) & 1u) bfs_distance<2>(b, l, slice, v0 + i / 16, i % 16, level, dist);
     }
 }
 
@@ -842,8 +1030,9 @@ BfsPlan bfs_plan(uint32_t n, uint32_t tasks, uint32_t sw, uint32_t slices, BfsMo
     p.o_any = take(p.any_stride * p.counts);
     p.o_part = take((size_t)slices * tasks * sw * 8);
     p.o_dist = take(mode == BfsMode::kLong ? p.rows_stride * 128 : 0);
-    // per source: reach, total, sum, found; per word: live, source count; per slice: done, levels
-    p.o_src = take((size_t)slices * (sw * (64 * 28 + 12) + 8));
+    // per source: reach, total, sum, found; per word: live, source count; per slice: front, done,
+    // levels, push
+    p.o_src = take((size_t)slices * (sw * (64 * 28 + 12) + 20));
     return p;
 }
 
@@ -876,10 +1065,12 @@ struct BfsGroup {
         b.total = b.reach + src;
         sums = (double *)(b.total + src);
         b.live = (u64 *)(sums + src);
-        b.found = (uint32_t *)(b.live + words);
+        b.front = b.live + words;
+        b.found = (uint32_t *)(b.front + p.slices);
         word_count = b.found + src;
         b.done = word_count + words;
         b.levels = b.done + p.slices;
+        b.push = b.levels + p.slices;
     }
 };
 
@@ -891,7 +1082,8 @@ unsigned bfs_grid(uint64_t threads, uint32_t slices)
 
 // levels from .. to of every slice; returns at once where a slice is done
 template <int SW>
-hipError_t bfs_levels(const BfsGroup &g, uint32_t from, uint32_t to, uint64_t source_arcs, BfsMode mode, hipStream_t s)
+hipError_t bfs_levels(const BfsGroup &g, uint32_t from, uint32_t to, uint64_t source_arcs, BfsMode mode, BfsDir dir,
+                      hipStream_t s)
 {
     const BfsDev &b = g.b;
     const uint32_t slices = g.plan.slices, chunks = (b.n + kBfsChunk - 1) / kBfsChunk;
@@ -904,21 +1096,66 @@ hipError_t bfs_levels(const BfsGroup &g, uint32_t from, uint32_t to, uint64_t so
                 k_bfs_keep_first<SW><<<dim3(bfs_grid((uint64_t)b.n * (SW / 2), slices), slices), kBfsBlock, 0, s>>>(b, next);
         } else {
             const BfsLevel prev = g.level(l - 1);
-            k_bfs_pull<SW><<<dim3(bfs_grid((uint64_t)b.n * (SW / 2), slices), slices), kBfsBlock, 0, s>>>(b, prev, next, l);
-            if (b.tasks) {
-                k_bfs_hub_tasks<SW><<<dim3(bfs_grid((uint64_t)b.tasks * 64, slices), slices), kBfsBlock, 0, s>>>(b, prev);
-                k_bfs_hubs<SW><<<dim3(bfs_grid((uint64_t)b.hubs * (SW / 2), slices), slices), kBfsBlock, 0, s>>>(b, next, l);
+            if (SW == 2 && dir != BfsDir::kPull)
+                k_bfs_push<<<dim3(std::min(bfs_grid(b.n, slices), 1024u), slices), kBfsBlock, 0, s>>>(b, prev, next, dir);
+            k_bfs_pull<SW><<<dim3(bfs_grid((uint64_t)b.n * (SW / 2), slices), slices), kBfsBlock, 0, s>>>(b, prev, next, l,
+                                                                                                      dir);
+            if (b.tasks && dir != BfsDir::kPush) {
+                k_bfs_hub_tasks<SW><<<dim3(bfs_grid((uint64_t)b.tasks * 64, slices), slices), kBfsBlock, 0, s>>>(b, prev,
+                                                                                                              dir);
+                k_bfs_hubs<SW><<<dim3(bfs_grid((uint64_t)b.hubs * (SW / 2), slices), slices), kBfsBlock, 0, s>>>(b, next, l,
+                                                                                                             dir);
             }
         }
-        k_bfs_count<SW><<<dim3(bfs_grid((uint64_t)chunks * SW, slices), slices), kBfsBlock, 0, s>>>(b, next);
-        k_bfs_totals<SW><<<dim3(bfs_grid((uint64_t)splits * 16 * SW, slices), slices), kBfsBlock, 0, s>>>(b, next, splits);
+        k_bfs_count<SW><<<dim3(bfs_grid((uint64_t)chunks * SW, slices), slices), kBfsBlock, 0, s>>>(
+            b, next, g.level(l > 1 ? l - 1 : 2), dir != BfsDir::kPull && l > 1);
+        if (SW == 2)
+            k_bfs_totals_narrow<<<dim3(std::min((chunks + 7) / 8, std::max(1u, 128u / slices)), slices), kBfsBlock, 0, s>>>(
+                b, next);
+        else
+            k_bfs_totals<SW><<<dim3(bfs_grid((uint64_t)splits * 16 * SW, slices), slices), kBfsBlock, 0, s>>>(b, next,
+                                                                                                          splits);
         k_bfs_level<SW><<<slices, std::min(1024, 64 * SW), 0, s>>>(b, l);
         // a level that found nothing has marked its slice done and records nothing
-        if (mode == BfsMode::kLong)
-            k_bfs_dist<SW><<<dim3(bfs_grid((uint64_t)b.n * SW * 8, slices), slices), kBfsBlock, 0, s>>>(b, next, l, g.dist);
+        if (mode == BfsMode::kLong) {
+            if (SW == 2 && b.n >= 1u << 17)
+                k_bfs_dist_narrow<<<dim3(bfs_grid((uint64_t)b.n * 4, slices), slices), kBfsBlock, 0, s>>>(b, next, l, g.dist);
+            else
+                k_bfs_dist<SW><<<dim3(bfs_grid((uint64_t)b.n * SW * 8, slices), slices), kBfsBlock, 0, s>>>(b, next, l, g.dist);
+        }
     }
     return hipGetLastError();
 }
+
+// nodes with long lists and the tasks those are cut into (hub h: tasks first[h] ..)
+struct BfsHubs {
+    std::vector<uint32_t> node, first, tnode, tbeg, tend;
+
+    BfsHubs(const uint32_t *off, uint32_t n)
+    {
+        for (uint64_t v0 = 0; v0 < n; v0 += 16) {  // most runs of 16 hold none (one vector loop)
+            const uint32_t v1 = (uint32_t)std::min<uint64_t>(n, v0 + 16);
+            uint32_t any = 0;
+            for (uint32_t v = (uint32_t)v0; v < v1; ++v) any |= off[v + 1] - off[v] > kBfsHubDeg;
+            if (!any) continue;
+            for (uint32_t v = (uint32_t)v0; v < v1; ++v)
+                if (off[v + 1] - off[v] > kBfsHubDeg) cut(v, off[v], off[v + 1]);
+        }
+        first.push_back((uint32_t)tnode.size());
+    }
+
+private:
+    void cut(uint32_t v, uint64_t beg, uint64_t end)
+    {
+        node.push_back(v);
+        first.push_back((uint32_t)tnode.size());
+        for (uint64_t e = beg; e < end; e += kBfsHubArcs) {
+            tnode.push_back(v);
+            tbeg.push_back((uint32_t)e);
+            tend.push_back((uint32_t)std::min<uint64_t>(e + kBfsHubArcs, end));
+        }
+    }
+};
 
 }  // namespace
 
@@ -990,26 +1227,14 @@ int exact_bfs(const uint32_t *off, const uint32_t *h_off, const uint32_t *nbr, u
     // hubs and their tasks
     Scoped hub;
     {
-        const uint32_t *ho = h_ioff.empty() ? h_off : h_ioff.data();
-        std::vector<uint32_t> node, first, tnode, tbeg, tend;
-        for (uint32_t v = 0; v < n; ++v) {
-            if (ho[v + 1] - ho[v] <= kBfsHubDeg) continue;
-            node.push_back(v);
-            first.push_back((uint32_t)tnode.size());
-            for (uint64_t e = ho[v]; e < ho[v + 1]; e += kBfsHubArcs) {
-                tnode.push_back(v);
-                tbeg.push_back((uint32_t)e);
-                tend.push_back((uint32_t)std::min<uint64_t>(e + kBfsHubArcs, ho[v + 1]));
-            }
-        }
-        b.hubs = (uint32_t)node.size();
-        b.tasks = (uint32_t)tnode.size();
-        first.push_back(b.tasks);
+        const BfsHubs h(h_ioff.empty() ? h_off : h_ioff.data(), n);
+        b.hubs = (uint32_t)h.node.size();
+        b.tasks = (uint32_t)h.tnode.size();
         if (b.hubs) {
-            std::vector<uint32_t> h;
-            for (const auto *v : {&node, &first, &tnode, &tbeg, &tend}) h.insert(h.end(), v->begin(), v->end());
-            HBX_TRY(device_alloc(&hub.p, h.size() * 4));
-            HBX_TRY(hipMemcpy(hub.p, h.data(), h.size() * 4, hipMemcpyHostToDevice));
+            std::vector<uint32_t> all;
+            for (const auto *v : {&h.node, &h.first, &h.tnode, &h.tbeg, &h.tend}) all.insert(all.end(), v->begin(), v->end());
+            HBX_TRY(device_alloc(&hub.p, all.size() * 4));
+            HBX_TRY(hipMemcpy(hub.p, all.data(), all.size() * 4, hipMemcpyHostToDevice));
             b.hub_node = (const uint32_t *)hub.p;
             b.hub_first = b.hub_node + b.hubs;
             b.task_node = b.hub_first + b.hubs + 1;
@@ -1017,6 +1242,9 @@ int exact_bfs(const uint32_t *off, const uint32_t *h_off, const uint32_t *nbr, u
             b.task_end = b.task_beg + b.tasks;
         }
     }
+    // the tasks are those of the lists that a push reads too
+    const bool may_push = symmetric && arcs >= kBfsPushArcs;
+    b.push_arcs = arcs / kBfsPush;
     BfsMode mode = inv_sum ? BfsMode::kKeep : BfsMode::kSums;
     Scoped inv;
     BfsMemory mem(s);
@@ -1077,32 +1305,45 @@ int exact_bfs(const uint32_t *off, const uint32_t *h_off, const uint32_t *nbr, u
         k_bfs_zero<uint4><<<zgrid, kBfsBlock, 0, s>>>((uint4 *)r.b.visited, row_words / 2);
         k_bfs_zero<uint4><<<zgrid, kBfsBlock, 0, s>>>((uint4 *)r.level(1).rows, row_words / 2);
         k_bfs_zero<uint4><<<zgrid, kBfsBlock, 0, s>>>((uint4 *)r.level(1).flag, (uint64_t)slices * r.b.npad / 16);
+        if (may_push && r.plan.sw == 2) {  // level 2 too finds them zero
+            k_bfs_zero<uint4><<<zgrid, kBfsBlock, 0, s>>>((uint4 *)r.level(2).rows, row_words / 2);
+            k_bfs_zero<uint4><<<zgrid, kBfsBlock, 0, s>>>((uint4 *)r.level(2).flag, (uint64_t)slices * r.b.npad / 16);
+        }
         if (mode == BfsMode::kLong) k_bfs_zero<uint4><<<zgrid, kBfsBlock, 0, s>>>((uint4 *)r.dist, row_words * 8);
         k_bfs_begin<<<slices, kBfsBlock, 0, s>>>(r.b, r.plan.sw);
         // launches past a slice's last level return at once, so the host looks every 4, 8, ..
         // levels only
-        std::vector<uint32_t> state(2 * (size_t)g.plan.slices);
+        std::vector<uint32_t> state(3 * (size_t)g.plan.slices);
         uint32_t at = 0;  // levels launched
-        bool all = false;
+        bool all = false, each = false;
         while (!all) {
             uint32_t to = at + (at < 8 ? 4 : std::min(64u, at / 2));
             if (mode == BfsMode::kKeep) to = std::min(to, kBfsKeep);
             if (mode == BfsMode::kLong) to = std::min(to, 65535u);
             if (to == at) break;
+            // Past the eighth level, where a frontier seldom grows at a stroke, the levels up to the
+            // next look push without being asked if all slices were to push at this one
+            BfsDir dir = BfsDir::kPull;
+            if (may_push && r.plan.sw == 2) dir = at >= 8 && each ? BfsDir::kPush : BfsDir::kEither;
+            if (dir == BfsDir::kPush) to = std::min(to, at + 16);
             hipError_t e = hipErrorInvalidValue;
             switch (r.plan.sw) {
-            case 2: e = bfs_levels<2>(r, at + 1, to, source_arcs, mode, s); break;
-            case 4: e = bfs_levels<4>(r, at + 1, to, source_arcs, mode, s); break;
-            case 8: e = bfs_levels<8>(r, at + 1, to, source_arcs, mode, s); break;
-            case 16: e = bfs_levels<16>(r, at + 1, to, source_arcs, mode, s); break;
-            case 32: e = bfs_levels<32>(r, at + 1, to, source_arcs, mode, s); break;
+            case 2: e = bfs_levels<2>(r, at + 1, to, source_arcs, mode, dir, s); break;
+            case 4: e = bfs_levels<4>(r, at + 1, to, source_arcs, mode, dir, s); break;
+            case 8: e = bfs_levels<8>(r, at + 1, to, source_arcs, mode, dir, s); break;
+            case 16: e = bfs_levels<16>(r, at + 1, to, source_arcs, mode, dir, s); break;
+            case 32: e = bfs_levels<32>(r, at + 1, to, source_arcs, mode, dir, s); break;
             }
             HBX_TRY(e);
             HBX_TRY(hipMemcpyAsync(state.data(), r.b.done, state.size() * 4, hipMemcpyDeviceToHost, s));
             HBX_TRY(hipStreamSynchronize(s));
             at = to;
             all = true;
-            for (uint32_t i = 0; i < slices; ++i) all = all && state[i];
+            each = true;
+            for (uint32_t i = 0; i < slices; ++i) {
+                all = all && state[i];
+                each = each && (state[i] || state[2 * (size_t)g.plan.slices + i]);
+            }
         }
         if (!all && mode == BfsMode::kKeep) {  // long searches: this group again, and the rest, by distances
             mode = BfsMode::kLong;
