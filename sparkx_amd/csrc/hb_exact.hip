@@ -46,6 +46,7 @@
 #include <algorithm>
 #include <cstdarg>
 #include <cstdio>
+#include <cstdlib>
 #include <mutex>
 #include <vector>
 
@@ -67,6 +68,11 @@ constexpr uint32_t kBfsKeep = (1u << kBfsPlanes) - 1;  // levels whose distances
 // beside R-MAT-18: 225 ms; 267 when passes of 64 pushed).
 constexpr uint32_t kBfsPush = 8;
 constexpr uint64_t kBfsPushArcs = 1ull << 20;
+// Directed graphs: up to this many sources (one row of two words) every level pushes and the arcs
+// are not reversed, which would take memory for 5 words an arc and, on R-MAT-20 with 8.4M arcs, most
+// of a call (1 / 64 / 128 sources: 0.97 / 1.45 / 1.86 ms, 2.66 / 2.78 / 2.76 when they were).  From
+// 129 on the wider rows' pulls pay for it: 129 and 256 sources 2.9 ms, 2.8 and 4.9 in passes of 64.
+constexpr uint32_t kBfsFew = 128;
 
 typedef unsigned long long u64;
 
@@ -936,6 +942,14 @@ constexpr uint64_t kBfsBudget = 16ull << 30;  // device memory of one group of s
 constexpr uint64_t kBfsHold = 2ull << 30;
 constexpr int kBfsDevices = 16;
 
+// SPARKX_HB_BFS_BYTES in the environment: a group of slices, and the reversed arcs, may take no
+// more device memory than this (tests run several groups and the ways out of too little memory)
+uint64_t bfs_limit()
+{
+    const char *e = getenv("SPARKX_HB_BFS_BYTES");
+    return e ? strtoull(e, nullptr, 10) : UINT64_MAX;
+}
+
 struct BfsHeld {
     std::mutex mu;
     void *p[kBfsDevices] = {};
@@ -952,6 +966,7 @@ struct BfsMemory {
     ~BfsMemory() { release(); }
     hipError_t take(size_t want)
     {
+        if (want > bfs_limit()) return hipErrorOutOfMemory;
         if (device < 0) {
             const hipError_t e = hipGetDevice(&device);
             if (e != hipSuccess) return e;
@@ -1127,6 +1142,45 @@ hipError_t bfs_levels(const BfsGroup &g, uint32_t from, uint32_t to, uint64_t so
     return hipGetLastError();
 }
 
+// The reversed CSR of directed arcs, offsets then tails, into `rev`, its offsets also to the host.
+// A stable sort by head (4M arcs: 0.3 ms; counting and placing them with atomics took 2); short of
+// memory nothing is kept.
+hipError_t bfs_reverse(const uint32_t *off, const uint32_t *nbr, uint32_t n, uint32_t arcs, Scoped &rev,
+                       std::vector<uint32_t> &h_ioff, hipStream_t s)
+{
+#define HB_REV_TRY(call)                   \
+    do {                                   \
+        const hipError_t e_ = (call);      \
+        if (e_ != hipSuccess) {            \
+            (void)hipStreamSynchronize(s); \
+            rev.release();                 \
+            return e_;                     \
+        }                                  \
+    } while (0)
+    Scoped tmp;
+    const unsigned bits = std::max(1u, 32u - (unsigned)__builtin_clz(std::max(n - 1, 1u)));
+    size_t bytes = 0;
+    HB_REV_TRY(rocprim::radix_sort_pairs(nullptr, bytes, nbr, (uint32_t *)nullptr, (uint32_t *)nullptr,
+                                         (uint32_t *)nullptr, (size_t)arcs, 0, bits, s));
+    const size_t words = (bytes + 255) / 4 / 64 * 64;
+    const size_t rev_bytes = ((size_t)n + 1 + arcs) * 4, tmp_bytes = (words + 2 * (size_t)arcs) * 4;
+    if (rev_bytes + tmp_bytes > bfs_limit()) return hipErrorOutOfMemory;
+    HB_REV_TRY(device_alloc(&rev.p, rev_bytes));
+    HB_REV_TRY(device_alloc(&tmp.p, tmp_bytes));
+    uint32_t *ioff = (uint32_t *)rev.p, *inbr = ioff + n + 1;
+    uint32_t *tail = (uint32_t *)tmp.p + words, *head = tail + arcs;
+    k_bfs_tails<<<(unsigned)std::min<uint64_t>(((uint64_t)n + 3) / 4, 16384), kBfsBlock, 0, s>>>(off, n, tail);
+    HB_REV_TRY(rocprim::radix_sort_pairs(tmp.p, bytes, nbr, head, tail, inbr, (size_t)arcs, 0, bits, s));
+    k_bfs_offsets<<<(unsigned)std::min<uint64_t>(((uint64_t)arcs + kBfsBlock - 1) / kBfsBlock, 16384), kBfsBlock, 0,
+                    s>>>(head, arcs, n, ioff);
+    HB_REV_TRY(hipGetLastError());
+    h_ioff.resize((size_t)n + 1);
+    HB_REV_TRY(hipMemcpyAsync(h_ioff.data(), ioff, ((size_t)n + 1) * 4, hipMemcpyDeviceToHost, s));
+    HB_REV_TRY(hipStreamSynchronize(s));
+#undef HB_REV_TRY
+    return hipSuccess;
+}
+
 // nodes with long lists and the tasks those are cut into (hub h: tasks first[h] ..)
 struct BfsHubs {
     std::vector<uint32_t> node, first, tnode, tbeg, tend;
@@ -1196,35 +1250,26 @@ int exact_bfs(const uint32_t *off, const uint32_t *h_off, const uint32_t *nbr, u
     b.nbr = nbr;
     b.n = n;
     b.npad = (n + kBfsChunk - 1) / kBfsChunk * kBfsChunk;
-    // tails of the arcs to each node: the lists themselves, or the reversed arcs
-    Scoped rev, tmp;
+    // tails of the arcs to each node: the lists themselves, or the reversed arcs; directed graphs
+    // with few sources, and those whose reversed arcs find no memory, only push
+    Scoped rev;
     std::vector<uint32_t> h_ioff;
-    if (symmetric || arcs == 0) {
-        b.ioff = off;
-        b.inbr = nbr;
-    } else {
-        // a stable sort by head (4M arcs: 0.3 ms; counting and placing them with atomics took 2)
-        HBX_TRY(device_alloc(&rev.p, ((size_t)n + 1 + arcs) * 4));
-        uint32_t *ioff = (uint32_t *)rev.p, *inbr = ioff + n + 1;
-        const unsigned bits = std::max(1u, 32u - (unsigned)__builtin_clz(std::max(n - 1, 1u)));
-        size_t bytes = 0;
-        HBX_TRY(rocprim::radix_sort_pairs(nullptr, bytes, nbr, inbr, inbr, inbr, (size_t)arcs, 0, bits, s));
-        const size_t words = (bytes + 255) / 4 / 64 * 64;
-        HBX_TRY(device_alloc(&tmp.p, (words + 2 * (size_t)arcs) * 4));
-        uint32_t *tail = (uint32_t *)tmp.p + words, *head = tail + arcs;
-        k_bfs_tails<<<(unsigned)std::min<uint64_t>(((uint64_t)n + 3) / 4, 16384), kBfsBlock, 0, s>>>(off, n, tail);
-        HBX_TRY(rocprim::radix_sort_pairs(tmp.p, bytes, nbr, head, tail, inbr, (size_t)arcs, 0, bits, s));
-        k_bfs_offsets<<<(unsigned)std::min<uint64_t>(((uint64_t)arcs + kBfsBlock - 1) / kBfsBlock, 16384), kBfsBlock, 0,
-                        s>>>(head, arcs, n, ioff);
-        HBX_TRY(hipGetLastError());
-        h_ioff.resize((size_t)n + 1);
-        HBX_TRY(hipMemcpyAsync(h_ioff.data(), ioff, ((size_t)n + 1) * 4, hipMemcpyDeviceToHost, s));
-        HBX_TRY(hipStreamSynchronize(s));
-        tmp.release();
-        b.ioff = ioff;
-        b.inbr = inbr;
+    b.ioff = off;
+    b.inbr = nbr;
+    const bool directed = !symmetric && arcs != 0;
+    bool push_only = directed && s_end - s_begin <= kBfsFew;
+    if (directed && !push_only) {
+        const hipError_t e = bfs_reverse(off, nbr, n, arcs, rev, h_ioff, s);
+        if (e == hipSuccess) {
+            b.ioff = (const uint32_t *)rev.p;
+            b.inbr = b.ioff + n + 1;
+        } else if (e == hipErrorOutOfMemory) {
+            push_only = true;
+        } else {
+            HBX_TRY(e);
+        }
     }
-    // hubs and their tasks
+    // hubs and their tasks, of the lists that pulls read or, where there are none, those that pushes do
     Scoped hub;
     {
         const BfsHubs h(h_ioff.empty() ? h_off : h_ioff.data(), n);
@@ -1242,8 +1287,8 @@ int exact_bfs(const uint32_t *off, const uint32_t *h_off, const uint32_t *nbr, u
             b.task_end = b.task_beg + b.tasks;
         }
     }
-    // the tasks are those of the lists that a push reads too
-    const bool may_push = symmetric && arcs >= kBfsPushArcs;
+    // both read the same lists, which the tasks are of
+    const bool may_push = push_only || (symmetric && arcs >= kBfsPushArcs);
     b.push_arcs = arcs / kBfsPush;
     BfsMode mode = inv_sum ? BfsMode::kKeep : BfsMode::kSums;
     Scoped inv;
@@ -1264,13 +1309,13 @@ int exact_bfs(const uint32_t *off, const uint32_t *h_off, const uint32_t *nbr, u
             const uint64_t words = (s_end - s0 + 63) / 64;
             auto bytes = [&](uint32_t w, uint32_t k) { return (uint64_t)bfs_plan(n, b.tasks, w, k, mode).bytes; };
             uint32_t wide = 2;
-            while (wide < 32 && wide < words) wide *= 2;
+            while (wide < 32 && wide < words && !push_only) wide *= 2;
             uint32_t sw = wide;
-            uint64_t budget = kBfsHold;
+            uint64_t budget = std::min(kBfsHold, bfs_limit());
             while (sw > 8 && bytes(sw, 1) > budget) sw /= 2;
             if (bytes(sw, 1) > budget) {
                 sw = wide;
-                budget = kBfsBudget;
+                budget = std::min(kBfsBudget, bfs_limit());
                 while (sw > 2 && bytes(sw, 1) > budget) sw /= 2;
             }
             uint32_t slices = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((words + sw - 1) / sw, budget / bytes(sw, 1)));
@@ -1324,7 +1369,7 @@ int exact_bfs(const uint32_t *off, const uint32_t *h_off, const uint32_t *nbr, u
             // Past the eighth level, where a frontier seldom grows at a stroke, the levels up to the
             // next look push without being asked if all slices were to push at this one
             BfsDir dir = BfsDir::kPull;
-            if (may_push && r.plan.sw == 2) dir = at >= 8 && each ? BfsDir::kPush : BfsDir::kEither;
+            if (may_push && r.plan.sw == 2) dir = push_only || (at >= 8 && each) ? BfsDir::kPush : BfsDir::kEither;
             if (dir == BfsDir::kPush) to = std::min(to, at + 16);
             hipError_t e = hipErrorInvalidValue;
             switch (r.plan.sw) {
