@@ -885,15 +885,24 @@ __global__ __launch_bounds__(kBfsBlock) void k_bfs_tails(const uint32_t *__restr
     }
 }
 
-// ioff from the ascending heads: arc e writes the offsets of the nodes after its predecessor's
-// head up to its own, the last arc those of the nodes past it too
-__global__ __launch_bounds__(kBfsBlock) void k_bfs_offsets(const uint32_t *__restrict__ head, uint64_t arcs,
-                                                           uint32_t n, uint32_t *ioff)
+// ioff from the ascending heads: for each of the n + 1 offsets the first arc whose head is not
+// below it, by a binary search.  (Filled from the arcs instead, a long run of nodes without an
+// arc to them is one thread's: a million of them took 32 ms.)
+__global__ __launch_bounds__(kBfsBlock) void k_bfs_offsets(const uint32_t *__restrict__ head, uint32_t arcs, uint32_t n,
+                                                           uint32_t *ioff)
 {
-    for (uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; e < arcs; e += (uint64_t)gridDim.x * blockDim.x) {
-        for (uint64_t v = e ? (uint64_t)head[e - 1] + 1 : 0; v <= head[e]; ++v) ioff[v] = (uint32_t)e;
-        if (e + 1 == arcs)
-            for (uint64_t v = (uint64_t)head[e] + 1; v <= n; ++v) ioff[v] = (uint32_t)arcs;
+    for (uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; v <= n; v += (uint64_t)gridDim.x * blockDim.x) {
+        uint32_t lo = 0, len = arcs;
+        while (len) {
+            const uint32_t half = len / 2;
+            if (head[(size_t)lo + half] < v) {
+                lo += half + 1;
+                len -= half + 1;
+            } else {
+                len = half;
+            }
+        }
+        ioff[v] = lo;
     }
 }
 
@@ -1171,8 +1180,7 @@ hipError_t bfs_reverse(const uint32_t *off, const uint32_t *nbr, uint32_t n, uin
     uint32_t *tail = (uint32_t *)tmp.p + words, *head = tail + arcs;
     k_bfs_tails<<<(unsigned)std::min<uint64_t>(((uint64_t)n + 3) / 4, 16384), kBfsBlock, 0, s>>>(off, n, tail);
     HB_REV_TRY(rocprim::radix_sort_pairs(tmp.p, bytes, nbr, head, tail, inbr, (size_t)arcs, 0, bits, s));
-    k_bfs_offsets<<<(unsigned)std::min<uint64_t>(((uint64_t)arcs + kBfsBlock - 1) / kBfsBlock, 16384), kBfsBlock, 0,
-                    s>>>(head, arcs, n, ioff);
+    k_bfs_offsets<<<(unsigned)std::min<uint64_t>((uint64_t)n / kBfsBlock + 1, 16384), kBfsBlock, 0, s>>>(head, arcs, n, ioff);
     HB_REV_TRY(hipGetLastError());
     h_ioff.resize((size_t)n + 1);
     HB_REV_TRY(hipMemcpyAsync(h_ioff.data(), ioff, ((size_t)n + 1) * 4, hipMemcpyDeviceToHost, s));

@@ -79,3 +79,25 @@ def test_large_directed_graph_is_not_reversed_for_one_source(hb):  # noqa: F811
     alone, _ = best(path + 1, path)
     say("beside 16 M arcs", one, "alone", alone)
     assert one < 3 * alone
+
+
+def test_long_runs_of_nodes_without_arcs_to_them(hb, oracle):  # noqa: F811
+    """129 sources of a directed graph of a million nodes, few of which are heads: the offsets of
+    the reversed arcs do not wait for one thread to cross the gaps."""
+    from sparkx_amd.exact import exact_bfs
+    n = 1 << 20
+    s = np.arange(300)
+    g = _directed(hb, n, s, np.where(s < 150, 0, n - 300 + s), "gaps")
+    say("gaps", g.size(), g.width())
+    _check_sources(hb, oracle, g, 0, 129, "gaps")
+    spread = _directed(hb, n, s, s * 3400 + 7, "spread")
+    times = {}
+    for x in (spread, g):
+        runs = []
+        for _ in range(4):
+            t = time.perf_counter()
+            exact_bfs(x, (0, 129), inv_sum=False)
+            runs.append(time.perf_counter() - t)
+        times[x.name] = min(runs)
+    say(times)
+    assert times["gaps"] < 3 * times["spread"]
