@@ -1022,6 +1022,7 @@ enum class BfsMode { kSums, kKeep, kLong };
 // the group's one allocation, cut up
 struct BfsPlan {
     uint32_t sw = 0, slices = 0;
+    uint32_t words = 0;  // of a row that hold sources: sw, or 1 of 2 where the distances of both do not fit
     size_t rows_stride = 0, flag_stride = 0, count_stride = 0, any_stride = 0;  // per level
     uint32_t counts = 0;  // count buffers; rows and flags have two, by level parity
     size_t bytes = 0;
@@ -1029,10 +1030,11 @@ struct BfsPlan {
     bool keep = false;
 };
 
-BfsPlan bfs_plan(uint32_t n, uint32_t tasks, uint32_t sw, uint32_t slices, BfsMode mode)
+BfsPlan bfs_plan(uint32_t n, uint32_t tasks, uint32_t sw, uint32_t words, uint32_t slices, BfsMode mode)
 {
     BfsPlan p;
     p.sw = sw;
+    p.words = words;
     p.slices = slices;
     p.keep = mode == BfsMode::kKeep;
     p.counts = p.keep ? kBfsKeep : 1;
@@ -1053,7 +1055,7 @@ BfsPlan bfs_plan(uint32_t n, uint32_t tasks, uint32_t sw, uint32_t slices, BfsMo
     p.o_count = take(p.count_stride * p.counts);
     p.o_any = take(p.any_stride * p.counts);
     p.o_part = take((size_t)slices * tasks * sw * 8);
-    p.o_dist = take(mode == BfsMode::kLong ? p.rows_stride * 128 : 0);
+    p.o_dist = take(mode == BfsMode::kLong ? (size_t)slices * n * words * 128 : 0);
     // per source: reach, total, sum, found; per word: live, source count; per slice: front, done,
     // levels, push
     p.o_src = take((size_t)slices * (sw * (64 * 28 + 12) + 20));
@@ -1315,7 +1317,7 @@ int exact_bfs(const uint32_t *off, const uint32_t *h_off, const uint32_t *nbr, u
             // the widest rows and then the most slices that fit into memory that is kept, with
             // rows of at least 64 bytes (half a cache line), else into the budget
             const uint64_t words = (s_end - s0 + 63) / 64;
-            auto bytes = [&](uint32_t w, uint32_t k) { return (uint64_t)bfs_plan(n, b.tasks, w, k, mode).bytes; };
+            auto bytes = [&](uint32_t w, uint32_t k) { return (uint64_t)bfs_plan(n, b.tasks, w, w, k, mode).bytes; };
             uint32_t wide = 2;
             while (wide < 32 && wide < words && !push_only) wide *= 2;
             uint32_t sw = wide;
@@ -1328,26 +1330,28 @@ int exact_bfs(const uint32_t *off, const uint32_t *h_off, const uint32_t *nbr, u
             }
             uint32_t slices = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((words + sw - 1) / sw, budget / bytes(sw, 1)));
             while (slices > 1 && bytes(sw, slices) > budget) --slices;
-            for (;;) {
-                const BfsPlan p = bfs_plan(n, b.tasks, sw, slices, mode);
+            for (uint32_t row = sw;;) {
+                const BfsPlan p = bfs_plan(n, b.tasks, sw, row, slices, mode);
                 const hipError_t e = mem.take(p.bytes);
                 if (e == hipSuccess) {
                     g.place((char *)mem.p, p);
                     break;
                 }
-                if (e != hipErrorOutOfMemory || (sw == 2 && slices == 1)) HBX_TRY(e);
+                if (e != hipErrorOutOfMemory) HBX_TRY(e);
                 if (slices > 1) slices /= 2;
-                else sw /= 2;
+                else if (sw > 2) row = sw /= 2;
+                else if (mode == BfsMode::kLong && row == 2) row = 1;
+                else HBX_TRY(e);
             }
         }
-        const uint32_t per_slice = 64 * g.plan.sw;
+        const uint32_t per_slice = 64 * g.plan.words;
         // the last group may need fewer slices; the buffers keep their strides
         const uint32_t slices = (uint32_t)std::min<uint64_t>(g.plan.slices, (s_end - s0 + per_slice - 1) / per_slice);
         BfsGroup r = g;
         r.plan.slices = slices;
         r.b.src0 = (uint32_t)s0;
-        r.b.src_end = (uint32_t)s_end;
         const uint64_t group_end = std::min<uint64_t>(s_end, s0 + (uint64_t)slices * per_slice);
+        r.b.src_end = (uint32_t)group_end;
         uint64_t source_arcs = 0;
         for (uint32_t i = 0; i < slices; ++i) {
             const uint64_t a = s0 + (uint64_t)i * per_slice, e = std::min<uint64_t>(a + per_slice, s_end);
@@ -1362,7 +1366,7 @@ int exact_bfs(const uint32_t *off, const uint32_t *h_off, const uint32_t *nbr, u
             k_bfs_zero<uint4><<<zgrid, kBfsBlock, 0, s>>>((uint4 *)r.level(2).rows, row_words / 2);
             k_bfs_zero<uint4><<<zgrid, kBfsBlock, 0, s>>>((uint4 *)r.level(2).flag, (uint64_t)slices * r.b.npad / 16);
         }
-        if (mode == BfsMode::kLong) k_bfs_zero<uint4><<<zgrid, kBfsBlock, 0, s>>>((uint4 *)r.dist, row_words * 8);
+        if (mode == BfsMode::kLong) k_bfs_zero<uint4><<<zgrid, kBfsBlock, 0, s>>>((uint4 *)r.dist, (uint64_t)slices * n * g.plan.words * 8);
         k_bfs_begin<<<slices, kBfsBlock, 0, s>>>(r.b, r.plan.sw);
         // launches past a slice's last level return at once, so the host looks every 4, 8, ..
         // levels only
@@ -1406,7 +1410,8 @@ int exact_bfs(const uint32_t *off, const uint32_t *h_off, const uint32_t *nbr, u
         if (!all)
             return efail(HB_ERANGE, "hb_exact_bfs: eccentricity above 65535 (harmonic sums need u16 distances)");
         const size_t sources = (size_t)(group_end - s0);
-        std::vector<u64> h_sums(2 * (size_t)g.plan.slices * per_slice);
+        const size_t cols = (size_t)g.plan.slices * 64 * g.plan.sw;
+        std::vector<u64> h_sums(2 * cols);
         if (reach || total)
             HBX_TRY(hipMemcpyAsync(h_sums.data(), r.b.reach, h_sums.size() * 8, hipMemcpyDeviceToHost, s));
         if (inv_sum) {
@@ -1441,10 +1446,9 @@ int exact_bfs(const uint32_t *off, const uint32_t *h_off, const uint32_t *nbr, u
             HBX_TRY(hipMemcpyAsync(inv_sum + (s0 - s_begin), r.sums, sources * 8, hipMemcpyDeviceToHost, s));
         }
         HBX_TRY(hipStreamSynchronize(s));
-        const size_t half = (size_t)g.plan.slices * per_slice;
         for (size_t i = 0; i < sources; ++i) {
             if (reach) reach[s0 - s_begin + i] = h_sums[i];
-            if (total) total[s0 - s_begin + i] = h_sums[half + i];
+            if (total) total[s0 - s_begin + i] = h_sums[cols + i];
         }
         s0 = group_end;
     }

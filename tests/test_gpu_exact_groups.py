@@ -67,3 +67,13 @@ def test_too_little_memory_is_reported(hb, monkeypatch):  # noqa: F811
     with pytest.raises(hb.HyperBallError) as e:
         ExactClosenessCentrality(_graph(hb, "hubs"), True)
     assert e.value.code == -2  # HB_ENOMEM
+
+
+def test_distances_of_one_word_at_a_time(hb, oracle, monkeypatch):  # noqa: F811
+    """Memory for the distances of 64 sources of a long search but not of 128: 64 at a time."""
+    g = _graph(hb, "ladder")
+    n = g.size()
+    monkeypatch.setenv("SPARKX_HB_BFS_BYTES", str(n * 250))  # 51 bytes a node and 128 per 64 sources
+    for lo, hi in ((0, 1), (5, 69), (100, 400)):
+        say("one word", lo, hi, n)
+        _check_sources(hb, oracle, g, lo, hi, (lo, hi))
