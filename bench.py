@@ -75,7 +75,8 @@ def algorithmic_bytes(slot, arcs, nodes, items, p, gathered, first_nodes=0):
     (`gathered`: none in an iteration 1 that hashes ids, and only the neighbours that
     changed outside dense iterations).  Hub chunks add one partial sketch write per
     task.  Where iteration 1 hashes (every bin but one that k_union_rows runs) the node's
-    own block is not read either with p <= 10 (first_nodes)."""
+    own block is not read either with p <= 10 (first_nodes).  A node that takes the bound of
+    all sketches from a neighbour counts in full, though its own block is not read."""
     R = 1 << p
     b = nodes * (8 + 2 * R + 8 + 32) + arcs * 4 + gathered * R - first_nodes * R
     if slot == 3:
@@ -86,8 +87,8 @@ def algorithmic_bytes(slot, arcs, nodes, items, p, gathered, first_nodes=0):
 def kernel_name(slot, p, team, layout):
     """The kernel that does a slot's work in the dense iterations (k_union has a second
     instantiation, in the same slot, for the first one).  In the chain layout at
-    p = 5 and 6 the single bin of one-copy teams (an id range from node 0) is run by
-    k_union_rows after the first iteration, which k_union still runs."""
+    p = 5 and 6 k_union_rows runs them, the first included, for the single bin of one-copy
+    teams (an id range from node 0)."""
     if slot == 0 and layout == "chain" and p in (5, 6) and team == (1 << p) // 16:
         return f"hb::k_union_rows<{p}>"
     if slot < 3:

@@ -157,8 +157,8 @@ hipError_t device_alloc(T **p, size_t bytes)
     return e;
 }
 // exact BFS sums of sources [s_begin, s_end) over a staged CSR (hb_exact.hip), h_off
-// the host copy of its offsets; symmetric: the CSR holds v -> u for every u -> v (levels
-// may then pull)
+// the host copy of its offsets; symmetric: the CSR holds v -> u for every u -> v (else levels that
+// pull need it reversed)
 int exact_bfs(const uint32_t *off, const uint32_t *h_off, const uint32_t *nbr, uint32_t n, bool symmetric,
               uint64_t s_begin,
               uint64_t s_end, uint64_t *reach, uint64_t *total, double *inv_sum, hipStream_t s);

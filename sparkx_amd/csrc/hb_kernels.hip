@@ -19,8 +19,10 @@
 // a symmetric graph without those that reach no other node).  A node whose sketch is B is
 // done for good, and a node with such a neighbour becomes B whatever the others hold, so
 // neither gathers anything.  Graphs of small diameter reach B within a few iterations:
-// R-MAT-24 (p = 7) iterations 4, 5 and 6 take 2.5, 1.0 and 0.4 ms instead of 7.9, 7.9 and
-// 4.5, its run 24.2 instead of 40.1 ms; R-MAT-20 (p = 8) 3.3 instead of 4.7 ms.
+// R-MAT-24 (p = 7) iterations 4, 5 and 6 take 1.6, 0.9 and 0.4 ms instead of 7.9, 7.9 and 4.5; the
+// rule alone took its run from 40.1 to 24.2 ms and R-MAT-20's (p = 8) from 4.7 to 3.3.  One bound
+// has to fit all: a component of three nodes or more that holds a register's maximum keeps the
+// others below B, and then nothing is saved.
 #include <algorithm>
 #include <cmath>
 #include <type_traits>

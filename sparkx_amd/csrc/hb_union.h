@@ -18,7 +18,7 @@ namespace hb {
 enum class Gather {
     kAll,      // every neighbour's registers
     kChanged,  // those of the neighbours in HbView::gather_bits
-    kFirst,    // iteration 1 with P <= 10: sketches hold only their own insertion, so ids are hashed
+    kFirst,    // iteration 1: sketches hold only their own insertion, so ids are hashed
 };
 
 // one graph's state as seen by one iteration
@@ -27,7 +27,7 @@ struct HbView {
     const uint32_t *orig;      // hashed id of each arc's head (iteration 1)
     const uint32_t *node_id;   // hashed id of each node (null: its index)
     const uint8_t *in;
-    uint32_t *scr;          // LDS, 16 u32 per lane of the block (Gather::kFirst only)
+    uint32_t *scr;          // LDS; Gather::kFirst with P <= 10: 16 u32 per lane of the block
     uint8_t *out;
     float *est;
     double *dist, *inv;
